@@ -55,7 +55,8 @@ __global__ void k_hash(uint64_t n, const double* __restrict__ pos, const uint32_
   if (i == 0) {
     if (ws_par) ws_par[0] = 1u - ws_par[0];
     if (refine_count) refine_count[0] = 0u;
-    if (obs_count) obs_count[0] = obs_count[1] = obs_count[2] = 0u;  // [1]: pend_count, [2]: obs_count2
+    // [1]: pend_count, [2]: obs_count2, [3]: queue_next
+    if (obs_count) obs_count[0] = obs_count[1] = obs_count[2] = obs_count[3] = 0u;
   }
   if (i < n) {
     const SimGrid& g = grids[sim[i]];

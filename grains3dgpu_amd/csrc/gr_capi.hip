@@ -839,6 +839,7 @@ static int finalize(grains_ctx* ctx) {
   const size_t S = ctx->shapes.size();
   std::vector<ShapeNP<double>> np64(S);
   std::vector<ShapeNP<float>> np32(S);
+  std::vector<SqPow> sq64(S, SqPow{});
   std::vector<ShapeDyn> dyn(S);
   std::vector<double> rcpf(S), v64, cv64;
   for (size_t i = 0; i < S; ++i) {
@@ -846,6 +847,11 @@ static int finalize(grains_ctx* ctx) {
     int32_t voff = (int32_t)(v64.size() / 3);
     np64[i] = to_np<double>(h, quirks, voff);
     np32[i] = to_np<float>(h, quirks, voff);
+    if (h.s.kind == GRAINS_SUPERQUADRIC) {
+      const double a = h.core[0], b = h.core[1], c = h.core[2], n1 = h.core[3], n2 = h.core[4];
+      sq64[i] = {1.0 / (n2 - 1.0), 1.0 / (n1 - 1.0), (n1 - n2) / (n2 * (n1 - 1.0)), n1 / n2, 1.0 / n1,
+                 b / a,            c / a,            c / b};
+    }
     dyn[i].mass = h.mass;
     std::copy(h.inertia, h.inertia + 6, dyn[i].inertia);
     std::copy(h.inv, h.inv + 6, dyn[i].inv);
@@ -883,6 +889,7 @@ static int finalize(grains_ctx* ctx) {
   int rc;
   ShapeNP<double>* p64;
   ShapeNP<float>* p32;
+  SqPow* psq;
   ShapeDyn* pdyn;
   double *prc, *pv64, *pcv64, *potr;
   float *pv32, *pcv32;
@@ -891,7 +898,7 @@ static int finalize(grains_ctx* ctx) {
   SimGrid* pgr;
   uint32_t* posh;
   if ((rc = dalloc(ctx, &p64, S * sizeof(ShapeNP<double>), L)) || (rc = dalloc(ctx, &p32, S * sizeof(ShapeNP<float>), L)) ||
-      (rc = dalloc(ctx, &pdyn, S * sizeof(ShapeDyn), L)) || (rc = dalloc(ctx, &prc, S * sizeof(double), L)) ||
+      (rc = dalloc(ctx, &psq, S * sizeof(SqPow), L)) || (rc = dalloc(ctx, &pdyn, S * sizeof(ShapeDyn), L)) || (rc = dalloc(ctx, &prc, S * sizeof(double), L)) ||
       (rc = dalloc(ctx, &pv64, v64.size() * sizeof(double), L)) || (rc = dalloc(ctx, &pcv64, cv64.size() * sizeof(double), L)) ||
       (rc = dalloc(ctx, &pv32, v32.size() * sizeof(float), L)) || (rc = dalloc(ctx, &pcv32, cv32.size() * sizeof(float), L)) ||
       (rc = dalloc(ctx, &ph64, hk64.size() * sizeof(HookeP<double>), L)) ||
@@ -922,6 +929,7 @@ static int finalize(grains_ctx* ctx) {
     return rc;
   d.pend_count = d.obs_count + 1;
   d.obs_count2 = d.obs_count + 2;
+  d.queue_next = d.obs_count + 3;
   // warm-start records: two buffers of ecap = K x N, zeroed (no direction)
   d.warm = ((ctx->cfg.flags & GRAINS_WARM_START) && ctx->cfg.precision == GRAINS_FP32_MIXED &&
             !(ctx->cfg.flags & GRAINS_REF_QUIRKS))
@@ -940,6 +948,7 @@ static int finalize(grains_ctx* ctx) {
   }
   GR_HIP(hipMemcpy(p64, np64.data(), S * sizeof(ShapeNP<double>), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(p32, np32.data(), S * sizeof(ShapeNP<float>), hipMemcpyHostToDevice));
+  GR_HIP(hipMemcpy(psq, sq64.data(), S * sizeof(SqPow), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(pdyn, dyn.data(), S * sizeof(ShapeDyn), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(prc, rcpf.data(), S * sizeof(double), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(pv64, v64.data(), v64.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -955,6 +964,7 @@ static int finalize(grains_ctx* ctx) {
   }
   d.np64 = p64;
   d.np32 = p32;
+  d.sq64 = psq;
   d.dyn = pdyn;
   d.rc_pf = prc;
   d.verts64 = pv64;

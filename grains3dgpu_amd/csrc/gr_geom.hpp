@@ -80,11 +80,15 @@ GR_D V3<T> sq_support_pow(const T* d, V3<T> v) {
     T yt = T(1) / pow(T(1) + pow(alpha, n1), T(1) / n1);
     return {T(0), sy * b * yt, sz * alpha * c * yt};
   }
-  T alpha = pow(b / a * ay / ax, T(1) / (n2 - T(1)));
-  T temp = T(1) + pow(alpha, n2);
-  T gamma = pow(temp, (n1 - n2) / (n2 * (n1 - T(1))));
-  T beta = gamma * pow(c / a * az / ax, T(1) / (n1 - T(1)));
-  T xt = T(1) / pow(pow(temp, n1 / n2) + pow(beta, n1), T(1) / n1);
+  // (independent pow calls side by side: their instruction chains interleave,
+  // five in sequence instead of seven)
+  const T alpha = pow(b / a * ay / ax, T(1) / (n2 - T(1)));
+  const T zeta = pow(c / a * az / ax, T(1) / (n1 - T(1)));
+  const T temp = T(1) + pow(alpha, n2);
+  const T gamma = pow(temp, (n1 - n2) / (n2 * (n1 - T(1))));
+  const T tr = pow(temp, n1 / n2);
+  const T beta = gamma * zeta;
+  const T xt = T(1) / pow(tr + pow(beta, n1), T(1) / n1);
   return {sx * a * xt, sy * alpha * b * xt, sz * beta * c * xt};
 }
 
@@ -1028,17 +1032,6 @@ struct NoWarm {
   template <class V>
   GR_D bool fetch(V&) const { return false; }
 };
-// A given first direction (world frame); ok = false: none.
-template <class T>
-struct GivenDir {
-  V3<T> w;
-  bool ok;
-  GR_D bool fetch(V3<T>& o) const {
-    o = w;
-    return ok;
-  }
-};
-
 // PAIR (physics semantics): two lanes per pair, as gjk_sv<PAIR>.
 template <class T, bool SV, bool SCREEN = false, bool PAIR = false, class W = NoWarm>
 GR_D CInfo<T> closest_points(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<T>& a2w,

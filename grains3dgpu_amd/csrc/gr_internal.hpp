@@ -91,6 +91,13 @@ struct alignas(16) ShapeDyn {
   double pad;
 };
 
+// Exponents and axis ratios of a superquadric's crust core as the FP64
+// support chain divides them out (sq_support_pow), once per shape.
+struct alignas(64) SqPow {
+  double k1, k2, g, r, in1;  // 1/(n2-1), 1/(n1-1), (n1-n2)/(n2 (n1-1)), n1/n2, 1/n1
+  double ba, ca, cb;         // b/a, c/a, c/b
+};
+
 template <class T>
 struct alignas(16) PairRes {
   T f[3];
@@ -113,6 +120,7 @@ struct DevScene {
   // shapes
   const ShapeNP<double>* np64;
   const ShapeNP<float>* np32;
+  const SqPow* sq64;
   const ShapeDyn* dyn;
   const double* rc_pf;          // prefilter radius per shape
   const double* verts64;        // full polyhedron vertices
@@ -143,6 +151,7 @@ struct DevScene {
   void* pair_res;               // PairRes<T>[ecap]
   uint32_t* refine_list;        // entries to re-run in FP64 (FP32-mixed)
   uint32_t* refine_count;
+  uint32_t* queue_next;         // FP64 searches: entries handed out past the dealt ones (reset by k_hash)
   uint32_t* defer_list;         // entries the screening pass left undecided: one
                                 // segment of defer_cap words per block
   uint32_t* defer_count;        // per block of the screen (narrow_blocks)

@@ -83,22 +83,55 @@ struct WarmLookup {
   }
 };
 
+// Hooke force and torque on particle i of the contact ci with j; the poses'
+// origins in the frame of ci, xi in the world.
+template <class T, class R>
+__device__ __forceinline__ void contact_force(const DevScene& d, const SimGrid& g, uint32_t i, uint32_t j,
+                                              int32_t matA, int32_t matB, T massA, T massB, V3<double> xi, V3<T> oA,
+                                              V3<T> oB, const CInfo<T>& ci, PairRes<R>& out) {
+  const uint64_t n = d.n;
+  const HookeP<T> h = hk_table<T>(d)[g.table + material_hash((uint32_t)matA, (uint32_t)matB)];
+  const V3<T> vi = cvt<T>(load3(d.vel, n, i)), wi = cvt<T>(load3(d.omega, n, i));
+  const V3<T> vj = cvt<T>(load3(d.vel, n, j)), wj = cvt<T>(load3(d.omega, n, j));
+  V3<T> li, lj;
+  if (d.flags & GRAINS_REF_QUIRKS) {
+    // reference lever: the world contact point (Kinematics.cpp:86-91)
+    V3<T> cpw;
+    if constexpr (sizeof(T) == 8)
+      cpw = ci.cp;
+    else
+      cpw = cvt<float>(xi + cvt<double>(ci.cp));
+    li = cpw;
+    lj = cpw;
+  } else {
+    li = ci.cp - oA;
+    lj = ci.cp - oB;
+  }
+  const V3<T> relVel = (vi + cross(wi, li)) - (vj + cross(wj, lj));
+  const V3<T> relAng = wi - wj;
+  V3<T> F, M;
+  hooke<T>(h, ci, relVel, relAng, massA, massB, ci.cp - oA, F, M);
+  out.f[0] = R(F.x);
+  out.f[1] = R(F.y);
+  out.f[2] = R(F.z);
+  out.m[0] = R(M.x);
+  out.m[1] = R(M.y);
+  out.m[2] = R(M.z);
+}
+
 // Narrow phase + Hooke force of entry (si, sj) -- sorted positions -- from
 // si's side (ComponentManagerCPU.cpp:384-419).  Poses come from the sorted
 // records; velocities, needed only for contacts, from the planes through the
 // particle ids.  Returns the pair flag.
 // e: the entry (its slot in si's candidate list keys the warm-start record);
 // ~0u for callers without one (the FP64 re-run).
-// start (FP64 re-run, physics semantics; may be null): GJK's first
-// direction in the world frame, the FP32 search's last one.
 // dir (FP32, physics semantics; may be null): receives the direction the
 // search ended on in the world frame (left alone when GJK did not run).
-// PAIR (the FP64 re-run, physics semantics): lanes 2k and 2k + 1 evaluate
+// PAIR (physics semantics): lanes 2k and 2k + 1 evaluate
 // the same entry, sharing GJK's support pairs (gjk_sv<PAIR>).
 template <class T, class R, bool SV, bool SCREEN = false, bool WARM = false, bool PAIR = false>
 __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, uint32_t sj, PairRes<R>& out,
-                                               NpStats& st, uint32_t e = ~0u,
-                                               const V3<double>* start = nullptr, V3<T>* dir = nullptr) {
+                                               NpStats& st, uint32_t e = ~0u, V3<T>* dir = nullptr) {
   const uint64_t n = d.n;
   const PoseRec pi = d.pk[si];
   const PoseRec pj = d.pk[sj];
@@ -131,9 +164,6 @@ __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, u
       ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, NoWarm(),
                                                dir);
     }
-  } else if constexpr (sizeof(T) == 8 && SV) {
-    const GivenDir<double> given = {start ? *start : V3<double>{0.0, 0.0, 0.0}, start != nullptr};
-    ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, given);
   } else {
     ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, NoWarm(), dir);
   }
@@ -141,34 +171,8 @@ __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, u
   if constexpr (SCREEN) return flag;  // decided pairs have no contact
   if (ci.overlap < T(0)) {
     flag |= kFlagContact;
-    const uint32_t i = d.sidx[si], j = d.sidx[sj];
-    const HookeP<T> h = hk_table<T>(d)[g.table + material_hash((uint32_t)A.material, (uint32_t)B.material)];
-    const V3<T> vi = cvt<T>(load3(d.vel, n, i)), wi = cvt<T>(load3(d.omega, n, i));
-    const V3<T> vj = cvt<T>(load3(d.vel, n, j)), wj = cvt<T>(load3(d.omega, n, j));
-    V3<T> li, lj;
-    if (d.flags & GRAINS_REF_QUIRKS) {
-      // reference lever: the world contact point (Kinematics.cpp:86-91)
-      V3<T> cpw;
-      if constexpr (sizeof(T) == 8)
-        cpw = ci.cp;
-      else
-        cpw = cvt<float>(xi + cvt<double>(ci.cp));
-      li = cpw;
-      lj = cpw;
-    } else {
-      li = ci.cp - a2w.o;
-      lj = ci.cp - b2w.o;
-    }
-    const V3<T> relVel = (vi + cross(wi, li)) - (vj + cross(wj, lj));
-    const V3<T> relAng = wi - wj;
-    V3<T> F, M;
-    hooke<T>(h, ci, relVel, relAng, A.mass, B.mass, ci.cp - a2w.o, F, M);
-    out.f[0] = R(F.x);
-    out.f[1] = R(F.y);
-    out.f[2] = R(F.z);
-    out.m[0] = R(M.x);
-    out.m[1] = R(M.y);
-    out.m[2] = R(M.z);
+    contact_force<T, R>(d, g, d.sidx[si], d.sidx[sj], A.material, B.material, A.mass, B.mass, xi, a2w.o, b2w.o, ci,
+                        out);
   }
   return flag;
 }
@@ -219,7 +223,7 @@ __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
     NpStats st = {0u, 0};
     PairRes<T> r;
     V3<T> dir = {T(0), T(0), T(0)};
-    uint32_t flag = pair_force<T, T, SV, screen, WARM, PAIR>(d, d.pair_i[e], d.pair_j[e], r, st, e, nullptr,
+    uint32_t flag = pair_force<T, T, SV, screen, WARM, PAIR>(d, d.pair_i[e], d.pair_j[e], r, st, e,
                                                               sizeof(T) == 4 && SV ? &dir : nullptr);
     if constexpr (screen) {
       block_append(seg, &seg_n, st.deferred() != 0, e);
@@ -275,11 +279,6 @@ __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
   count_add(d.counters, kCntNear, c_near);
   count_max(d.counters, kCntMaxIters, c_maxit);
 }
-
-// FP64 re-run of the entries queued by k_narrow<float>; results stored in
-// FP32, or in FP64 with GRAINS_FP64_CONTACTS (d.res64).
-template <bool SV, bool PAIR>
-__global__ void __launch_bounds__(kBlock) k_refine64(DevScene d);
 
 // Particle x obstacle of any other kind than Rectangle: closestPointsRigidBodies
 // (bounding spheres, OBB, GJK) against the obstacle at rest, with its zero

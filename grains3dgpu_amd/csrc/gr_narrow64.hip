@@ -4,68 +4,46 @@
 // code (and the oracle).
 #include <algorithm>
 
-#include "gr_narrow.hpp"
+#include "gr_search.hpp"
 
 namespace gr {
 
-// The FP32-mixed path's FP64 re-runs.  Under the physics semantics each
-// search starts from the direction the entry's FP32 search of this step
-// ended on (left in the entry's result slot by k_narrow): near the optimum
-// already, so the FP64 search needs a few iterations instead of a cold
-// search's tens, and it meets the same FP64 gap test.  A zero direction (no
-// FP32 GJK ran) starts cold.  PAIR (physics semantics): the re-runs are few
-// and the step waits for the longest, so two lanes take each entry and share
-// its support evaluations (pair_force<PAIR>), halving that chain; the PAIR
-// launch runs when the grid holds every entry twice over, the other when it
-// does not (each returns at once in the other's case).
-template <bool SV, bool PAIR>
-__global__ void __launch_bounds__(kBlock) k_refine64(DevScene d) {
-  constexpr uint32_t L = PAIR ? 2u : 1u;  // lanes per entry
+// The FP32-mixed path's FP64 re-runs under the reference semantics, one lane
+// per entry from scratch (physics semantics: k_search64).
+__global__ void __launch_bounds__(kBlock) k_refine64_ref(DevScene d) {
   const uint32_t cnt = *d.refine_count;
-  const bool paired = SV && (uint64_t)cnt * 2 <= (uint64_t)gridDim.x * blockDim.x;
-  if (paired != PAIR) return;
-  PairRes<float>* res = (PairRes<float>*)d.pair_res;
-  PairRes<double>* res64 = (PairRes<double>*)d.pair_res;  // d.res64: results kept in FP64
-  const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x / L;
-  const bool lead = gid % L == 0;  // the lane that stores the entry's results
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   uint32_t c_it = 0, c_maxit = 0;
-  for (uint64_t k = gid / L; k < cnt; k += stride) {
+  for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < cnt; k += stride) {
     const uint32_t e = d.refine_list[k];
     NpStats st = {0u, 0};
-    V3<double> start = {0.0, 0.0, 0.0};
-    bool warm = false;
-    if (SV) {
+    PairRes<double> r;
+    const uint32_t flag = pair_force<double, double, false>(d, d.pair_i[e], d.pair_j[e], r, st);
+    if (flag & kFlagContact) {
       if (d.res64) {
-        const PairRes<double> q = res64[e];
-        start = {q.f[0], q.f[1], q.f[2]};
+        ((PairRes<double>*)d.pair_res)[e] = r;
       } else {
-        const PairRes<float> q = res[e];
-        start = {(double)q.f[0], (double)q.f[1], (double)q.f[2]};
+        PairRes<float> q;
+#pragma unroll
+        for (int k3 = 0; k3 < 3; ++k3) q.f[k3] = (float)r.f[k3], q.m[k3] = (float)r.m[k3];
+        ((PairRes<float>*)d.pair_res)[e] = q;
       }
-      const double nn = dot(start, start);
-      warm = nn > 0.0 && nn < INFINITY;
     }
-    uint32_t flag;
-    if (d.res64) {
-      PairRes<double> r;
-      flag = pair_force<double, double, SV, false, false, PAIR>(d, d.pair_i[e], d.pair_j[e], r, st, ~0u,
-                                                                 warm ? &start : nullptr);
-      if (lead && (flag & kFlagContact)) res64[e] = r;
-    } else {
-      PairRes<float> r;
-      flag = pair_force<double, float, SV, false, false, PAIR>(d, d.pair_i[e], d.pair_j[e], r, st, ~0u,
-                                                                warm ? &start : nullptr);
-      if (lead && (flag & kFlagContact)) res[e] = r;
-    }
-    if (lead) {
-      d.pair_flag[e] = flag | kFlagRefine;
-      c_it += st.iters;
-      c_maxit = c_maxit > (uint32_t)st.iters ? c_maxit : (uint32_t)st.iters;
-    }
+    d.pair_flag[e] = flag | kFlagRefine;
+    c_it += st.iters;
+    c_maxit = c_maxit > (uint32_t)st.iters ? c_maxit : (uint32_t)st.iters;
   }
   count_add(d.counters, kCntRefIters, c_it);
   count_max(d.counters, kCntRefMaxIters, c_maxit);
+}
+
+// One wave per block, two per SIMD (the registers' limit); the queue's length
+// decides on the device which form runs.
+template <int MODE>
+static void launch_search64(const DevScene& d, hipStream_t s) {
+  const dim3 grid((unsigned)cu_count() * 8);
+  hipLaunchKernelGGL((k_search64<MODE, 4>), grid, dim3(64), 0, s, d);
+  hipLaunchKernelGGL((k_search64<MODE, 1>), grid, dim3(64), 0, s, d);
 }
 
 void launch_narrow64(const DevScene& d, int pass, hipStream_t s) {
@@ -80,19 +58,14 @@ void launch_narrow64(const DevScene& d, int pass, hipStream_t s) {
       hipLaunchKernelGGL((k_narrow<double, false, 0>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
   } else if (two) {
     launch_defer_flatten(d, s);
-    // the queue's paired and single forms: one of them runs
-    hipLaunchKernelGGL((k_narrow<double, true, 1, false, true>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
-    hipLaunchKernelGGL((k_narrow<double, true, 1, false, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
+    launch_search64<0>(d, s);
   }
 }
 void launch_refine64(const DevScene& d, hipStream_t s) {
-  const dim3 grid(d.narrow_blocks / 4 + 1);
-  if (d.flags & GRAINS_REF_QUIRKS) {
-    hipLaunchKernelGGL((k_refine64<false, false>), grid, dim3(kBlock), 0, s, d);
-  } else {
-    hipLaunchKernelGGL((k_refine64<true, true>), grid, dim3(kBlock), 0, s, d);
-    hipLaunchKernelGGL((k_refine64<true, false>), grid, dim3(kBlock), 0, s, d);
-  }
+  if (d.flags & GRAINS_REF_QUIRKS)
+    hipLaunchKernelGGL(k_refine64_ref, dim3(d.narrow_blocks / 4 + 1), dim3(kBlock), 0, s, d);
+  else
+    launch_search64<1>(d, s);
 }
 void launch_integrate64(const DevScene& d, hipStream_t s, int part) { launch_integrate_t<double>(d, s, part); }
 void launch_gjk_batch64(const ShapeNP<double>* shapes, const double* verts, const uint32_t* sa,
