@@ -34,69 +34,60 @@ void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s) {
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, p, n, v);
 }
 
+// ---- the start of a run -------------------------------------------------------------
+__global__ void k_run_begin(DevScene d, uint32_t n, int sort) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < (uint32_t)kNumCounters * kCntSlots) d.counters[i] = 0ull;
+  if (i == 0) {
+    d.nl[kNlDone] = 0u;
+    d.nl[kNlTarget] = n;
+    if (sort) d.sort_state[0] = d.sort_state[2] = 0u;
+  }
+}
+void launch_run_begin(const DevScene& d, uint32_t n, bool sort, hipStream_t s) {
+  constexpr unsigned words = kNumCounters * kCntSlots;
+  hipLaunchKernelGGL(k_run_begin, dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d, n, sort ? 1 : 0);
+}
+
 // ---- cell hash --------------------------------------------------------------------
-// The first kernel of a step (no other kernel runs beside it on the
-// stream): ws_par (warm starts on), the step's warm-start buffer index, is
-// flipped here, and the step's queue counters (FP64 re-runs, particles near
-// obstacles; may be null) are cleared.
-// With a sorted order of the previous step in place (sort_state[0]), a
+// The first kernel of a list build (no other kernel runs beside it on the
+// stream): ws_par (warm starts on), the warm-start buffer of the lists, is
+// flipped here.  Keys are those of the search's cells (d.sgrids).
+// With a sorted order of the previous build in place (sort_state[0]), a
 // particle whose key differs from its key there (ks_prev at its previous
 // position rank[i]) has changed cell: it is counted in sort_state[2] and the
 // first kMaxMovers are listed in mv_list.
-__global__ void k_hash(uint64_t n, const double* __restrict__ pos, const uint32_t* __restrict__ sim,
-                       const SimGrid* __restrict__ grids, uint32_t* __restrict__ key,
-                       unsigned long long* __restrict__ counters, uint32_t* __restrict__ ws_par,
-                       uint32_t* __restrict__ refine_count, uint32_t* __restrict__ obs_count,
-                       const uint32_t* __restrict__ ks_prev, const uint32_t* __restrict__ rank,
-                       uint32_t* __restrict__ sort_state, uint32_t* __restrict__ mv_list) {
+__global__ void k_hash(DevScene d, const uint32_t* __restrict__ ks_prev) {
+  const uint64_t n = d.n;
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t ood = 0;
   bool mover = false;
   if (i == 0) {
-    if (ws_par) ws_par[0] = 1u - ws_par[0];
-    if (refine_count) refine_count[0] = 0u;
-    // [1]: pend_count, [2]: obs_count2, [3]: queue_next
-    if (obs_count) obs_count[0] = obs_count[1] = obs_count[2] = obs_count[3] = 0u;
+    if (d.warm) d.ws_par[0] = 1u - d.ws_par[0];
+    d.nl[kNlValid] = 0u;
+    d.nl[kNlOver] = 0u;
+    d.nl[kNlOutside] = 0u;
   }
   if (i < n) {
-    const SimGrid& g = grids[sim[i]];
-    const double p[3] = {pos[i], pos[n + i], pos[2 * n + i]};
+    const SimGrid& g = d.sgrids[d.sim[i]];
+    const double p[3] = {d.pos[i], d.pos[n + i], d.pos[2 * n + i]};
     uint32_t c[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      double f = floor((p[k] - g.lo[k]) / g.h);
-      // centres outside [lo, hi] are counted; the partial last cell beyond
-      // n3*h (the domain is rarely a multiple of h) folds into cell n3-1.
-      // A NaN centre (cell 0 here) is counted by the integration as a
-      // non-finite state, not as out of the domain.
-      if (p[k] < g.lo[k] || p[k] > g.hi[k]) ood = 1;
-      if (!(f >= 0.0))
-        c[k] = 0;
-      else if (f >= (double)g.n3[k])
-        c[k] = g.n3[k] - 1;
-      else
-        c[k] = (uint32_t)f;
-    }
-    const uint32_t k = g.base + (c[2] * g.n3[1] + c[1]) * g.n3[0] + c[0];
-    key[i] = k;
-    if (sort_state[0]) mover = k != ks_prev[rank[i]];
+    cell_of(g, p, c);
+    const uint32_t k = cell_key(g, c);
+    d.skey[i] = k;
+    if (d.sort_state[0]) mover = k != ks_prev[d.rank[i]];
   }
   const unsigned long long mb = __ballot(mover);
   if (mb) {
     const int leader = __ffsll(mb) - 1;
     uint32_t base = 0;
-    if ((int)__lane_id() == leader) base = atomicAdd(&sort_state[2], (uint32_t)__popcll(mb));
+    if ((int)__lane_id() == leader) base = atomicAdd(&d.sort_state[2], (uint32_t)__popcll(mb));
     base = __shfl(base, leader) + (uint32_t)__popcll(mb & ((1ull << __lane_id()) - 1ull));
-    if (mover && base < (uint32_t)kMaxMovers) mv_list[base] = (uint32_t)i;
+    if (mover && base < (uint32_t)kMaxMovers) d.mv_list[base] = (uint32_t)i;
   }
-  count_add(counters, kCntOod, ood);
 }
 
-
 void launch_hash(const DevScene& d, const uint32_t* keys_prev, hipStream_t s) {
-  hipLaunchKernelGGL(k_hash, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d.n,
-                     d.pos, d.sim, d.grids, d.key, d.counters, d.warm ? d.ws_par : nullptr, d.refine_count,
-                     d.obs_count, keys_prev, d.rank, d.sort_state, d.mv_list);
+  hipLaunchKernelGGL(k_hash, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d, keys_prev);
 }
 
 // ---- block-wide exclusive scan of one value per thread ---------------------------
@@ -326,7 +317,7 @@ __global__ void __launch_bounds__(1024) k_merge_movers(DevScene d, const uint32_
   for (uint32_t m = t; m < P; m += blockDim.x) {
     if (m < cnt) {
       const uint32_t i = d.mv_list[m];
-      km[m] = ((uint64_t)d.key[i] << 32) | i;
+      km[m] = ((uint64_t)d.skey[i] << 32) | i;
       om[m] = d.rank[i];
     } else {
       km[m] = ~0ull;
@@ -393,7 +384,7 @@ __global__ void __launch_bounds__(kBlock) k_merge_stayers(DevScene d, const uint
   const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= d.n) return;
   const uint32_t i = is[s], k = ks[s];
-  if (d.key[i] != k) return;
+  if (d.skey[i] != k) return;
   const uint32_t cnt = d.sort_state[2];
   const uint64_t me = ((uint64_t)k << 32) | i;
   uint32_t a = 0, b = cnt;
@@ -450,7 +441,7 @@ __global__ void __launch_bounds__(1024) k_sort_small(DevScene d, uint32_t* __res
   const uint32_t n = (uint32_t)d.n, t = threadIdx.x;
   uint32_t P = 2;
   while (P < n) P <<= 1;
-  for (uint32_t m = t; m < P; m += blockDim.x) km[m] = m < n ? ((uint64_t)d.key[m] << 32) | m : ~0ull;
+  for (uint32_t m = t; m < P; m += blockDim.x) km[m] = m < n ? ((uint64_t)d.skey[m] << 32) | m : ~0ull;
   __syncthreads();
   for (uint32_t size = 2; size <= P; size <<= 1)
     for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
@@ -481,7 +472,7 @@ void launch_sort(DevScene& d, int passes, int digit_bits, uint32_t** keys_sorted
     *idx_sorted = d.idxA;
     return;
   }
-  const uint32_t* kin = d.key;
+  const uint32_t* kin = d.skey;
   const uint32_t* iin = nullptr;
   switch (digit_bits) {
     case 8: run_sort_passes<8>(d, passes, kin, iin, s); break;
@@ -582,16 +573,16 @@ __global__ void k_cell_off(const uint32_t* __restrict__ ks, const float4* __rest
 }
 
 // One thread per sorted position s: the inverse permutation and the
-// particle's records in cell order -- the only gather of the state per step;
-// the candidate and narrow phases read bp / pk of neighbouring cells, which
-// are neighbouring lines.
+// particle's records in cell order -- the only gather of the state per list
+// build; the candidate and narrow phases read bp / pk of neighbouring cells,
+// which are neighbouring lines.
 __global__ void k_cells(DevScene d, const uint32_t* __restrict__ ks, const uint32_t* __restrict__ is) {
   const uint64_t n = d.n;
   const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
   const uint32_t i = is[s];
   d.rank[i] = (uint32_t)s;
-  if (s == 0) {  // an order and its inverse stand; the next step counts its movers afresh
+  if (s == 0) {  // an order and its inverse stand; the next build counts its movers afresh
     d.sort_state[0] = 1u;
     d.sort_state[2] = 0u;
   }
@@ -610,9 +601,22 @@ __global__ void k_cells(DevScene d, const uint32_t* __restrict__ ks, const uint3
   r.sim = d.sim[i];
   d.pk[s] = r;
   const double rc = d.rc_pf[shp];
-  d.bp[s] = make_double4(r.x, r.y, r.z, rc);
-  const SimGrid& g = d.grids[r.sim];
-  d.bp32[s] = make_float4((float)(r.x - g.lo[0]), (float)(r.y - g.lo[1]), (float)(r.z - g.lo[2]), (float)rc);
+  const SimGrid& g = d.sgrids[r.sim];
+  const double reach = rc + g.half_skin;
+  d.rcs[s] = rc;
+  d.bp[s] = make_double4(r.x, r.y, r.z, reach);
+  d.bp32[s] = make_float4((float)(r.x - g.lo[0]), (float)(r.y - g.lo[1]), (float)(r.z - g.lo[2]), (float)reach);
+  const double p[3] = {r.x, r.y, r.z};
+  uint32_t c[3];
+  const SimGrid& gr = d.grids[r.sim];
+  cell_of(gr, p, c);
+  d.rkey[s] = cell_key(gr, c);
+  // a centre outside a periodic side is folded into a border cell now and
+  // wrapped by the step: these lists hold for that step only
+  bool out = false;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) out |= ((g.periodic >> k) & 1) && (p[k] < g.lo[k] || p[k] >= g.hi[k]);
+  if (out) d.nl[kNlOutside] = 1u;
 }
 
 void launch_cells(const DevScene& d, const uint32_t* keys_s, const uint32_t* idx_s, hipStream_t s) {
@@ -626,6 +630,19 @@ void launch_cells(const DevScene& d, const uint32_t* keys_s, const uint32_t* idx
 }
 
 // ---- candidates -------------------------------------------------------------------
+// The search finds the pairs whose list spheres overlap: prefilter radii
+// grown by half the skin, so the lists hold every pair whose bounding spheres
+// can overlap until some particle has moved by half the skin.  The steps
+// apply the prefilter itself to them (narrow phase).  Without a skin the two
+// are the same.
+__device__ __forceinline__ void list_overflow(const DevScene& d, uint32_t over, uint32_t cnt) {
+  if (over) d.nl[kNlOver] = 1u;
+  if (!d.skin) {  // the lists are the step's candidates: an overflow is an error
+    count_add(d.counters, kCntOverflow, over);
+    count_max(d.counters, kCntMaxCand, over ? cnt : 0u);
+  }
+}
+
 // One thread per sorted position s (spatially coherent waves).  Writes the
 // sorted positions of its candidates, in the reference visit order, into
 // cand[k * N + s] (k-major, so the lanes of a wave write neighbouring words)
@@ -701,7 +718,7 @@ __global__ void __launch_bounds__(kBlock) k_candidates_direct(DevScene d, const 
     const double4 bi = d.bp[s];
     const float4 fi = d.bp32[s];
     // one sim: no need to read the pose record (a 64-byte line) for its id
-    const SimGrid g = d.grids[d.nsims > 1 ? d.pk[s].sim : 0u];
+    const SimGrid g = d.sgrids[d.nsims > 1 ? d.pk[s].sim : 0u];
     const V3<double> xi = {bi.x, bi.y, bi.z};
     const bool px = g.periodic & 1, py = g.periodic & 2, pz = g.periodic & 4;
     const float Lx = (float)g.L[0], Ly = (float)g.L[1], Lz = (float)g.L[2];
@@ -733,8 +750,7 @@ __global__ void __launch_bounds__(kBlock) k_candidates_direct(DevScene d, const 
     });
     d.cand_count[s] = cnt < d.K ? cnt : d.K;
   }
-  count_add(d.counters, kCntOverflow, over);
-  count_max(d.counters, kCntMaxCand, cnt);
+  list_overflow(d, over, cnt);
 }
 
 // Half shell.  The prefilter is symmetric -- the FP64 test of cand_scan
@@ -833,7 +849,7 @@ __device__ __forceinline__ void half_decide(const DevScene& d, HalfLds& L, uint3
   for (uint32_t k = lane; k < nw; k += 64) {
     const uint2 p = L.pair[wv][k];
     const double4 bi = d.bp[p.x];
-    const SimGrid& gp = d.grids[MULTI ? d.pk[p.x].sim : 0u];
+    const SimGrid& gp = d.sgrids[MULTI ? d.pk[p.x].sim : 0u];
     half_pair(d, p.x, p.y, V3<double>{bi.x, bi.y, bi.z}, bi.w, gp, over);
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // read before the list is refilled
@@ -858,7 +874,7 @@ __device__ __forceinline__ void half_group(const DevScene& d, HalfLds& L, uint64
     a1 = d.cell_off[c + 1];
   }
   const bool busy = a1 > a0;
-  const SimGrid& g = d.grids[MULTI && busy ? d.pk[a0].sim : 0u];
+  const SimGrid& g = d.sgrids[MULTI && busy ? d.pk[a0].sim : 0u];
   // lane k < 14 of the group: the k-th range (k = 0: the cell; 1: (0, 0, +1);
   // 2..4: (0, +1, -1..+1); 5..13: (+1, -1..+1, -1..+1)), [t0, t1), and the
   // image shift of a range reached across a periodic side
@@ -1016,7 +1032,7 @@ __global__ void __launch_bounds__(kBlock) k_candidates_half(DevScene d) {
   const uint64_t c = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kCellLanes;
   half_group<MULTI>(d, L, c, 0u, 0u, 1u, 1u, nw, over);
   if (nw) half_decide<MULTI>(d, L, nw, over);
-  count_add(d.counters, kCntOverflow, over);
+  list_overflow(d, over, 0u);
 }
 
 // the work list: groups per cell, their exclusive scan (half_goff, total at
@@ -1057,7 +1073,7 @@ __global__ void __launch_bounds__(kBlock) k_candidates_half_wl(DevScene d) {
     half_group<MULTI>(d, L, c, part / sp, part % sp, sc, sp, nw, over);
   }
   if (nw) half_decide<MULTI>(d, L, nw, over);
-  count_add(d.counters, kCntOverflow, over);
+  list_overflow(d, over, 0u);
 }
 
 // The block's neighbour records are staged in LDS first.  The block holds
@@ -1086,7 +1102,7 @@ __global__ void __launch_bounds__(kBlock) k_candidates_staged(DevScene d, const 
   const uint64_t s = b0 + threadIdx.x;
   if (threadIdx.x < 9) {
     const uint64_t last = b0 + blockDim.x - 1 < n ? b0 + blockDim.x - 1 : n - 1;
-    const SimGrid& g0 = d.grids[d.pk[b0].sim];
+    const SimGrid& g0 = d.sgrids[d.pk[b0].sim];
     const int64_t dz = (int64_t)(threadIdx.x / 3) - 1, dy = (int64_t)(threadIdx.x % 3) - 1;
     const int64_t o = (dz * (int64_t)g0.n3[1] + dy) * (int64_t)g0.n3[0];
     int64_t lo = (int64_t)ks[b0] + o - 1, hi = (int64_t)ks[last] + o + 1;
@@ -1138,7 +1154,7 @@ __global__ void __launch_bounds__(kBlock) k_candidates_staged(DevScene d, const 
   uint32_t cnt = 0, over = 0;
   if (s < n) {
     const double4 bi = d.bp[s];
-    const SimGrid g = d.grids[d.pk[s].sim];
+    const SimGrid g = d.sgrids[d.pk[s].sim];
     const V3<double> xi = {bi.x, bi.y, bi.z};
     const double ri = bi.w;
     const bool px = g.periodic & 1, py = g.periodic & 2, pz = g.periodic & 4;
@@ -1174,8 +1190,7 @@ __global__ void __launch_bounds__(kBlock) k_candidates_staged(DevScene d, const 
     });
     d.cand_count[s] = cnt < d.K ? cnt : d.K;
   }
-  count_add(d.counters, kCntOverflow, over);
-  count_max(d.counters, kCntMaxCand, cnt);
+  list_overflow(d, over, cnt);
 }
 
 void launch_candidates(const DevScene& d, const uint32_t* keys_s, hipStream_t s) {
@@ -1205,22 +1220,18 @@ void launch_candidates(const DevScene& d, const uint32_t* keys_s, hipStream_t s)
     hipLaunchKernelGGL(k_candidates_direct, grid, block, 0, s, d, keys_s);
 }
 
-// flat entry list in sorted positions: entry e = entry_off[s] + k holds
-// (s, cand[k * N + s]).  SORT (half-shell lists, filled in no fixed order):
-// each list is put in the reference visit order first -- the 27 neighbour
-// cells z outer, y, x inner, ascending sorted position within a cell
-// (LinkedCell.cpp:41-70, ComponentManagerCPU.cpp:364-421) -- by placing each
-// candidate at its rank (the lists are short).  Away from a periodic side
-// the neighbour cells' keys ascend in visit order, so the rank is that of
-// the sorted position; a cell on a periodic side ranks by (neighbour slot,
-// sorted position).  Counts beyond K (an overflow, reported by the step)
-// are clamped as the scan clamps them.
+// flat entry list in sorted positions: entry e = entry_off[s] + k.  Each list
+// is put in the reference visit order of the positions it was built from --
+// the 27 neighbour cells z outer, y, x inner, ascending id within a cell
+// (LinkedCell.cpp:41-70, ComponentManagerCPU.cpp:364-421; cells further away,
+// which a skin can reach, where their clamped offset puts them) -- by a
+// sorting network over (slot, id).  Counts beyond K (an overflow) are clamped
+// as the scan clamps them.
 // Batcher's odd-even merge sort of kSortNet keys, ascending; every index a
 // compile-time constant once the loops unroll, so the keys stay in registers.
-// Lists of up to 16 keys take the 16-key network, longer ones rank each
-// candidate; WIDE (dense beds, whose lists often pass 16) adds the 32-key
-// network, whose registers cost the kernel three of its seven waves per SIMD
-// where it is not needed.
+// Lists of up to 16 keys take the 16-key network, up to 32 the 32-key one
+// (32-bit keys, up to 2^27 particles: the slot above the id), longer ones
+// rank each candidate.
 constexpr int kSortNet = 16;
 template <int N, class K>
 __device__ __forceinline__ void sort_network(K (&key)[N]) {
@@ -1239,122 +1250,126 @@ __device__ __forceinline__ void sort_network(K (&key)[N]) {
           }
 }
 
-template <bool SORT, bool WIDE = false>
-__global__ void k_expand(DevScene d, const uint32_t* __restrict__ ks) {
+__global__ void k_expand(DevScene d) {
   const uint64_t n = d.n;
   const uint32_t* cand = d.cand;
   const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t c = 0, raw = 0;
+  if (s == 0) d.nl[kNlValid] = d.nl[kNlOver] && d.skin ? 0u : (d.nl[kNlOutside] || !d.skin ? 2u : 1u);
+  uint32_t raw = 0;
   if (s < n) {
     raw = d.cand_count[s];
-    c = raw < d.K ? raw : d.K;
+    const uint32_t c = raw < d.K ? raw : d.K;
     const uint32_t e0 = d.entry_off[s];
-    if constexpr (!SORT) {
-      // four candidates loaded together: one load latency per four entries
-      for (uint32_t k0 = 0; k0 < c; k0 += 4) {
-        uint32_t v[4];
+    const uint32_t id = d.sidx[s];
+    if (d.warm) d.ws_nb[(uint64_t)(*d.ws_par) * n + id] = make_uint2(e0, c);
+    const SimGrid& g = d.grids[d.nsims > 1 ? d.pk[s].sim : 0u];
+    const uint32_t nx = g.n3[0], ny = g.n3[1];
+    auto cell = [&](uint32_t key, int* o) {
+      const uint32_t l = key - g.base;
+      o[0] = (int)(l % nx);
+      o[1] = (int)((l / nx) % ny);
+      o[2] = (int)(l / (nx * ny));
+    };
+    int ci[3];
+    cell(d.rkey[s], ci);
+    auto order = [&](uint32_t t) -> uint64_t {
+      int cj[3], v[3];
+      cell(d.rkey[t], cj);
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) v[u] = k0 + u < c ? cand[(uint64_t)(k0 + u) * n + s] : 0u;
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u)
-          if (k0 + u < c) {
-            d.pair_i[e0 + k0 + u] = (uint32_t)s;
-            d.pair_j[e0 + k0 + u] = v[u];
-          }
+      for (int k = 0; k < 3; ++k) {
+        int x = cj[k] - ci[k];
+        const int m = (int)g.n3[k];
+        if ((g.periodic >> k) & 1) x = 2 * x > m ? x - m : (2 * x < -m ? x + m : x);
+        v[k] = x > 1 ? 1 : (x < -1 ? -1 : x);
       }
+      return ((uint64_t)(uint32_t)(((v[2] + 1) * 3 + v[1] + 1) * 3 + v[0] + 1) << 32) | d.sidx[t];
+    };
+    constexpr uint32_t kId27 = (1u << 27) - 1u;
+    auto net = [&](auto& key) {
+      using K = typename std::decay<decltype(key[0])>::type;
+      constexpr int N = (int)(sizeof(key) / sizeof(key[0]));
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        K v = ~(K)0;
+        if ((uint32_t)k < c) {
+          const uint64_t o = order(cand[(uint64_t)k * n + s]);
+          v = sizeof(K) == 4 ? (K)(((o >> 32) << 27) | (o & kId27)) : (K)o;
+        }
+        key[k] = v;
+      }
+      sort_network<N>(key);
+#pragma unroll
+      for (int k = 0; k < N; ++k)
+        if ((uint32_t)k < c) {
+          d.pair_i[e0 + k] = (uint32_t)s;
+          d.pair_j[e0 + k] = d.rank[sizeof(K) == 4 ? (uint32_t)key[k] & kId27 : (uint32_t)key[k]];
+        }
+    };
+    if (c <= kSortNet) {
+      uint64_t key[kSortNet];
+      net(key);
+    } else if (c <= 2 * kSortNet && n <= (1ull << 27)) {
+      uint32_t key[2 * kSortNet];
+      net(key);
     } else {
-      const SimGrid& g = d.grids[d.nsims > 1 ? d.pk[s].sim : 0u];
-      const int nx = (int)g.n3[0], ny = (int)g.n3[1], nz = (int)g.n3[2];
-      const uint32_t ls = ks[s] - g.base;
-      const int cx = (int)(ls % (uint32_t)nx), cy = (int)((ls / (uint32_t)nx) % (uint32_t)ny),
-                cz = (int)(ls / ((uint32_t)nx * (uint32_t)ny));
-      const bool wraps = ((g.periodic & 1) && (cx == 0 || cx == nx - 1)) ||
-                         ((g.periodic & 2) && (cy == 0 || cy == ny - 1)) ||
-                         ((g.periodic & 4) && (cz == 0 || cz == nz - 1));
-      // order key: the sorted position, after the neighbour slot on a periodic side
-      auto order = [&](uint32_t t) -> uint64_t {
-        if (!wraps) return t;
-        const uint32_t lt = ks[t] - g.base;
-        int dx = (int)(lt % (uint32_t)nx) - cx, dy = (int)((lt / (uint32_t)nx) % (uint32_t)ny) - cy,
-            dz = (int)(lt / ((uint32_t)nx * (uint32_t)ny)) - cz;
-        dx = dx > 1 ? -1 : (dx < -1 ? 1 : dx);  // across the periodic side
-        dy = dy > 1 ? -1 : (dy < -1 ? 1 : dy);
-        dz = dz > 1 ? -1 : (dz < -1 ? 1 : dz);
-        return ((uint64_t)(((dz + 1) * 3 + (dy + 1)) * 3 + (dx + 1)) << 32) | t;
-      };
-      // in registers: the list padded with keys that sort last, a sorting
-      // network with compile-time indices
-      // (32-bit keys, up to 2^27 particles: the neighbour slot above the
-      // 27-bit sorted position, so the 32-key network holds 32 registers)
-      constexpr uint32_t kPos27 = (1u << 27) - 1u;
-      auto net = [&](auto& key) {
-        using K = typename std::decay<decltype(key[0])>::type;
-        constexpr int N = (int)(sizeof(key) / sizeof(key[0]));
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-          K v = ~(K)0;
-          if ((uint32_t)k < c) {
-            const uint64_t o = order(cand[(uint64_t)k * n + s]);
-            v = sizeof(K) == 4 ? (K)(((o >> 32) << 27) | (o & kPos27)) : (K)o;
-          }
-          key[k] = v;
-        }
-        sort_network<N>(key);
-#pragma unroll
-        for (int k = 0; k < N; ++k)
-          if ((uint32_t)k < c) {
-            d.pair_i[e0 + k] = (uint32_t)s;
-            d.pair_j[e0 + k] = sizeof(K) == 4 ? (uint32_t)key[k] & kPos27 : (uint32_t)key[k];  // the sorted position
-          }
-      };
-      if (c <= kSortNet) {
-        uint64_t key[kSortNet];
-        net(key);
-      } else if (WIDE && c <= 2 * kSortNet && n <= (1ull << 27)) {
-        uint32_t key[2 * kSortNet];
-        net(key);
-      } else {
-        // a long list: each candidate at its rank
-        for (uint32_t k = 0; k < c; ++k) {
-          const uint32_t tk = cand[(uint64_t)k * n + s];
-          const uint64_t ok = order(tk);
-          uint32_t rank = 0;
-          for (uint32_t j = 0; j < c; ++j) rank += j != k && order(cand[(uint64_t)j * n + s]) < ok;
-          d.pair_i[e0 + rank] = (uint32_t)s;
-          d.pair_j[e0 + rank] = tk;
-        }
+      // a long list: each candidate at its rank
+      for (uint32_t k = 0; k < c; ++k) {
+        const uint32_t tk = cand[(uint64_t)k * n + s];
+        const uint64_t ok = order(tk);
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < c; ++j) rank += j != k && order(cand[(uint64_t)j * n + s]) < ok;
+        d.pair_i[e0 + rank] = (uint32_t)s;
+        d.pair_j[e0 + rank] = tk;
       }
     }
   }
-  count_add(d.counters, kCntCandidates, c);
-  if constexpr (SORT) count_max(d.counters, kCntMaxCand, raw);
+  if (!d.skin) count_max(d.counters, kCntMaxCand, raw > d.K ? raw : 0u);
 }
 
-// ---- the screening pass's queue ------------------------------------------------
-// Block b copies its segment of the screen's queue (defer_count[b] entries
-// at defer_list + b * defer_cap) to defer_flat[defer_off[b] ...], coalesced:
-// the complete pass then reads entry k directly instead of searching for
-// its segment.
-__global__ void __launch_bounds__(kBlock) k_defer_flatten(DevScene d) {
-  const uint32_t b = blockIdx.x;
-  const uint32_t cnt = d.defer_count[b], off = d.defer_off[b];
-  const uint32_t* seg = d.defer_list + (uint64_t)b * d.defer_cap;
-  for (uint32_t k = threadIdx.x; k < cnt; k += blockDim.x) d.defer_flat[off + k] = seg[k];
+// Warm starts: each new entry takes the record its pair had in the lists
+// before (the same slot first: a particle's list keeps its order while its
+// neighbours stay, then the others, four loads in flight), or none.
+__global__ void __launch_bounds__(kBlock) k_warm_carry(DevScene d) {
+  const uint64_t n = d.n, KN = (uint64_t)d.K * n;
+  const uint32_t E = d.entry_off[n];
+  const uint32_t cur = *d.ws_par;
+  const float4* old = d.ws + (uint64_t)(1u - cur) * KN;
+  float4* now = d.ws + (uint64_t)cur * KN;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E; e += stride) {
+    const uint32_t s = d.pair_i[e];
+    const uint32_t wj = d.sidx[d.pair_j[e]];
+    const uint2 nb = d.ws_nb[(uint64_t)(1u - cur) * n + d.sidx[s]];
+    const uint32_t wk = (uint32_t)e - d.entry_off[s];
+    const float4* pr = old + nb.x;
+    float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+    bool hit = false;
+    if (wk < nb.y) {
+      r = pr[wk];
+      hit = __float_as_uint(r.w) == wj;
+    }
+    for (uint32_t k0 = 0; !hit && k0 < nb.y; k0 += 4) {
+      float4 q[4];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) q[u] = k0 + u < nb.y ? pr[k0 + u] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        if (!hit && k0 + u < nb.y && __float_as_uint(q[u].w) == wj) {
+          r = q[u];
+          hit = true;
+        }
+    }
+    if (!hit) r = make_float4(0.f, 0.f, 0.f, 0.f);
+    r.w = __uint_as_float(wj);
+    now[e] = r;
+    d.pair_flag[e] = kFlagCand;  // a record that may have to be forgotten
+  }
 }
 
-void launch_defer_flatten(const DevScene& d, hipStream_t s) {
-  launch_scan(d.defer_count, d.defer_off, d.narrow_blocks, d.scan_blocks, s);
-  hipLaunchKernelGGL(k_defer_flatten, dim3(d.narrow_blocks), dim3(kBlock), 0, s, d);
-}
-
-void launch_expand(const DevScene& d, const uint32_t* keys_s, hipStream_t s) {
+void launch_expand(const DevScene& d, const uint32_t*, hipStream_t s) {
   const dim3 grid((unsigned)((d.n + d.block - 1) / d.block)), block(d.block);
-  if (d.cand_half && !d.cand_staged && d.half_wl)
-    hipLaunchKernelGGL((k_expand<true, true>), grid, block, 0, s, d, keys_s);
-  else if (d.cand_half && !d.cand_staged)
-    hipLaunchKernelGGL((k_expand<true, false>), grid, block, 0, s, d, keys_s);
-  else
-    hipLaunchKernelGGL(k_expand<false>, grid, block, 0, s, d, keys_s);
+  hipLaunchKernelGGL(k_expand, grid, block, 0, s, d);
+  if (d.warm) hipLaunchKernelGGL(k_warm_carry, dim3((unsigned)cu_count() * 8), dim3(kBlock), 0, s, d);
 }
 
 int cu_count() {

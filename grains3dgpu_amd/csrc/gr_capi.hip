@@ -367,14 +367,26 @@ struct grains_ctx {
   std::vector<void*> state_allocs; // particle state
   int passes = 1;      // LSD radix passes of the cell keys
   int digit_bits = 8;  // bits per pass
+  int ref_passes = 1;  // passes the reference's cell keys take (grains_stats_t.sort_passes)
   uint32_t *keys_s = nullptr, *idx_s = nullptr;
   hipGraph_t graph = nullptr;            // one step
   hipGraphExec_t graph_exec = nullptr;
   hipGraph_t graph_multi = nullptr;      // graph_steps steps
   hipGraphExec_t graph_multi_exec = nullptr;
   uint32_t graph_steps = 1;
+  hipGraph_t graph_build = nullptr;      // the neighbour lists' build
+  hipGraphExec_t graph_build_exec = nullptr;
   grains_stats_t stats;
-  std::vector<SimGrid> grids;
+  std::vector<SimGrid> grids;   // the reference's cells
+  std::vector<SimGrid> sgrids;  // the search's
+  // Neighbour lists.  They stand from one call to the next while nothing but
+  // the steps themselves moves the particles; lists_ok is cleared wherever
+  // the state or the layout is set.
+  bool lists_ok = false;
+  uint32_t since_build = 0;     // steps taken since they were built
+  uint32_t interval = 8;        // steps they are expected to hold, and whether a build has shown it
+  bool interval_known = false;
+  unsigned char* host_words = nullptr;  // pinned: the counters and the list words, read back together
   // profiling: events around the phases of each step
   bool profiling = false;
   bool capturing = false;
@@ -469,9 +481,16 @@ static void drop_graph(grains_ctx* ctx) {
   if (ctx->graph_multi) (void)hipGraphDestroy(ctx->graph_multi);
   ctx->graph_exec = nullptr;
   ctx->graph = nullptr;
+  if (ctx->graph_build_exec) (void)hipGraphExecDestroy(ctx->graph_build_exec);
+  if (ctx->graph_build) (void)hipGraphDestroy(ctx->graph_build);
   ctx->graph_multi_exec = nullptr;
   ctx->graph_multi = nullptr;
+  ctx->graph_build_exec = nullptr;
+  ctx->graph_build = nullptr;
 }
+
+constexpr size_t kCounterBytes = (size_t)kNumCounters * kCntSlots * 8;
+constexpr size_t kWordBytes = kCounterBytes + kNlWords * 4;
 
 extern "C" const char* grains_version(void) { return "grains_hip 0.1 gfx950"; }
 
@@ -561,7 +580,8 @@ extern "C" int grains_create(const grains_config_t* cfg, grains_ctx_t** out) {
       hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
       hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess) {
+      hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess ||
+      hipHostMalloc((void**)&ctx->host_words, kWordBytes, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     grains_destroy(ctx);
     return GRAINS_EDEVICE;
@@ -582,6 +602,7 @@ extern "C" void grains_destroy(grains_ctx_t* ctx) {
   adj_drop(ctx);
   free_list(ctx->allocs);
   free_list(ctx->state_allocs);
+  if (ctx->host_words) (void)hipHostFree(ctx->host_words);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
@@ -668,9 +689,11 @@ static int hist_reset(grains_ctx* ctx) {
   return GRAINS_OK;
 }
 
-// Warm-start records forgotten: the next step searches cold (a new state is
-// not the continuation of the recorded directions).
+// A new state: the neighbour lists no longer hold, and the warm-start records
+// are forgotten: the next step searches cold (it is not the continuation of
+// the recorded directions).
 static int warm_reset(grains_ctx* ctx) {
+  ctx->lists_ok = false;
   if (!ctx->d.ws_nb) return GRAINS_OK;
   launch_fill_u32((uint32_t*)ctx->d.ws_nb, 4 * ctx->n, 0u, ctx->stream);
   GR_HIP(hipGetLastError());
@@ -736,14 +759,21 @@ extern "C" int grains_set_particles(grains_ctx_t* ctx, const uint32_t* shape, co
 }
 
 // cell layout, obstacle ranges, shape tables and work buffers
-// Segment of the screening pass's queue per block: a block of the persistent
-// narrow launch visits at most ceil(ecap / (blocks * threads)) * threads
-// entries, so blocks * defer_cap <= ecap + blocks * threads, within the
-// allocation (ecap + kMaxNarrowPerCu blocks per CU * 256 threads).
+// One of the screening pass's queues: a block of the persistent narrow launch
+// visits at most ceil(ecap / (blocks * threads)) * threads entries, and every
+// kDeferQueues-th block fills the same queue.  For any launch shape the
+// queues together hold at most (blocks + kDeferQueues - 1) (ecap / blocks +
+// threads) words, which defer_words bounds (a launch has at least one block
+// per CU and at most kMaxNarrowPerCu).
 static void set_defer_cap(grains_ctx* ctx) {
   DevScene& d = ctx->d;
   const uint64_t per = (uint64_t)d.narrow_blocks * d.block;
-  d.defer_cap = (uint32_t)(((d.ecap + per - 1) / per) * d.block);
+  const uint64_t block_cap = ((d.ecap + per - 1) / per) * d.block;
+  d.defer_cap = (uint32_t)(block_cap * ((d.narrow_blocks + kDeferQueues - 1) / kDeferQueues));
+}
+static uint64_t defer_words(uint64_t ecap) {
+  const uint64_t cus = (uint64_t)cu_count();
+  return ecap + (kDeferQueues - 1) * (ecap / cus + 1) + (cus * kMaxNarrowPerCu + kDeferQueues) * 256;
 }
 
 static void adj_drop(grains_ctx* ctx) {
@@ -828,12 +858,64 @@ static int finalize(grains_ctx* ctx) {
     if (g.obs_end == g.obs_begin) g.obs_begin = (uint32_t)k;
     g.obs_end = (uint32_t)k + 1;
   }
-  d.ncells = (uint32_t)base;
+  // The search's cells: the reference's, or wider where the lists' reach --
+  // the largest two radii and the skin -- asks for it.  The skin is a tenth of
+  // the sim's mean radius: on the superquadric beds it grows the lists by a
+  // fifth, and grains at 0.2 m/s (dt = 1e-6) take about 60 steps to use it up.
+  // Measured (ms/step, skin 0.02 / 0.05 / 0.1 / 0.2 of the mean radius): bed of
+  // 10^6 at rest 0.355 / 0.364 / 0.380 / 0.400, 50,653 agitated grains 0.456 /
+  // 0.452 / 0.447 / 0.447, 100,003 polyhedra 0.290 / 0.279 / 0.270 / 0.273, 64
+  // beds (369,564) 0.358 / 0.356 / 0.354 / 0.367; lists built every step:
+  // 0.58, 0.52, 0.40, 0.58.
+  // A periodic axis that would hold fewer than three such cells leaves the
+  // whole context without a skin: the lists are then built every step, in
+  // cells at least two radii wide, or where even those do not fit, in the
+  // reference's.
+  std::vector<double> rmean(ns, 0.0);
+  std::vector<uint64_t> rnum(ns, 0);
+  for (uint64_t i = 0; i < ctx->n; ++i) {
+    const HostShape& h = ctx->shapes[ctx->pshape[i]];
+    rmean[ctx->psim[i]] += quirks ? h.rc : h.rc_exact;
+    ++rnum[ctx->psim[i]];
+  }
+  uint64_t sbase = 0;
+  for (int with = 1; with >= 0; --with) {
+    ctx->sgrids = ctx->grids;
+    d.skin = with;
+    sbase = 0;
+    for (uint32_t s = 0; s < ns; ++s) {
+      SimGrid& g = ctx->sgrids[s];
+      const double skin = with && rnum[s] ? 0.1 * rmean[s] / (double)rnum[s] : 0.0;
+      double h = std::max(g.h, (2.0 * lc[s] + skin) * (1.0 + 1e-9));
+      for (int k = 0; k < 3; ++k) {
+        if (!(skin > 1e-9 * g.L[k]) && rnum[s]) d.skin = 0;
+        if (((g.periodic >> k) & 1) && g.L[k] < 3.0 * h) {
+          d.skin = 0;
+          h = g.h;  // (without a skin: the reference's cells)
+        }
+      }
+      if (h != g.h)
+        for (int k = 0; k < 3; ++k) g.n3[k] = (uint32_t)std::max(1.0, g.L[k] / h);
+      g.h = h;
+      g.half_skin = 0.5 * skin;
+      g.move2 = 0.25 * skin * skin * (1.0 - 1e-6) * (1.0 - 1e-6);
+      g.base = (uint32_t)sbase;
+      sbase += (uint64_t)g.n3[0] * g.n3[1] * g.n3[2];
+      ctx->grids[s].move2 = g.move2;
+    }
+    if (d.skin == with) break;
+  }
+  d.ncells = (uint32_t)sbase;
   int bits = 1;
-  while (bits < 32 && (1ull << bits) < base) ++bits;
+  while (bits < 32 && (1ull << bits) < sbase) ++bits;
   // fewest LSD passes of digits up to kRadixMaxBits wide, digits at least 8
   // bits: an 18-bit key sorts in 2 passes of 9 bits instead of 3 of 8
   ctx->passes = (bits + kRadixMaxBits - 1) / kRadixMaxBits;
+  {
+    int ref = 1;
+    while (ref < 32 && (1ull << ref) < base) ++ref;
+    ctx->ref_passes = (ref + kRadixMaxBits - 1) / kRadixMaxBits;
+  }
   ctx->digit_bits = std::max(8, (bits + ctx->passes - 1) / ctx->passes);
   // shape tables
   const size_t S = ctx->shapes.size();
@@ -895,7 +977,7 @@ static int finalize(grains_ctx* ctx) {
   float *pv32, *pcv32;
   HookeP<double>* ph64;
   HookeP<float>* ph32;
-  SimGrid* pgr;
+  SimGrid *pgr, *psg;
   uint32_t* posh;
   if ((rc = dalloc(ctx, &p64, S * sizeof(ShapeNP<double>), L)) || (rc = dalloc(ctx, &p32, S * sizeof(ShapeNP<float>), L)) ||
       (rc = dalloc(ctx, &psq, S * sizeof(SqPow), L)) || (rc = dalloc(ctx, &pdyn, S * sizeof(ShapeDyn), L)) || (rc = dalloc(ctx, &prc, S * sizeof(double), L)) ||
@@ -903,7 +985,8 @@ static int finalize(grains_ctx* ctx) {
       (rc = dalloc(ctx, &pv32, v32.size() * sizeof(float), L)) || (rc = dalloc(ctx, &pcv32, cv32.size() * sizeof(float), L)) ||
       (rc = dalloc(ctx, &ph64, hk64.size() * sizeof(HookeP<double>), L)) ||
       (rc = dalloc(ctx, &ph32, hk32.size() * sizeof(HookeP<float>), L)) ||
-      (rc = dalloc(ctx, &pgr, ns * sizeof(SimGrid), L)) || (rc = dalloc(ctx, &posh, (osh.size() + 1) * sizeof(uint32_t), L)) ||
+      (rc = dalloc(ctx, &pgr, ns * sizeof(SimGrid), L)) || (rc = dalloc(ctx, &psg, ns * sizeof(SimGrid), L)) ||
+      (rc = dalloc(ctx, &d.skey, n * 4, L)) || (rc = dalloc(ctx, &d.rkey, n * 4, L)) || (rc = dalloc(ctx, &d.rcs, n * 8, L)) || (rc = dalloc(ctx, &posh, (osh.size() + 1) * sizeof(uint32_t), L)) ||
       (rc = dalloc(ctx, &potr, (otr.size() + 12) * sizeof(double), L)) ||
       (rc = dalloc(ctx, &d.key, n * 4, L)) || (rc = dalloc(ctx, &d.keyA, n * 4, L)) || (rc = dalloc(ctx, &d.idxA, n * 4, L)) ||
       (rc = dalloc(ctx, &d.keyB, n * 4, L)) || (rc = dalloc(ctx, &d.idxB, n * 4, L)) || (rc = dalloc(ctx, &d.rank, n * 4, L)) ||
@@ -922,14 +1005,14 @@ static int finalize(grains_ctx* ctx) {
       (rc = dalloc(ctx, &d.obs_count, 16, L)) || (rc = dalloc(ctx, &d.pend, n * 4, L)) ||
       (rc = dalloc(ctx, &d.pend_list, n * 4, L)) || (rc = dalloc(ctx, &d.sort_state, 16, L)) ||
       (rc = dalloc(ctx, &d.mv_list, kMaxMovers * 4, L)) || (rc = dalloc(ctx, &d.mv_keys, kMaxMovers * 8, L)) ||
-      (rc = dalloc(ctx, &d.mv_old, kMaxMovers * 4, L)) || (rc = dalloc(ctx, &d.mv_dst, kMaxMovers * 4, L)) ||  (rc = dalloc(ctx, &d.defer_list, (ecap + max_nb * 256) * 4, L)) ||
-      (rc = dalloc(ctx, &d.defer_count, max_nb * 4, L)) || (rc = dalloc(ctx, &d.defer_off, (max_nb + 1) * 4, L)) ||
-      (rc = dalloc(ctx, &d.defer_flat, (ecap + 1) * 4, L)) ||
-      (rc = dalloc(ctx, &d.counters, (size_t)kNumCounters * kCntSlots * 8, L)))
+      (rc = dalloc(ctx, &d.mv_old, kMaxMovers * 4, L)) || (rc = dalloc(ctx, &d.mv_dst, kMaxMovers * 4, L)) ||
+      (rc = dalloc(ctx, &d.defer_list, defer_words(ecap) * 4, L)) ||
+      (rc = dalloc(ctx, &d.defer_count, kDeferQueues * 64, L)) || (rc = dalloc(ctx, &d.counters, kWordBytes, L)))
     return rc;
   d.pend_count = d.obs_count + 1;
   d.obs_count2 = d.obs_count + 2;
   d.queue_next = d.obs_count + 3;
+  d.nl = (uint32_t*)((unsigned char*)d.counters + kCounterBytes);
   // warm-start records: two buffers of ecap = K x N, zeroed (no direction)
   d.warm = ((ctx->cfg.flags & GRAINS_WARM_START) && ctx->cfg.precision == GRAINS_FP32_MIXED &&
             !(ctx->cfg.flags & GRAINS_REF_QUIRKS))
@@ -958,6 +1041,7 @@ static int finalize(grains_ctx* ctx) {
   GR_HIP(hipMemcpy(ph64, hk64.data(), hk64.size() * sizeof(HookeP<double>), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(ph32, hk32.data(), hk32.size() * sizeof(HookeP<float>), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(pgr, ctx->grids.data(), ns * sizeof(SimGrid), hipMemcpyHostToDevice));
+  GR_HIP(hipMemcpy(psg, ctx->sgrids.data(), ns * sizeof(SimGrid), hipMemcpyHostToDevice));
   if (!osh.empty()) {
     GR_HIP(hipMemcpy(posh, osh.data(), osh.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     GR_HIP(hipMemcpy(potr, otr.data(), otr.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -974,6 +1058,8 @@ static int finalize(grains_ctx* ctx) {
   d.hooke64 = ph64;
   d.hooke32 = ph32;
   d.grids = pgr;
+  d.sgrids = psg;
+  d.keep_torce = 0;
   d.obs_shape = posh;
   d.obs_tr = potr;
   d.nsims = ns;
@@ -992,7 +1078,7 @@ static int finalize(grains_ctx* ctx) {
   d.narrow_blocks = (uint32_t)(cu_count() * ctx->cfg.narrow_blocks_per_cu);
   d.split = ctx->cfg.narrow_passes == 2 ? 1 : 0;
   d.overlap = 1;
-  d.cand_half = half_of(ctx->cfg.candidate_staging, ctx->grids);
+  d.cand_half = half_of(ctx->cfg.candidate_staging, ctx->sgrids);
   d.cand_staged = staging_of(ctx->cfg.candidate_staging, n, d.ncells, d.cand_half);
   // dense cells on average: the half-shell search takes its groups (several
   // on a dense cell) from a work list built each step
@@ -1010,12 +1096,15 @@ static int finalize(grains_ctx* ctx) {
   launch_fill_u32(d.refine_count, 4, 0u, ctx->stream);
   launch_fill_u32(d.sort_state, 4, 0u, ctx->stream);
   launch_fill_u32(d.obs_count, 4, 0u, ctx->stream);
-  launch_fill_u32(d.defer_count, max_nb, 0u, ctx->stream);
+  launch_fill_u32(d.defer_count, kDeferQueues * 16, 0u, ctx->stream);
   set_defer_cap(ctx);
-  launch_fill_u32((uint32_t*)d.counters, 2 * kNumCounters * kCntSlots, 0u, ctx->stream);
+  launch_fill_u32((uint32_t*)d.counters, kWordBytes / 4, 0u, ctx->stream);
   GR_HIP(hipGetLastError());
   GR_HIP(hipStreamSynchronize(ctx->stream));
   ctx->layout_ok = true;
+  ctx->lists_ok = false;
+  ctx->interval = 8;
+  ctx->interval_known = false;
   return GRAINS_OK;
 }
 
@@ -1127,14 +1216,14 @@ static void mark(grains_ctx* ctx) {
   (void)hipEventRecord(ctx->pev[ctx->pev_used++], ctx->stream);
 }
 
-// one step, enqueued on ctx->stream (also what a graph captures)
-static void enqueue_step(grains_ctx* ctx) {
+// the neighbour lists built from the current positions, enqueued on
+// ctx->stream (also what a graph captures)
+static void enqueue_build(grains_ctx* ctx) {
   DevScene& d = ctx->d;
   hipStream_t s = ctx->stream;
-  mark(ctx);
-  // (the sort's output pair: the last of its ping-pong passes)
-  // (the previous order's keys: where the last sort left them)
-  launch_hash(d, (d.small_sort || (ctx->passes & 1)) ? d.keyA : d.keyB, s);  // also clears the step's queue counters
+  // (the sort's output pair: the last of its ping-pong passes; the previous
+  // order's keys: where the last sort left them)
+  launch_hash(d, (d.small_sort || (ctx->passes & 1)) ? d.keyA : d.keyB, s);
   mark(ctx);
   launch_sort(d, ctx->passes, ctx->digit_bits, &ctx->keys_s, &ctx->idx_s, s);
   mark(ctx);
@@ -1146,6 +1235,18 @@ static void enqueue_step(grains_ctx* ctx) {
   launch_scan(d.cand_count, d.entry_off, d.n, d.scan_blocks, s, d.K);
   launch_expand(d, ctx->keys_s, s);
   mark(ctx);
+}
+
+// one step over the lists (returning at once, kernel by kernel, when they no
+// longer hold), after a build when `build`
+static void enqueue_step(grains_ctx* ctx, bool build) {
+  DevScene& d = ctx->d;
+  hipStream_t s = ctx->stream;
+  mark(ctx);
+  if (build)
+    enqueue_build(ctx);
+  else
+    for (int k = 0; k < 5; ++k) mark(ctx);  // the build's phases: nothing
   // the integration split around the narrow phase's second pass: two
   // passes (physics semantics), the step not profiled phase by phase
   const bool split = d.overlap && d.split > 0 && !(d.flags & GRAINS_REF_QUIRKS) && !ctx->adj_rec &&
@@ -1190,9 +1291,16 @@ static void enqueue_step(grains_ctx* ctx) {
   mark(ctx);
 }
 
-static int read_stats(grains_ctx* ctx, uint32_t steps) {
-  std::vector<unsigned long long> slots((size_t)kNumCounters * kCntSlots);
-  GR_HIP(hipMemcpy(slots.data(), ctx->d.counters, slots.size() * 8, hipMemcpyDeviceToHost));
+// the counters and list words, read back (the stream is then idle)
+static int read_words(grains_ctx* ctx, uint32_t* nl) {
+  GR_HIP(hipMemcpyAsync(ctx->host_words, ctx->d.counters, kWordBytes, hipMemcpyDeviceToHost, ctx->stream));
+  GR_HIP(hipStreamSynchronize(ctx->stream));
+  std::memcpy(nl, ctx->host_words + kCounterBytes, kNlWords * 4);
+  return GRAINS_OK;
+}
+
+static void read_stats(grains_ctx* ctx, uint32_t steps) {
+  const unsigned long long* slots = (const unsigned long long*)ctx->host_words;
   unsigned long long c[kNumCounters];
   for (int k = 0; k < kNumCounters; ++k) {
     c[k] = 0;
@@ -1219,7 +1327,20 @@ static int read_stats(grains_ctx* ctx, uint32_t steps) {
   st.fp64_refine_max_iterations = c[kCntRefMaxIters];
   st.neighbor_overflow = c[kCntOverflow];
   st.max_candidates = (uint32_t)c[kCntMaxCand];
-  st.sort_passes = (uint32_t)ctx->passes;
+  st.sort_passes = (uint32_t)ctx->ref_passes;
+}
+
+// The lists with their skin (on) or without: every build then holds for its
+// step alone, and a list is the step's own candidates.
+static int use_skin(grains_ctx* ctx, bool on) {
+  std::vector<SimGrid> g = ctx->sgrids;
+  if (!on)
+    for (SimGrid& x : g) x.half_skin = 0.0;
+  GR_HIP(hipStreamSynchronize(ctx->stream));
+  GR_HIP(hipMemcpy((void*)ctx->d.sgrids, g.data(), g.size() * sizeof(SimGrid), hipMemcpyHostToDevice));
+  ctx->d.skin = on ? 1 : 0;
+  ctx->lists_ok = false;
+  drop_graph(ctx);  // captured kernels hold the flag
   return GRAINS_OK;
 }
 
@@ -1243,56 +1364,120 @@ static int state_from(grains_ctx* ctx, const double* src) {
   GR_HIP(hipMemcpyAsync(ctx->d.omega, src + 10 * n, 3 * n * 8, hipMemcpyDeviceToDevice, s));
   return GRAINS_OK;
 }
-// after each recorded step: a checkpoint every adj_every steps
-static int adj_after_step(grains_ctx* ctx) {
-  ++ctx->adj_steps;
-  if (ctx->adj_steps % ctx->adj_every) return GRAINS_OK;
+// after recorded steps (never past a checkpoint): a checkpoint every
+// adj_every steps
+static int adj_after_steps(grains_ctx* ctx, uint32_t steps) {
+  ctx->adj_steps += steps;
+  if (!steps || ctx->adj_steps % ctx->adj_every) return GRAINS_OK;
   double* cp;
   int rc = dalloc(ctx, &cp, 13 * ctx->n * 8, ctx->adj_cp);
   if (rc) return rc;
   return state_to(ctx, cp);
 }
 
+// Steps are launched in chunks of as many as the lists are expected to hold
+// for; the kernels of a step whose lists no longer hold return at once, and
+// after each chunk the host reads how many were taken, builds new lists when
+// they ran out, and goes on.
 static int run_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
   int rc = finalize(ctx);
   if (rc) return rc;
   hipStream_t s = ctx->stream;
-  launch_fill_u32((uint32_t*)ctx->d.counters, 2 * kNumCounters * kCntSlots, 0u, s);
-  // the first step of a run sorts in full (the state may have been set
-  // since the last sorted order), the others merge their movers
-  launch_fill_u32(ctx->d.sort_state, 3, 0u, s);
-  // chunks of graph_steps steps in one graph (not while the adjoint
-  // records: it copies the state after every step)
-  const uint32_t chunk = graph && !ctx->adj_rec ? ctx->graph_steps : 1u;
-  const uint32_t n_multi = chunk > 1 ? n_steps / chunk : 0u;
+  launch_run_begin(ctx->d, n_steps, !ctx->lists_ok, s);
+  // 0: the lists' build; otherwise that many steps
   auto capture = [&](uint32_t steps, hipGraph_t* g, hipGraphExec_t* ge) -> int {
+    if (*ge) return GRAINS_OK;
     ctx->capturing = true;
     GR_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    for (uint32_t k = 0; k < steps; ++k) enqueue_step(ctx);
+    if (!steps) enqueue_build(ctx);
+    for (uint32_t k = 0; k < steps; ++k) enqueue_step(ctx, false);
     hipError_t ec = hipStreamEndCapture(s, g);
     ctx->capturing = false;
     GR_HIP(ec);
     GR_HIP(hipGraphInstantiate(ge, *g, nullptr, nullptr, 0));
     return GRAINS_OK;
   };
-  if (graph && n_steps > n_multi * chunk && !ctx->graph_exec &&
-      (rc = capture(1, &ctx->graph, &ctx->graph_exec)))
-    return rc;
-  if (n_multi && !ctx->graph_multi_exec && (rc = capture(chunk, &ctx->graph_multi, &ctx->graph_multi_exec)))
-    return rc;
+  // profiled steps are launched one by one with their builds' phases
+  auto build = [&]() -> int {
+    if (!graph) {
+      enqueue_build(ctx);
+      return GRAINS_OK;
+    }
+    if (int r = capture(0, &ctx->graph_build, &ctx->graph_build_exec)) return r;
+    GR_HIP(hipGraphLaunch(ctx->graph_build_exec, s));
+    return GRAINS_OK;
+  };
+  auto steps = [&](uint32_t m) -> int {
+    if (!graph) {
+      for (uint32_t k = 0; k < m; ++k) enqueue_step(ctx, false);
+      return GRAINS_OK;
+    }
+    const uint32_t chunk = ctx->graph_steps;
+    if (chunk > 1 && m >= chunk) {
+      if (int r = capture(chunk, &ctx->graph_multi, &ctx->graph_multi_exec)) return r;
+      for (; m >= chunk; m -= chunk) GR_HIP(hipGraphLaunch(ctx->graph_multi_exec, s));
+    }
+    if (m)
+      if (int r = capture(1, &ctx->graph, &ctx->graph_exec)) return r;
+    for (; m; --m) GR_HIP(hipGraphLaunch(ctx->graph_exec, s));
+    return GRAINS_OK;
+  };
   ctx->pev_used = 0;
   GR_HIP(hipEventRecord(ctx->ev0, s));
-  for (uint32_t k = 0; k < n_multi; ++k) GR_HIP(hipGraphLaunch(ctx->graph_multi_exec, s));
-  for (uint32_t k = n_multi * chunk; k < n_steps; ++k) {
-    if (graph)
-      GR_HIP(hipGraphLaunch(ctx->graph_exec, s));
-    else
-      enqueue_step(ctx);
-    if (ctx->adj_rec && (rc = adj_after_step(ctx))) return rc;
+  uint32_t done = 0, nl[kNlWords] = {0};
+  while (done < n_steps) {
+    uint32_t m = n_steps - done;
+    if (ctx->adj_rec) m = std::min<uint32_t>(m, ctx->adj_every - (uint32_t)(ctx->adj_steps % ctx->adj_every));
+    const bool each = !ctx->d.skin || ctx->interval <= 1;  // lists for one step at a time
+    if (each) {
+      m = std::min(m, 64u);
+      for (uint32_t k = 0; k < m; ++k) {
+        if (ctx->profiling && !graph) {
+          enqueue_step(ctx, true);
+        } else {
+          if ((rc = build()) || (rc = steps(1))) return rc;
+        }
+      }
+      ctx->interval = 4;
+    } else {
+      bool fresh = !ctx->lists_ok;
+      if (fresh) ctx->since_build = 0;
+      m = std::min(m, ctx->interval > ctx->since_build ? ctx->interval - ctx->since_build : 1u);
+      if (fresh && ctx->profiling && !graph) {
+        enqueue_step(ctx, true);
+        if ((rc = steps(m - 1))) return rc;
+      } else if ((fresh && (rc = build())) || (rc = steps(m))) {
+        return rc;
+      }
+    }
+    GR_HIP(hipGetLastError());
+    if (done + m == n_steps) GR_HIP(hipEventRecord(ctx->ev1, s));
+    if ((rc = read_words(ctx, nl))) return rc;
+    const uint32_t took = nl[kNlDone] - done;
+    if (ctx->d.skin && nl[kNlOver]) {
+      // a list outgrew max_neighbors with the skin; the step's own
+      // candidates may still fit
+      if ((rc = use_skin(ctx, false))) return rc;
+    } else {
+      if (!took) return fail(ctx, GRAINS_EDEVICE, "a step did not run");
+      ctx->lists_ok = nl[kNlValid] != 0;
+      ctx->since_build = each ? 1u : ctx->since_build + took;
+      if (!each && !ctx->lists_ok) {
+        ctx->interval = ctx->since_build;
+        ctx->interval_known = true;
+      } else if (!each && ctx->since_build >= ctx->interval) {
+        // they outlast the estimate: a little more once a build has shown
+        // how long they last, else twice as long
+        ctx->interval = ctx->since_build + (ctx->interval_known ? 1 + ctx->since_build / 8 : ctx->since_build);
+      }
+    }
+    done += took;
+    if (ctx->adj_rec && (rc = adj_after_steps(ctx, took))) return rc;
   }
-  GR_HIP(hipGetLastError());
-  GR_HIP(hipEventRecord(ctx->ev1, s));
-  GR_HIP(hipStreamSynchronize(s));
+  if (!n_steps) {
+    GR_HIP(hipEventRecord(ctx->ev1, s));
+    if ((rc = read_words(ctx, nl))) return rc;
+  }
   float ms = 0;
   GR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   for (int p = 0; p < GRAINS_NUM_PHASES; ++p) ctx->phase_ms[p] = 0;
@@ -1305,9 +1490,8 @@ static int run_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
         ctx->phase_ms[p] += t;
       }
   }
-  rc = read_stats(ctx, n_steps);
+  read_stats(ctx, n_steps);
   ctx->stats.elapsed_ms = ms;
-  if (rc) return rc;
   if (ctx->stats.neighbor_overflow)
     return fail(ctx, GRAINS_EOVERFLOW, "candidate capacity max_neighbors exceeded (" +
                                            std::to_string(ctx->stats.max_candidates) + " needed)");
@@ -1359,9 +1543,10 @@ extern "C" int grains_set_narrow_passes(grains_ctx_t* ctx, int passes) {
 extern "C" int grains_set_candidate_staging(grains_ctx_t* ctx, int mode) {
   if (!ctx || mode < 0 || mode > 3) return GRAINS_EINVAL;
   ctx->cfg.candidate_staging = mode;
-  ctx->d.cand_half = half_of(mode, ctx->grids);
+  ctx->d.cand_half = half_of(mode, ctx->sgrids);
   ctx->d.cand_staged = staging_of(mode, ctx->d.n, ctx->d.ncells, ctx->d.cand_half);
-  drop_graph(ctx);  // a captured step holds the old kernel
+  drop_graph(ctx);  // a captured build holds the old kernel
+  ctx->lists_ok = false;
   return GRAINS_OK;
 }
 
@@ -1381,8 +1566,27 @@ extern "C" int grains_get_cell_keys(grains_ctx_t* ctx, uint32_t* keys, uint32_t*
   if (!ctx) return GRAINS_EINVAL;
   if (n != ctx->n || !ctx->layout_ok || !ctx->idx_s) return fail(ctx, GRAINS_ESTATE, "no step run yet");
   GR_HIP(hipStreamSynchronize(ctx->stream));
-  if (keys) GR_HIP(hipMemcpy(keys, ctx->d.key, n * 4, hipMemcpyDeviceToHost));
-  if (sorted) GR_HIP(hipMemcpy(sorted, ctx->idx_s, n * 4, hipMemcpyDeviceToHost));
+  std::vector<uint32_t> own;
+  uint32_t* k = keys;
+  if (!k) {
+    own.resize(n);
+    k = own.data();
+  }
+  GR_HIP(hipMemcpy(k, ctx->d.key, n * 4, hipMemcpyDeviceToHost));
+  if (sorted) {  // stable, two counting passes of 16 bits
+    std::vector<uint32_t> tmp(n);
+    for (int p = 0; p < 2; ++p) {
+      std::vector<uint32_t> off(65537, 0u);
+      const uint32_t* in = p ? tmp.data() : nullptr;
+      uint32_t* out = p ? sorted : tmp.data();
+      for (uint64_t i = 0; i < n; ++i) ++off[((k[i] >> (16 * p)) & 0xffffu) + 1];
+      for (int v = 0; v < 65536; ++v) off[v + 1] += off[v];
+      for (uint64_t i = 0; i < n; ++i) {
+        const uint32_t id = in ? in[i] : (uint32_t)i;
+        out[off[(k[id] >> (16 * p)) & 0xffffu]++] = id;
+      }
+    }
+  }
   return GRAINS_OK;
 }
 
@@ -1396,19 +1600,48 @@ extern "C" int grains_get_pairs(grains_ctx_t* ctx, int which, uint32_t* ij, uint
   GR_HIP(hipMemcpy(rank.data(), ctx->d.rank, n * 4, hipMemcpyDeviceToHost));
   GR_HIP(hipMemcpy(sidx.data(), ctx->idx_s, n * 4, hipMemcpyDeviceToHost));
   const uint64_t E = off[n];
-  std::vector<uint32_t> pj(E), fl(E);
+  std::vector<uint32_t> pj(E), fl(E), key(n);
+  GR_HIP(hipMemcpy(key.data(), ctx->d.key, n * 4, hipMemcpyDeviceToHost));
   if (E) {
     GR_HIP(hipMemcpy(pj.data(), ctx->d.pair_j, E * 4, hipMemcpyDeviceToHost));
     GR_HIP(hipMemcpy(fl.data(), ctx->d.pair_flag, E * 4, hipMemcpyDeviceToHost));
   }
+  const uint32_t want = which == GRAINS_PAIRS_CONTACT ? kFlagContact : kFlagCand;
   uint64_t k = 0;
+  std::vector<uint64_t> row;
   for (uint64_t i = 0; i < n; ++i) {
+    // the particle's pairs by (neighbour cell in the visit order, id), at the
+    // positions of the step
     const uint32_t s = rank[i];
+    const SimGrid& g = ctx->grids[ctx->psim[i]];
+    auto cell = [&](uint32_t id, uint32_t* c) {
+      const uint32_t l = key[id] - g.base;
+      c[0] = l % g.n3[0];
+      c[1] = (l / g.n3[0]) % g.n3[1];
+      c[2] = l / (g.n3[0] * g.n3[1]);
+    };
+    uint32_t ci[3];
+    cell((uint32_t)i, ci);
+    row.clear();
     for (uint32_t e = off[s]; e < off[s + 1]; ++e) {
-      if (which == GRAINS_PAIRS_CONTACT && !(fl[e] & kFlagContact)) continue;
-      if (ij && k < cap) {  // entries hold sorted positions
+      if (!(fl[e] & want)) continue;
+      const uint32_t j = sidx[pj[e]];  // entries hold sorted positions
+      uint32_t cj[3];
+      cell(j, cj);
+      uint64_t slot = 0;
+      for (int a = 2; a >= 0; --a) {
+        const int m = (int)g.n3[a];
+        int v = (int)cj[a] - (int)ci[a];
+        if ((g.periodic >> a) & 1) v = v == m - 1 ? -1 : (v == 1 - m ? 1 : v);
+        slot = slot * 3 + (uint64_t)(v + 1);
+      }
+      row.push_back((slot << 32) | j);
+    }
+    std::sort(row.begin(), row.end());
+    for (uint64_t r : row) {
+      if (ij && k < cap) {
         ij[2 * k] = (uint32_t)i;
-        ij[2 * k + 1] = sidx[pj[e]];
+        ij[2 * k + 1] = (uint32_t)r;
       }
       ++k;
     }
@@ -1741,25 +1974,33 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
   GR_HIP(hipMemcpyAsync(ctx->adj_count, ctx->d.contact_count, n * 4, hipMemcpyDeviceToDevice, s));
   const bool prof = ctx->profiling;
   ctx->profiling = false;
+  // every step below sets its state: its lists are built for it alone
+  const bool skin = ctx->d.skin != 0;
+  if (skin && (rc = use_skin(ctx, false))) return rc;
+  ctx->lists_ok = false;
+  ctx->d.keep_torce = 1;
+  launch_run_begin(ctx->d, 0u, true, s);
   const uint64_t nblocks = (T + K - 1) / K;
   for (uint64_t bb = nblocks; bb-- > 0;) {
     const uint64_t t0 = bb * K, t1 = std::min(t0 + K, T);
     if ((rc = state_from(ctx, (const double*)ctx->adj_cp[bb]))) break;
     for (uint64_t t = t0; t < t1 && !rc; ++t) {
       if ((rc = state_to(ctx, ctx->adj_blk + (t - t0) * 13 * n))) break;
-      enqueue_step(ctx);
+      enqueue_step(ctx, true);
     }
     for (uint64_t t = t1; t-- > t0 && !rc;) {
       double* st = ctx->adj_blk + (t - t0) * 13 * n;
       if ((rc = state_from(ctx, st))) break;
-      enqueue_step(ctx);  // entries, contact flags, force and torque of step t
+      enqueue_step(ctx, true);  // entries, contact flags, force and torque of step t
       a.state = st;
       launch_adjoint_step(ctx->d, a, ntab, s);
     }
     if (rc) break;
   }
   ctx->profiling = prof;
+  ctx->d.keep_torce = 0;
   int rc2 = state_from(ctx, ctx->adj_save);
+  if (skin && !rc2) rc2 = use_skin(ctx, true);
   if (rc) return rc;
   if (rc2) return rc2;
   GR_HIP(hipMemcpyAsync(ctx->d.contact_count, ctx->adj_count, n * 4, hipMemcpyDeviceToDevice, s));

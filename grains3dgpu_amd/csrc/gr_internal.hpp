@@ -5,14 +5,17 @@
 // HBM layout (N particles, E candidate entries, C cells):
 //   state    pos[3][N], quat[4][N] (x,y,z,w), vel[3][N], omega[3][N]   FP64 planes
 //   ids      shape[N], sim[N]                                          u32
-//   broad    key[N] (by particle), key/idx ping-pong [2][N], rank[N],
-//            cell_off[C+1] (first sorted position of each cell)      u32
-//   sorted   bp[N] = {x, y, z, prefilter radius}   32 B, cell order
+//   broad    key[N] (by particle: the reference's cell, each step),
+//            skey[N] (the search's cell), key/idx ping-pong [2][N], rank[N],
+//            cell_off[C+1] (first sorted position of each search cell) u32
+//   sorted   bp[N] = {x, y, z, list radius}   32 B, cell order, as the lists
+//            were built; rcs[N] = prefilter radius
 //            bp32[N] = bp in FP32, relative to the sim's domain minimum, 16 B
 //            cell_sph[C] = bounding sphere of each cell's residents, 16 B
 //            pk[N] = PoseRec {pos, quat, shape, sim}  64 B, cell order
-//            (rebuilt every step from the planes; neighbours of a cell are
-//            contiguous, so the gathers of a wave share cache lines)
+//            (gathered from the planes when the lists are built, then kept
+//            up by the integration; neighbours of a cell are contiguous, so
+//            the gathers of a wave share cache lines)
 //   pairs    cand[K][N] (k-major: lanes write consecutive words),
 //            cand_count[N], entry_off[N+1]                            u32
 //            pair_i[E], pair_j[E] (sorted positions), pair_flag[E]     u32
@@ -45,6 +48,8 @@ constexpr uint32_t kFlagContact = 1u;
 constexpr uint32_t kFlagGjk = 2u;
 constexpr uint32_t kFlagDeep = 4u;
 constexpr uint32_t kFlagRefine = 8u;
+constexpr uint32_t kFlagCand = 16u;     // passed the bounding-sphere prefilter this step
+constexpr int kFlagSlot = 8;            // contacts: the neighbour cell's slot in the visit order, from this bit on
 
 // device counters (u64), summed over the steps of one grains_step call.
 // Each counter is spread over kCntSlots words (slot = block index mod
@@ -72,6 +77,19 @@ enum Counter {
   kNumCounters = 18
 };
 
+// State of the neighbour lists and of the run of steps (device words, read
+// back with the counters).
+enum ListState {
+  kNlValid = 0,   // the lists cover the current positions (2: for one step only)
+  kNlRun,         // this step runs (latched from kNlValid by its first kernel)
+  kNlLast,        // it is the run's last step
+  kNlDone,        // steps of the run taken
+  kNlTarget,      // steps of the run asked for
+  kNlOver,        // a list outgrew max_neighbors when the lists were built
+  kNlOutside,     // a centre lay outside a periodic side when they were built
+  kNlWords = 8
+};
+
 // One simulation's linked cell and forces.
 struct SimGrid {
   double lo[3], hi[3], L[3];
@@ -82,6 +100,8 @@ struct SimGrid {
   int32_t periodic;      // bitmask x=1, y=2, z=4
   uint32_t table;        // first entry of its contact table block
   uint32_t obs_begin, obs_end;  // its obstacles (obstacles sorted by sim)
+  double half_skin;      // half the lists' skin: added to every list radius
+  double move2;          // squared displacement since the lists were built up to which they hold
 };
 
 // Dynamics of one shape (RigidBody mass properties, RigidBody.cpp:19-59).
@@ -129,14 +149,20 @@ struct DevScene {
   const float* cverts32;
   const HookeP<double>* hooke64;
   const HookeP<float>* hooke32;
-  const SimGrid* grids;
+  const SimGrid* grids;         // the reference's cells (keys, adjacency, visit order)
+  const SimGrid* sgrids;        // the search's cells (at least a list reach wide)
   const uint32_t* obs_shape;    // sorted by sim
   const double* obs_tr;         // 12 doubles each
   // broad phase
-  uint32_t *key, *keyA, *idxA, *keyB, *idxB, *rank;
+  uint32_t *key, *skey, *keyA, *idxA, *keyB, *idxB, *rank;
+  uint32_t* rkey;               // reference cell by sorted position when the lists were built
+  double* rcs;                  // prefilter radius by sorted position
+  uint32_t* nl;                 // ListState words
+  int32_t skin;                 // 1: the lists hold for several steps; 0: for the step they are built in
+  int32_t keep_torce;           // 1: every step's total force and torque are stored (the adjoint reads them)
   const uint32_t* sidx;         // particle at each sorted position (this step)
   uint32_t* cell_off;           // CSR over cells: residents of c are [off[c], off[c+1])
-  double4* bp;                  // {x, y, z, prefilter radius} by sorted position
+  double4* bp;                  // {x, y, z, list radius} by sorted position when the lists were built
   float4* bp32;                 // bp in FP32, positions relative to the sim's domain minimum
   float4* cell_sph;             // per cell: bounding sphere of its residents' spheres (bp32 frame)
   PoseRec* pk;                  // pose by sorted position
@@ -151,12 +177,10 @@ struct DevScene {
   void* pair_res;               // PairRes<T>[ecap]
   uint32_t* refine_list;        // entries to re-run in FP64 (FP32-mixed)
   uint32_t* refine_count;
-  uint32_t* queue_next;         // FP64 searches: entries handed out past the dealt ones (reset by k_hash)
-  uint32_t* defer_list;         // entries the screening pass left undecided: one
-                                // segment of defer_cap words per block
-  uint32_t* defer_count;        // per block of the screen (narrow_blocks)
-  uint32_t* defer_off;          // exclusive scan of defer_count (+ total)
-  uint32_t* defer_flat;         // the segments flattened in order (the complete pass's input)
+  uint32_t* queue_next;         // FP64 searches: entries handed out past the dealt ones
+  uint32_t* defer_list;         // entries the screening pass left undecided: kDeferQueues
+                                // queues of defer_cap words, block b filling queue b % kDeferQueues
+  uint32_t* defer_count;        // their lengths (one 64-byte line each)
   uint32_t defer_cap;
   int32_t split;                // 1: screening pass + pass over the queued entries
   int32_t cand_staged;          // 1: candidate search stages neighbour windows in LDS
@@ -171,17 +195,17 @@ struct DevScene {
   int32_t integrator;
   double* ab_hist;
   // GRAINS_WARM_START (FP32-mixed, physics semantics): each entry's GJK
-  // direction of the step, in the world frame, in two buffers of K x N
+  // direction of its last step, in the world frame, in two buffers of K x N
   // records {x, y, z, neighbour id as bits} in entry order, and per particle
-  // id the first entry and the entry count of each step (ws_nb); ws_par =
-  // the buffer this step writes (flipped at the start of every step), the
-  // other holds the previous step
+  // id the first entry and the entry count (ws_nb); ws_par = the buffer of
+  // the current lists (flipped when they are built: the other holds the
+  // records of the lists before, k_warm_carry)
   int32_t warm;
   float4* ws;
   uint2* ws_nb;
   uint32_t* ws_par;
   // particles within reach of an obstacle, queued by k_integrate for
-  // k_integrate_obs (count reset by k_hash at the start of every step)
+  // k_integrate_obs (count reset by the step's first kernel)
   uint32_t* obs_list;
   uint32_t* obs_count;
   // the particles k_integrate_pend queues for k_integrate_obs (steps with
@@ -192,13 +216,13 @@ struct DevScene {
   uint32_t* obs_count2;
   // Two narrow passes: pend[s] = 1 when the screen left an entry of sorted
   // position s undecided (both particles of the entry are marked; cleared by
-  // k_cells).  With `overlap`, the integration of the other particles runs
+  // the integration).  With `overlap`, the integration of the other particles runs
   // while the complete pass and the FP64 re-runs settle those entries, and
   // the marked particles (queued in pend_list, count pend_count, reset by
-  // k_hash) are integrated after both.
+  // the screen) are integrated after both.
   // Sorting by merge.  sort_state[0] = 1 once a sorted order and its
-  // inverse permutation stand (k_cells; cleared before each run of steps),
-  // [2] = the particles that changed cell (k_hash; at most kMaxMovers of
+  // inverse permutation stand (k_cells; cleared when the state is set),
+  // [2] = the particles that changed search cell (k_hash; at most kMaxMovers of
   // their ids kept in mv_list); the step's sort follows from the two
   // (sort_mode: 0 radix, 1 merge the movers into the previous order, 2 no
   // particle changed cell), evaluated by each sort kernel itself.  The
@@ -261,9 +285,9 @@ void launch_candidates(const DevScene& d, const uint32_t* keys_s, hipStream_t s)
 // the kernels return at once unless *gate == 0
 void launch_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* block_sums, hipStream_t s,
                  uint32_t clamp = 0xffffffffu, const uint32_t* gate = nullptr);
-// the screening pass's queue: scan of the segment counts, then the segments
-// copied into defer_flat in order
-void launch_defer_flatten(const DevScene& d, hipStream_t s);
+// the start of a run of n steps: counters cleared, run words set; sort:
+// the sorted order no longer stands
+void launch_run_begin(const DevScene& d, uint32_t n, bool sort, hipStream_t s);
 void launch_expand(const DevScene& d, const uint32_t* keys_s, hipStream_t s);
 int cu_count();
 // gr_narrow64.hip / gr_narrow32.hip
@@ -290,6 +314,62 @@ void launch_gjk_batch32(const ShapeNP<float>* shapes, const float* verts, const 
                         hipStream_t s);
 
 // ---- small device helpers --------------------------------------------------------
+// The screening pass's queues: one counter would serialise a block's append
+// at a single address (~12 ns each).
+constexpr uint32_t kDeferQueues = 16;
+__device__ __forceinline__ uint32_t defer_total(const DevScene& d) {
+  uint32_t t = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < kDeferQueues; ++q) t += d.defer_count[16 * q];
+  return t;
+}
+// the k-th queued entry, the queues end to end
+__device__ __forceinline__ uint32_t defer_entry(const DevScene& d, uint32_t k) {
+  uint32_t q = 0;
+#pragma unroll
+  for (uint32_t i = 0; i + 1 < kDeferQueues; ++i) {
+    const uint32_t c = d.defer_count[16 * i];
+    if (q == i && k >= c) {
+      k -= c;
+      q = i + 1;
+    }
+  }
+  return d.defer_list[(uint64_t)q * d.defer_cap + k];
+}
+// The reference's cell of a centre (LinkedCell::computeLinearCellHash,
+// LinkedCell.cpp:117-149), FP64 divide + floor; the partial last cell beyond
+// n3 h (the domain is rarely a multiple of h) folds into cell n3 - 1, and
+// centres outside (a NaN: cell 0) into the border cells.
+__device__ __forceinline__ void cell_of(const SimGrid& g, const double* p, uint32_t* c) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double f = floor((p[k] - g.lo[k]) / g.h);
+    if (!(f >= 0.0))
+      c[k] = 0;
+    else if (f >= (double)g.n3[k])
+      c[k] = g.n3[k] - 1;
+    else
+      c[k] = (uint32_t)f;
+  }
+}
+__device__ __forceinline__ uint32_t cell_key(const SimGrid& g, const uint32_t* c) {
+  return g.base + (c[2] * g.n3[1] + c[1]) * g.n3[0] + c[0];
+}
+// Slot of cell cj among the 27 neighbour cells of ci in the visit order (z
+// outer, then y, then x: LinkedCell.cpp:41-70), periodic axes wrapped; -1:
+// not a neighbour.
+__device__ __forceinline__ int cell_slot(const SimGrid& g, const uint32_t* ci, const uint32_t* cj) {
+  int dd[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int n = (int)g.n3[k];
+    int v = (int)cj[k] - (int)ci[k];
+    if ((g.periodic >> k) & 1) v = v == n - 1 ? -1 : (v == 1 - n ? 1 : v);
+    if (v < -1 || v > 1) return -1;
+    dd[k] = v;
+  }
+  return ((dd[2] + 1) * 3 + dd[1] + 1) * 3 + dd[0] + 1;
+}
 // The step's sort from sort_state (DevScene::sort_state): radix when no
 // previous order stands or too many particles changed cell, a merge when a
 // few did, nothing when none did.  Read between k_hash and k_cells, which

@@ -5,6 +5,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gr_internal.hpp"
 #include "gr_move.hpp"
@@ -45,43 +46,59 @@ __device__ __forceinline__ void pair_frames(const SimGrid& g, V3<double> xi, Qt<
   }
 }
 
-// The previous step's GJK direction of the pair (wi, wj), looked up only
-// when the pair reaches GJK: wi's entry wk of the previous step first (a
-// particle's list keeps its order while its neighbours stay), then its other
-// entries, four loads in flight at a time.  Records: float4 {direction in the
-// world frame, neighbour id bits} in entry order; nb = {first entry, count}
-// of wi in the previous step.
+// The GJK direction of the entry's last step (world frame), read only when
+// the pair reaches GJK; a zero direction: none.
 struct WarmLookup {
-  const float4* prev;
-  const uint2* prev_nb;
-  uint32_t wi, wj, wk;
+  const float4* rec;
   GR_D bool fetch(V3<float>& w) const {
-    const uint2 nb = prev_nb[wi];
-    const uint32_t np = nb.y;
-    const float4* pr = prev + nb.x;
-    float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
-    bool hit = false;
-    if (wk < np) {
-      r = pr[wk];
-      hit = __float_as_uint(r.w) == wj;
-    }
-    for (uint32_t k0 = 0; !hit && k0 < np; k0 += 4) {
-      float4 q[4];
-#pragma unroll
-      for (uint32_t u = 0; u < 4; ++u)
-        q[u] = k0 + u < np ? pr[k0 + u] : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-      for (uint32_t u = 0; u < 4; ++u)
-        if (!hit && k0 + u < np && __float_as_uint(q[u].w) == wj) {
-          r = q[u];
-          hit = true;
-        }
-    }
+    const float4 r = *rec;
     w = {r.x, r.y, r.z};
     const float nn = dot(w, w);
-    return hit && nn > 0.f && nn < INFINITY;
+    return nn > 0.f && nn < INFINITY;
   }
 };
+
+// a rounded product: the FP32 unit is built with FMA contraction, which would
+// fold it into the sum it goes into
+__device__ __forceinline__ double product(double a, double b) {
+  double p = a * b;
+  asm("" : "+v"(p));
+  return p;
+}
+
+// The bounding-sphere prefilter of the reference's particle loop
+// (ComponentManagerCPU.cpp:384-396) for a list entry at the current
+// positions: spheres overlapping, particles in neighbouring cells.  FP64
+// without contraction in both precisions.  Spheres that overlap by less than
+// a cell's side lie in neighbouring cells (any cell is at least that wide
+// unless the caller asked for smaller ones), so the cells are worked out only
+// for offsets within rounding of the side or more, and when a centre lay
+// outside a periodic side (`outside`: its cell is a folded one).
+__device__ __forceinline__ bool is_candidate(const SimGrid& g, V3<double> xi, V3<double> xj, double ri, double rj,
+                                             bool outside) {
+  double ex = xj.x - xi.x, ey = xj.y - xi.y, ez = xj.z - xi.z;
+  if (g.periodic & 1) ex -= product(g.L[0], rint(ex / g.L[0]));
+  if (g.periodic & 2) ey -= product(g.L[1], rint(ey / g.L[1]));
+  if (g.periodic & 4) ez -= product(g.L[2], rint(ez / g.L[2]));
+  const double rs = ri + rj;
+  const double d2 = product(ex, ex) + product(ey, ey) + product(ez, ez);
+  if (!(d2 < rs * rs * (1.0 + kPrefilterSlack))) return false;
+  if (fmax(fabs(ex), fmax(fabs(ey), fabs(ez))) <= g.h * (1.0 - 1e-9) && !outside) return true;
+  const double pi[3] = {xi.x, xi.y, xi.z}, pj[3] = {xj.x, xj.y, xj.z};
+  uint32_t ci[3], cj[3];
+  cell_of(g, pi, ci);
+  cell_of(g, pj, cj);
+  return cell_slot(g, ci, cj) >= 0;
+}
+
+// flag bits of a contact: its neighbour cell's slot in the visit order
+__device__ __forceinline__ uint32_t slot_bits(const SimGrid& g, V3<double> xi, V3<double> xj) {
+  const double pi[3] = {xi.x, xi.y, xi.z}, pj[3] = {xj.x, xj.y, xj.z};
+  uint32_t ci[3], cj[3];
+  cell_of(g, pi, ci);
+  cell_of(g, pj, cj);
+  return (uint32_t)max(cell_slot(g, ci, cj), 0) << kFlagSlot;
+}
 
 // Hooke force and torque on particle i of the contact ci with j; the poses'
 // origins in the frame of ci, xi in the world.
@@ -123,22 +140,27 @@ __device__ __forceinline__ void contact_force(const DevScene& d, const SimGrid& 
 // si's side (ComponentManagerCPU.cpp:384-419).  Poses come from the sorted
 // records; velocities, needed only for contacts, from the planes through the
 // particle ids.  Returns the pair flag.
-// e: the entry (its slot in si's candidate list keys the warm-start record);
-// ~0u for callers without one (the FP64 re-run).
+// e: the entry.  FILTER: apply the prefilter first (a list entry); the
+// returned flag is 0 for a pair it leaves out.
 // dir (FP32, physics semantics; may be null): receives the direction the
 // search ended on in the world frame (left alone when GJK did not run).
 // PAIR (physics semantics): lanes 2k and 2k + 1 evaluate
 // the same entry, sharing GJK's support pairs (gjk_sv<PAIR>).
-template <class T, class R, bool SV, bool SCREEN = false, bool WARM = false, bool PAIR = false>
+template <class T, class R, bool SV, bool SCREEN = false, bool WARM = false, bool PAIR = false, bool FILTER = false>
 __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, uint32_t sj, PairRes<R>& out,
-                                               NpStats& st, uint32_t e = ~0u, V3<T>* dir = nullptr) {
+                                               NpStats& st, uint32_t e, V3<T>* dir = nullptr) {
   const uint64_t n = d.n;
   const PoseRec pi = d.pk[si];
   const PoseRec pj = d.pk[sj];
+  const SimGrid& g = d.grids[pi.sim];
+  if constexpr (FILTER) {
+    if (!is_candidate(g, V3<double>{pi.x, pi.y, pi.z}, V3<double>{pj.x, pj.y, pj.z}, d.rcs[si], d.rcs[sj],
+                      d.nl[kNlOutside] != 0))
+      return 0u;
+  }
   const ShapeNP<T>* np = np_table<T>(d);
   const ShapeNP<T> A = np[pi.shape];
   const ShapeNP<T> B = np[pj.shape];
-  const SimGrid& g = d.grids[pi.sim];
   const V3<double> xi = {pi.x, pi.y, pi.z};
   Tr<T> a2w, b2w;
   pair_frames<T>(g, xi, Qt<double>{pi.qx, pi.qy, pi.qz, pi.qw}, V3<double>{pj.x, pj.y, pj.z},
@@ -148,49 +170,102 @@ __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, u
   const GjkArgs args = {d.flags, sizeof(T) == 8 && d.precision == GRAINS_FP32_MIXED ? d.gjk_rel64 : d.gjk_rel};
   CInfo<T> ci;
   if constexpr (sizeof(T) == 4 && SV && WARM) {
-    if (e != ~0u) {
-      const uint64_t KN = (uint64_t)d.K * n;
-      const uint32_t cur = *d.ws_par;
-      const uint32_t wj = d.sidx[sj];
-      const WarmLookup wl{d.ws + (uint64_t)(1u - cur) * KN, d.ws_nb + (uint64_t)(1u - cur) * n, d.sidx[si], wj,
-                          e - d.entry_off[si]};
-      V3<T> dw = {T(0), T(0), T(0)};
-      ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, wl, &dw);
-      // every decided entry writes its record (a zero direction when GJK
-      // did not run), so an entry never holds a record of an earlier step
-      if (!st.deferred()) d.ws[(uint64_t)cur * KN + e] = make_float4(dw.x, dw.y, dw.z, __uint_as_float(wj));
-      if (dir) *dir = dw;
-    } else {
-      ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, NoWarm(),
-                                               dir);
-    }
+    float4* rec = d.ws + (uint64_t)(*d.ws_par) * ((uint64_t)d.K * n) + e;
+    V3<T> dw = {T(0), T(0), T(0)};
+    ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, WarmLookup{rec},
+                                             &dw);
+    // every decided entry writes its record (a zero direction when GJK did
+    // not run), so an entry never holds a record of an earlier step
+    if (!st.deferred()) *rec = make_float4(dw.x, dw.y, dw.z, __uint_as_float(d.sidx[sj]));
+    if (dir) *dir = dw;
   } else {
     ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, NoWarm(), dir);
   }
-  uint32_t flag = (st.gjk() ? kFlagGjk : 0u) | (st.deep() ? kFlagDeep : 0u);
+  uint32_t flag = kFlagCand | (st.gjk() ? kFlagGjk : 0u) | (st.deep() ? kFlagDeep : 0u);
   if constexpr (SCREEN) return flag;  // decided pairs have no contact
   if (ci.overlap < T(0)) {
-    flag |= kFlagContact;
+    flag |= kFlagContact | slot_bits(g, xi, V3<double>{pj.x, pj.y, pj.z});
     contact_force<T, R>(d, g, d.sidx[si], d.sidx[sj], A.material, B.material, A.mass, B.mass, xi, a2w.o, b2w.o, ci,
                         out);
   }
   return flag;
 }
 
-// One lane per candidate entry, grid-stride.  SV: physics semantics
-// (signed-volume GJK); !SV: REF_QUIRKS.
+// The step's first kernel, block 0: latch whether the step runs (the lists
+// hold) and whether it is the run's last, and clear the integration's queues.
+__device__ __forceinline__ bool step_begin(const DevScene& d) {
+  const bool run = d.nl[kNlValid] != 0u;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    d.nl[kNlRun] = run ? 1u : 0u;
+    d.nl[kNlLast] = d.nl[kNlDone] + 1u == d.nl[kNlTarget] ? 1u : 0u;
+    d.obs_count[0] = d.obs_count[1] = d.obs_count[2] = 0u;  // [1]: pend_count, [2]: obs_count2
+  }
+  return run;
+}
+// The last kernel of the step that every step launches once, one thread: the
+// step is taken; the narrow phase's queues (no kernel reads them any more).
+__device__ __forceinline__ void step_end(const DevScene& d) {
+  if (blockIdx.x || threadIdx.x) return;
+  d.nl[kNlDone] += 1u;
+  if (d.nl[kNlValid] == 2u) d.nl[kNlValid] = 0u;  // lists for one step
+  *d.refine_count = 0u;
+  *d.queue_next = 0u;
+#pragma unroll
+  for (uint32_t q = 0; q < kDeferQueues; ++q) d.defer_count[16 * q] = 0u;
+}
+
+// The screen's undecided entries: collected per wave in LDS, appended to the
+// block's queue 64 or more at a time and at the end.  Called by whole waves;
+// cnt is wave-uniform.
+struct DeferLds {
+  uint32_t buf[kBlock / 64][128];
+  uint32_t cnt[kBlock / 64];
+  uint32_t base;
+};
+__device__ __forceinline__ void defer_push(const DevScene& d, DeferLds& L, uint32_t& cnt, bool pred, uint32_t e) {
+  const uint64_t m = __ballot(pred);
+  if (!m) return;
+  const uint32_t lane = __lane_id(), wv = threadIdx.x / 64;
+  if (pred) L.buf[wv][cnt + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = e;
+  cnt += (uint32_t)__popcll(m);
+  if (cnt < 64) return;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the wave's LDS writes are done
+  const uint32_t q = blockIdx.x % kDeferQueues;
+  uint32_t base = 0;
+  if (lane == 0) base = atomicAdd(&d.defer_count[16 * q], cnt);
+  base = __shfl(base, 0);
+  uint32_t* list = d.defer_list + (uint64_t)q * d.defer_cap + base;
+  for (uint32_t k = lane; k < cnt; k += 64) list[k] = L.buf[wv][k];
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // read before the buffer is refilled
+  cnt = 0;
+}
+__device__ __forceinline__ void defer_flush(const DevScene& d, DeferLds& L, uint32_t cnt) {  // the whole block
+  const uint32_t lane = __lane_id(), wv = threadIdx.x / 64, nw = blockDim.x / 64;
+  if (lane == 0) L.cnt[wv] = cnt;
+  __syncthreads();
+  uint32_t off = 0, tot = 0;
+  for (uint32_t w = 0; w < nw; ++w) {
+    if (w < wv) off += L.cnt[w];
+    tot += L.cnt[w];
+  }
+  const uint32_t q = blockIdx.x % kDeferQueues;
+  if (threadIdx.x == 0 && tot) L.base = atomicAdd(&d.defer_count[16 * q], tot);
+  __syncthreads();
+  if (!tot) return;
+  uint32_t* list = d.defer_list + (uint64_t)q * d.defer_cap + L.base + off;
+  for (uint32_t k = lane; k < cnt; k += 64) list[k] = L.buf[wv][k];
+}
+
+// One lane per list entry, grid-stride.  SV: physics semantics (signed-volume
+// GJK); !SV: REF_QUIRKS.
 // PASS 0: every entry, complete.  With two passes (physics semantics):
-// PASS 2 screens every entry -- bounding sphere, OBB and GJK's first support
-// pair decide most pairs of a resting or loose packing (no contact) with a
-// small kernel -- and queues the rest; PASS 1 runs the queued entries, packed
-// lane-dense, complete.  A wave costs as much as its slowest lane, so the
-// long searches are kept together and the screen's waves stay short.  The
-// queued searches start from scratch with the same arithmetic: results equal
-// those of PASS 0 bit for bit.
-// The screen queues into one segment per block (an LDS counter, no global
-// atomic: a single queue counter would serialise one atomic per wave); the
-// segments are copied into one list at the offsets of an exclusive scan of
-// their counts (launch_defer_flatten), which PASS 1 reads in order.
+// PASS 2 screens every entry -- prefilter, bounding sphere, OBB and GJK's
+// first support pair decide most pairs of a resting or loose packing (no
+// contact) with a small kernel -- and queues the rest; PASS 1 runs the queued
+// entries, packed lane-dense, complete.  A wave costs as much as its slowest
+// lane, so the long searches are kept together and the screen's waves stay
+// short.  The queued searches start from scratch with the same arithmetic:
+// results equal those of PASS 0 bit for bit.
 // WARM: FP32 searches start from the pair's previous direction (d.warm).
 // PAIR (PASS 1, physics semantics): two lanes per queued entry, sharing its
 // support evaluations (pair_force<PAIR>): the queue is short on beds, and
@@ -200,77 +275,94 @@ __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, u
 template <class T, bool SV, int PASS, bool WARM = false, bool PAIR = false>
 __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
   constexpr bool screen = SV && PASS == 2;
-  __shared__ uint32_t seg_n;
-  uint32_t* seg = d.defer_list + (uint64_t)blockIdx.x * d.defer_cap;
-  if constexpr (screen) {
-    if (threadIdx.x == 0) seg_n = 0;
-    __syncthreads();
+  constexpr bool first = PASS != 1;  // the step's first kernel
+  if constexpr (first) {
+    if (!step_begin(d)) return;
   }
+  __shared__ std::conditional_t<screen, DeferLds, char> L;
+  uint32_t nq = 0;  // the wave's entries in L.buf
   PairRes<T>* res = (PairRes<T>*)d.pair_res;
-  const uint32_t E = PASS == 1 ? d.defer_off[gridDim.x] : d.entry_off[d.n];
+  const uint32_t E = PASS == 1 ? defer_total(d) : d.entry_off[d.n];
   if constexpr (PASS == 1) {
     const bool paired = SV && (uint64_t)E * 2 <= (uint64_t)gridDim.x * blockDim.x;
     if (paired != PAIR) return;
   }
-  constexpr uint32_t L = PAIR ? 2u : 1u;  // lanes per entry
-  uint32_t c_gjk = 0, c_it = 0, c_deep = 0, c_ref = 0, c_bk = 0, c_maxit = 0, c_near = 0;
+  constexpr uint32_t L2 = PAIR ? 2u : 1u;  // lanes per entry
+  uint32_t c_cand = 0, c_def = 0, c_gjk = 0, c_it = 0, c_deep = 0, c_ref = 0, c_bk = 0, c_maxit = 0, c_near = 0;
   const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x / L;
-  const bool lead = gid % L == 0;  // the lane that stores the entry's results
-  for (uint64_t k = gid / L; k < E; k += stride) {
-    uint32_t e = (uint32_t)k;
-    if constexpr (PASS == 1) e = d.defer_flat[k];
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x / L2;
+  const bool lead = gid % L2 == 0;  // the lane that stores the entry's results
+  const uint32_t lane = __lane_id();
+  // whole waves take turns (the queue appends are wave-wide)
+  for (uint64_t kw = (gid - lane) / L2; kw < E; kw += stride) {
+    const uint64_t k = kw + lane / L2;
+    const bool in = k < E;
+    uint32_t e = 0, flag = 0;
     NpStats st = {0u, 0};
-    PairRes<T> r;
-    V3<T> dir = {T(0), T(0), T(0)};
-    uint32_t flag = pair_force<T, T, SV, screen, WARM, PAIR>(d, d.pair_i[e], d.pair_j[e], r, st, e,
+    bool refine = false;
+    if (in) {
+      e = PASS == 1 ? defer_entry(d, (uint32_t)k) : (uint32_t)k;
+      PairRes<T> r;
+      V3<T> dir = {T(0), T(0), T(0)};
+      flag = pair_force<T, T, SV, screen, WARM, PAIR, first>(d, d.pair_i[e], d.pair_j[e], r, st, e,
                                                               sizeof(T) == 4 && SV ? &dir : nullptr);
-    if constexpr (screen) {
-      block_append(seg, &seg_n, st.deferred() != 0, e);
-      if (st.deferred()) d.pend[d.pair_i[e]] = d.pend[d.pair_j[e]] = 1u;
-    }
-    // FP32-mixed: re-run in FP64 when the search ended on rounding instead
-    // of the gap test, the cores overlap (the contact normal switches to the
-    // centre line there), the contact decision lay within FP32's rounding
-    // band (its FP64 decision may differ), or (GRAINS_FP64_CONTACTS) the
-    // pair is in contact
-    const bool refine = sizeof(T) == 4 && !st.deferred() &&
-                        (st.backup() || st.deep() || st.near() ||
-                         ((d.flags & GRAINS_FP64_CONTACTS) && (flag & kFlagContact)));
-    if (!st.deferred() && lead) {
-      if (refine) {
-        // the FP64 re-run replaces this entry's result: its slot carries the
-        // direction the FP32 search ended on, the re-run's first direction
-        if (d.res64) {
-          PairRes<double> q = {{(double)dir.x, (double)dir.y, (double)dir.z}, {0.0, 0.0, 0.0}};
-          ((PairRes<double>*)d.pair_res)[e] = q;
-        } else {
-          PairRes<T> q;
-          q.f[0] = dir.x, q.f[1] = dir.y, q.f[2] = dir.z;
-          q.m[0] = q.m[1] = q.m[2] = T(0);
-          res[e] = q;
+      if constexpr (first) {
+        c_cand += (flag & kFlagCand) != 0;
+        if constexpr (WARM) {
+          // a pair that left the prefilter's reach forgets its direction
+          if (!flag && (d.pair_flag[e] & kFlagCand))
+            d.ws[(uint64_t)(*d.ws_par) * ((uint64_t)d.K * d.n) + e] =
+                make_float4(0.f, 0.f, 0.f, __uint_as_float(d.sidx[d.pair_j[e]]));
         }
-        flag |= kFlagRefine;
-      } else if (flag & kFlagContact) {
-        // (FP32-mixed with FP64 contact geometry refines every contact)
-        res[e] = r;
       }
-      d.pair_flag[e] = flag;
-      c_gjk += st.gjk();
-      c_it += st.iters;
-      c_maxit = c_maxit > (uint32_t)st.iters ? c_maxit : (uint32_t)st.iters;
-      c_deep += st.deep();
-      c_bk += st.backup();
-      c_ref += refine;
-      c_near += st.near();
+      // FP32-mixed: re-run in FP64 when the search ended on rounding instead
+      // of the gap test, the cores overlap (the contact normal switches to the
+      // centre line there), the contact decision lay within FP32's rounding
+      // band (its FP64 decision may differ), or (GRAINS_FP64_CONTACTS) the
+      // pair is in contact
+      refine = sizeof(T) == 4 && !st.deferred() &&
+               (st.backup() || st.deep() || st.near() ||
+                ((d.flags & GRAINS_FP64_CONTACTS) && (flag & kFlagContact)));
+      if (!st.deferred() && lead) {
+        if (refine) {
+          // the FP64 re-run replaces this entry's result: its slot carries the
+          // direction the FP32 search ended on, the re-run's first direction
+          if (d.res64) {
+            PairRes<double> q = {{(double)dir.x, (double)dir.y, (double)dir.z}, {0.0, 0.0, 0.0}};
+            ((PairRes<double>*)d.pair_res)[e] = q;
+          } else {
+            PairRes<T> q;
+            q.f[0] = dir.x, q.f[1] = dir.y, q.f[2] = dir.z;
+            q.m[0] = q.m[1] = q.m[2] = T(0);
+            res[e] = q;
+          }
+          flag |= kFlagRefine;
+        } else if (flag & kFlagContact) {
+          // (FP32-mixed with FP64 contact geometry refines every contact)
+          res[e] = r;
+        }
+        d.pair_flag[e] = flag;
+        c_gjk += st.gjk();
+        c_it += st.iters;
+        c_maxit = c_maxit > (uint32_t)st.iters ? c_maxit : (uint32_t)st.iters;
+        c_deep += st.deep();
+        c_bk += st.backup();
+        c_ref += refine;
+        c_near += st.near();
+      }
+    }
+    if constexpr (screen) {
+      defer_push(d, L, nq, st.deferred() != 0, e);
+      c_def += st.deferred();
+      if (st.deferred()) d.pend[d.pair_i[e]] = d.pend[d.pair_j[e]] = 1u;
     }
     if constexpr (sizeof(T) == 4 && !screen) wave_append(d.refine_list, d.refine_count, refine && lead, e);
   }
   if constexpr (screen) {
-    __syncthreads();
-    if (threadIdx.x == 0) d.defer_count[blockIdx.x] = seg_n;
-    count_add(d.counters, kCntDeferred, threadIdx.x == 0 ? seg_n : 0u);  // every lane: a wave reduction
+    defer_flush(d, L, nq);
+    count_add(d.counters, kCntDeferred, c_def);
   }
+  if constexpr (first) count_add(d.counters, kCntCandidates, c_cand);
   count_add(d.counters, kCntGjk, c_gjk);
   count_add(d.counters, kCntGjkIters, c_it);
   count_add(d.counters, kCntDeep, c_deep);
@@ -353,7 +445,17 @@ __device__ __forceinline__ bool obstacle_in_reach(const DevScene& d, const SimGr
 }
 
 struct IntegCounts {
-  uint32_t walls = 0, contacts = 0, gjk = 0, iters = 0, deep = 0, nonfinite = 0;
+  uint32_t walls = 0, contacts = 0, gjk = 0, iters = 0, deep = 0, nonfinite = 0, outside = 0, max_cand = 0;
+  __device__ __forceinline__ void add(const IntegCounts& c) {
+    walls += c.walls;
+    contacts += c.contacts;
+    gjk += c.gjk;
+    iters += c.iters;
+    deep += c.deep;
+    nonfinite += c.nonfinite;
+    outside += c.outside;
+    max_cand = max(max_cand, c.max_cand);
+  }
 };
 
 // One particle's step from its sorted position s: sum its entries in visit
@@ -369,28 +471,66 @@ __device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i
   const uint32_t e0 = d.entry_off[s], e1 = d.entry_off[s + 1];
   V3<double> F = {0.0, 0.0, 0.0}, M = {0.0, 0.0, 0.0};
   int32_t ncon = 0;
-  // in entry order; four flags loaded together (one load latency per four)
+  uint32_t ncand = 0;
+  auto add = [&](uint32_t e) {
+    if (sizeof(T) == 4 && d.res64) {
+      const PairRes<double> r = res64[e];
+      F = F + V3<double>{r.f[0], r.f[1], r.f[2]};
+      M = M + V3<double>{r.m[0], r.m[1], r.m[2]};
+    } else {
+      const PairRes<T> r = res[e];
+      F = F + V3<double>{(double)r.f[0], (double)r.f[1], (double)r.f[2]};
+      M = M + V3<double>{(double)r.m[0], (double)r.m[1], (double)r.m[2]};
+    }
+  };
+  auto order = [&](uint32_t fl, uint32_t e) {  // (slot, id) in the visit order
+    return ((uint64_t)((fl >> kFlagSlot) & 31u) << 32) | d.sidx[d.pair_j[e]];
+  };
+  // The contacts, summed in the reference's visit order.  The list stands in
+  // the visit order of the positions it was built from; particles that have
+  // changed cell since can leave contacts out of order, and then the sum is
+  // taken again in order (two contacts sum the same either way).
+  bool sorted = true;
+  uint32_t last_fl = 0, last_e = 0;
+  // four flags loaded together (one load latency per four)
   for (uint32_t e = e0; e < e1; e += 4) {
     uint32_t fl[4];
 #pragma unroll
     for (uint32_t u = 0; u < 4; ++u) fl[u] = e + u < e1 ? d.pair_flag[e + u] : 0u;
 #pragma unroll
-    for (uint32_t u = 0; u < 4; ++u)
+    for (uint32_t u = 0; u < 4; ++u) {
+      ncand += (fl[u] & kFlagCand) != 0;
       if (fl[u] & kFlagContact) {
-        if (sizeof(T) == 4 && d.res64) {
-          const PairRes<double> r = res64[e + u];
-          F = F + V3<double>{r.f[0], r.f[1], r.f[2]};
-          M = M + V3<double>{r.m[0], r.m[1], r.m[2]};
-        } else {
-          const PairRes<T> r = res[e + u];
-          F = F + V3<double>{(double)r.f[0], (double)r.f[1], (double)r.f[2]};
-          M = M + V3<double>{(double)r.m[0], (double)r.m[1], (double)r.m[2]};
+        add(e + u);
+        if (ncon) {
+          const uint32_t a = last_fl >> kFlagSlot, b = fl[u] >> kFlagSlot;
+          sorted &= a < b || (a == b && order(last_fl, last_e) < order(fl[u], e + u));
         }
+        last_fl = fl[u];
+        last_e = e + u;
         ++ncon;
       }
+    }
+  }
+  if (!sorted && ncon > 2) {
+    F = M = {0.0, 0.0, 0.0};
+    uint64_t done = 0;
+    for (int32_t k = 0; k < ncon; ++k) {
+      uint64_t best = ~0ull;
+      uint32_t be = e0;
+      for (uint32_t e = e0; e < e1; ++e) {
+        const uint32_t fl = d.pair_flag[e];
+        if (!(fl & kFlagContact)) continue;
+        const uint64_t o = order(fl, e);
+        if ((k == 0 || o > done) && o < best) best = o, be = e;
+      }
+      add(be);
+      done = best;
+    }
   }
   const uint32_t si = d.shape[i];
-  const SimGrid& g = d.grids[d.sim[i]];
+  const uint32_t sim = d.sim[i];
+  const SimGrid& g = d.grids[sim];
   const V3<double> xi = load3(d.pos, n, i);
   const Qt<double> qi = load_quat(d.quat, n, i);
   const V3<double> vel = load3(d.vel, n, i);
@@ -427,10 +567,22 @@ __device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i
   // addExternalForces (ComponentManagerCPU.cpp:448-460)
   const ShapeDyn dy = d.dyn[si];
   F = F + dy.mass * V3<double>{g.g[0], g.g[1], g.g[2]};
-  store3(d.last_force, n, i, F);
-  store3(d.last_torque, n, i, M);
-  d.contact_count[i] += ncon;
+  if (d.nl[kNlLast] || d.keep_torce) {  // only the run's last step can be asked for
+    store3(d.last_force, n, i, F);
+    store3(d.last_torque, n, i, M);
+  }
+  if (ncon) d.contact_count[i] += ncon;
   c.contacts = (uint32_t)ncon;
+  c.max_cand = ncand;
+  // the reference's cell of the step's positions, and whether the centre
+  // lies in its grid (the keys and counts a caller can ask for)
+  {
+    const double p[3] = {xi.x, xi.y, xi.z};
+    uint32_t cc[3];
+    cell_of(g, p, cc);
+    d.key[i] = cell_key(g, cc);
+    c.outside = p[0] < g.lo[0] || p[0] > g.hi[0] || p[1] < g.lo[1] || p[1] > g.hi[1] || p[2] < g.lo[2] || p[2] > g.hi[2];
+  }
   V3<double> x = xi, vnew = vel, onew = om;
   Qt<double> qn = qi;
   if constexpr (!SO) {
@@ -454,6 +606,26 @@ __device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i
     };
     x = {wrap(x.x, 0), wrap(x.y, 1), wrap(x.z, 2)};
   }
+  // the pose record in list order; the lists hold while every particle is
+  // within half the skin of where they were built, inside its periodic sides
+  PoseRec pr;
+  pr.x = x.x, pr.y = x.y, pr.z = x.z;
+  pr.qx = qn.x, pr.qy = qn.y, pr.qz = qn.z, pr.qw = qn.w;
+  pr.shape = si;
+  pr.sim = sim;
+  d.pk[s] = pr;
+  if (d.skin) {
+    const double4 b = d.bp[s];
+    V3<double> mv = {x.x - b.x, x.y - b.y, x.z - b.z};
+    if (g.periodic) mv = min_image(g, mv);
+    bool out = mv.x * mv.x + mv.y * mv.y + mv.z * mv.z > g.move2;
+    if (g.periodic) {
+      const double p[3] = {x.x, x.y, x.z};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) out |= ((g.periodic >> k) & 1) && (p[k] < g.lo[k] || p[k] >= g.hi[k]);
+    }
+    if (out) d.nl[kNlValid] = 0u;
+  }
   store3(d.pos, n, i, x);
   store3(d.vel, n, i, vnew);
   store3(d.omega, n, i, onew);
@@ -472,6 +644,8 @@ __device__ __forceinline__ void integrate_counts(const DevScene& d, const IntegC
   count_add(d.counters, kCntWall, c.walls);
   // contacts are counted after any FP64 re-run has settled each entry
   count_add(d.counters, kCntContacts, c.contacts);
+  count_add(d.counters, kCntOod, c.outside);
+  count_max(d.counters, kCntMaxCand, c.max_cand);
   if (gen) {
     count_add(d.counters, kCntGjk, c.gjk);
     count_add(d.counters, kCntGjkIters, c.iters);
@@ -484,7 +658,6 @@ __device__ __forceinline__ void integrate_counts(const DevScene& d, const IntegC
 template <class T, bool SO>
 __device__ __forceinline__ bool integrate_or_queue(const DevScene& d, uint32_t i, uint32_t s, IntegCounts& c) {
   const uint64_t n = d.n;
-  if (d.warm) d.ws_nb[(uint64_t)(*d.ws_par) * n + i] = make_uint2(d.entry_off[s], d.entry_off[s + 1] - d.entry_off[s]);
   const SimGrid& g = d.grids[d.sim[i]];
   const bool queue =
       g.obs_end > g.obs_begin && obstacle_in_reach(d, g, d.np64[d.shape[i]].rc_max, load3(d.pos, n, i));
@@ -499,13 +672,17 @@ __device__ __forceinline__ bool integrate_or_queue(const DevScene& d, uint32_t i
 // (d.pend) is queued in pend_list for k_integrate_pend instead.
 template <class T, bool SO, bool SPLIT = false>
 __global__ void __launch_bounds__(kBlock) k_integrate(DevScene d) {
+  if (!d.nl[kNlRun]) return;
+  if (!SPLIT) step_end(d);
   const uint64_t n = d.n;
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   IntegCounts c;
   bool queue = false, later = false;
   if (i < n) {
     const uint32_t s = d.rank[i];
-    later = SPLIT && d.pend[s];
+    const bool marked = d.pend[s] != 0u;
+    if (!SPLIT && marked) d.pend[s] = 0u;
+    later = SPLIT && marked;
     if (!later) queue = integrate_or_queue<T, SO>(d, (uint32_t)i, s, c);
   }
   if (SPLIT) wave_append(d.pend_list, d.pend_count, later, (uint32_t)i);
@@ -518,6 +695,8 @@ __global__ void __launch_bounds__(kBlock) k_integrate(DevScene d) {
 // a wave takes the same number of turns (the queue appends are wave-wide).
 template <class T, bool SO>
 __global__ void __launch_bounds__(kBlock) k_integrate_pend(DevScene d) {
+  if (!d.nl[kNlRun]) return;
+  step_end(d);
   const uint32_t cnt = *d.pend_count;
   IntegCounts tot;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -527,11 +706,11 @@ __global__ void __launch_bounds__(kBlock) k_integrate_pend(DevScene d) {
     uint32_t i = 0;
     if (k < cnt) {
       i = d.pend_list[k];
+      const uint32_t s = d.rank[i];
+      d.pend[s] = 0u;
       IntegCounts c;
-      queue = integrate_or_queue<T, SO>(d, i, d.rank[i], c);
-      tot.walls += c.walls;
-      tot.contacts += c.contacts;
-      tot.nonfinite += c.nonfinite;
+      queue = integrate_or_queue<T, SO>(d, i, s, c);
+      tot.add(c);
     }
     if (d.nobs) wave_append(d.obs_list2, d.obs_count2, queue, i);
   }
@@ -545,6 +724,7 @@ __global__ void __launch_bounds__(kBlock) k_integrate_pend(DevScene d) {
 template <class T, bool GEN, bool SO>
 __global__ void __launch_bounds__(kBlock) k_integrate_obs(DevScene d, const uint32_t* __restrict__ list,
                                                          const uint32_t* __restrict__ count) {
+  if (!d.nl[kNlRun]) return;
   const uint32_t cnt = *count;
   IntegCounts tot;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -552,12 +732,7 @@ __global__ void __launch_bounds__(kBlock) k_integrate_obs(DevScene d, const uint
     const uint32_t i = list[k];
     IntegCounts c;
     integrate_particle<T, true, GEN, SO>(d, i, d.rank[i], c);
-    tot.walls += c.walls;
-    tot.contacts += c.contacts;
-    tot.gjk += c.gjk;
-    tot.iters += c.iters;
-    tot.deep += c.deep;
-    tot.nonfinite += c.nonfinite;
+    tot.add(c);
   }
   integrate_counts(d, tot, GEN);
 }

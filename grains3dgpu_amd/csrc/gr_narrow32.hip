@@ -23,7 +23,6 @@ void launch_narrow32(const DevScene& d, int pass, hipStream_t s) {
     else
       hipLaunchKernelGGL((k_narrow<float, false, 0>), grid, block, 0, s, d);
   } else if (two) {
-    launch_defer_flatten(d, s);
     // the queue's paired and single forms: one of them runs
     if (warm) {
       hipLaunchKernelGGL((k_narrow<float, true, 1, true, true>), grid, block, 0, s, d);

@@ -18,7 +18,7 @@ __global__ void __launch_bounds__(kBlock) k_refine64_ref(DevScene d) {
     const uint32_t e = d.refine_list[k];
     NpStats st = {0u, 0};
     PairRes<double> r;
-    const uint32_t flag = pair_force<double, double, false>(d, d.pair_i[e], d.pair_j[e], r, st);
+    const uint32_t flag = pair_force<double, double, false>(d, d.pair_i[e], d.pair_j[e], r, st, e);
     if (flag & kFlagContact) {
       if (d.res64) {
         ((PairRes<double>*)d.pair_res)[e] = r;
@@ -57,7 +57,6 @@ void launch_narrow64(const DevScene& d, int pass, hipStream_t s) {
     else
       hipLaunchKernelGGL((k_narrow<double, false, 0>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
   } else if (two) {
-    launch_defer_flatten(d, s);
     launch_search64<0>(d, s);
   }
 }

@@ -353,11 +353,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   constexpr uint32_t NE = 64 / L;           // entries a wave holds
   constexpr int NP = L == 1 ? 9 : 6;        // doubles per simplex point: y, own (L = 4: the lane's body's; 1: both)
   __shared__ double pts[4][NP][64];
-  const uint32_t E = MODE == 0 ? d.defer_off[d.narrow_blocks] : *d.refine_count;
+  const uint32_t E = MODE == 0 ? defer_total(d) : *d.refine_count;
   if ((E <= kSearchQuad) != (L == 4)) return;
   const uint32_t W = gridDim.x, w = blockIdx.x;  // one wave per block
   if (w >= E) return;
-  const uint32_t* list = MODE == 0 ? d.defer_flat : d.refine_list;
   const uint32_t lane = threadIdx.x, slot = lane / L;
   const bool odd = L == 4 && (lane & 2u);  // L = 4: the lane's body is B
   const bool lead = lane % L == 0;
@@ -411,9 +410,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         pair_frames<T>(g, xi, Qt<T>{pi.qx, pi.qy, pi.qz, pi.qw}, V3<T>{pj.x, pj.y, pj.z},
                        Qt<T>{pj.qx, pj.qy, pj.qz, pj.qw}, a2w, b2w);
         CInfo<T> ci = no_contact<T>();
-        uint32_t flag = 0;
+        uint32_t flag = kFlagCand;
         if (gjk) {
-          flag = kFlagGjk;
+          flag |= kFlagGjk;
           const T ctSum = A.crust + B.crust;
           const bool deep = inside || dist <= Eps<T>::HIGH;
           const T inv = T(1) / sc;
@@ -456,7 +455,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
           ci = cp_spheres(A.rc, B.rc, a2w, b2w);
         }
         if (ci.overlap < T(0)) {
-          flag |= kFlagContact;
+          flag |= kFlagContact | slot_bits(g, xi, V3<T>{pj.x, pj.y, pj.z});
           PairRes<T> r;
           contact_force<T, T>(d, g, d.sidx[si], d.sidx[sj], A.material, B.material, A.mass, B.mass, xi, a2w.o,
                               b2w.o, ci, r);
@@ -498,7 +497,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         }
       }
       if (k < E) {
-        e = list[k];
+        e = MODE == 0 ? defer_entry(d, k) : d.refine_list[k];
         active = true;
         const uint32_t si = d.pair_i[e], sj = d.pair_j[e];
         const PoseRec pi = d.pk[si], pj = d.pk[sj];

@@ -1,0 +1,119 @@
+"""Neighbour lists kept over several steps.  A run that keeps its lists equals
+one whose lists are built anew for every step (the state set between steps:
+positions and orientations unchanged, so the next step starts from the same
+bits), bit for bit: state, forces, contact counts, cell keys, pair lists and
+counters."""
+import numpy as np
+import pytest
+
+from grains3dgpu_amd import _abi as A
+from grains3dgpu_amd import scene as S
+from tests.scenes import bimodal_spheres, dense_cylinders_cones, dense_spheres, dense_superquadrics
+
+pytestmark = pytest.mark.gpu
+
+
+def two_beds():
+    a = dense_spheres(n=300, seed=3, vel=4.0, periodic=0b011)
+    b = dense_spheres(n=500, seed=4, vel=0.5, periodic=0)
+    n = len(a.pos)
+    return S.Scene(shapes=a.shapes, tables=a.tables, n_materials=1, sims=[a.sims[0], b.sims[0]],
+                   particle_shape=np.r_[a.particle_shape, b.particle_shape],
+                   particle_sim=np.r_[np.zeros(n, np.uint32), np.ones(len(b.pos), np.uint32)],
+                   pos=np.r_[a.pos, b.pos], quat=np.r_[a.quat, b.quat], vel=np.r_[a.vel, b.vel],
+                   omega=np.r_[a.omega, b.omega], dt=1e-6)
+
+
+def small_cells():
+    # cells of 0.7 of the largest diameter: pairs in reach but not in
+    # neighbouring cells are no candidates
+    sc = dense_spheres(n=600, seed=5, vel=6.0)
+    sc.sims[0]["cell_size"] = 0.7e-3
+    return sc
+
+
+def outside():
+    # centres beyond periodic and open sides
+    sc = dense_spheres(n=500, seed=6, vel=3.0, periodic=0b001)
+    sc.pos[::7] += sc.sims[0]["domain_max"][0] * 0.3 * np.random.default_rng(1).uniform(-1, 1, sc.pos[::7].shape)
+    return sc
+
+
+SCENES = {
+    "fast": lambda: dense_spheres(n=700, seed=2, vel=8.0, periodic=0b011),
+    "slow": lambda: dense_spheres(n=400, seed=7, vel=0.01, walls=True),
+    "two_beds": two_beds,
+    "small_cells": small_cells,
+    "wide_cells": lambda: _factor(dense_spheres(n=800, seed=8, vel=5.0), 1.6),
+    "outside": outside,
+    "superquadrics": lambda: dense_superquadrics(n=300, seed=9, vel=4.0),
+    "cylinders": lambda: dense_cylinders_cones(n=300, seed=10, vel=4.0),
+    "bimodal": lambda: bimodal_spheres(n_small=4000),
+    "few_cells": lambda: dense_spheres(n=60, seed=11, vel=3.0, periodic=0b111),  # three or four cells a side
+}
+
+
+def _factor(sc, f):
+    sc.sims[0]["cell_size_factor"] = f
+    return sc
+
+
+def result(e):
+    return [*e.get_state(), *e.get_torce(), e.get_contact_count(), *e.get_cell_keys(),
+            e.get_pairs(A.PAIRS_CANDIDATE), e.get_pairs(A.PAIRS_CONTACT)]
+
+
+@pytest.mark.parametrize("name", SCENES)
+@pytest.mark.parametrize("precision,flags,mode", [(A.FP64, 0, 0), (A.FP32_MIXED, 0, 3), (A.FP64, A.REF_QUIRKS, 2)])
+def test_kept_lists_equal_fresh_ones(name, precision, flags, mode):
+    from grains3dgpu_amd import engine
+    sc = SCENES[name]()
+    steps = 25
+
+    def make():
+        return S.load(engine.Engine(dt=sc.dt, precision=precision, flags=flags, max_neighbors=96,
+                                    gjk_rel_tol=1e-6 if precision == A.FP32_MIXED else 0.0,
+                                    candidate_staging=mode), sc)
+    kept, fresh, graph = make(), make(), make()
+    kept.step(steps)
+    graph.step(steps, graph=True)
+    cand = contacts = outside = 0
+    for k in range(steps):
+        if k:
+            fresh.set_state(*fresh.get_state())
+        fresh.step(1)
+        st = fresh.get_stats()
+        cand, contacts, outside = (cand + st["candidate_pairs"], contacts + st["contacts"],
+                                   outside + st["out_of_domain"])
+    want = result(fresh)
+    for e in (kept, graph):
+        for a, b in zip(result(e), want):
+            np.testing.assert_array_equal(a, b)
+        st = e.get_stats()
+        assert (st["steps"], st["candidate_pairs"], st["contacts"], st["out_of_domain"]) == (steps, cand, contacts,
+                                                                                           outside)
+        # single steps go on from the same lists
+        e.step(1)
+        e.step(2)
+    for a, b in zip(result(kept), result(graph)):
+        np.testing.assert_array_equal(a, b)
+
+
+def test_lists_too_long_with_the_skin():
+    """max_neighbors holds every step's candidates but not the lists with
+    their skin: the run goes on without one and equals one with room; one
+    short of the candidates is an overflow, as before."""
+    from grains3dgpu_amd import engine
+    from grains3dgpu_amd.engine import GrainsError
+    sc = dense_spheres(n=500, seed=12, vel=0.01)
+    full = S.load(engine.Engine(dt=sc.dt, max_neighbors=96), sc)
+    full.step(5)
+    most = full.get_stats()["max_candidates"]
+    tight = S.load(engine.Engine(dt=sc.dt, max_neighbors=most), sc)
+    tight.step(5)
+    for a, b in zip(result(tight), result(full)):
+        np.testing.assert_array_equal(a, b)
+    assert tight.get_stats()["max_candidates"] == most
+    short = S.load(engine.Engine(dt=sc.dt, max_neighbors=most - 1), sc)
+    with pytest.raises(GrainsError, match="max_neighbors"):
+        short.step(5)
