@@ -1248,8 +1248,9 @@ static void enqueue_step(grains_ctx* ctx, bool build) {
   else
     for (int k = 0; k < 5; ++k) mark(ctx);  // the build's phases: nothing
   // the integration split around the narrow phase's second pass: two
-  // passes (physics semantics), the step not profiled phase by phase
-  const bool split = d.overlap && d.split > 0 && !(d.flags & GRAINS_REF_QUIRKS) && !ctx->adj_rec &&
+  // passes (physics semantics), the step not profiled phase by phase; a
+  // small bed's integration is too short to be worth the second stream
+  const bool split = d.overlap && d.n > kWideIntegrate && d.split > 0 && !(d.flags & GRAINS_REF_QUIRKS) && !ctx->adj_rec &&
                      !(ctx->profiling && !ctx->capturing);
   if (d.precision == GRAINS_FP64 && split) {
     launch_narrow64(d, 0, s);

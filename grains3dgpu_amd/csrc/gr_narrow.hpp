@@ -269,11 +269,9 @@ __device__ __forceinline__ void defer_flush(const DevScene& d, DeferLds& L, uint
 // WARM: FP32 searches start from the pair's previous direction (d.warm).
 // PAIR (PASS 1, physics semantics): two lanes per queued entry, sharing its
 // support evaluations (pair_force<PAIR>): the queue is short on beds, and
-// the pass lasts as long as its longest search.  The PAIR launch runs when
-// the grid holds the queue twice over, the other when it does not (each
-// returns at once in the other's case).
+// the pass lasts as long as its longest search (k_complete chooses).
 template <class T, bool SV, int PASS, bool WARM = false, bool PAIR = false>
-__global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
+__device__ __forceinline__ void narrow(const DevScene& d) {
   constexpr bool screen = SV && PASS == 2;
   constexpr bool first = PASS != 1;  // the step's first kernel
   if constexpr (first) {
@@ -283,10 +281,6 @@ __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
   uint32_t nq = 0;  // the wave's entries in L.buf
   PairRes<T>* res = (PairRes<T>*)d.pair_res;
   const uint32_t E = PASS == 1 ? defer_total(d) : d.entry_off[d.n];
-  if constexpr (PASS == 1) {
-    const bool paired = SV && (uint64_t)E * 2 <= (uint64_t)gridDim.x * blockDim.x;
-    if (paired != PAIR) return;
-  }
   constexpr uint32_t L2 = PAIR ? 2u : 1u;  // lanes per entry
   uint32_t c_cand = 0, c_def = 0, c_gjk = 0, c_it = 0, c_deep = 0, c_ref = 0, c_bk = 0, c_maxit = 0, c_near = 0;
   const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -372,6 +366,23 @@ __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
   count_max(d.counters, kCntMaxIters, c_maxit);
 }
 
+template <class T, bool SV, int PASS, bool WARM = false>
+__global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
+  narrow<T, SV, PASS, WARM>(d);
+}
+// The complete pass over the screen's queue: two lanes per entry when the
+// grid holds the queue twice over, else one.  (One launch: the two forms as
+// launches of their own cost a graph node of ~5 us each, and the one with
+// nothing to do had to wait for room beside the integration: 0.13 ms on the
+// bed of 10^6.)
+template <class T, bool WARM>
+__global__ void __launch_bounds__(kBlock) k_complete(DevScene d) {
+  if ((uint64_t)defer_total(d) * 2 <= (uint64_t)gridDim.x * blockDim.x)
+    narrow<T, true, 1, WARM, true>(d);
+  else
+    narrow<T, true, 1, WARM, false>(d);
+}
+
 // Particle x obstacle of any other kind than Rectangle: closestPointsRigidBodies
 // (bounding spheres, OBB, GJK) against the obstacle at rest, with its zero
 // kinematics and mass (ComponentManagerCPU.cpp:301-351), in FP64 for both
@@ -408,22 +419,31 @@ __device__ __forceinline__ void obstacle_contact64(const DevScene& d, uint32_t s
 
 // Particle x Rectangle wall at rest: the plane branch of
 // closestPointsRigidBodies (CollisionDetection.cpp:203-206) and the Hooke
-// force, in FP64; adds to F and M and returns 1 on contact.
-__device__ __forceinline__ uint32_t wall_contact64(const DevScene& d, const ShapeNP<double>& A, uint32_t os,
-                                                   uint32_t table, const Tr<double>& a2w, const Tr<double>& b2w,
-                                                   V3<double> vel, V3<double> om, V3<double>& F, V3<double>& M) {
+// force f and torque m, in FP64; returns whether they touch.  Walls whose plane is
+// farther from the centre than every point of the particle leave the support
+// point on its side: no contact, decided without it.
+__device__ __forceinline__ bool wall_contact64(const DevScene& d, const ShapeNP<double>& A, uint32_t o,
+                                               uint32_t table, V3<double> xi, Qt<double> qi, V3<double> vel,
+                                               V3<double> om, V3<double>& f, V3<double>& m) {
+  const double* t = d.obs_tr + 12 * (size_t)o;
+  const uint32_t os = d.obs_shape[o];
+  Tr<double> a2w, b2w;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) b2w.R.m[k] = t[k];
+  b2w.o = {t[9], t[10], t[11]};
+  const V3<double> rn = {t[2], t[5], t[8]};
+  if (fabs(dot(rn, xi - b2w.o)) > A.rc_max * (1.0 + 1e-9)) return false;
+  a2w.R = rot(qi);
+  a2w.o = xi;
   const CInfo<double> ci = cp_rectangle(sup_ctx(A, false, d.verts64, d.cverts64), a2w, b2w);
-  if (!(ci.overlap < 0.0)) return 0;
+  if (!(ci.overlap < 0.0)) return false;
   const ShapeNP<double> B = d.np64[os];
   const HookeP<double> h = d.hooke64[table + material_hash((uint32_t)A.material, (uint32_t)B.material)];
   // reference lever: the world contact point (Kinematics.cpp:86-91)
   const V3<double> lever = (d.flags & GRAINS_REF_QUIRKS) ? ci.cp : ci.cp - a2w.o;
   const V3<double> relVel = vel + cross(om, lever);
-  V3<double> f, m;
   hooke<double>(h, ci, relVel, om, A.mass, B.mass, ci.cp - a2w.o, f, m);
-  F = F + f;
-  M = M + m;
-  return 1;
+  return true;
 }
 
 // Can particle i (centre xi, every point within rc_max of it) touch an
@@ -458,20 +478,19 @@ struct IntegCounts {
   }
 };
 
-// One particle's step from its sorted position s: sum its entries in visit
-// order, obstacles (OBS; FP64 for both precisions, GEN: some are not
-// Rectangles), gravity, then moveParticles (ComponentManagerCPU.cpp:428-500)
-// on the quaternion state.  SO: a second-order scheme (d.integrator);
-// otherwise FirstOrderExplicit.
-template <class T, bool OBS, bool GEN, bool SO>
-__device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i, uint32_t s, IntegCounts& c) {
-  const uint64_t n = d.n;
+// The contacts of sorted position s, summed in the reference's visit order.
+// The list stands in the visit order of the positions it was built from;
+// particles that have changed cell since can leave contacts out of order, and
+// then the sum is taken again in order (two contacts sum the same either way).
+template <class T>
+__device__ __forceinline__ void sum_contacts(const DevScene& d, uint32_t s, V3<double>& F, V3<double>& M,
+                                             int32_t& ncon, uint32_t& ncand) {
   const PairRes<T>* res = (const PairRes<T>*)d.pair_res;
   const PairRes<double>* res64 = (const PairRes<double>*)d.pair_res;  // d.res64
   const uint32_t e0 = d.entry_off[s], e1 = d.entry_off[s + 1];
-  V3<double> F = {0.0, 0.0, 0.0}, M = {0.0, 0.0, 0.0};
-  int32_t ncon = 0;
-  uint32_t ncand = 0;
+  F = M = {0.0, 0.0, 0.0};
+  ncon = 0;
+  ncand = 0;
   auto add = [&](uint32_t e) {
     if (sizeof(T) == 4 && d.res64) {
       const PairRes<double> r = res64[e];
@@ -486,10 +505,6 @@ __device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i
   auto order = [&](uint32_t fl, uint32_t e) {  // (slot, id) in the visit order
     return ((uint64_t)((fl >> kFlagSlot) & 31u) << 32) | d.sidx[d.pair_j[e]];
   };
-  // The contacts, summed in the reference's visit order.  The list stands in
-  // the visit order of the positions it was built from; particles that have
-  // changed cell since can leave contacts out of order, and then the sum is
-  // taken again in order (two contacts sum the same either way).
   bool sorted = true;
   uint32_t last_fl = 0, last_e = 0;
   // four flags loaded together (one load latency per four)
@@ -528,42 +543,30 @@ __device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i
       done = best;
     }
   }
-  const uint32_t si = d.shape[i];
-  const uint32_t sim = d.sim[i];
+}
+
+// A particle's state at the step's start.
+struct ParticleState {
+  uint32_t si, sim;
+  V3<double> xi, vel, om;
+  Qt<double> qi;
+  __device__ __forceinline__ ParticleState(const DevScene& d, uint64_t i)
+      : si(d.shape[i]), sim(d.sim[i]), xi(load3(d.pos, d.n, i)), vel(load3(d.vel, d.n, i)),
+        om(load3(d.omega, d.n, i)), qi(load_quat(d.quat, d.n, i)) {}
+};
+
+// Gravity, then moveParticles (ComponentManagerCPU.cpp:428-500) on the
+// quaternion state, from the total contact force F and torque M.  SO: a
+// second-order scheme (d.integrator); otherwise FirstOrderExplicit.
+template <bool SO>
+__device__ __forceinline__ void finish_step(const DevScene& d, uint64_t i, uint32_t s, const ParticleState& p0,
+                                            V3<double> F, V3<double> M, int32_t ncon, uint32_t ncand,
+                                            IntegCounts& c) {
+  const uint64_t n = d.n;
+  const uint32_t si = p0.si, sim = p0.sim;
   const SimGrid& g = d.grids[sim];
-  const V3<double> xi = load3(d.pos, n, i);
-  const Qt<double> qi = load_quat(d.quat, n, i);
-  const V3<double> vel = load3(d.vel, n, i);
-  const V3<double> om = load3(d.omega, n, i);
-  // particle x obstacle (ComponentManagerCPU.cpp:301-351)
-  if constexpr (OBS) {
-    const ShapeNP<double> A = d.np64[si];
-    for (uint32_t o = g.obs_begin; o < g.obs_end; ++o) {
-      const double* t = d.obs_tr + 12 * (size_t)o;
-      const uint32_t os = d.obs_shape[o];
-      if constexpr (GEN) {
-        if (d.np64[os].kind != GRAINS_RECTANGLE) {
-          NpStats st = {0u, 0};
-          obstacle_contact64(d, si, os, t, g.table, xi, qi, vel, om, F, M, c.walls, st);
-          c.gjk += st.gjk();
-          c.iters += st.iters;
-          c.deep += st.deep();
-          continue;
-        }
-      }
-      Tr<double> a2w, b2w;
-#pragma unroll
-      for (int k = 0; k < 9; ++k) b2w.R.m[k] = t[k];
-      b2w.o = {t[9], t[10], t[11]};
-      // a centre farther from the plane than every point of the particle
-      // leaves the support point on its side: no contact, decided without it
-      const V3<double> rn = {t[2], t[5], t[8]};
-      if (fabs(dot(rn, xi - b2w.o)) > A.rc_max * (1.0 + 1e-9)) continue;
-      a2w.R = rot(qi);
-      a2w.o = xi;
-      c.walls += wall_contact64(d, A, os, g.table, a2w, b2w, vel, om, F, M);
-    }
-  }
+  const V3<double> xi = p0.xi, vel = p0.vel, om = p0.om;
+  const Qt<double> qi = p0.qi;
   // addExternalForces (ComponentManagerCPU.cpp:448-460)
   const ShapeDyn dy = d.dyn[si];
   F = F + dy.mass * V3<double>{g.g[0], g.g[1], g.g[2]};
@@ -639,6 +642,40 @@ __device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i
   c.nonfinite = !isfinite(all);
 }
 
+// One particle's step from its sorted position s: its contacts, obstacles
+// (OBS: one lane takes them in turn, some not Rectangles; FP64 for both
+// precisions; ComponentManagerCPU.cpp:301-351), gravity and the move.
+template <class T, bool OBS, bool SO>
+__device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i, uint32_t s, IntegCounts& c) {
+  V3<double> F, M;
+  int32_t ncon;
+  uint32_t ncand;
+  sum_contacts<T>(d, s, F, M, ncon, ncand);
+  const ParticleState p(d, i);
+  if constexpr (OBS) {
+    const SimGrid& g = d.grids[p.sim];
+    const ShapeNP<double> A = d.np64[p.si];
+    for (uint32_t o = g.obs_begin; o < g.obs_end; ++o) {
+      const uint32_t os = d.obs_shape[o];
+      if (d.np64[os].kind != GRAINS_RECTANGLE) {
+        NpStats st = {0u, 0};
+        obstacle_contact64(d, p.si, os, d.obs_tr + 12 * (size_t)o, g.table, p.xi, p.qi, p.vel, p.om, F, M, c.walls, st);
+        c.gjk += st.gjk();
+        c.iters += st.iters;
+        c.deep += st.deep();
+      } else {
+        V3<double> f, m;
+        if (wall_contact64(d, A, o, g.table, p.xi, p.qi, p.vel, p.om, f, m)) {
+          F = F + f;
+          M = M + m;
+          ++c.walls;
+        }
+      }
+    }
+  }
+  finish_step<SO>(d, i, s, p, F, M, ncon, ncand, c);
+}
+
 __device__ __forceinline__ void integrate_counts(const DevScene& d, const IntegCounts& c, bool gen) {
   count_add(d.counters, kCntNan, c.nonfinite);
   count_add(d.counters, kCntWall, c.walls);
@@ -661,7 +698,7 @@ __device__ __forceinline__ bool integrate_or_queue(const DevScene& d, uint32_t i
   const SimGrid& g = d.grids[d.sim[i]];
   const bool queue =
       g.obs_end > g.obs_begin && obstacle_in_reach(d, g, d.np64[d.shape[i]].rc_max, load3(d.pos, n, i));
-  if (!queue) integrate_particle<T, false, false, SO>(d, i, s, c);
+  if (!queue) integrate_particle<T, false, SO>(d, i, s, c);
   return queue;
 }
 
@@ -718,10 +755,10 @@ __global__ void __launch_bounds__(kBlock) k_integrate_pend(DevScene d) {
 }
 
 // The particles k_integrate (list obs_list) or k_integrate_pend (obs_list2)
-// queued: the same step with their obstacle contacts (FP64; GEN: some
-// obstacles are not Rectangles).  Grid-stride over the queue, whose length
-// the device holds.
-template <class T, bool GEN, bool SO>
+// queued: the same step with their obstacle contacts (FP64; some obstacles
+// are not Rectangles).  Grid-stride over the queue, whose length the device
+// holds.
+template <class T, bool SO>
 __global__ void __launch_bounds__(kBlock) k_integrate_obs(DevScene d, const uint32_t* __restrict__ list,
                                                          const uint32_t* __restrict__ count) {
   if (!d.nl[kNlRun]) return;
@@ -731,48 +768,98 @@ __global__ void __launch_bounds__(kBlock) k_integrate_obs(DevScene d, const uint
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < cnt; k += stride) {
     const uint32_t i = list[k];
     IntegCounts c;
-    integrate_particle<T, true, GEN, SO>(d, i, d.rank[i], c);
+    integrate_particle<T, true, SO>(d, i, d.rank[i], c);
     tot.add(c);
   }
-  integrate_counts(d, tot, GEN);
+  integrate_counts(d, tot, true);
+}
+
+// The same where every obstacle is a Rectangle, by eight lanes per particle:
+// each takes one wall (a superquadric's support is a chain of seven FP64 pow
+// calls: one lane taking a corner grain's walls in turn held its wave ~25 us),
+// and the contacts are added in the walls' order.
+// ALL: every particle instead of a queue -- a small bed's whole integration
+// in one launch, the step's last (1,000 spheres: 16 + 25 us in two launches -> 18 us;
+// 8,191 touching superquadrics: 22 + 90 us -> 27 us).
+template <class T, bool SO, bool ALL>
+__global__ void __launch_bounds__(kBlock) k_integrate_walls(DevScene d, const uint32_t* __restrict__ list,
+                                                           const uint32_t* __restrict__ count) {
+  if (!d.nl[kNlRun]) return;
+  if (ALL) step_end(d);
+  constexpr uint32_t G = 8;
+  const uint32_t cnt = ALL ? (uint32_t)d.n : *count;
+  const uint32_t lane = __lane_id(), sub = lane % G;
+  IntegCounts tot;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x / G;
+  for (uint64_t k = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; k < cnt; k += stride) {
+    const uint32_t i = ALL ? (uint32_t)k : list[k];
+    const uint32_t s = d.rank[i];
+    V3<double> F, M;
+    int32_t ncon;
+    uint32_t ncand;
+    sum_contacts<T>(d, s, F, M, ncon, ncand);
+    const ParticleState p(d, i);
+    const SimGrid& g = d.grids[p.sim];
+    uint32_t walls = 0;
+    for (uint32_t o0 = g.obs_begin; o0 < g.obs_end; o0 += G) {
+      V3<double> f = {0.0, 0.0, 0.0}, m = f;
+      const bool hit = o0 + sub < g.obs_end &&
+                       wall_contact64(d, d.np64[p.si], o0 + sub, g.table, p.xi, p.qi, p.vel, p.om, f, m);
+      uint32_t hits = (uint32_t)(__ballot(hit) >> (lane - sub)) & ((1u << G) - 1u);
+      for (; hits; hits &= hits - 1) {
+        const int w = (int)(lane - sub) + __ffs(hits) - 1;
+        F = F + V3<double>{__shfl(f.x, w), __shfl(f.y, w), __shfl(f.z, w)};
+        M = M + V3<double>{__shfl(m.x, w), __shfl(m.y, w), __shfl(m.z, w)};
+        ++walls;
+      }
+    }
+    if (sub == 0) {
+      if (ALL && d.pend[s]) d.pend[s] = 0u;
+      IntegCounts c;
+      c.walls = walls;
+      finish_step<SO>(d, i, s, p, F, M, ncon, ncand, c);
+      tot.add(c);
+    }
+  }
+  integrate_counts(d, tot, false);
 }
 
 // The integration launches of one precision (launch_integrate32/64).
 // part 1 (second stream): the particles the screen settled, then their
 // obstacle queue; part 2 (after the join): the marked particles, then
-// theirs; part 0: every particle, then the obstacle queue.
-template <class T>
-inline void launch_integrate_t(const DevScene& d, hipStream_t s, int part) {
-  const dim3 grid((unsigned)((d.n + d.block - 1) / d.block));
-  const bool so = d.integrator != GRAINS_FIRST_ORDER_EXPLICIT;
+// theirs; part 0: every particle (a bed of at most kWideIntegrate by eight
+// lanes each where all obstacles are Rectangles), then the obstacle queue.
+template <class T, bool SO>
+inline void launch_integrate_so(const DevScene& d, hipStream_t s, int part) {
+  const dim3 grid((unsigned)((d.n + d.block - 1) / d.block)), block(d.block);
   // queues are walked grid-stride over their device-held counts
   const dim3 og(std::min<unsigned>(grid.x, (unsigned)cu_count() * 8));
-  if (part == 1) {
-    if (so)
-      hipLaunchKernelGGL((k_integrate<T, true, true>), grid, dim3(d.block), 0, s, d);
-    else
-      hipLaunchKernelGGL((k_integrate<T, false, true>), grid, dim3(d.block), 0, s, d);
-  } else if (part == 2) {
-    if (so)
-      hipLaunchKernelGGL((k_integrate_pend<T, true>), og, dim3(d.block), 0, s, d);
-    else
-      hipLaunchKernelGGL((k_integrate_pend<T, false>), og, dim3(d.block), 0, s, d);
-  } else if (so) {
-    hipLaunchKernelGGL((k_integrate<T, true>), grid, dim3(d.block), 0, s, d);
-  } else {
-    hipLaunchKernelGGL((k_integrate<T, false>), grid, dim3(d.block), 0, s, d);
+  if (part == 0 && d.nobs && !d.gen_obs && d.n <= kWideIntegrate) {
+    hipLaunchKernelGGL((k_integrate_walls<T, SO, true>), dim3((unsigned)((d.n * 8 + kBlock - 1) / kBlock)),
+                       dim3(kBlock), 0, s, d, nullptr, nullptr);
+    return;
   }
+  if (part == 1)
+    hipLaunchKernelGGL((k_integrate<T, SO, true>), grid, block, 0, s, d);
+  else if (part == 2)
+    hipLaunchKernelGGL((k_integrate_pend<T, SO>), og, block, 0, s, d);
+  else
+    hipLaunchKernelGGL((k_integrate<T, SO>), grid, block, 0, s, d);
   if (!d.nobs) return;
   const uint32_t* list = part == 2 ? d.obs_list2 : d.obs_list;
   const uint32_t* count = part == 2 ? d.obs_count2 : d.obs_count;
-  if (d.gen_obs && so)
-    hipLaunchKernelGGL((k_integrate_obs<T, true, true>), og, dim3(d.block), 0, s, d, list, count);
-  else if (d.gen_obs)
-    hipLaunchKernelGGL((k_integrate_obs<T, true, false>), og, dim3(d.block), 0, s, d, list, count);
-  else if (so)
-    hipLaunchKernelGGL((k_integrate_obs<T, false, true>), og, dim3(d.block), 0, s, d, list, count);
+  if (d.gen_obs)
+    hipLaunchKernelGGL((k_integrate_obs<T, SO>), og, block, 0, s, d, list, count);
   else
-    hipLaunchKernelGGL((k_integrate_obs<T, false, false>), og, dim3(d.block), 0, s, d, list, count);
+    hipLaunchKernelGGL((k_integrate_walls<T, SO, false>), dim3((unsigned)cu_count() * 2), dim3(kBlock), 0, s, d, list,
+                       count);
+}
+template <class T>
+inline void launch_integrate_t(const DevScene& d, hipStream_t s, int part) {
+  if (d.integrator != GRAINS_FIRST_ORDER_EXPLICIT)
+    launch_integrate_so<T, true>(d, s, part);
+  else
+    launch_integrate_so<T, false>(d, s, part);
 }
 
 // GrainsTestDev workload: GJK distance of independent pairs of full shapes.

@@ -23,14 +23,10 @@ void launch_narrow32(const DevScene& d, int pass, hipStream_t s) {
     else
       hipLaunchKernelGGL((k_narrow<float, false, 0>), grid, block, 0, s, d);
   } else if (two) {
-    // the queue's paired and single forms: one of them runs
-    if (warm) {
-      hipLaunchKernelGGL((k_narrow<float, true, 1, true, true>), grid, block, 0, s, d);
-      hipLaunchKernelGGL((k_narrow<float, true, 1, true, false>), grid, block, 0, s, d);
-    } else {
-      hipLaunchKernelGGL((k_narrow<float, true, 1, false, true>), grid, block, 0, s, d);
-      hipLaunchKernelGGL((k_narrow<float, true, 1, false, false>), grid, block, 0, s, d);
-    }
+    if (warm)
+      hipLaunchKernelGGL((k_complete<float, true>), grid, block, 0, s, d);
+    else
+      hipLaunchKernelGGL((k_complete<float, false>), grid, block, 0, s, d);
   }
 }
 void launch_integrate32(const DevScene& d, hipStream_t s, int part) { launch_integrate_t<float>(d, s, part); }

@@ -37,13 +37,10 @@ __global__ void __launch_bounds__(kBlock) k_refine64_ref(DevScene d) {
   count_max(d.counters, kCntRefMaxIters, c_maxit);
 }
 
-// One wave per block, two per SIMD (the registers' limit); the queue's length
-// decides on the device which form runs.
+// One wave per block, two per SIMD (the registers' limit).
 template <int MODE>
 static void launch_search64(const DevScene& d, hipStream_t s) {
-  const dim3 grid((unsigned)cu_count() * 8);
-  hipLaunchKernelGGL((k_search64<MODE, 4>), grid, dim3(64), 0, s, d);
-  hipLaunchKernelGGL((k_search64<MODE, 1>), grid, dim3(64), 0, s, d);
+  hipLaunchKernelGGL(k_search64<MODE>, dim3((unsigned)cu_count() * 8), dim3(64), 0, s, d);
 }
 
 void launch_narrow64(const DevScene& d, int pass, hipStream_t s) {

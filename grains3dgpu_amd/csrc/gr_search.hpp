@@ -330,8 +330,7 @@ __device__ __forceinline__ SvBest sv_closest_quad(V3<double> a, V3<double> b, V3
 // body, which take the independent pow calls of a support side by side, one
 // per face of the simplex (L = 4).  Four lanes issue about twice the
 // instructions per entry: the line lies where one lane per entry fills the
-// waves (46,700 entries: 0.56 ms by four; 173,000: 1.10 ms by one).  Both
-// forms are launched; each returns at once when the queue is the other's.
+// waves (46,700 entries: 0.56 ms by four; 173,000: 1.10 ms by one).
 //
 // A lane whose search has ended waits until a quarter of the wave's entries
 // have, then those store their results and take the next entries together
@@ -348,13 +347,11 @@ __device__ __forceinline__ SvBest sv_closest_quad(V3<double> a, V3<double> b, V3
 // 0.128 -> 0.080 ms (both bound by the longest search).
 constexpr uint32_t kSearchQuad = 98304;  // longest queue taken by four lanes per entry
 template <int MODE, int L>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) k_search64(DevScene d) {
+__device__ __forceinline__ void search64(const DevScene& d, const uint32_t E, double (*pts)[9][64]) {
   using T = double;
   constexpr uint32_t NE = 64 / L;           // entries a wave holds
-  constexpr int NP = L == 1 ? 9 : 6;        // doubles per simplex point: y, own (L = 4: the lane's body's; 1: both)
-  __shared__ double pts[4][NP][64];
-  const uint32_t E = MODE == 0 ? defer_total(d) : *d.refine_count;
-  if ((E <= kSearchQuad) != (L == 4)) return;
+  // (doubles per simplex point in LDS: the difference, the lane's body's
+  // point; L = 1: both bodies')
   const uint32_t W = gridDim.x, w = blockIdx.x;  // one wave per block
   if (w >= E) return;
   const uint32_t lane = threadIdx.x, slot = lane / L;
@@ -714,6 +711,16 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     count_add(d.counters, kCntRefIters, c_it);
     count_max(d.counters, kCntRefMaxIters, c_maxit);
   }
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) k_search64(DevScene d) {
+  __shared__ double pts[4][9][64];
+  const uint32_t E = MODE == 0 ? defer_total(d) : *d.refine_count;
+  if (E <= kSearchQuad)
+    search64<MODE, 4>(d, E, pts);
+  else
+    search64<MODE, 1>(d, E, pts);
 }
 
 }  // namespace gr
