@@ -759,21 +759,22 @@ extern "C" int grains_set_particles(grains_ctx_t* ctx, const uint32_t* shape, co
 }
 
 // cell layout, obstacle ranges, shape tables and work buffers
-// One of the screening pass's queues: a block of the persistent narrow launch
-// visits at most ceil(ecap / (blocks * threads)) * threads entries, and every
+// One of the screening pass's queues: the blocks on one of the kXcds dies
+// share ecap / kXcds + 64 entries, in turns of a block's threads, and every
 // kDeferQueues-th block fills the same queue.  For any launch shape the
-// queues together hold at most (blocks + kDeferQueues - 1) (ecap / blocks +
-// threads) words, which defer_words bounds (a launch has at least one block
-// per CU and at most kMaxNarrowPerCu).
+// queues together hold at most (blocks + kDeferQueues - 1) ((ecap + 64 kXcds)
+// / blocks + threads) words, which defer_words bounds (a launch has at least
+// one block per CU and at most kMaxNarrowPerCu).
 static void set_defer_cap(grains_ctx* ctx) {
   DevScene& d = ctx->d;
   const uint64_t per = (uint64_t)d.narrow_blocks * d.block;
-  const uint64_t block_cap = ((d.ecap + per - 1) / per) * d.block;
+  const uint64_t block_cap = ((d.ecap + 64 * kXcds + per - 1) / per) * d.block;
   d.defer_cap = (uint32_t)(block_cap * ((d.narrow_blocks + kDeferQueues - 1) / kDeferQueues));
 }
 static uint64_t defer_words(uint64_t ecap) {
   const uint64_t cus = (uint64_t)cu_count();
-  return ecap + (kDeferQueues - 1) * (ecap / cus + 1) + (cus * kMaxNarrowPerCu + kDeferQueues) * 256;
+  return ecap + (kDeferQueues - 1) * (ecap / cus + 1) + (cus * kMaxNarrowPerCu + kDeferQueues) * 256 +
+         64 * kXcds * kDeferQueues;
 }
 
 static void adj_drop(grains_ctx* ctx) {

@@ -449,7 +449,6 @@ struct GjkOut {
   bool backup;    // Johnson: the backup procedure was taken; signed volumes:
                   // the search ended on rounding or the cap, not the gap test
   bool separated; // signed volumes: the lower bound passed `sep` (no contact)
-  bool deferred;  // screening search: not separated by the first support pair
   V3<T> vdir;     // signed volumes: the search's last direction in A's frame
                   // (the closest-point direction of a converged search)
   bool has_v;     // vdir is a direction (not inside, not degenerate)
@@ -539,7 +538,6 @@ GR_D GjkOut<T> gjk_jh(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
   out.deep = false;
   out.backup = backup;
   out.separated = false;
-  out.deferred = false;
   return out;
 }
 
@@ -716,11 +714,6 @@ constexpr int kNesterovIters = 8;
 // stops with `separated` (INFINITY for a plain distance query).  Contact
 // decisions equal those of the full search, which reports no contact exactly
 // when its distance, an upper bound, is above sep -- implied by mu > sep.
-// SCREEN: stop after the first support pair's separation test; a pair it
-// does not separate returns `deferred` (no result: the full search repeats it
-// from the start).  Everything up to that test is this same code, so the
-// screen separates exactly the pairs the full search separates at its first
-// support pair.
 // warm (optional): a first search direction in A's frame, e.g. the pair's
 // closest-point direction of the previous step.  Its support pair seeds the
 // simplex (v = w, |v| and the lower bound from it); a search whose gap test
@@ -733,7 +726,7 @@ constexpr int kNesterovIters = 8;
 // search is then the same on both lanes, and a search's chain of dependent
 // support evaluations is half as long (the FP64 supports of superquadrics
 // are chains of pow).
-template <class T, bool SCREEN = false, bool PAIR = false>
+template <class T, bool PAIR = false>
 GR_D GjkOut<T> gjk_sv(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, const Tr<T>& b2w,
                       const GjkArgs& args, T rsum, T sep, const V3<T>* warm = nullptr) {
   const bool nesterov = (args.flags & GRAINS_NESTEROV) != 0;
@@ -756,7 +749,6 @@ GR_D GjkOut<T> gjk_sv(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
   T dist = norm(v), mu = T(0);
   V3<T> dir = v, wprev = v, last_d = v;
   bool accel = nesterov, inside = false, ran = false, stalled = false, separated = false, done = false;
-  bool screened = false;
   int num_iter = 0;
   // the support pair in direction d: pl = s_A(-d), ql = s_B(R^T d) (A's frame, scaled)
   auto supports = [&](const V3<T>& d) {
@@ -790,8 +782,6 @@ GR_D GjkOut<T> gjk_sv(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
     if (mu > sep_s) {
       separated = true;
       done = true;
-    } else if (SCREEN) {
-      screened = true;
     } else {
       S.y[0] = w;
       S.p[0] = pl;
@@ -806,7 +796,7 @@ GR_D GjkOut<T> gjk_sv(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
       if (dist - mu <= dist * rel) done = true;
     }
   }
-  while (!done && !screened && dist > Eps<T>::HIGH && num_iter < kGjkMaxIter) {
+  while (!done && dist > Eps<T>::HIGH && num_iter < kGjkMaxIter) {
     V3<T> d = v;
     if (accel && num_iter >= kNesterovIters) accel = false;
     if (accel) {
@@ -828,7 +818,6 @@ GR_D GjkOut<T> gjk_sv(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
       done = true;
       break;
     }
-    if constexpr (SCREEN) break;
     if (dist - mu <= dist * rel) {
       done = true;
       break;
@@ -909,8 +898,7 @@ GR_D GjkOut<T> gjk_sv(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
     dist = nd;
   }
   // the loop ran out of support points (iteration cap)
-  if (!SCREEN && !done && dist > Eps<T>::HIGH) stalled = true;
-  const bool deferred = SCREEN && !separated;
+  if (!done && dist > Eps<T>::HIGH) stalled = true;
   GjkOut<T> out;
   if (n == 0) {
     out.pa = ran ? pl : zero;
@@ -934,7 +922,6 @@ GR_D GjkOut<T> gjk_sv(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
   out.deep = inside || dist <= Eps<T>::HIGH;
   out.backup = stalled;
   out.separated = separated;
-  out.deferred = deferred;
   // the direction to start from next time: the converged closest-point
   // direction, else the last one searched
   out.vdir = (done && !separated && !inside && n > 0 && dist > Eps<T>::HIGH) ? v : last_d;
@@ -1021,9 +1008,6 @@ template <class T> GR_D T near_band(T rsum) {
 // semantics run GJK on the crust cores (the commented intent of lines 231-236).
 // SV selects the physics semantics (signed-volume GJK on the crust cores);
 // !SV is REF_QUIRKS (Johnson's sub-algorithm on the full shapes).
-// SCREEN (physics semantics): decide only the pairs without contact that the
-// bounding sphere, the OBB or GJK's first support pair settle; every other
-// pair returns kNpDeferred for the full pass.
 // warm (physics semantics): asked for a first GJK direction in the world
 // frame only when the pair reaches GJK (fetch returns false: none); dir_w
 // (optional): receives the search's direction in the world frame when GJK
@@ -1033,7 +1017,7 @@ struct NoWarm {
   GR_D bool fetch(V&) const { return false; }
 };
 // PAIR (physics semantics): two lanes per pair, as gjk_sv<PAIR>.
-template <class T, bool SV, bool SCREEN = false, bool PAIR = false, class W = NoWarm>
+template <class T, bool SV, bool PAIR = false, class W = NoWarm>
 GR_D CInfo<T> closest_points(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<T>& a2w,
                              const Tr<T>& b2w, const GjkArgs& args, const T* verts_full,
                              const T* verts_core, NpStats& st, const W& warm = W(),
@@ -1041,10 +1025,6 @@ GR_D CInfo<T> closest_points(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<
   constexpr bool quirks = !SV;
   const T band = near_band(A.rc + B.rc);  // 0 in FP64
   if ((A.kind == GRAINS_SPHERE && B.kind == GRAINS_SPHERE) || B.kind == GRAINS_RECTANGLE) {
-    if constexpr (SCREEN) {
-      st.bits |= kNpDeferred;
-      return no_contact<T>();
-    }
     T margin;
     const CInfo<T> c = B.kind == GRAINS_RECTANGLE
                            ? cp_rectangle(sup_ctx(A, false, verts_full, verts_core), a2w, b2w, &margin)
@@ -1061,16 +1041,12 @@ GR_D CInfo<T> closest_points(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<
   // leave such pairs to the re-run at once.
   const bool sphere_near = band > T(0) && overlap >= T(0) && overlap <= band;
   if (sphere_near && !SV) {
-    if constexpr (SCREEN) st.bits |= kNpDeferred;
-    else st.bits |= kNpNear;
+    st.bits |= kNpNear;
     return no_contact<T>();
   }
   if (overlap < T(0) || sphere_near) {
     if (!obb_intersect(A.bbox, B.bbox, a2w, b2w)) {
-      if (sphere_near) {
-        if constexpr (SCREEN) st.bits |= kNpDeferred;
-        else st.bits |= kNpNear;
-      }
+      if (sphere_near) st.bits |= kNpNear;
       return no_contact<T>();
     }
     {
@@ -1083,17 +1059,13 @@ GR_D CInfo<T> closest_points(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<
         V3<T> warm_w;
         if (warm.fetch(warm_w)) {
           const V3<T> wa = vm(warm_w, a2w.R);  // into A's frame
-          g = gjk_sv<T, SCREEN, PAIR>(ca, cb, a2w, b2w, args, A.rc + B.rc, ctSum + band, &wa);
+          g = gjk_sv<T, PAIR>(ca, cb, a2w, b2w, args, A.rc + B.rc, ctSum + band, &wa);
         } else {
-          g = gjk_sv<T, SCREEN, PAIR>(ca, cb, a2w, b2w, args, A.rc + B.rc, ctSum + band);
+          g = gjk_sv<T, PAIR>(ca, cb, a2w, b2w, args, A.rc + B.rc, ctSum + band);
         }
         if (dir_w && g.has_v) *dir_w = mv(a2w.R, g.vdir);
       } else {
         g = gjk_jh(ca, cb, a2w, b2w, args);
-      }
-      if (g.deferred) {
-        st.bits |= kNpDeferred;
-        return no_contact<T>();
       }
       st.bits |= kNpGjk;
       st.iters = g.iters;
@@ -1131,6 +1103,48 @@ GR_D CInfo<T> closest_points(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<
     }
   }
   return no_contact<T>();
+}
+
+// What of a pair the bounding spheres, the OBB or GJK's first support pair
+// settle (physics semantics): most pairs of a resting or loose packing, none
+// in contact.  Returns kNpGjk or 0 for a settled pair, kNpDeferred for one
+// left to closest_points, which repeats it from the start with the same
+// arithmetic (closest_points and gjk_sv up to the first separation test), so
+// exactly the pairs it separates there are settled here.  warm_w: the first
+// direction, in the world frame (zero or not finite: the centre difference);
+// dir_w receives the direction of a pair GJK separates.
+template <class T>
+GR_D uint32_t screen_pair(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<T>& a2w, const Tr<T>& b2w,
+                          const T* verts_full, const T* verts_core, V3<T> warm_w, V3<T>& dir_w) {
+  if ((A.kind == GRAINS_SPHERE && B.kind == GRAINS_SPHERE) || B.kind == GRAINS_RECTANGLE) return kNpDeferred;
+  const T rsum = A.rc + B.rc;
+  const T band = near_band(rsum);  // 0 in FP64
+  const T overlap = norm(b2w.o - a2w.o) - rsum;
+  const bool sphere_near = band > T(0) && overlap >= T(0) && overlap <= band;
+  if (!(overlap < T(0) || sphere_near)) return 0u;
+  if (!obb_intersect(A.bbox, B.bbox, a2w, b2w)) return sphere_near ? kNpDeferred : 0u;
+  SupCtx<T> ca = sup_ctx(A, true, verts_full, verts_core);
+  SupCtx<T> cb = sup_ctx(B, true, verts_full, verts_core);
+  const T ctSum = A.crust + B.crust;
+  Tr<T> b2a = relative(a2w, b2w);
+  int ex;
+  frexp(rsum, &ex);
+  const T sc = ldexp(T(1), -ex);
+  b2a.o = sc * b2a.o;
+  const T sep_s = sc * (ctSum + band);
+  const T nn = dot(warm_w, warm_w);
+  const bool warm = nn > T(0) && nn < T(INFINITY);
+  const V3<T> wa = vm(warm_w, a2w.R), v = -b2a.o;  // into A's frame
+  const V3<T> dir = {warm ? wa.x : v.x, warm ? wa.y : v.y, warm ? wa.z : v.z};
+  const T nd = norm(dir);
+  if (!warm && !(nd > Eps<T>::HIGH)) return kNpDeferred;
+  const V3<T> w = sc * support(ca, -dir) - apply(b2a, sc * support(cb, vm(dir, b2a.R)));
+  const T lb = dot(dir, w) / nd;
+  T mu = T(0);
+  if (mu < lb) mu = lb;
+  if (!(mu > sep_s)) return kNpDeferred;
+  if (nd > T(0)) dir_w = mv(a2w.R, dir);
+  return kNpGjk;
 }
 
 // Hooke::performForcesCalculus + computeForces (HookeContactForceModel.cpp:91-186).

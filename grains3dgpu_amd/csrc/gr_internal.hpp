@@ -42,6 +42,7 @@ constexpr int kMaxMovers = 4096;     // particles that change cell in a step, me
 constexpr uint32_t kSmallSort = 8192; // the most particles k_sort_small can hold (64 KB of LDS)
 constexpr uint32_t kSmallSortDefault = 1024;  // beds up to this size sort in one block by default
 constexpr uint64_t kWideIntegrate = 16384;  // beds up to this size integrate every particle with its walls in one launch
+constexpr uint32_t kXcds = 8;          // dies of the card, each with its own L2; blocks go to them in turn
 constexpr int kMaxNarrowPerCu = 64;  // resident narrow-phase blocks per CU the queue buffers are sized for
 
 // per-pair flag bits

@@ -28,6 +28,24 @@ template <> __device__ __forceinline__ const HookeP<float>* hk_table<float>(cons
 // Poses of A and B for the narrow phase.  FP64: world coordinates, with B's
 // periodic image placed next to A exactly as the oracle does.  FP32: a frame
 // translated to A's centre, B's offset taken in FP64 before rounding.
+// dm: from A's centre to B's nearest image.  (The form below repeats the
+// body: calling this one from it changes which products the compiler
+// contracts in the FP32 search that follows, and so its results' last bits.)
+template <class T>
+__device__ __forceinline__ void pair_frames(V3<double> xi, Qt<double> qi, V3<double> xj, Qt<double> qj,
+                                            V3<double> dm, Tr<T>& a2w, Tr<T>& b2w) {
+  if constexpr (sizeof(T) == 8) {
+    a2w.R = rot(qi);
+    a2w.o = xi;
+    b2w.R = rot(qj);
+    b2w.o = same(dm, xj - xi) ? xj : xi + dm;
+  } else {
+    a2w.R = cvt<float>(rot(qi));
+    a2w.o = {0.0f, 0.0f, 0.0f};
+    b2w.R = cvt<float>(rot(qj));
+    b2w.o = cvt<float>(dm);
+  }
+}
 template <class T>
 __device__ __forceinline__ void pair_frames(const SimGrid& g, V3<double> xi, Qt<double> qi, V3<double> xj,
                                             Qt<double> qj, Tr<T>& a2w, Tr<T>& b2w) {
@@ -64,6 +82,18 @@ __device__ __forceinline__ double product(double a, double b) {
   double p = a * b;
   asm("" : "+v"(p));
   return p;
+}
+
+// A sim's grid through the scalar cache (a wave-uniform address; grids do
+// not change while kernels run).
+__device__ __forceinline__ SimGrid uniform_grid(const SimGrid* p) {
+  const auto* w = (const __attribute__((address_space(4))) uint32_t*)p;
+  uint32_t v[sizeof(SimGrid) / 4];
+#pragma unroll
+  for (uint32_t k = 0; k < sizeof(SimGrid) / 4; ++k) v[k] = w[k];
+  SimGrid g;
+  __builtin_memcpy(&g, v, sizeof(g));
+  return g;
 }
 
 // The bounding-sphere prefilter of the reference's particle loop
@@ -146,7 +176,7 @@ __device__ __forceinline__ void contact_force(const DevScene& d, const SimGrid& 
 // search ended on in the world frame (left alone when GJK did not run).
 // PAIR (physics semantics): lanes 2k and 2k + 1 evaluate
 // the same entry, sharing GJK's support pairs (gjk_sv<PAIR>).
-template <class T, class R, bool SV, bool SCREEN = false, bool WARM = false, bool PAIR = false, bool FILTER = false>
+template <class T, class R, bool SV, bool WARM = false, bool PAIR = false, bool FILTER = false>
 __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, uint32_t sj, PairRes<R>& out,
                                                NpStats& st, uint32_t e, V3<T>* dir = nullptr) {
   const uint64_t n = d.n;
@@ -172,17 +202,16 @@ __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, u
   if constexpr (sizeof(T) == 4 && SV && WARM) {
     float4* rec = d.ws + (uint64_t)(*d.ws_par) * ((uint64_t)d.K * n) + e;
     V3<T> dw = {T(0), T(0), T(0)};
-    ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, WarmLookup{rec},
+    ci = closest_points<T, SV, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, WarmLookup{rec},
                                              &dw);
-    // every decided entry writes its record (a zero direction when GJK did
-    // not run), so an entry never holds a record of an earlier step
-    if (!st.deferred()) *rec = make_float4(dw.x, dw.y, dw.z, __uint_as_float(d.sidx[sj]));
+    // every entry writes its record (a zero direction when GJK did not run),
+    // so none holds the direction of an earlier step
+    *rec = make_float4(dw.x, dw.y, dw.z, __uint_as_float(d.sidx[sj]));
     if (dir) *dir = dw;
   } else {
-    ci = closest_points<T, SV, SCREEN, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, NoWarm(), dir);
+    ci = closest_points<T, SV, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, NoWarm(), dir);
   }
   uint32_t flag = kFlagCand | (st.gjk() ? kFlagGjk : 0u) | (st.deep() ? kFlagDeep : 0u);
-  if constexpr (SCREEN) return flag;  // decided pairs have no contact
   if (ci.overlap < T(0)) {
     flag |= kFlagContact | slot_bits(g, xi, V3<double>{pj.x, pj.y, pj.z});
     contact_force<T, R>(d, g, d.sidx[si], d.sidx[sj], A.material, B.material, A.mass, B.mass, xi, a2w.o, b2w.o, ci,
@@ -258,10 +287,8 @@ __device__ __forceinline__ void defer_flush(const DevScene& d, DeferLds& L, uint
 
 // One lane per list entry, grid-stride.  SV: physics semantics (signed-volume
 // GJK); !SV: REF_QUIRKS.
-// PASS 0: every entry, complete.  With two passes (physics semantics):
-// PASS 2 screens every entry -- prefilter, bounding sphere, OBB and GJK's
-// first support pair decide most pairs of a resting or loose packing (no
-// contact) with a small kernel -- and queues the rest; PASS 1 runs the queued
+// PASS 0: every entry, complete.  With two passes (physics semantics) the
+// screen settles most entries and queues the rest; PASS 1 runs the queued
 // entries, packed lane-dense, complete.  A wave costs as much as its slowest
 // lane, so the long searches are kept together and the screen's waves stay
 // short.  The queued searches start from scratch with the same arithmetic:
@@ -272,17 +299,14 @@ __device__ __forceinline__ void defer_flush(const DevScene& d, DeferLds& L, uint
 // the pass lasts as long as its longest search (k_complete chooses).
 template <class T, bool SV, int PASS, bool WARM = false, bool PAIR = false>
 __device__ __forceinline__ void narrow(const DevScene& d) {
-  constexpr bool screen = SV && PASS == 2;
   constexpr bool first = PASS != 1;  // the step's first kernel
   if constexpr (first) {
     if (!step_begin(d)) return;
   }
-  __shared__ std::conditional_t<screen, DeferLds, char> L;
-  uint32_t nq = 0;  // the wave's entries in L.buf
   PairRes<T>* res = (PairRes<T>*)d.pair_res;
   const uint32_t E = PASS == 1 ? defer_total(d) : d.entry_off[d.n];
   constexpr uint32_t L2 = PAIR ? 2u : 1u;  // lanes per entry
-  uint32_t c_cand = 0, c_def = 0, c_gjk = 0, c_it = 0, c_deep = 0, c_ref = 0, c_bk = 0, c_maxit = 0, c_near = 0;
+  uint32_t c_cand = 0, c_gjk = 0, c_it = 0, c_deep = 0, c_ref = 0, c_bk = 0, c_maxit = 0, c_near = 0;
   const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x / L2;
   const bool lead = gid % L2 == 0;  // the lane that stores the entry's results
@@ -298,7 +322,7 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
       e = PASS == 1 ? defer_entry(d, (uint32_t)k) : (uint32_t)k;
       PairRes<T> r;
       V3<T> dir = {T(0), T(0), T(0)};
-      flag = pair_force<T, T, SV, screen, WARM, PAIR, first>(d, d.pair_i[e], d.pair_j[e], r, st, e,
+      flag = pair_force<T, T, SV, WARM, PAIR, first>(d, d.pair_i[e], d.pair_j[e], r, st, e,
                                                               sizeof(T) == 4 && SV ? &dir : nullptr);
       if constexpr (first) {
         c_cand += (flag & kFlagCand) != 0;
@@ -314,10 +338,10 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
       // centre line there), the contact decision lay within FP32's rounding
       // band (its FP64 decision may differ), or (GRAINS_FP64_CONTACTS) the
       // pair is in contact
-      refine = sizeof(T) == 4 && !st.deferred() &&
+      refine = sizeof(T) == 4 &&
                (st.backup() || st.deep() || st.near() ||
                 ((d.flags & GRAINS_FP64_CONTACTS) && (flag & kFlagContact)));
-      if (!st.deferred() && lead) {
+      if (lead) {
         if (refine) {
           // the FP64 re-run replaces this entry's result: its slot carries the
           // direction the FP32 search ended on, the re-run's first direction
@@ -345,16 +369,7 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
         c_near += st.near();
       }
     }
-    if constexpr (screen) {
-      defer_push(d, L, nq, st.deferred() != 0, e);
-      c_def += st.deferred();
-      if (st.deferred()) d.pend[d.pair_i[e]] = d.pend[d.pair_j[e]] = 1u;
-    }
-    if constexpr (sizeof(T) == 4 && !screen) wave_append(d.refine_list, d.refine_count, refine && lead, e);
-  }
-  if constexpr (screen) {
-    defer_flush(d, L, nq);
-    count_add(d.counters, kCntDeferred, c_def);
+    if constexpr (sizeof(T) == 4) wave_append(d.refine_list, d.refine_count, refine && lead, e);
   }
   if constexpr (first) count_add(d.counters, kCntCandidates, c_cand);
   count_add(d.counters, kCntGjk, c_gjk);
@@ -366,10 +381,114 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
   count_max(d.counters, kCntMaxIters, c_maxit);
 }
 
-template <class T, bool SV, int PASS, bool WARM = false>
+template <class T, bool SV, bool WARM = false>
 __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
-  narrow<T, SV, PASS, WARM>(d);
+  narrow<T, SV, 0, WARM>(d);
 }
+
+// the screen's part of a shape, in registers from here on
+template <class T>
+__device__ __forceinline__ void load_now(ShapeNP<T>& s) {
+  asm volatile("" : "+v"(s.kind), "+v"(s.rc), "+v"(s.crust), "+v"(s.bbox[0]), "+v"(s.bbox[1]), "+v"(s.bbox[2]));
+  asm volatile("" : "+v"(s.core[0]), "+v"(s.core[1]), "+v"(s.core[2]), "+v"(s.core[3]), "+v"(s.core[4]));
+}
+
+// The screening pass (physics semantics): screen_pair on every entry; the
+// entries it leaves undecided go to the complete pass's queues.
+// What it costs is waiting for its gathers (a wave of the form that read each
+// piece where it was used waited nine loads in turn, 74 % of its time) and,
+// behind that, some 700 VALU instructions per entry.  So what is stored by
+// entry is read a turn ahead, the shapes at once with what the tests need of
+// them, the grid through the scalar cache and a neighbour's id not at all
+// (the record keeps it): three waits in turn.  4.2e6 entries of 10^6
+// superquadrics: 180 -> 142 us; 128 VGPRs, four waves per SIMD (at 96 it
+// spills).  The dies' shares halve what is read past the L2s (710 -> 408 MB).
+template <class T, bool WARM>
+__global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 2) k_screen(DevScene d) {
+  if (!step_begin(d)) return;
+  __shared__ DeferLds L;
+  uint32_t nq = 0;  // the wave's entries in L.buf
+  const uint32_t E = d.entry_off[d.n], lane = __lane_id();
+  float4* const ws = WARM ? d.ws + (uint64_t)(*d.ws_par) * ((uint64_t)d.K * d.n) : nullptr;
+  const bool outside = d.nl[kNlOutside] != 0;
+  // each die takes a share of the entries (neighbours meet in its L2), its
+  // blocks in turn
+  const uint32_t dies = gridDim.x % kXcds == 0 ? kXcds : 1;
+  const uint32_t share = (E / dies / 64 + 1) * 64, x = blockIdx.x % dies;
+  const uint32_t end = min(E, (x + 1) * share), turn = gridDim.x / dies * blockDim.x;
+  uint32_t c_cand = 0, c_def = 0, c_gjk = 0;
+  uint32_t e = x * share + blockIdx.x / dies * blockDim.x + threadIdx.x;
+  uint32_t si = 0, sj = 0;
+  float4 rec = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto fetch = [&](uint32_t k) {  // what is stored by entry, a turn ahead
+    if (k >= end) return;
+    si = d.pair_i[k];
+    sj = d.pair_j[k];
+    if constexpr (WARM) rec = ws[k];
+  };
+  fetch(e);
+  // whole waves take turns (the queue appends are wave-wide)
+  for (uint32_t ew = e - lane; ew < end; ew += turn, e += turn) {
+    const bool in = e < end;
+    const uint32_t ci = si, cj = sj;
+    const float4 r = rec;
+    uint32_t bits = 0;
+    V3<float> dw = {0.f, 0.f, 0.f};
+    const PoseRec pi = d.pk[ci], pj = d.pk[cj];
+    const double ri = d.rcs[ci], rj = d.rcs[cj];
+    fetch(e + turn);
+    // what the tests read of the shapes, loaded before the first of them
+    ShapeNP<T> A = np_table<T>(d)[pi.shape], B = np_table<T>(d)[pj.shape];
+    load_now(A);
+    load_now(B);
+    bool cand = false;
+    V3<double> dm;  // from A's centre to B's nearest image
+    for (bool done = !in; !done;) {  // one turn per sim among the wave's entries
+      const uint32_t sim = __builtin_amdgcn_readfirstlane(pi.sim);
+      uint32_t us = sim;
+      asm("" : "+s"(us));  // (sim would become the lane's pi.sim where they are equal)
+      if (pi.sim == sim) {
+        const SimGrid g = uniform_grid(d.grids + us);
+        const V3<double> xi = {pi.x, pi.y, pi.z}, xj = {pj.x, pj.y, pj.z};
+        cand = is_candidate(g, xi, xj, ri, rj, outside);
+        dm = g.periodic ? min_image(g, xj - xi) : xj - xi;
+        done = true;
+      }
+    }
+    if (cand) {
+      Tr<T> a2w, b2w;
+      pair_frames<T>(V3<double>{pi.x, pi.y, pi.z}, Qt<double>{pi.qx, pi.qy, pi.qz, pi.qw}, V3<double>{pj.x, pj.y, pj.z},
+                     Qt<double>{pj.qx, pj.qy, pj.qz, pj.qw}, dm, a2w, b2w);
+      V3<T> dir = {T(0), T(0), T(0)};
+      bits = screen_pair<T>(A, B, a2w, b2w, vt_full<T>(d), vt_core<T>(d), V3<T>{T(r.x), T(r.y), T(r.z)}, dir);
+      if constexpr (WARM) {
+        // a settled pair keeps the direction of this step or none (the
+        // record's fourth word, the neighbour, stays)
+        if (!(bits & kNpDeferred)) dw = dir;
+      }
+    }
+    if (in) {
+      if (bits & kNpDeferred) {
+        d.pend[ci] = d.pend[cj] = 1u;
+      } else {
+        d.pair_flag[e] = cand ? kFlagCand | (bits & kNpGjk ? kFlagGjk : 0u) : 0u;
+        if constexpr (WARM) {
+          if (dw.x != 0.f || dw.y != 0.f || dw.z != 0.f || r.x != 0.f || r.y != 0.f || r.z != 0.f)
+            ws[e] = make_float4(dw.x, dw.y, dw.z, r.w);
+        }
+      }
+    }
+    c_cand += cand;
+    c_gjk += (bits & kNpGjk) != 0;
+    c_def += (bits & kNpDeferred) != 0;
+    defer_push(d, L, nq, (bits & kNpDeferred) != 0, e);
+  }
+  defer_flush(d, L, nq);
+  count_add(d.counters, kCntDeferred, c_def);
+  count_add(d.counters, kCntCandidates, c_cand);
+  count_add(d.counters, kCntGjk, c_gjk);
+}
+
 // The complete pass over the screen's queue: two lanes per entry when the
 // grid holds the queue twice over, else one.  (One launch: the two forms as
 // launches of their own cost a graph node of ~5 us each, and the one with

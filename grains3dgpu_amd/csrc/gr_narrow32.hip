@@ -13,15 +13,15 @@ void launch_narrow32(const DevScene& d, int pass, hipStream_t s) {
   const dim3 grid(d.narrow_blocks), block(d.block);
   if (pass == 0) {
     if (two && warm)
-      hipLaunchKernelGGL((k_narrow<float, true, 2, true>), grid, block, 0, s, d);
+      hipLaunchKernelGGL((k_screen<float, true>), grid, block, 0, s, d);
     else if (two)
-      hipLaunchKernelGGL((k_narrow<float, true, 2>), grid, block, 0, s, d);
+      hipLaunchKernelGGL((k_screen<float, false>), grid, block, 0, s, d);
     else if (warm)
-      hipLaunchKernelGGL((k_narrow<float, true, 0, true>), grid, block, 0, s, d);
+      hipLaunchKernelGGL((k_narrow<float, true, true>), grid, block, 0, s, d);
     else if (sv)
-      hipLaunchKernelGGL((k_narrow<float, true, 0>), grid, block, 0, s, d);
+      hipLaunchKernelGGL((k_narrow<float, true>), grid, block, 0, s, d);
     else
-      hipLaunchKernelGGL((k_narrow<float, false, 0>), grid, block, 0, s, d);
+      hipLaunchKernelGGL((k_narrow<float, false>), grid, block, 0, s, d);
   } else if (two) {
     if (warm)
       hipLaunchKernelGGL((k_complete<float, true>), grid, block, 0, s, d);

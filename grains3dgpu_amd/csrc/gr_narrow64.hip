@@ -48,11 +48,11 @@ void launch_narrow64(const DevScene& d, int pass, hipStream_t s) {
   const bool two = sv && d.split > 0;
   if (pass == 0) {
     if (two)
-      hipLaunchKernelGGL((k_narrow<double, true, 2>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
+      hipLaunchKernelGGL((k_screen<double, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
     else if (sv)
-      hipLaunchKernelGGL((k_narrow<double, true, 0>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
+      hipLaunchKernelGGL((k_narrow<double, true>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
     else
-      hipLaunchKernelGGL((k_narrow<double, false, 0>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
+      hipLaunchKernelGGL((k_narrow<double, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
   } else if (two) {
     launch_search64<0>(d, s);
   }
