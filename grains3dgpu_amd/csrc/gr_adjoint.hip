@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_particle(DevScene d, AdjBufs a) 
   const Qt<double> q = st.q(i);
   const V3<double> Mt = load3(d.last_torque, n, i);
   const uint32_t si = d.shape[i];
-  const ShapeDyn dy = d.dyn[si];
+  const Dynamics dy = load_dyn(d.dyn + si);
   StateBar s1, s0;
   s1.x = nb.v3(0, i);
   s1.q = nb.q(i);

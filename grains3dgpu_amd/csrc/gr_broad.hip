@@ -57,6 +57,8 @@ void launch_run_begin(const DevScene& d, uint32_t n, bool sort, hipStream_t s) {
 // particle whose key differs from its key there (ks_prev at its previous
 // position rank[i]) has changed cell: it is counted in sort_state[2] and the
 // first kMaxMovers are listed in mv_list.
+// The steps since the last build have advanced the records by sorted position
+// only (kNlStale): the planes take them here.
 __global__ void k_hash(DevScene d, const uint32_t* __restrict__ ks_prev) {
   const uint64_t n = d.n;
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -69,7 +71,15 @@ __global__ void k_hash(DevScene d, const uint32_t* __restrict__ ks_prev) {
   }
   if (i < n) {
     const SimGrid& g = d.sgrids[d.sim[i]];
-    const double p[3] = {d.pos[i], d.pos[n + i], d.pos[2 * n + i]};
+    double p[3];
+    if (d.nl[kNlStale]) {
+      const uint32_t r = d.rank[i];
+      const PoseRec q = d.pk[r];
+      store_state(d, i, r, q, d.vk[r]);
+      p[0] = q.x, p[1] = q.y, p[2] = q.z;
+    } else {
+      p[0] = d.pos[i], p[1] = d.pos[n + i], p[2] = d.pos[2 * n + i];
+    }
     uint32_t c[3];
     cell_of(g, p, c);
     const uint32_t k = cell_key(g, c);
@@ -88,6 +98,18 @@ __global__ void k_hash(DevScene d, const uint32_t* __restrict__ ks_prev) {
 
 void launch_hash(const DevScene& d, const uint32_t* keys_prev, hipStream_t s) {
   hipLaunchKernelGGL(k_hash, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d, keys_prev);
+}
+
+// the planes of a run's state between two of its steps
+__global__ void k_store_state(DevScene d) {
+  if (!d.nl[kNlStale]) return;
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= d.n) return;
+  const uint32_t r = d.rank[i];
+  store_state(d, i, r, d.pk[r], d.vk[r]);
+}
+void launch_store_state(const DevScene& d, hipStream_t s) {
+  hipLaunchKernelGGL(k_store_state, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d);
 }
 
 // ---- block-wide exclusive scan of one value per thread ---------------------------
@@ -585,6 +607,7 @@ __global__ void k_cells(DevScene d, const uint32_t* __restrict__ ks, const uint3
   if (s == 0) {  // an order and its inverse stand; the next build counts its movers afresh
     d.sort_state[0] = 1u;
     d.sort_state[2] = 0u;
+    d.nl[kNlStale] = 0u;
   }
   d.cand_count[s] = 0u;  // the half-shell search adds to it from both sides
   d.pend[s] = 0u;
@@ -600,6 +623,16 @@ __global__ void k_cells(DevScene d, const uint32_t* __restrict__ ks, const uint3
   r.shape = shp;
   r.sim = d.sim[i];
   d.pk[s] = r;
+  VelRec v;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    v.v[k] = d.vel[k * n + i];
+    v.w[k] = d.omega[k * n + i];
+  }
+  d.vk[s] = v;
+  if (d.hk)
+    for (int k = 0; k < 12; ++k) d.hk[12 * s + k] = d.ab_hist[k * n + i];
+  if (d.nobs) d.rws[s] = d.np64[shp].rc_max;
   const double rc = d.rc_pf[shp];
   const SimGrid& g = d.sgrids[r.sim];
   const double reach = rc + g.half_skin;

@@ -935,10 +935,15 @@ static int finalize(grains_ctx* ctx) {
       sq64[i] = {1.0 / (n2 - 1.0), 1.0 / (n1 - 1.0), (n1 - n2) / (n2 * (n1 - 1.0)), n1 / n2, 1.0 / n1,
                  b / a,            c / a,            c / b};
     }
-    dyn[i].mass = h.mass;
-    std::copy(h.inertia, h.inertia + 6, dyn[i].inertia);
-    std::copy(h.inv, h.inv + 6, dyn[i].inv);
-    dyn[i].pad = 0;
+    ShapeDyn& y = dyn[i];
+    y = ShapeDyn{};
+    y.mass = h.mass;
+    for (int k = 0; k < 3; ++k) {
+      constexpr int on[3] = {0, 3, 5}, off[3] = {1, 2, 4};
+      y.diag[k] = h.inertia[on[k]], y.inv_diag[k] = h.inv[on[k]];
+      y.off[k] = h.inertia[off[k]], y.inv_off[k] = h.inv[off[k]];
+      if (y.off[k] != 0.0 || y.inv_off[k] != 0.0) y.off_axis = 1.0;
+    }
     rcpf[i] = quirks ? h.rc : h.rc_exact;
     v64.insert(v64.end(), h.verts.begin(), h.verts.end());
     cv64.insert(cv64.end(), h.core_verts.begin(), h.core_verts.end());
@@ -993,6 +998,7 @@ static int finalize(grains_ctx* ctx) {
       (rc = dalloc(ctx, &d.keyB, n * 4, L)) || (rc = dalloc(ctx, &d.idxB, n * 4, L)) || (rc = dalloc(ctx, &d.rank, n * 4, L)) ||
       (rc = dalloc(ctx, &d.cell_off, ((size_t)d.ncells + 1) * 4, L)) ||
       (rc = dalloc(ctx, &d.bp, n * sizeof(double4), L)) || (rc = dalloc(ctx, &d.pk, n * sizeof(PoseRec), L)) ||
+      (rc = dalloc(ctx, &d.vk, n * sizeof(VelRec), L)) || (rc = dalloc(ctx, &d.rws, n * 8, L)) ||
       (rc = dalloc(ctx, &d.bp32, n * sizeof(float4), L)) ||
       (rc = dalloc(ctx, &d.cell_sph, ((size_t)d.ncells + 1) * sizeof(float4), L)) ||
       (rc = dalloc(ctx, &d.half_goff, ((size_t)d.ncells + 1) * 4, L)) || (rc = dalloc(ctx, &d.half_glist, n * 4, L)) ||
@@ -1010,6 +1016,8 @@ static int finalize(grains_ctx* ctx) {
       (rc = dalloc(ctx, &d.defer_list, defer_words(ecap) * 4, L)) ||
       (rc = dalloc(ctx, &d.defer_count, kDeferQueues * 64, L)) || (rc = dalloc(ctx, &d.counters, kWordBytes, L)))
     return rc;
+  d.hk = nullptr;
+  if (d.ab_hist && (rc = dalloc(ctx, &d.hk, 12 * n * sizeof(double), L))) return rc;
   d.pend_count = d.obs_count + 1;
   d.obs_count2 = d.obs_count + 2;
   d.queue_next = d.obs_count + 3;
@@ -1374,6 +1382,7 @@ static int adj_after_steps(grains_ctx* ctx, uint32_t steps) {
   double* cp;
   int rc = dalloc(ctx, &cp, 13 * ctx->n * 8, ctx->adj_cp);
   if (rc) return rc;
+  launch_store_state(ctx->d, ctx->stream);
   return state_to(ctx, cp);
 }
 

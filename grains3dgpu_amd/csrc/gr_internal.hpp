@@ -12,10 +12,12 @@
 //            were built; rcs[N] = prefilter radius
 //            bp32[N] = bp in FP32, relative to the sim's domain minimum, 16 B
 //            cell_sph[C] = bounding sphere of each cell's residents, 16 B
-//            pk[N] = PoseRec {pos, quat, shape, sim}  64 B, cell order
-//            (gathered from the planes when the lists are built, then kept
-//            up by the integration; neighbours of a cell are contiguous, so
-//            the gathers of a wave share cache lines)
+//            pk[N] = PoseRec {pos, quat, shape, sim}  64 B, vk[N] = VelRec
+//            {vel, omega}  48 B, cell order (gathered from the planes when
+//            the lists are built; the steps advance these, and the planes
+//            are written by a run's last step and before the next build:
+//            neighbours of a cell are contiguous, so the gathers of a wave
+//            share cache lines)
 //   pairs    cand[K][N] (k-major: lanes write consecutive words),
 //            cand_count[N], entry_off[N+1]                            u32
 //            pair_i[E], pair_j[E] (sorted positions), pair_flag[E]     u32
@@ -44,6 +46,11 @@ constexpr uint32_t kSmallSortDefault = 1024;  // beds up to this size sort in on
 constexpr uint64_t kWideIntegrate = 16384;  // beds up to this size integrate every particle with its walls in one launch
 constexpr uint32_t kXcds = 8;          // dies of the card, each with its own L2; blocks go to them in turn
 constexpr int kMaxNarrowPerCu = 64;  // resident narrow-phase blocks per CU the queue buffers are sized for
+
+// Velocities of the particle at one sorted position.
+struct alignas(16) VelRec {
+  double v[3], w[3];
+};
 
 // per-pair flag bits
 constexpr uint32_t kFlagContact = 1u;
@@ -89,6 +96,7 @@ enum ListState {
   kNlTarget,      // steps of the run asked for
   kNlOver,        // a list outgrew max_neighbors when the lists were built
   kNlOutside,     // a centre lay outside a periodic side when they were built
+  kNlStale,       // the records by sorted position are ahead of the state's planes
   kNlWords = 8
 };
 
@@ -106,11 +114,19 @@ struct SimGrid {
   double move2;          // squared displacement since the lists were built up to which they hold
 };
 
-// Dynamics of one shape (RigidBody mass properties, RigidBody.cpp:19-59).
-struct alignas(16) ShapeDyn {
+// Dynamics of one shape (RigidBody mass properties, RigidBody.cpp:19-59);
+// inertia and its inverse as upper triangles xx xy xz yy yz zz.
+struct Dynamics {
   double mass;
   double inertia[6], inv[6];
-  double pad;
+};
+// As the device stores it: one 64-byte line for the shapes whose principal
+// axes are their own (all but general polyhedra), a second for the rest.
+struct alignas(64) ShapeDyn {
+  double mass;
+  double diag[3], inv_diag[3];
+  double off_axis;  // 1: the second line holds products of inertia
+  double off[3], inv_off[3], pad[2];
 };
 
 // Exponents and axis ratios of a superquadric's crust core as the FP64
@@ -168,6 +184,9 @@ struct DevScene {
   float4* bp32;                 // bp in FP32, positions relative to the sim's domain minimum
   float4* cell_sph;             // per cell: bounding sphere of its residents' spheres (bp32 frame)
   PoseRec* pk;                  // pose by sorted position
+  VelRec* vk;                   // velocities by sorted position
+  double* hk;                   // integration history by sorted position (12 values each; d.ab_hist)
+  double* rws;                  // largest radius by sorted position (with obstacles)
   uint32_t ncells;
   uint32_t *hist;               // 256 * n_tiles (+1)
   uint32_t *scan_blocks;        // block sums of scans
@@ -206,7 +225,7 @@ struct DevScene {
   float4* ws;
   uint2* ws_nb;
   uint32_t* ws_par;
-  // particles within reach of an obstacle, queued by k_integrate for
+  // particles (sorted positions) within reach of an obstacle, queued by k_integrate for
   // k_integrate_obs (count reset by the step's first kernel)
   uint32_t* obs_list;
   uint32_t* obs_count;
@@ -275,6 +294,7 @@ struct AdjBufs {
 // gr_broad.hip
 void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 // keys_prev: the sort's output buffer (the previous step's sorted keys)
+void launch_store_state(const DevScene& d, hipStream_t s);
 void launch_hash(const DevScene& d, const uint32_t* keys_prev, hipStream_t s);
 // sorts (d.key, identity) into the returned buffers: `passes` LSD passes of
 // `digit_bits` (8 .. kRadixMaxBits) bits each
@@ -438,6 +458,30 @@ __device__ __forceinline__ void store3(double* p, uint64_t n, uint64_t i, V3<dou
   p[i] = v.x;
   p[n + i] = v.y;
   p[2 * n + i] = v.z;
+}
+// particle i's state into the planes, from its records at sorted position s
+__device__ __forceinline__ void store_state(const DevScene& d, uint64_t i, uint64_t s, const PoseRec& p,
+                                            const VelRec& v) {
+  const uint64_t n = d.n;
+  store3(d.pos, n, i, {p.x, p.y, p.z});
+  d.quat[i] = p.qx;
+  d.quat[n + i] = p.qy;
+  d.quat[2 * n + i] = p.qz;
+  d.quat[3 * n + i] = p.qw;
+  store3(d.vel, n, i, {v.v[0], v.v[1], v.v[2]});
+  store3(d.omega, n, i, {v.w[0], v.w[1], v.w[2]});
+  if (d.hk)
+    for (int k = 0; k < 12; ++k) d.ab_hist[k * n + i] = d.hk[12 * s + k];
+}
+__device__ __forceinline__ Dynamics load_dyn(const ShapeDyn* p) {
+  const double4* q = (const double4*)p;  // the first line at once
+  const double4 a = q[0], b = q[1];
+  Dynamics r = {a.x, {a.y, 0.0, 0.0, a.z, 0.0, a.w}, {b.x, 0.0, 0.0, b.y, 0.0, b.z}};
+  if (b.w != 0.0) {
+    r.inertia[1] = p->off[0], r.inertia[2] = p->off[1], r.inertia[4] = p->off[2];
+    r.inv[1] = p->inv_off[0], r.inv[2] = p->inv_off[1], r.inv[4] = p->inv_off[2];
+  }
+  return r;
 }
 // minimum-image offset along periodic directions
 __device__ __forceinline__ V3<double> min_image(const SimGrid& g, V3<double> d) {

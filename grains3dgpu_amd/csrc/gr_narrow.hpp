@@ -130,16 +130,16 @@ __device__ __forceinline__ uint32_t slot_bits(const SimGrid& g, V3<double> xi, V
   return (uint32_t)max(cell_slot(g, ci, cj), 0) << kFlagSlot;
 }
 
-// Hooke force and torque on particle i of the contact ci with j; the poses'
-// origins in the frame of ci, xi in the world.
+// Hooke force and torque on the particle at sorted position si of the contact
+// ci with the one at sj; the poses' origins in the frame of ci, xi in the world.
 template <class T, class R>
-__device__ __forceinline__ void contact_force(const DevScene& d, const SimGrid& g, uint32_t i, uint32_t j,
+__device__ __forceinline__ void contact_force(const DevScene& d, const SimGrid& g, uint32_t si, uint32_t sj,
                                               int32_t matA, int32_t matB, T massA, T massB, V3<double> xi, V3<T> oA,
                                               V3<T> oB, const CInfo<T>& ci, PairRes<R>& out) {
-  const uint64_t n = d.n;
   const HookeP<T> h = hk_table<T>(d)[g.table + material_hash((uint32_t)matA, (uint32_t)matB)];
-  const V3<T> vi = cvt<T>(load3(d.vel, n, i)), wi = cvt<T>(load3(d.omega, n, i));
-  const V3<T> vj = cvt<T>(load3(d.vel, n, j)), wj = cvt<T>(load3(d.omega, n, j));
+  const VelRec ri = d.vk[si], rj = d.vk[sj];
+  const V3<T> vi = cvt<T>(V3<double>{ri.v[0], ri.v[1], ri.v[2]}), wi = cvt<T>(V3<double>{ri.w[0], ri.w[1], ri.w[2]});
+  const V3<T> vj = cvt<T>(V3<double>{rj.v[0], rj.v[1], rj.v[2]}), wj = cvt<T>(V3<double>{rj.w[0], rj.w[1], rj.w[2]});
   V3<T> li, lj;
   if (d.flags & GRAINS_REF_QUIRKS) {
     // reference lever: the world contact point (Kinematics.cpp:86-91)
@@ -168,8 +168,7 @@ __device__ __forceinline__ void contact_force(const DevScene& d, const SimGrid& 
 
 // Narrow phase + Hooke force of entry (si, sj) -- sorted positions -- from
 // si's side (ComponentManagerCPU.cpp:384-419).  Poses come from the sorted
-// records; velocities, needed only for contacts, from the planes through the
-// particle ids.  Returns the pair flag.
+// records; so do velocities, needed only for contacts.  Returns the pair flag.
 // e: the entry.  FILTER: apply the prefilter first (a list entry); the
 // returned flag is 0 for a pair it leaves out.
 // dir (FP32, physics semantics; may be null): receives the direction the
@@ -214,7 +213,7 @@ __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, u
   uint32_t flag = kFlagCand | (st.gjk() ? kFlagGjk : 0u) | (st.deep() ? kFlagDeep : 0u);
   if (ci.overlap < T(0)) {
     flag |= kFlagContact | slot_bits(g, xi, V3<double>{pj.x, pj.y, pj.z});
-    contact_force<T, R>(d, g, d.sidx[si], d.sidx[sj], A.material, B.material, A.mass, B.mass, xi, a2w.o, b2w.o, ci,
+    contact_force<T, R>(d, g, si, sj, A.material, B.material, A.mass, B.mass, xi, a2w.o, b2w.o, ci,
                         out);
   }
   return flag;
@@ -236,6 +235,7 @@ __device__ __forceinline__ bool step_begin(const DevScene& d) {
 __device__ __forceinline__ void step_end(const DevScene& d) {
   if (blockIdx.x || threadIdx.x) return;
   d.nl[kNlDone] += 1u;
+  d.nl[kNlStale] = d.nl[kNlLast] || d.keep_torce || !d.skin ? 0u : 1u;
   if (d.nl[kNlValid] == 2u) d.nl[kNlValid] = 0u;  // lists for one step
   *d.refine_count = 0u;
   *d.queue_next = 0u;
@@ -664,46 +664,50 @@ __device__ __forceinline__ void sum_contacts(const DevScene& d, uint32_t s, V3<d
   }
 }
 
-// A particle's state at the step's start.
+// The state at the step's start of the particle at sorted position s.
 struct ParticleState {
   uint32_t si, sim;
   V3<double> xi, vel, om;
   Qt<double> qi;
-  __device__ __forceinline__ ParticleState(const DevScene& d, uint64_t i)
-      : si(d.shape[i]), sim(d.sim[i]), xi(load3(d.pos, d.n, i)), vel(load3(d.vel, d.n, i)),
-        om(load3(d.omega, d.n, i)), qi(load_quat(d.quat, d.n, i)) {}
+  __device__ __forceinline__ ParticleState(const DevScene& d, uint32_t s) {
+    const PoseRec p = d.pk[s];
+    const VelRec v = d.vk[s];
+    si = p.shape, sim = p.sim;
+    xi = {p.x, p.y, p.z};
+    qi = {p.qx, p.qy, p.qz, p.qw};
+    vel = {v.v[0], v.v[1], v.v[2]};
+    om = {v.w[0], v.w[1], v.w[2]};
+  }
 };
 
 // Gravity, then moveParticles (ComponentManagerCPU.cpp:428-500) on the
 // quaternion state, from the total contact force F and torque M.  SO: a
 // second-order scheme (d.integrator); otherwise FirstOrderExplicit.
 template <bool SO>
-__device__ __forceinline__ void finish_step(const DevScene& d, uint64_t i, uint32_t s, const ParticleState& p0,
+__device__ __forceinline__ void finish_step(const DevScene& d, const SimGrid& g, uint32_t s, const ParticleState& p0,
                                             V3<double> F, V3<double> M, int32_t ncon, uint32_t ncand,
                                             IntegCounts& c) {
   const uint64_t n = d.n;
-  const uint32_t si = p0.si, sim = p0.sim;
-  const SimGrid& g = d.grids[sim];
+  const uint32_t si = p0.si;
   const V3<double> xi = p0.xi, vel = p0.vel, om = p0.om;
   const Qt<double> qi = p0.qi;
   // addExternalForces (ComponentManagerCPU.cpp:448-460)
-  const ShapeDyn dy = d.dyn[si];
+  const Dynamics dy = load_dyn(d.dyn + si);
   F = F + dy.mass * V3<double>{g.g[0], g.g[1], g.g[2]};
-  if (d.nl[kNlLast] || d.keep_torce) {  // only the run's last step can be asked for
-    store3(d.last_force, n, i, F);
-    store3(d.last_torque, n, i, M);
-  }
-  if (ncon) d.contact_count[i] += ncon;
   c.contacts = (uint32_t)ncon;
   c.max_cand = ncand;
-  // the reference's cell of the step's positions, and whether the centre
-  // lies in its grid (the keys and counts a caller can ask for)
-  {
+  c.outside = xi.x < g.lo[0] || xi.x > g.hi[0] || xi.y < g.lo[1] || xi.y > g.hi[1] || xi.z < g.lo[2] || xi.z > g.hi[2];
+  const bool asked = d.nl[kNlLast] || d.keep_torce;  // the results of the run's last step can be asked for
+  const uint64_t i = asked || ncon || !d.skin ? d.sidx[s] : 0u;
+  if (ncon) d.contact_count[i] += ncon;
+  if (asked) {
+    store3(d.last_force, n, i, F);
+    store3(d.last_torque, n, i, M);
+    // the reference's cell of the step's positions
     const double p[3] = {xi.x, xi.y, xi.z};
     uint32_t cc[3];
     cell_of(g, p, cc);
     d.key[i] = cell_key(g, cc);
-    c.outside = p[0] < g.lo[0] || p[0] > g.hi[0] || p[1] < g.lo[1] || p[1] > g.hi[1] || p[2] < g.lo[2] || p[2] > g.hi[2];
   }
   V3<double> x = xi, vnew = vel, onew = om;
   Qt<double> qn = qi;
@@ -714,9 +718,10 @@ __device__ __forceinline__ void finish_step(const DevScene& d, uint64_t i, uint3
     const int nh = d.integrator == GRAINS_SECOND_ORDER_ADAMS_BASHFORTH ? 4
                    : d.integrator == GRAINS_SECOND_ORDER_LEAPFROG    ? 1
                                                                      : 0;
-    for (int k = 0; k < nh; ++k) hist[k] = load3(d.ab_hist + 3 * k * n, n, i);
+    double* h = d.hk + 12 * (uint64_t)s;
+    for (int k = 0; k < nh; ++k) hist[k] = {h[3 * k], h[3 * k + 1], h[3 * k + 2]};
     move_particle_scheme(d.integrator, dy.mass, dy.inertia, dy.inv, d.dt, F, M, x, qn, vnew, onew, hist);
-    for (int k = 0; k < nh; ++k) store3(d.ab_hist + 3 * k * n, n, i, hist[k]);
+    for (int k = 0; k < nh; ++k) h[3 * k] = hist[k].x, h[3 * k + 1] = hist[k].y, h[3 * k + 2] = hist[k].z;
   }
   if (g.periodic) {
     // periodic wrap of the centre (not in the reference)
@@ -734,8 +739,10 @@ __device__ __forceinline__ void finish_step(const DevScene& d, uint64_t i, uint3
   pr.x = x.x, pr.y = x.y, pr.z = x.z;
   pr.qx = qn.x, pr.qy = qn.y, pr.qz = qn.z, pr.qw = qn.w;
   pr.shape = si;
-  pr.sim = sim;
+  pr.sim = p0.sim;
+  const VelRec vr = {{vnew.x, vnew.y, vnew.z}, {onew.x, onew.y, onew.z}};
   d.pk[s] = pr;
+  d.vk[s] = vr;
   if (d.skin) {
     const double4 b = d.bp[s];
     V3<double> mv = {x.x - b.x, x.y - b.y, x.z - b.z};
@@ -748,13 +755,8 @@ __device__ __forceinline__ void finish_step(const DevScene& d, uint64_t i, uint3
     }
     if (out) d.nl[kNlValid] = 0u;
   }
-  store3(d.pos, n, i, x);
-  store3(d.vel, n, i, vnew);
-  store3(d.omega, n, i, onew);
-  d.quat[i] = qn.x;
-  d.quat[n + i] = qn.y;
-  d.quat[2 * n + i] = qn.z;
-  d.quat[3 * n + i] = qn.w;
+  // the planes, when they are read before another build (step_end tells it)
+  if (asked || !d.skin) store_state(d, i, s, pr, vr);
   // a non-finite state (NaN or infinity anywhere in it) is counted; the
   // reference has no such check and carries NaN on silently
   const double all = x.x + x.y + x.z + qn.x + qn.y + qn.z + qn.w + vnew.x + vnew.y + vnew.z + onew.x + onew.y + onew.z;
@@ -762,37 +764,35 @@ __device__ __forceinline__ void finish_step(const DevScene& d, uint64_t i, uint3
 }
 
 // One particle's step from its sorted position s: its contacts, obstacles
-// (OBS: one lane takes them in turn, some not Rectangles; FP64 for both
+// (one lane takes them in turn, some not Rectangles; FP64 for both
 // precisions; ComponentManagerCPU.cpp:301-351), gravity and the move.
-template <class T, bool OBS, bool SO>
-__device__ __forceinline__ void integrate_particle(const DevScene& d, uint64_t i, uint32_t s, IntegCounts& c) {
+template <class T, bool SO>
+__device__ __forceinline__ void integrate_obs(const DevScene& d, uint32_t s, IntegCounts& c) {
   V3<double> F, M;
   int32_t ncon;
   uint32_t ncand;
   sum_contacts<T>(d, s, F, M, ncon, ncand);
-  const ParticleState p(d, i);
-  if constexpr (OBS) {
-    const SimGrid& g = d.grids[p.sim];
-    const ShapeNP<double> A = d.np64[p.si];
-    for (uint32_t o = g.obs_begin; o < g.obs_end; ++o) {
-      const uint32_t os = d.obs_shape[o];
-      if (d.np64[os].kind != GRAINS_RECTANGLE) {
-        NpStats st = {0u, 0};
-        obstacle_contact64(d, p.si, os, d.obs_tr + 12 * (size_t)o, g.table, p.xi, p.qi, p.vel, p.om, F, M, c.walls, st);
-        c.gjk += st.gjk();
-        c.iters += st.iters;
-        c.deep += st.deep();
-      } else {
-        V3<double> f, m;
-        if (wall_contact64(d, A, o, g.table, p.xi, p.qi, p.vel, p.om, f, m)) {
-          F = F + f;
-          M = M + m;
-          ++c.walls;
-        }
+  const ParticleState p(d, s);
+  const SimGrid& g = d.grids[p.sim];
+  const ShapeNP<double> A = d.np64[p.si];
+  for (uint32_t o = g.obs_begin; o < g.obs_end; ++o) {
+    const uint32_t os = d.obs_shape[o];
+    if (d.np64[os].kind != GRAINS_RECTANGLE) {
+      NpStats st = {0u, 0};
+      obstacle_contact64(d, p.si, os, d.obs_tr + 12 * (size_t)o, g.table, p.xi, p.qi, p.vel, p.om, F, M, c.walls, st);
+      c.gjk += st.gjk();
+      c.iters += st.iters;
+      c.deep += st.deep();
+    } else {
+      V3<double> f, m;
+      if (wall_contact64(d, A, o, g.table, p.xi, p.qi, p.vel, p.om, f, m)) {
+        F = F + f;
+        M = M + m;
+        ++c.walls;
       }
     }
   }
-  finish_step<SO>(d, i, s, p, F, M, ncon, ncand, c);
+  finish_step<SO>(d, g, s, p, F, M, ncon, ncand, c);
 }
 
 __device__ __forceinline__ void integrate_counts(const DevScene& d, const IntegCounts& c, bool gen) {
@@ -809,40 +809,57 @@ __device__ __forceinline__ void integrate_counts(const DevScene& d, const IntegC
   }
 }
 
-// One particle (id i, sorted position s) without obstacle contacts, or its
-// queueing for k_integrate_obs; returns whether it was queued.
+// One particle (sorted position s) without obstacle contacts, or its queueing
+// for k_integrate_obs; returns whether it was queued.
 template <class T, bool SO>
-__device__ __forceinline__ bool integrate_or_queue(const DevScene& d, uint32_t i, uint32_t s, IntegCounts& c) {
-  const uint64_t n = d.n;
-  const SimGrid& g = d.grids[d.sim[i]];
-  const bool queue =
-      g.obs_end > g.obs_begin && obstacle_in_reach(d, g, d.np64[d.shape[i]].rc_max, load3(d.pos, n, i));
-  if (!queue) integrate_particle<T, false, SO>(d, i, s, c);
-  return queue;
+__device__ __forceinline__ bool integrate_or_queue(const DevScene& d, const SimGrid& g, uint32_t s,
+                                                   const ParticleState& p, double reach, IntegCounts& c) {
+  if (g.obs_end > g.obs_begin && obstacle_in_reach(d, g, reach, p.xi)) return true;
+  V3<double> F, M;
+  int32_t ncon;
+  uint32_t ncand;
+  sum_contacts<T>(d, s, F, M, ncon, ncand);
+  finish_step<SO>(d, g, s, p, F, M, ncon, ncand, c);
+  return false;
 }
 
-// One thread per particle.  A particle within reach of an obstacle of its
+// One thread per particle, in list order.  A particle within reach of an obstacle of its
 // sim is queued for k_integrate_obs instead (obs_list); the others need no
 // obstacle code, so this kernel does not carry the FP64 support maps and
 // GJK that obstacle contacts take.  SPLIT: a particle the screen marked
 // (d.pend) is queued in pend_list for k_integrate_pend instead.
+// Bound by what it moves, ~360 B a particle from and to its records in list
+// order; one thread per particle id, with the state in planes, the pose
+// record scattered beside them and 176 B of shape read for one radius, moved
+// 684 B and took 154 us for 10^6 superquadrics (beside the complete pass);
+// now 105 us.
 template <class T, bool SO, bool SPLIT = false>
 __global__ void __launch_bounds__(kBlock) k_integrate(DevScene d) {
   if (!d.nl[kNlRun]) return;
   if (!SPLIT) step_end(d);
-  const uint64_t n = d.n;
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   IntegCounts c;
   bool queue = false, later = false;
-  if (i < n) {
-    const uint32_t s = d.rank[i];
+  if (s < d.n) {
     const bool marked = d.pend[s] != 0u;
     if (!SPLIT && marked) d.pend[s] = 0u;
     later = SPLIT && marked;
-    if (!later) queue = integrate_or_queue<T, SO>(d, (uint32_t)i, s, c);
+    if (!later) {
+      const ParticleState p(d, (uint32_t)s);
+      const double reach = d.nobs ? d.rws[s] : 0.0;
+      for (bool done = false; !done;) {  // one turn per sim among the wave's particles
+        const uint32_t sim = __builtin_amdgcn_readfirstlane(p.sim);
+        uint32_t us = sim;
+        asm("" : "+s"(us));  // (sim would become the lane's p.sim where they are equal)
+        if (p.sim == sim) {
+          queue = integrate_or_queue<T, SO>(d, uniform_grid(d.grids + us), (uint32_t)s, p, reach, c);
+          done = true;
+        }
+      }
+    }
   }
-  if (SPLIT) wave_append(d.pend_list, d.pend_count, later, (uint32_t)i);
-  if (d.nobs) wave_append(d.obs_list, d.obs_count, queue, (uint32_t)i);
+  if (SPLIT) wave_append(d.pend_list, d.pend_count, later, (uint32_t)s);
+  if (d.nobs) wave_append(d.obs_list, d.obs_count, queue, (uint32_t)s);
   integrate_counts(d, c, false);
 }
 
@@ -859,16 +876,17 @@ __global__ void __launch_bounds__(kBlock) k_integrate_pend(DevScene d) {
   for (uint64_t b = (uint64_t)blockIdx.x * blockDim.x; b < cnt; b += stride) {
     const uint64_t k = b + threadIdx.x;
     bool queue = false;
-    uint32_t i = 0;
+    uint32_t s = 0;
     if (k < cnt) {
-      i = d.pend_list[k];
-      const uint32_t s = d.rank[i];
+      s = d.pend_list[k];
       d.pend[s] = 0u;
       IntegCounts c;
-      queue = integrate_or_queue<T, SO>(d, i, s, c);
+      // (a queued wave holds particles of many sims)
+      const ParticleState p(d, s);
+      queue = integrate_or_queue<T, SO>(d, d.grids[p.sim], s, p, d.nobs ? d.rws[s] : 0.0, c);
       tot.add(c);
     }
-    if (d.nobs) wave_append(d.obs_list2, d.obs_count2, queue, i);
+    if (d.nobs) wave_append(d.obs_list2, d.obs_count2, queue, s);
   }
   integrate_counts(d, tot, false);
 }
@@ -885,9 +903,8 @@ __global__ void __launch_bounds__(kBlock) k_integrate_obs(DevScene d, const uint
   IntegCounts tot;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < cnt; k += stride) {
-    const uint32_t i = list[k];
     IntegCounts c;
-    integrate_particle<T, true, SO>(d, i, d.rank[i], c);
+    integrate_obs<T, SO>(d, list[k], c);
     tot.add(c);
   }
   integrate_counts(d, tot, true);
@@ -911,13 +928,12 @@ __global__ void __launch_bounds__(kBlock) k_integrate_walls(DevScene d, const ui
   IntegCounts tot;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x / G;
   for (uint64_t k = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; k < cnt; k += stride) {
-    const uint32_t i = ALL ? (uint32_t)k : list[k];
-    const uint32_t s = d.rank[i];
+    const uint32_t s = ALL ? (uint32_t)k : list[k];
     V3<double> F, M;
     int32_t ncon;
     uint32_t ncand;
     sum_contacts<T>(d, s, F, M, ncon, ncand);
-    const ParticleState p(d, i);
+    const ParticleState p(d, s);
     const SimGrid& g = d.grids[p.sim];
     uint32_t walls = 0;
     for (uint32_t o0 = g.obs_begin; o0 < g.obs_end; o0 += G) {
@@ -936,7 +952,7 @@ __global__ void __launch_bounds__(kBlock) k_integrate_walls(DevScene d, const ui
       if (ALL && d.pend[s]) d.pend[s] = 0u;
       IntegCounts c;
       c.walls = walls;
-      finish_step<SO>(d, i, s, p, F, M, ncon, ncand, c);
+      finish_step<SO>(d, g, s, p, F, M, ncon, ncand, c);
       tot.add(c);
     }
   }

@@ -454,7 +454,7 @@ __device__ __forceinline__ void search64(const DevScene& d, const uint32_t E, do
         if (ci.overlap < T(0)) {
           flag |= kFlagContact | slot_bits(g, xi, V3<T>{pj.x, pj.y, pj.z});
           PairRes<T> r;
-          contact_force<T, T>(d, g, d.sidx[si], d.sidx[sj], A.material, B.material, A.mass, B.mass, xi, a2w.o,
+          contact_force<T, T>(d, g, si, sj, A.material, B.material, A.mass, B.mass, xi, a2w.o,
                               b2w.o, ci, r);
           if (lead) {
             if (store64) {

@@ -117,3 +117,32 @@ def test_lists_too_long_with_the_skin():
     short = S.load(engine.Engine(dt=sc.dt, max_neighbors=most - 1), sc)
     with pytest.raises(GrainsError, match="max_neighbors"):
         short.step(5)
+
+
+@pytest.mark.parametrize("scheme", [A.FIRST_ORDER_EXPLICIT, A.SECOND_ORDER_EXPLICIT, A.SECOND_ORDER_LEAPFROG,
+                                    A.SECOND_ORDER_ADAMS_BASHFORTH])
+@pytest.mark.parametrize("which", ["fast", "slow", "cylinders"])
+def test_state_between_the_steps_of_a_run(which, scheme):
+    """The steps of a run advance the records in list order; the state (and a
+    two-step scheme's history) is written back at the run's end and before
+    every build.  A run cut in two by a snapshot taken and put back, which
+    builds anew from the state, and one cut into single steps equal it."""
+    from grains3dgpu_amd import engine
+    sc = SCENES[which]()
+
+    def eng():
+        return S.load(engine.Engine(dt=sc.dt, precision=A.FP64, integrator=scheme), sc)
+
+    whole, cut, single = eng(), eng(), eng()
+    whole.step(40)
+    cut.step(13)
+    cut.restore(cut.snapshot())
+    cut.step(27)
+    for _ in range(40):
+        single.step(1)
+    for a, b, c in zip(whole.get_state(), cut.get_state(), single.get_state()):
+        np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(a, c)
+    for a, b, c in zip(whole.get_torce(), cut.get_torce(), single.get_torce()):
+        np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(a, c)
