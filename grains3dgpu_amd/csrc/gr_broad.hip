@@ -112,6 +112,20 @@ void launch_store_state(const DevScene& d, hipStream_t s) {
   hipLaunchKernelGGL(k_store_state, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d);
 }
 
+// Particles [i0, i0 + m) of the state's planes as rows, into the host's
+// pinned memory: out = pos[m][3], quat[m][4], vel[m][3], omega[m][3].
+__global__ void k_state_rows(DevScene d, uint64_t i0, uint64_t m, double* __restrict__ out) {
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 13 * m) return;
+  const double* src = t < 3 * m ? d.pos : t < 7 * m ? d.quat : t < 10 * m ? d.vel : d.omega;
+  const uint64_t base = t < 3 * m ? 0 : t < 7 * m ? 3 * m : t < 10 * m ? 7 * m : 10 * m;
+  const uint32_t comps = base == 3 * m ? 4u : 3u, r = (uint32_t)(t - base);  // (13 m < 2^32: kRowsMax)
+  out[t] = src[(uint64_t)(r % comps) * d.n + i0 + r / comps];
+}
+void launch_state_rows(const DevScene& d, uint64_t i0, uint64_t m, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_state_rows, dim3((unsigned)((13 * m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d, i0, m, out);
+}
+
 // ---- block-wide exclusive scan of one value per thread ---------------------------
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* lds_waves, uint32_t& total) {
   const int lane = __lane_id();

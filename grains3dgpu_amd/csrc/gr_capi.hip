@@ -11,6 +11,7 @@
 #include <string>
 #include <limits>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "../../include/grains_hip.h"
@@ -387,6 +388,12 @@ struct grains_ctx {
   uint32_t interval = 8;        // steps they are expected to hold, and whether a build has shown it
   bool interval_known = false;
   unsigned char* host_words = nullptr;  // pinned: the counters and the list words, read back together
+  // grains_get_state: rows of up to rows_cap particles in pinned memory, two
+  // of them when the state takes several
+  std::mutex rows_mu;
+  double* rows[2] = {nullptr, nullptr};
+  hipEvent_t rows_ev[2] = {nullptr, nullptr};
+  uint64_t rows_cap = 0;
   // profiling: events around the phases of each step
   bool profiling = false;
   bool capturing = false;
@@ -412,6 +419,7 @@ struct grains_ctx {
   std::vector<float> na_v32;
 };
 
+static void free_rows(grains_ctx* ctx);
 #define GR_HIP(call)                                                                    \
   do {                                                                                  \
     hipError_t e_ = (call);                                                             \
@@ -603,6 +611,7 @@ extern "C" void grains_destroy(grains_ctx_t* ctx) {
   free_list(ctx->allocs);
   free_list(ctx->state_allocs);
   if (ctx->host_words) (void)hipHostFree(ctx->host_words);
+  free_rows(ctx);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
@@ -1136,23 +1145,92 @@ extern "C" int grains_set_state(grains_ctx_t* ctx, const double* pos, const doub
   return hist_reset(ctx);
 }
 
+constexpr uint64_t kRowsMax = 1u << 18;        // particles per pinned buffer (27 MB)
+constexpr uint64_t kRowsPerThread = 1u << 14;  // particles worth a thread of their own (1.7 MB)
+
+// a part of a get_state: particles [i0, i0 + m) from the rows in `rows`
+struct StateDst {
+  double *pos, *quat, *vel, *omega;
+};
+static void copy_rows(const StateDst& o, const double* rows, uint64_t i0, uint64_t m, uint64_t a, uint64_t b) {
+  auto put = [&](double* dst, uint64_t base, uint64_t comps) {
+    if (dst) std::memcpy(dst + comps * (i0 + a), rows + base * m + comps * a, comps * (b - a) * sizeof(double));
+  };
+  put(o.pos, 0, 3), put(o.quat, 3, 4), put(o.vel, 7, 3), put(o.omega, 10, 3);
+}
+// The same by several threads: a caller's array that has not been written
+// before costs a page fault per 4 KB, 104 MB of them 20 ms on one thread.
+static void copy_rows_threads(const StateDst& o, const double* rows, uint64_t i0, uint64_t m) {
+  const uint64_t parts = std::min<uint64_t>(std::max(1u, std::min(8u, std::thread::hardware_concurrency())),
+                                            m / kRowsPerThread + 1);
+  uint64_t left = parts;  // parts [0, left) are this thread's
+  std::vector<std::thread> th;
+  try {
+    th.reserve(parts);
+    while (left > 1) {
+      const uint64_t a = m * (left - 1) / parts, b = m * left / parts;
+      th.emplace_back([=] { copy_rows(o, rows, i0, m, a, b); });
+      --left;
+    }
+  } catch (const std::exception&) {  // no more threads: the rest is copied here
+  }
+  copy_rows(o, rows, i0, m, 0, m * left / parts);
+  for (std::thread& t : th) t.join();
+}
+
+static void free_rows(grains_ctx* ctx) {
+  for (int k = 0; k < 2; ++k) {
+    if (ctx->rows[k]) (void)hipHostFree(ctx->rows[k]);
+    if (ctx->rows_ev[k]) (void)hipEventDestroy(ctx->rows_ev[k]);
+    ctx->rows[k] = nullptr;
+    ctx->rows_ev[k] = nullptr;
+  }
+  ctx->rows_cap = 0;
+}
+static bool alloc_rows(grains_ctx* ctx, uint64_t cap, int count) {
+  for (int k = 0; k < count; ++k)
+    if (hipHostMalloc((void**)&ctx->rows[k], 13 * cap * sizeof(double), hipHostMallocDefault) != hipSuccess ||
+        hipEventCreateWithFlags(&ctx->rows_ev[k], hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();
+      free_rows(ctx);
+      return false;
+    }
+  ctx->rows_cap = cap;
+  return true;
+}
+
+// The planes turn into rows on the device, written into one of two pinned
+// buffers while the other is copied out: 10^6 particles 20 -> 3.7 ms (planes
+// copied to pageable memory and turned into rows by the host).
 extern "C" int grains_get_state(grains_ctx_t* ctx, double* pos, double* quat, double* vel, double* omega,
                                 uint64_t n) {
   if (!ctx) return GRAINS_EINVAL;
   if (n != ctx->n || !n) return fail(ctx, GRAINS_EINVAL, "particle count mismatch");
-  GR_HIP(hipStreamSynchronize(ctx->stream));
-  std::vector<double> buf(4 * n);
-  auto get = [&](double* dst, const double* src, int comps) -> int {
-    if (!dst) return GRAINS_OK;
-    GR_HIP(hipMemcpy(buf.data(), src, comps * n * sizeof(double), hipMemcpyDeviceToHost));
-    for (uint64_t i = 0; i < n; ++i)
-      for (int k = 0; k < comps; ++k) dst[comps * i + k] = buf[k * n + i];
-    return GRAINS_OK;
+  const StateDst out = {pos, quat, vel, omega};
+  std::lock_guard<std::mutex> lock(ctx->rows_mu);
+  if (ctx->rows_cap < std::min(n, kRowsMax) || (n > ctx->rows_cap && !ctx->rows[1])) {
+    free_rows(ctx);
+    uint64_t cap = std::min(n, kRowsMax);
+    // less at a time where so much cannot be pinned
+    while (!alloc_rows(ctx, cap, cap < n ? 2 : 1)) {
+      if (cap <= 256) return fail(ctx, GRAINS_EDEVICE, "no pinned memory for the state");
+      cap = std::max<uint64_t>(256, cap / 2);
+    }
+  }
+  const uint64_t cap = ctx->rows_cap;
+  hipStream_t s = ctx->stream;
+  auto start = [&](uint64_t c) -> hipError_t {
+    launch_state_rows(ctx->d, c * cap, std::min(cap, n - c * cap), ctx->rows[c & 1], s);
+    hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : hipEventRecord(ctx->rows_ev[c & 1], s);
   };
-  int rc;
-  if ((rc = get(pos, ctx->d.pos, 3)) || (rc = get(quat, ctx->d.quat, 4)) || (rc = get(vel, ctx->d.vel, 3)) ||
-      (rc = get(omega, ctx->d.omega, 3)))
-    return rc;
+  const uint64_t chunks = (n + cap - 1) / cap;
+  GR_HIP(start(0));
+  for (uint64_t c = 0; c < chunks; ++c) {
+    GR_HIP(hipEventSynchronize(ctx->rows_ev[c & 1]));
+    if (c + 1 < chunks) GR_HIP(start(c + 1));
+    copy_rows_threads(out, ctx->rows[c & 1], c * cap, std::min(cap, n - c * cap));
+  }
   return GRAINS_OK;
 }
 

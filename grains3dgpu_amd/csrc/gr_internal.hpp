@@ -295,6 +295,7 @@ struct AdjBufs {
 void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 // keys_prev: the sort's output buffer (the previous step's sorted keys)
 void launch_store_state(const DevScene& d, hipStream_t s);
+void launch_state_rows(const DevScene& d, uint64_t i0, uint64_t m, double* out, hipStream_t s);
 void launch_hash(const DevScene& d, const uint32_t* keys_prev, hipStream_t s);
 // sorts (d.key, identity) into the returned buffers: `passes` LSD passes of
 // `digit_bits` (8 .. kRadixMaxBits) bits each
