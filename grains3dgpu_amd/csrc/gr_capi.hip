@@ -721,13 +721,16 @@ static int alloc_state(grains_ctx* ctx) {
        ctx->cfg.integrator == GRAINS_SECOND_ORDER_LEAPFROG) &&
       ((rc = dalloc(ctx, &d.ab_hist, 12 * n * sizeof(double), L)) || (rc = hist_reset(ctx))))
     return rc;
-  if ((rc = dalloc(ctx, &d.pos, 3 * n * sizeof(double), L)) || (rc = dalloc(ctx, &d.quat, 4 * n * sizeof(double), L)) ||
-      (rc = dalloc(ctx, &d.vel, 3 * n * sizeof(double), L)) || (rc = dalloc(ctx, &d.omega, 3 * n * sizeof(double), L)) ||
+  // the state's 13 planes in one block: copied at once (snapshots, checkpoints)
+  if ((rc = dalloc(ctx, &d.pos, 13 * n * sizeof(double), L)) ||
       (rc = dalloc(ctx, &d.shape, n * sizeof(uint32_t), L)) || (rc = dalloc(ctx, &d.sim, n * sizeof(uint32_t), L)) ||
       (rc = dalloc(ctx, &d.contact_count, n * sizeof(int32_t), L)) ||
       (rc = dalloc(ctx, &d.last_force, 3 * n * sizeof(double), L)) ||
       (rc = dalloc(ctx, &d.last_torque, 3 * n * sizeof(double), L)))
     return rc;
+  d.quat = d.pos + 3 * n;
+  d.vel = d.pos + 7 * n;
+  d.omega = d.pos + 10 * n;
   std::vector<double> zero(4 * n, 0.0), q(4 * n, 0.0);
   for (uint64_t i = 0; i < n; ++i) q[3 * n + i] = 1.0;
   GR_HIP(hipMemcpy(d.pos, zero.data(), 3 * n * sizeof(double), hipMemcpyHostToDevice));
@@ -1025,6 +1028,7 @@ static int finalize(grains_ctx* ctx) {
       (rc = dalloc(ctx, &d.defer_list, defer_words(ecap) * 4, L)) ||
       (rc = dalloc(ctx, &d.defer_count, kDeferQueues * 64, L)) || (rc = dalloc(ctx, &d.counters, kWordBytes, L)))
     return rc;
+  d.gjk_rec = nullptr;
   d.hk = nullptr;
   if (d.ab_hist && (rc = dalloc(ctx, &d.hk, 12 * n * sizeof(double), L))) return rc;
   d.pend_count = d.obs_count + 1;
@@ -1435,21 +1439,11 @@ static int use_skin(grains_ctx* ctx, bool on) {
 // ---- differentiation: recorded trajectory --------------------------------------
 // the live state <-> 13 planes (pos 3, quat 4, vel 3, omega 3), on the stream
 static int state_to(grains_ctx* ctx, double* dst) {
-  const uint64_t n = ctx->n;
-  hipStream_t s = ctx->stream;
-  GR_HIP(hipMemcpyAsync(dst, ctx->d.pos, 3 * n * 8, hipMemcpyDeviceToDevice, s));
-  GR_HIP(hipMemcpyAsync(dst + 3 * n, ctx->d.quat, 4 * n * 8, hipMemcpyDeviceToDevice, s));
-  GR_HIP(hipMemcpyAsync(dst + 7 * n, ctx->d.vel, 3 * n * 8, hipMemcpyDeviceToDevice, s));
-  GR_HIP(hipMemcpyAsync(dst + 10 * n, ctx->d.omega, 3 * n * 8, hipMemcpyDeviceToDevice, s));
+  GR_HIP(hipMemcpyAsync(dst, ctx->d.pos, 13 * ctx->n * 8, hipMemcpyDeviceToDevice, ctx->stream));
   return GRAINS_OK;
 }
 static int state_from(grains_ctx* ctx, const double* src) {
-  const uint64_t n = ctx->n;
-  hipStream_t s = ctx->stream;
-  GR_HIP(hipMemcpyAsync(ctx->d.pos, src, 3 * n * 8, hipMemcpyDeviceToDevice, s));
-  GR_HIP(hipMemcpyAsync(ctx->d.quat, src + 3 * n, 4 * n * 8, hipMemcpyDeviceToDevice, s));
-  GR_HIP(hipMemcpyAsync(ctx->d.vel, src + 7 * n, 3 * n * 8, hipMemcpyDeviceToDevice, s));
-  GR_HIP(hipMemcpyAsync(ctx->d.omega, src + 10 * n, 3 * n * 8, hipMemcpyDeviceToDevice, s));
+  GR_HIP(hipMemcpyAsync(ctx->d.pos, src, 13 * ctx->n * 8, hipMemcpyDeviceToDevice, ctx->stream));
   return GRAINS_OK;
 }
 // after recorded steps (never past a checkpoint): a checkpoint every
@@ -1947,14 +1941,8 @@ extern "C" int grains_snapshot(grains_ctx_t* ctx, void* bytes, size_t* size) {
   char* p = (char*)bytes;
   std::memcpy(p, &n, 8);
   p += 8;
-  GR_HIP(hipMemcpy(p, ctx->d.pos, 3 * n * 8, hipMemcpyDeviceToHost));
-  p += 3 * n * 8;
-  GR_HIP(hipMemcpy(p, ctx->d.quat, 4 * n * 8, hipMemcpyDeviceToHost));
-  p += 4 * n * 8;
-  GR_HIP(hipMemcpy(p, ctx->d.vel, 3 * n * 8, hipMemcpyDeviceToHost));
-  p += 3 * n * 8;
-  GR_HIP(hipMemcpy(p, ctx->d.omega, 3 * n * 8, hipMemcpyDeviceToHost));
-  p += 3 * n * 8;
+  GR_HIP(hipMemcpy(p, ctx->d.pos, 13 * n * 8, hipMemcpyDeviceToHost));
+  p += 13 * n * 8;
   GR_HIP(hipMemcpy(p, ctx->d.contact_count, n * 4, hipMemcpyDeviceToHost));
   p += n * 4;
   if (nh) GR_HIP(hipMemcpy(p, ctx->d.ab_hist, nh, hipMemcpyDeviceToHost));
@@ -1972,14 +1960,8 @@ extern "C" int grains_restore(grains_ctx_t* ctx, const void* bytes, size_t size)
   if (n0 != n || size < 8 + 13 * n * 8 + n * 4 + nh) return fail(ctx, GRAINS_EINVAL, "snapshot does not match");
   GR_HIP(hipStreamSynchronize(ctx->stream));
   const char* p = (const char*)bytes + 8;
-  GR_HIP(hipMemcpy(ctx->d.pos, p, 3 * n * 8, hipMemcpyHostToDevice));
-  p += 3 * n * 8;
-  GR_HIP(hipMemcpy(ctx->d.quat, p, 4 * n * 8, hipMemcpyHostToDevice));
-  p += 4 * n * 8;
-  GR_HIP(hipMemcpy(ctx->d.vel, p, 3 * n * 8, hipMemcpyHostToDevice));
-  p += 3 * n * 8;
-  GR_HIP(hipMemcpy(ctx->d.omega, p, 3 * n * 8, hipMemcpyHostToDevice));
-  p += 3 * n * 8;
+  GR_HIP(hipMemcpy(ctx->d.pos, p, 13 * n * 8, hipMemcpyHostToDevice));
+  p += 13 * n * 8;
   GR_HIP(hipMemcpy(ctx->d.contact_count, p, n * 4, hipMemcpyHostToDevice));
   p += n * 4;
   if (nh) GR_HIP(hipMemcpy(ctx->d.ab_hist, p, nh, hipMemcpyHostToDevice));
@@ -2041,6 +2023,10 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
         (rc = dalloc(ctx, &a.entry_tidx, ecap * 4, L)) || (rc = dalloc(ctx, &a.wall_theta, n * max_obs * 4 * 8, L)) ||
         (rc = dalloc(ctx, &a.wall_tidx, n * max_obs * 4, L)) || (rc = dalloc(ctx, &a.dtheta, (size_t)ntab * 4 * 8, L)))
       return rc;
+    // the FP64 searches leave their results for the adjoint of their contacts
+    a.gjk = nullptr;
+    if (ctx->d.precision == GRAINS_FP64 && ctx->d.split > 0 && (rc = dalloc(ctx, &a.gjk, ecap * sizeof(GjkRec), L)))
+      return rc;
     a.max_obs = max_obs;
   }
   // the state adjoint, rows -> planes
@@ -2069,6 +2055,7 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
   ctx->lists_ok = false;
   ctx->d.keep_torce = 1;
   launch_run_begin(ctx->d, 0u, true, s);
+  ctx->d.gjk_rec = a.gjk;
   const uint64_t nblocks = (T + K - 1) / K;
   for (uint64_t bb = nblocks; bb-- > 0;) {
     const uint64_t t0 = bb * K, t1 = std::min(t0 + K, T);
@@ -2088,6 +2075,7 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
   }
   ctx->profiling = prof;
   ctx->d.keep_torce = 0;
+  ctx->d.gjk_rec = nullptr;
   int rc2 = state_from(ctx, ctx->adj_save);
   if (skin && !rc2) rc2 = use_skin(ctx, true);
   if (rc) return rc;

@@ -114,6 +114,12 @@ struct SimGrid {
   double move2;          // squared displacement since the lists were built up to which they hold
 };
 
+// What an FP64 search found of a contact: the closest points of the cores in
+// their own frames, their distance, and whether they overlap.
+struct alignas(64) GjkRec {
+  double pa[3], pb[3], dist, deep;
+};
+
 // Dynamics of one shape (RigidBody mass properties, RigidBody.cpp:19-59);
 // inertia and its inverse as upper triangles xx xy xz yy yz zz.
 struct Dynamics {
@@ -196,6 +202,7 @@ struct DevScene {
   uint32_t *cand, *cand_count, *entry_off;
   uint32_t *pair_i, *pair_j, *pair_flag;
   void* pair_res;               // PairRes<T>[ecap]
+  GjkRec* gjk_rec;              // by entry: the contacts' searches (reverse sweep of the adjoint; else null)
   uint32_t* refine_list;        // entries to re-run in FP64 (FP32-mixed)
   uint32_t* refine_count;
   uint32_t* queue_next;         // FP64 searches: entries handed out past the dealt ones
@@ -287,6 +294,7 @@ struct AdjBufs {
   double* wall_theta;     // 4 per (particle, wall slot)
   uint32_t* wall_tidx;
   uint32_t max_obs;       // wall slots per particle
+  GjkRec* gjk;            // d.gjk_rec during the sweep, or null: k_adj_entry searches again
   double* dtheta;         // 4 per contact-table entry, summed over the sweep
 };
 

@@ -447,6 +447,8 @@ __device__ __forceinline__ void search64(const DevScene& d, const uint32_t E, do
             cv = round_tol(cv, Eps<T>::MID);
             ci.cv = (-distance) * cv;
             ci.overlap = distance;
+            if (MODE == 0 && d.gjk_rec && lead)
+              d.gjk_rec[e] = {{p.x, p.y, p.z}, {q.x, q.y, q.z}, inv * dist, deep ? 1.0 : 0.0};
           }
         } else if (A.kind == GRAINS_SPHERE && B.kind == GRAINS_SPHERE) {
           ci = cp_spheres(A.rc, B.rc, a2w, b2w);
