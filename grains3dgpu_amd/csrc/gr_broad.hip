@@ -112,6 +112,33 @@ void launch_store_state(const DevScene& d, hipStream_t s) {
   hipLaunchKernelGGL(k_store_state, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d);
 }
 
+// the state after the step just taken, into its slot of the log
+__global__ void k_log_state(DevScene d) {
+  if (!d.nl[kNlRun] || !d.log->base) return;
+  const int64_t slot = d.log->first + (int64_t)d.nl[kNlDone];
+  if (slot < 1 || slot >= (int64_t)d.log->slots) return;
+  const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, n = d.n;
+  if (s >= n) return;
+  const uint32_t i = d.sidx[s];
+  const PoseRec p = d.pk[s];
+  const VelRec v = d.vk[s];
+  double* o = d.log->base + 13 * n * (uint64_t)slot + i;
+  o[0] = p.x, o[n] = p.y, o[2 * n] = p.z;
+  o[3 * n] = p.qx, o[4 * n] = p.qy, o[5 * n] = p.qz, o[6 * n] = p.qw;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    o[(7 + k) * n] = v.v[k];
+    o[(10 + k) * n] = v.w[k];
+  }
+}
+void launch_log_state(const DevScene& d, hipStream_t s) {
+  hipLaunchKernelGGL(k_log_state, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d);
+}
+__global__ void k_log_set(StateLog* log, StateLog v) { *log = v; }
+void launch_log_set(const DevScene& d, StateLog v, hipStream_t s) {
+  hipLaunchKernelGGL(k_log_set, dim3(1), dim3(1), 0, s, d.log, v);
+}
+
 // Particles [i0, i0 + m) of the state's planes as rows, into the host's
 // pinned memory: out = pos[m][3], quat[m][4], vel[m][3], omega[m][3].
 __global__ void k_state_rows(DevScene d, uint64_t i0, uint64_t m, double* __restrict__ out) {

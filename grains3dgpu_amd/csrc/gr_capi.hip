@@ -406,6 +406,9 @@ struct grains_ctx {
   uint64_t adj_steps = 0;
   std::vector<void*> adj_cp;      // state every adj_every steps (13 planes)
   std::vector<void*> adj_allocs;  // sweep buffers
+  std::vector<double*> adj_log;   // per block of adj_every steps, the states between (null: run again from its checkpoint)
+  std::vector<void*> adj_log_allocs;
+  bool adj_log_ok = false;        // the logged steps followed each other (no state set between)
   AdjBufs ab{};
   double *adj_blk = nullptr, *adj_save = nullptr;
   int32_t* adj_count = nullptr;
@@ -703,6 +706,7 @@ static int hist_reset(grains_ctx* ctx) {
 // the recorded directions).
 static int warm_reset(grains_ctx* ctx) {
   ctx->lists_ok = false;
+  ctx->adj_log_ok = false;
   if (!ctx->d.ws_nb) return GRAINS_OK;
   launch_fill_u32((uint32_t*)ctx->d.ws_nb, 4 * ctx->n, 0u, ctx->stream);
   GR_HIP(hipGetLastError());
@@ -790,8 +794,11 @@ static uint64_t defer_words(uint64_t ecap) {
 }
 
 static void adj_drop(grains_ctx* ctx) {
+  if (ctx->adj_rec) drop_graph(ctx);  // a recorded step logs its state
   free_list(ctx->adj_cp);
   free_list(ctx->adj_allocs);
+  free_list(ctx->adj_log_allocs);
+  ctx->adj_log.clear();
   ctx->adj_rec = false;
   ctx->adj_steps = 0;
   ctx->ab = AdjBufs{};
@@ -1029,6 +1036,8 @@ static int finalize(grains_ctx* ctx) {
       (rc = dalloc(ctx, &d.defer_count, kDeferQueues * 64, L)) || (rc = dalloc(ctx, &d.counters, kWordBytes, L)))
     return rc;
   d.gjk_rec = nullptr;
+  if ((rc = dalloc(ctx, &d.log, sizeof(StateLog), L))) return rc;
+  launch_fill_u32((uint32_t*)d.log, sizeof(StateLog) / 4, 0u, ctx->stream);
   d.hk = nullptr;
   if (d.ab_hist && (rc = dalloc(ctx, &d.hk, 12 * n * sizeof(double), L))) return rc;
   d.pend_count = d.obs_count + 1;
@@ -1380,6 +1389,7 @@ static void enqueue_step(grains_ctx* ctx, bool build) {
     mark(ctx);
     launch_integrate32(d, s);
   }
+  if (ctx->adj_rec && !d.keep_torce) launch_log_state(d, s);
   mark(ctx);
 }
 
@@ -1458,6 +1468,25 @@ static int adj_after_steps(grains_ctx* ctx, uint32_t steps) {
   return state_to(ctx, cp);
 }
 
+// The states of a recorded trajectory's steps are kept beside its checkpoints
+// while they fit kLogBytes (and the device), so that the sweep need not run
+// them again: its block's memory (null: no more), and the place of the steps
+// of a run of which `done` are taken.
+constexpr uint64_t kLogBytes = 4ull << 30;
+static int log_chunk(grains_ctx* ctx, uint32_t done) {
+  const uint64_t K = ctx->adj_every, blk = ctx->adj_steps / K, bytes = 13 * ctx->n * 8 * K;
+  while (ctx->adj_log.size() <= blk) {
+    double* p = nullptr;
+    const uint64_t used = ctx->adj_log_allocs.size() * bytes;
+    if (K > 1 && bytes / K / 13 / 8 == ctx->n && bytes <= kLogBytes && used <= kLogBytes - bytes)
+      (void)dalloc(ctx, &p, bytes, ctx->adj_log_allocs);
+    ctx->adj_log.push_back(p);
+  }
+  launch_log_set(ctx->d, {ctx->adj_log[blk], (int64_t)(ctx->adj_steps % K) - (int64_t)done, K}, ctx->stream);
+  GR_HIP(hipGetLastError());
+  return GRAINS_OK;
+}
+
 // Steps are launched in chunks of as many as the lists are expected to hold
 // for; the kernels of a step whose lists no longer hold return at once, and
 // after each chunk the host reads how many were taken, builds new lists when
@@ -1511,6 +1540,7 @@ static int run_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
   while (done < n_steps) {
     uint32_t m = n_steps - done;
     if (ctx->adj_rec) m = std::min<uint32_t>(m, ctx->adj_every - (uint32_t)(ctx->adj_steps % ctx->adj_every));
+    if (ctx->adj_rec && (rc = log_chunk(ctx, done))) return rc;
     const bool each = !ctx->d.skin || ctx->interval <= 1;  // lists for one step at a time
     if (each) {
       m = std::min(m, 64u);
@@ -1991,9 +2021,13 @@ extern "C" int grains_adjoint_record(grains_ctx_t* ctx, uint32_t checkpoint_ever
   // the sweep's buffers are sized by checkpoint_every: drop them
   free_list(ctx->adj_cp);
   free_list(ctx->adj_allocs);
+  free_list(ctx->adj_log_allocs);
+  ctx->adj_log.clear();
+  ctx->adj_log_ok = true;
   ctx->ab = AdjBufs{};
   ctx->adj_blk = ctx->adj_save = nullptr;
   ctx->adj_count = nullptr;
+  if (!ctx->adj_rec) drop_graph(ctx);  // a recorded step logs its state
   ctx->adj_every = checkpoint_every;
   ctx->adj_steps = 0;
   ctx->adj_rec = true;
@@ -2011,24 +2045,31 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
   hipStream_t s = ctx->stream;
   int rc;
   AdjBufs& a = ctx->ab;
-  if (!ctx->adj_blk) {
+  if (!ctx->adj_save) {
     uint32_t max_obs = 1;
     for (const SimGrid& g : ctx->grids) max_obs = std::max(max_obs, g.obs_end - g.obs_begin);
     auto& L = ctx->adj_allocs;
-    if ((rc = dalloc(ctx, &ctx->adj_blk, K * 13 * n * 8, L)) || (rc = dalloc(ctx, &ctx->adj_save, 13 * n * 8, L)) ||
+    if ((rc = dalloc(ctx, &ctx->adj_save, 13 * n * 8, L)) ||
         (rc = dalloc(ctx, &ctx->adj_count, n * 4, L)) || (rc = dalloc(ctx, &a.abar, 13 * n * 8, L)) ||
         (rc = dalloc(ctx, &a.own, 13 * n * 8, L)) || (rc = dalloc(ctx, &a.Fb, 3 * n * 8, L)) ||
         (rc = dalloc(ctx, &a.Mb, 3 * n * 8, L)) || (rc = dalloc(ctx, &a.part_i, ecap * 13 * 8, L)) ||
         (rc = dalloc(ctx, &a.part_j, ecap * 13 * 8, L)) || (rc = dalloc(ctx, &a.entry_theta, ecap * 4 * 8, L)) ||
         (rc = dalloc(ctx, &a.entry_tidx, ecap * 4, L)) || (rc = dalloc(ctx, &a.wall_theta, n * max_obs * 4 * 8, L)) ||
-        (rc = dalloc(ctx, &a.wall_tidx, n * max_obs * 4, L)) || (rc = dalloc(ctx, &a.dtheta, (size_t)ntab * 4 * 8, L)))
+        (rc = dalloc(ctx, &a.wall_tidx, n * max_obs * 4, L)) || (rc = dalloc(ctx, &a.dtheta, (size_t)ntab * 4 * 8, L))) {
+      free_list(L);
+      a = AdjBufs{};
+      ctx->adj_save = ctx->adj_blk = nullptr;
       return rc;
+    }
     // the FP64 searches leave their results for the adjoint of their contacts
-    a.gjk = nullptr;
-    if (ctx->d.precision == GRAINS_FP64 && ctx->d.split > 0 && (rc = dalloc(ctx, &a.gjk, ecap * sizeof(GjkRec), L)))
-      return rc;
+    // (without the memory for them it searches again)
+    if (ctx->d.precision == GRAINS_FP64 && ctx->d.split > 0) (void)dalloc(ctx, &a.gjk, ecap * sizeof(GjkRec), L);
     a.max_obs = max_obs;
   }
+  // blocks whose steps have to be run again from their checkpoint
+  auto logged = [&](uint64_t bb) { return K == 1 || (ctx->adj_log_ok && ctx->adj_log[bb]); };
+  for (uint64_t bb = 0; bb * K < T; ++bb)
+    if (!logged(bb) && !ctx->adj_blk && (rc = dalloc(ctx, &ctx->adj_blk, K * 13 * n * 8, ctx->adj_allocs))) return rc;
   // the state adjoint, rows -> planes
   {
     std::vector<double> planes(13 * n);
@@ -2059,13 +2100,17 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
   const uint64_t nblocks = (T + K - 1) / K;
   for (uint64_t bb = nblocks; bb-- > 0;) {
     const uint64_t t0 = bb * K, t1 = std::min(t0 + K, T);
-    if ((rc = state_from(ctx, (const double*)ctx->adj_cp[bb]))) break;
-    for (uint64_t t = t0; t < t1 && !rc; ++t) {
-      if ((rc = state_to(ctx, ctx->adj_blk + (t - t0) * 13 * n))) break;
-      enqueue_step(ctx, true);
+    double* first = (double*)ctx->adj_cp[bb];
+    double* states = logged(bb) ? ctx->adj_log[bb] : ctx->adj_blk;
+    if (!logged(bb)) {
+      if ((rc = state_from(ctx, first))) break;
+      for (uint64_t t = t0; t < t1 && !rc; ++t) {
+        if ((rc = state_to(ctx, states + (t - t0) * 13 * n))) break;
+        enqueue_step(ctx, true);
+      }
     }
     for (uint64_t t = t1; t-- > t0 && !rc;) {
-      double* st = ctx->adj_blk + (t - t0) * 13 * n;
+      double* st = t == t0 ? first : states + (t - t0) * 13 * n;
       if ((rc = state_from(ctx, st))) break;
       enqueue_step(ctx, true);  // entries, contact flags, force and torque of step t
       a.state = st;

@@ -120,6 +120,15 @@ struct alignas(64) GjkRec {
   double pa[3], pb[3], dist, deep;
 };
 
+// Where the steps of a recorded trajectory leave their states (device memory,
+// set before each chunk of steps): 13 planes per slot, step number kNlDone of
+// the run in slot first + kNlDone, slots [1, slots).
+struct StateLog {
+  double* base;
+  int64_t first;
+  uint64_t slots;
+};
+
 // Dynamics of one shape (RigidBody mass properties, RigidBody.cpp:19-59);
 // inertia and its inverse as upper triangles xx xy xz yy yz zz.
 struct Dynamics {
@@ -202,6 +211,7 @@ struct DevScene {
   uint32_t *cand, *cand_count, *entry_off;
   uint32_t *pair_i, *pair_j, *pair_flag;
   void* pair_res;               // PairRes<T>[ecap]
+  StateLog* log;                // recorded trajectories
   GjkRec* gjk_rec;              // by entry: the contacts' searches (reverse sweep of the adjoint; else null)
   uint32_t* refine_list;        // entries to re-run in FP64 (FP32-mixed)
   uint32_t* refine_count;
@@ -303,6 +313,8 @@ struct AdjBufs {
 void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 // keys_prev: the sort's output buffer (the previous step's sorted keys)
 void launch_store_state(const DevScene& d, hipStream_t s);
+void launch_log_state(const DevScene& d, hipStream_t s);
+void launch_log_set(const DevScene& d, StateLog v, hipStream_t s);
 void launch_state_rows(const DevScene& d, uint64_t i0, uint64_t m, double* out, hipStream_t s);
 void launch_hash(const DevScene& d, const uint32_t* keys_prev, hipStream_t s);
 // sorts (d.key, identity) into the returned buffers: `passes` LSD passes of

@@ -1,6 +1,8 @@
 """The reverse sweep takes its contacts' closest points from the step's
 searches where the two-pass FP64 narrow phase leaves them, and searches again
-otherwise.  Both run the same arithmetic, so the gradients are equal bit for
+otherwise; it takes the states between checkpoints from the log of the
+recorded steps, and runs them again where the log does not stand (a state set
+while recording).  All run the same arithmetic, so the gradients are equal bit for
 bit: touching ellipsoids, spheres among ellipsoids, several checkpoint blocks."""
 import numpy as np
 import pytest
@@ -22,13 +24,16 @@ def test_recorded_searches_give_the_same_gradients(which):
     rng = np.random.default_rng(5)
     w = [rng.standard_normal((sc.n, k)) for k in (3, 4, 3, 3)]
     out = []
-    for passes in (1, 2):
+    for passes, log in ((1, True), (2, True), (2, False)):
         e = S.load(engine.Engine(dt=sc.dt, precision=A.FP64, gjk_rel_tol=1e-12, narrow_passes=passes), sc)
         e.adjoint_record(10)
+        if not log:
+            e.set_state(*e.get_state())
         e.step(42)
         assert e.get_stats()["contacts"] > 0
         g, g0 = e.adjoint(*w, want_state0=True)
         out.append([g, *g0])
     assert np.abs(out[0][0]).max() > 0
-    for a, b in zip(*out):
+    for a, b, c in zip(*out):
         np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(a, c)
