@@ -816,6 +816,12 @@ static int finalize(grains_ctx* ctx) {
   DevScene& d = ctx->d;
   const bool quirks = (ctx->cfg.flags & GRAINS_REF_QUIRKS) != 0;
   const uint32_t ns = (uint32_t)ctx->sims.size();
+  d.balls = 1;
+  for (uint32_t k : ctx->pshape)
+    if (ctx->shapes[k].s.kind != GRAINS_SPHERE) {
+      d.balls = 0;
+      break;
+    }
   d.gen_obs = 0;
   for (uint32_t s : ctx->obs_shape) {
     if (s >= ctx->shapes.size()) return fail(ctx, GRAINS_EINVAL, "obstacle shape index out of range");
@@ -1349,8 +1355,9 @@ static void enqueue_step(grains_ctx* ctx, bool build) {
     for (int k = 0; k < 5; ++k) mark(ctx);  // the build's phases: nothing
   // the integration split around the narrow phase's second pass: two
   // passes (physics semantics), the step not profiled phase by phase; a
-  // small bed's integration is too short to be worth the second stream
-  const bool split = d.overlap && d.n > kWideIntegrate && d.split > 0 && !(d.flags & GRAINS_REF_QUIRKS) && !ctx->adj_rec &&
+  // small bed's integration is too short to be worth the second stream, and
+  // spheres in FP64 have no second pass
+  const bool split = d.overlap && d.n > kWideIntegrate && !(d.balls && d.precision == GRAINS_FP64) && d.split > 0 && !(d.flags & GRAINS_REF_QUIRKS) && !ctx->adj_rec &&
                      !(ctx->profiling && !ctx->capturing);
   if (d.precision == GRAINS_FP64 && split) {
     launch_narrow64(d, 0, s);

@@ -166,6 +166,18 @@ GR_D SupCtx<T> sup_ctx(const ShapeNP<T>& s, bool core, const T* verts_full, cons
   return c;
 }
 
+// A's context on even lanes, B's on odd ones, field by field
+template <class T>
+GR_D SupCtx<T> lane_ctx(bool odd, const SupCtx<T>& A, const SupCtx<T>& B) {
+  SupCtx<T> c;
+  c.kind = odd ? B.kind : A.kind;
+  c.nv = odd ? B.nv : A.nv;
+  c.d = odd ? B.d : A.d;
+  c.verts = odd ? B.verts : A.verts;
+  if constexpr (sizeof(T) == 4) c.lg = odd ? B.lg : A.lg;
+  return c;
+}
+
 // Sphere.cpp:111-114, Box.cpp:129-134, Rectangle.cpp:115-120,
 // Superquadric.cpp:169-205, Cylinder.cpp:118-131 (dims r, h/2),
 // Cone.cpp:126-141 (dims r, h/4, sine of the half angle); polyhedron: first
@@ -461,7 +473,8 @@ constexpr int kGjkMaxIter = 1000;
 // (the REF_QUIRKS semantics): full shapes, v0 = s_A(0) - b2a(s_B(0)), the
 // break on mu < 1e-4*rel, the stale |v| kept when Johnson's backup procedure
 // is taken.  The physics semantics use gjk_sv.
-template <class T>
+// PAIR: two lanes per pair, as gjk_sv<PAIR>.
+template <class T, bool PAIR = false>
 GR_D GjkOut<T> gjk_jh(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, const Tr<T>& b2w,
                       const GjkArgs& args) {
   const T rel = args.rel > 0 ? T(args.rel) : Eps<T>::LOW;
@@ -483,7 +496,23 @@ GR_D GjkOut<T> gjk_jh(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
   int num_iter = 0;
   const Tr<T> b2a = relative(a2w, b2w);
   const V3<T> zero = {T(0), T(0), T(0)};
-  V3<T> v = support(A, zero) - apply(b2a, support(B, zero));
+  // the support pair in directions da (A's frame) and db (B's)
+  V3<T> pl, ql;
+  auto supports = [&](const V3<T>& da, const V3<T>& db) {
+    if constexpr (PAIR) {
+      const bool odd = (__lane_id() & 1u) != 0;
+      const SupCtx<T> C = lane_ctx(odd, A, B);
+      const V3<T> r = support(C, V3<T>{odd ? db.x : da.x, odd ? db.y : da.y, odd ? db.z : da.z});
+      const V3<T> o = {__shfl_xor(r.x, 1), __shfl_xor(r.y, 1), __shfl_xor(r.z, 1)};
+      pl = {odd ? o.x : r.x, odd ? o.y : r.y, odd ? o.z : r.z};
+      ql = {odd ? r.x : o.x, odd ? r.y : o.y, odd ? r.z : o.z};
+    } else {
+      pl = support(A, da);
+      ql = support(B, db);
+    }
+  };
+  supports(zero, zero);
+  V3<T> v = pl - apply(b2a, ql);
   T dist = norm(v);
   bool backup = false;
   while (bits < 15 && dist > Eps<T>::HIGH && num_iter < 1000) {
@@ -493,8 +522,7 @@ GR_D GjkOut<T> gjk_jh(const SupCtx<T>& A, const SupCtx<T>& B, const Tr<T>& a2w, 
       ++last;
       last_bit <<= 1;
     }
-    const V3<T> pl = support(A, -v);
-    const V3<T> ql = support(B, vm(v, b2a.R));
+    supports(-v, vm(v, b2a.R));
     const V3<T> w = pl - apply(b2a, ql);
     const T lb = dot(v, w) / dist;
     if (mu < lb) mu = lb;
@@ -1065,7 +1093,7 @@ GR_D CInfo<T> closest_points(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<
         }
         if (dir_w && g.has_v) *dir_w = mv(a2w.R, g.vdir);
       } else {
-        g = gjk_jh(ca, cb, a2w, b2w, args);
+        g = gjk_jh<T, PAIR>(ca, cb, a2w, b2w, args);
       }
       st.bits |= kNpGjk;
       st.iters = g.iters;
@@ -1145,6 +1173,17 @@ GR_D uint32_t screen_pair(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<T>&
   if (!(mu > sep_s)) return kNpDeferred;
   if (nd > T(0)) dir_w = mv(a2w.R, dir);
   return kNpGjk;
+}
+
+// The same under the reference semantics: the bounding spheres and the OBB
+// (closest_points<T, false> up to its search).
+template <class T>
+GR_D uint32_t screen_ref(const ShapeNP<T>& A, const ShapeNP<T>& B, const Tr<T>& a2w, const Tr<T>& b2w) {
+  if ((A.kind == GRAINS_SPHERE && B.kind == GRAINS_SPHERE) || B.kind == GRAINS_RECTANGLE) return kNpDeferred;
+  const T rsum = A.rc + B.rc, band = near_band(rsum);  // 0 in FP64
+  const T overlap = norm(b2w.o - a2w.o) - rsum;
+  if (band > T(0) && overlap >= T(0) && overlap <= band) return kNpDeferred;
+  return overlap < T(0) && obb_intersect(A.bbox, B.bbox, a2w, b2w) ? kNpDeferred : 0u;
 }
 
 // Hooke::performForcesCalculus + computeForces (HookeContactForceModel.cpp:91-186).

@@ -226,6 +226,7 @@ struct DevScene {
   int32_t half_wl;              // 1: the half-shell search takes its groups from a work list (dense cells)
   uint32_t* half_goff;          // work list: groups per cell, scanned (ncells + 1)
   uint32_t* half_glist;         // work list: each group's cell (n)
+  int32_t balls;                // 1: every particle is a sphere
   int32_t gen_obs;              // 1: some obstacle is not a Rectangle (GJK in the integration kernel)
   // time integration: scheme, and its history (12 planes of n): for
   // ADAMS_BASHFORTH the previous step's v, w, a, alpha (NaN: none yet), for

@@ -175,7 +175,8 @@ __device__ __forceinline__ void contact_force(const DevScene& d, const SimGrid& 
 // search ended on in the world frame (left alone when GJK did not run).
 // PAIR (physics semantics): lanes 2k and 2k + 1 evaluate
 // the same entry, sharing GJK's support pairs (gjk_sv<PAIR>).
-template <class T, class R, bool SV, bool WARM = false, bool PAIR = false, bool FILTER = false>
+// BALLS: every particle is a sphere.
+template <class T, class R, bool SV, bool WARM = false, bool PAIR = false, bool FILTER = false, bool BALLS = false>
 __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, uint32_t sj, PairRes<R>& out,
                                                NpStats& st, uint32_t e, V3<T>* dir = nullptr) {
   const uint64_t n = d.n;
@@ -198,7 +199,9 @@ __device__ __forceinline__ uint32_t pair_force(const DevScene& d, uint32_t si, u
   // tolerance, so it decides as that path does
   const GjkArgs args = {d.flags, sizeof(T) == 8 && d.precision == GRAINS_FP32_MIXED ? d.gjk_rel64 : d.gjk_rel};
   CInfo<T> ci;
-  if constexpr (sizeof(T) == 4 && SV && WARM) {
+  if constexpr (BALLS) {
+    ci = cp_spheres(A.rc, B.rc, a2w, b2w);
+  } else if constexpr (sizeof(T) == 4 && SV && WARM) {
     float4* rec = d.ws + (uint64_t)(*d.ws_par) * ((uint64_t)d.K * n) + e;
     V3<T> dw = {T(0), T(0), T(0)};
     ci = closest_points<T, SV, PAIR>(A, B, a2w, b2w, args, vt_full<T>(d), vt_core<T>(d), st, WarmLookup{rec},
@@ -297,7 +300,8 @@ __device__ __forceinline__ void defer_flush(const DevScene& d, DeferLds& L, uint
 // PAIR (PASS 1, physics semantics): two lanes per queued entry, sharing its
 // support evaluations (pair_force<PAIR>): the queue is short on beds, and
 // the pass lasts as long as its longest search (k_complete chooses).
-template <class T, bool SV, int PASS, bool WARM = false, bool PAIR = false>
+// BALLS (PASS 0, FP64): every particle is a sphere -- no search, no second pass.
+template <class T, bool SV, int PASS, bool WARM = false, bool PAIR = false, bool BALLS = false>
 __device__ __forceinline__ void narrow(const DevScene& d) {
   constexpr bool first = PASS != 1;  // the step's first kernel
   if constexpr (first) {
@@ -322,8 +326,8 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
       e = PASS == 1 ? defer_entry(d, (uint32_t)k) : (uint32_t)k;
       PairRes<T> r;
       V3<T> dir = {T(0), T(0), T(0)};
-      flag = pair_force<T, T, SV, WARM, PAIR, first>(d, d.pair_i[e], d.pair_j[e], r, st, e,
-                                                              sizeof(T) == 4 && SV ? &dir : nullptr);
+      flag = pair_force<T, T, SV, WARM, PAIR, first, BALLS>(d, d.pair_i[e], d.pair_j[e], r, st, e,
+                                                            sizeof(T) == 4 && SV ? &dir : nullptr);
       if constexpr (first) {
         c_cand += (flag & kFlagCand) != 0;
         if constexpr (WARM) {
@@ -386,6 +390,13 @@ __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
   narrow<T, SV, 0, WARM>(d);
 }
 
+// Beds of spheres in FP64 (either semantics) take one small pass: screen and
+// search passes 6.6 + 13 us on 1,000 spheres, this 7.2 us.
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_narrow_balls(DevScene d) {
+  narrow<T, true, 0, false, false, true>(d);
+}
+
 // the screen's part of a shape, in registers from here on
 template <class T>
 __device__ __forceinline__ void load_now(ShapeNP<T>& s) {
@@ -393,7 +404,7 @@ __device__ __forceinline__ void load_now(ShapeNP<T>& s) {
   asm volatile("" : "+v"(s.core[0]), "+v"(s.core[1]), "+v"(s.core[2]), "+v"(s.core[3]), "+v"(s.core[4]));
 }
 
-// The screening pass (physics semantics): screen_pair on every entry; the
+// The screening pass: screen_pair (REF_QUIRKS: screen_ref) on every entry; the
 // entries it leaves undecided go to the complete pass's queues.
 // What it costs is waiting for its gathers (a wave of the form that read each
 // piece where it was used waited nine loads in turn, 74 % of its time) and,
@@ -403,7 +414,7 @@ __device__ __forceinline__ void load_now(ShapeNP<T>& s) {
 // (the record keeps it): three waits in turn.  4.2e6 entries of 10^6
 // superquadrics: 180 -> 142 us; 128 VGPRs, four waves per SIMD (at 96 it
 // spills).  The dies' shares halve what is read past the L2s (710 -> 408 MB).
-template <class T, bool WARM>
+template <class T, bool WARM, bool SV = true>
 __global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 2) k_screen(DevScene d) {
   if (!step_begin(d)) return;
   __shared__ DeferLds L;
@@ -460,7 +471,7 @@ __global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 2) k_screen(DevSc
       pair_frames<T>(V3<double>{pi.x, pi.y, pi.z}, Qt<double>{pi.qx, pi.qy, pi.qz, pi.qw}, V3<double>{pj.x, pj.y, pj.z},
                      Qt<double>{pj.qx, pj.qy, pj.qz, pj.qw}, dm, a2w, b2w);
       V3<T> dir = {T(0), T(0), T(0)};
-      bits = screen_pair<T>(A, B, a2w, b2w, vt_full<T>(d), vt_core<T>(d), V3<T>{T(r.x), T(r.y), T(r.z)}, dir);
+      bits = !SV ? screen_ref<T>(A, B, a2w, b2w) : screen_pair<T>(A, B, a2w, b2w, vt_full<T>(d), vt_core<T>(d), V3<T>{T(r.x), T(r.y), T(r.z)}, dir);
       if constexpr (WARM) {
         // a settled pair keeps the direction of this step or none (the
         // record's fourth word, the neighbour, stays)
@@ -494,12 +505,15 @@ __global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 2) k_screen(DevSc
 // launches of their own cost a graph node of ~5 us each, and the one with
 // nothing to do had to wait for room beside the integration: 0.13 ms on the
 // bed of 10^6.)
-template <class T, bool WARM>
+// REF_QUIRKS in FP64 takes the two passes too: in one pass a wave searched
+// with the fifth of its lanes that reach GJK.  4,001 boxes and superquadrics
+// 149 -> 8 + 93 us.
+template <class T, bool WARM, bool SV = true>
 __global__ void __launch_bounds__(kBlock) k_complete(DevScene d) {
   if ((uint64_t)defer_total(d) * 2 <= (uint64_t)gridDim.x * blockDim.x)
-    narrow<T, true, 1, WARM, true>(d);
+    narrow<T, SV, 1, WARM, true>(d);
   else
-    narrow<T, true, 1, WARM, false>(d);
+    narrow<T, SV, 1, WARM, false>(d);
 }
 
 // Particle x obstacle of any other kind than Rectangle: closestPointsRigidBodies
@@ -929,12 +943,12 @@ __global__ void __launch_bounds__(kBlock) k_integrate_walls(DevScene d, const ui
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x / G;
   for (uint64_t k = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; k < cnt; k += stride) {
     const uint32_t s = ALL ? (uint32_t)k : list[k];
+    const ParticleState p(d, s);
+    const SimGrid& g = d.grids[p.sim];
     V3<double> F, M;
     int32_t ncon;
     uint32_t ncand;
     sum_contacts<T>(d, s, F, M, ncon, ncand);
-    const ParticleState p(d, s);
-    const SimGrid& g = d.grids[p.sim];
     uint32_t walls = 0;
     for (uint32_t o0 = g.obs_begin; o0 < g.obs_end; o0 += G) {
       V3<double> f = {0.0, 0.0, 0.0}, m = f;

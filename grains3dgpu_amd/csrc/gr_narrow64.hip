@@ -45,16 +45,22 @@ static void launch_search64(const DevScene& d, hipStream_t s) {
 
 void launch_narrow64(const DevScene& d, int pass, hipStream_t s) {
   const bool sv = !(d.flags & GRAINS_REF_QUIRKS);
-  const bool two = sv && d.split > 0;
-  if (pass == 0) {
-    if (two)
+  const bool two = d.split > 0;
+  if (d.balls) {
+    if (pass == 0) hipLaunchKernelGGL(k_narrow_balls<double>, dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
+  } else if (pass == 0) {
+    if (two && sv)
       hipLaunchKernelGGL((k_screen<double, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
+    else if (two)
+      hipLaunchKernelGGL((k_screen<double, false, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
     else if (sv)
       hipLaunchKernelGGL((k_narrow<double, true>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
     else
       hipLaunchKernelGGL((k_narrow<double, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
-  } else if (two) {
+  } else if (two && sv) {
     launch_search64<0>(d, s);
+  } else if (two) {
+    hipLaunchKernelGGL((k_complete<double, false, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
   }
 }
 void launch_refine64(const DevScene& d, hipStream_t s) {

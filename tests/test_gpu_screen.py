@@ -7,7 +7,7 @@ import pytest
 
 from grains3dgpu_amd import _abi as A
 from grains3dgpu_amd import scene as S
-from tests.scenes import dense_cylinders_cones, dense_superquadrics
+from tests.scenes import dense_cylinders_cones, dense_spheres, dense_superquadrics
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +37,54 @@ def test_screen_settles_what_one_pass_does(which, block, per_cu):
     for k in ("candidate_pairs", "gjk_calls", "contacts"):
         assert one[1][k] == two[1][k], k
     assert two[1]["candidate_pairs"] > 0
+
+
+@pytest.mark.parametrize("block,per_cu", [(64, 1), (256, 8)])
+@pytest.mark.parametrize("which", sorted(SCENES))
+def test_reference_semantics_in_two_passes(which, block, per_cu):
+    """REF_QUIRKS in FP64: the screen settles by spheres and OBB what one pass
+    does; the rest are searched by two lanes each, with the same results."""
+    from grains3dgpu_amd import engine
+    sc = SCENES[which]()
+    out = []
+    for passes in (1, 2):
+        e = S.load(engine.Engine(dt=sc.dt, precision=A.FP64, flags=A.REF_QUIRKS, narrow_passes=passes,
+                                 block_size=block, narrow_blocks_per_cu=per_cu), sc)
+        e.step(5)
+        out.append((e.get_state(), e.get_stats(), e.get_pairs(A.PAIRS_CONTACT)))
+    one, two = out
+    for a, b in zip(one[0], two[0]):
+        np.testing.assert_array_equal(a, b)
+    np.testing.assert_array_equal(one[2], two[2])
+    for k in ("candidate_pairs", "gjk_calls", "gjk_iterations", "contacts"):
+        assert one[1][k] == two[1][k], k
+
+
+@pytest.mark.parametrize("flags", [0, A.REF_QUIRKS])
+@pytest.mark.parametrize("n", [2, 300, 17000])
+def test_spheres_alone_equal_spheres_beside_a_box(n, flags):
+    """A bed of spheres takes the pass without a search; one more particle, a
+    box out of reach of all others, sends it through the general passes."""
+    import dataclasses
+    from grains3dgpu_amd import engine
+    sc = dense_spheres(n=max(n, 300), seed=35, vel=0.5)
+    if n < 300:
+        sc = dataclasses.replace(sc, pos=sc.pos[:n], quat=sc.quat[:n], vel=sc.vel[:n], omega=sc.omega[:n],
+                                 particle_shape=sc.particle_shape[:n])
+    L = np.array(sc.sims[0]["domain_max"], float)
+    sims = [dict(sc.sims[0], domain_max=tuple(L * [1, 1, 3]))]
+    alone = dataclasses.replace(sc, sims=sims)
+    box = [dict(kind=A.BOX, material=0, dims=(1e-4, 1e-4, 1e-4), density=2500.0)]
+    beside = dataclasses.replace(
+        sc, sims=sims, shapes=list(sc.shapes) + box, pos=np.r_[sc.pos, [L * [0.5, 0.5, 2.5]]],
+        quat=np.r_[sc.quat, [[0, 0, 0, 1.0]]], vel=np.r_[sc.vel, [[0, 0, 0.0]]], omega=np.r_[sc.omega, [[0, 0, 0.0]]],
+        particle_shape=np.r_[sc.particle_shape, len(sc.shapes)].astype(np.uint32))
+    out = []
+    for s in (alone, beside):
+        e = S.load(engine.Engine(dt=s.dt, precision=A.FP64, flags=flags), s)
+        e.step(8)
+        out.append((e.get_state(), e.get_torce(), e.get_stats()["contacts"]))
+    m = len(alone.pos)
+    assert out[0][2] == out[1][2] and (n < 300 or out[0][2] > 0)
+    for a, b in zip(out[0][0] + out[0][1], out[1][0] + out[1][1]):
+        np.testing.assert_array_equal(a, b[:m])
