@@ -1806,6 +1806,13 @@ extern "C" int grains_get_stats(grains_ctx_t* ctx, grains_stats_t* st) {
   return GRAINS_OK;
 }
 
+// the shape set rides in the batch kernel's arguments
+static bool shapes_in_args(const grains_ctx* ctx) {
+  bool in_args = ctx->na_np64.size() <= (size_t)kArgShapes;
+  for (size_t k = 0; in_args && k < ctx->na_np64.size(); ++k) in_args = ctx->na_np64[k].kind != GRAINS_POLYHEDRON;
+  return in_args;
+}
+
 extern "C" int grains_gjk_batch_device(grains_ctx_t* ctx, const uint32_t* sa, const uint32_t* sb, const double* ta,
                                        const double* tb, uint64_t n, double* dist, int32_t* iters, float* ms) {
   if (!ctx || !sa || !sb || !ta || !tb || !dist) return GRAINS_EINVAL;
@@ -1816,25 +1823,32 @@ extern "C" int grains_gjk_batch_device(grains_ctx_t* ctx, const uint32_t* sa, co
   const std::vector<ShapeNP<float>>& np32 = ctx->na_np32;
   const std::vector<double>& v64 = ctx->na_v64;
   const std::vector<float>& v32 = ctx->na_v32;
+  const bool in_args = shapes_in_args(ctx);
   std::vector<void*> tmp;
-  ShapeNP<double>* p64;
-  ShapeNP<float>* p32;
-  double* pv64;
-  float* pv32;
-  int rc;
-  if ((rc = dalloc(ctx, &p64, S * sizeof(ShapeNP<double>), tmp)) || (rc = dalloc(ctx, &p32, S * sizeof(ShapeNP<float>), tmp)) ||
-      (rc = dalloc(ctx, &pv64, v64.size() * 8, tmp)) || (rc = dalloc(ctx, &pv32, v32.size() * 4, tmp))) {
-    free_list(tmp);
-    return rc;
-  }
+  ShapeNP<double>* p64 = nullptr;
+  ShapeNP<float>* p32 = nullptr;
+  double* pv64 = nullptr;
+  float* pv32 = nullptr;
   hipStream_t s = ctx->stream;
-  (void)hipMemcpy(p64, np64.data(), S * sizeof(ShapeNP<double>), hipMemcpyHostToDevice);
-  (void)hipMemcpy(p32, np32.data(), S * sizeof(ShapeNP<float>), hipMemcpyHostToDevice);
-  (void)hipMemcpy(pv64, v64.data(), v64.size() * 8, hipMemcpyHostToDevice);
-  (void)hipMemcpy(pv32, v32.data(), v32.size() * 4, hipMemcpyHostToDevice);
+  int rc;
+  if (!in_args) {
+    if ((rc = dalloc(ctx, &p64, S * sizeof(ShapeNP<double>), tmp)) || (rc = dalloc(ctx, &p32, S * sizeof(ShapeNP<float>), tmp)) ||
+        (rc = dalloc(ctx, &pv64, v64.size() * 8, tmp)) || (rc = dalloc(ctx, &pv32, v32.size() * 4, tmp))) {
+      free_list(tmp);
+      return rc;
+    }
+    (void)hipMemcpy(p64, np64.data(), S * sizeof(ShapeNP<double>), hipMemcpyHostToDevice);
+    (void)hipMemcpy(p32, np32.data(), S * sizeof(ShapeNP<float>), hipMemcpyHostToDevice);
+    (void)hipMemcpy(pv64, v64.data(), v64.size() * 8, hipMemcpyHostToDevice);
+    (void)hipMemcpy(pv32, v32.data(), v32.size() * 4, hipMemcpyHostToDevice);
+  }
   const GjkArgs args = {ctx->cfg.flags, ctx->cfg.gjk_rel_tol};
   (void)hipEventRecord(ctx->ev0, s);
-  if (ctx->cfg.precision == GRAINS_FP64)
+  if (in_args && ctx->cfg.precision == GRAINS_FP64)
+    launch_gjk_batch_args64(np64.data(), S, sa, sb, ta, tb, n, args, dist, iters, s);
+  else if (in_args)
+    launch_gjk_batch_args32(np32.data(), S, sa, sb, ta, tb, n, args, dist, iters, s);
+  else if (ctx->cfg.precision == GRAINS_FP64)
     launch_gjk_batch64(p64, pv64, sa, sb, ta, tb, n, args, dist, nullptr, nullptr, iters, s);
   else
     launch_gjk_batch32(p32, pv32, sa, sb, ta, tb, n, args, dist, nullptr, nullptr, iters, s);
@@ -1938,16 +1952,20 @@ extern "C" int grains_gjk_batch_device_noalloc(grains_ctx_t* ctx, const uint32_t
   hipStream_t s = ctx->stream;
   unsigned char* tab = ctx->scratch;
   unsigned char* ver = ctx->scratch + bt;
-  if (fp64) {
-    GR_HIP(hipMemcpyAsync(tab, ctx->na_np64.data(), S * sizeof(ShapeNP<double>), hipMemcpyHostToDevice, s));
-  } else {
-    GR_HIP(hipMemcpyAsync(tab, ctx->na_np32.data(), S * sizeof(ShapeNP<float>), hipMemcpyHostToDevice, s));
+  const bool in_args = shapes_in_args(ctx);
+  if (!in_args) {
+    GR_HIP(hipMemcpyAsync(tab, fp64 ? (const void*)ctx->na_np64.data() : (const void*)ctx->na_np32.data(),
+                          S * (fp64 ? sizeof(ShapeNP<double>) : sizeof(ShapeNP<float>)), hipMemcpyHostToDevice, s));
+    GR_HIP(hipMemcpyAsync(ver, fp64 ? (const void*)ctx->na_v64.data() : (const void*)ctx->na_v32.data(), bv,
+                          hipMemcpyHostToDevice, s));
   }
-  GR_HIP(hipMemcpyAsync(ver, fp64 ? (const void*)ctx->na_v64.data() : (const void*)ctx->na_v32.data(), bv,
-                        hipMemcpyHostToDevice, s));
   const GjkArgs args = {ctx->cfg.flags, ctx->cfg.gjk_rel_tol};
   GR_HIP(hipEventRecord(ctx->ev0, s));
-  if (fp64)
+  if (in_args && fp64)
+    launch_gjk_batch_args64(ctx->na_np64.data(), S, sa, sb, ta, tb, n, args, dist, iters, s);
+  else if (in_args)
+    launch_gjk_batch_args32(ctx->na_np32.data(), S, sa, sb, ta, tb, n, args, dist, iters, s);
+  else if (fp64)
     launch_gjk_batch64((const ShapeNP<double>*)tab, (const double*)ver, sa, sb, ta, tb, n, args, dist, nullptr,
                        nullptr, iters, s);
   else

@@ -348,6 +348,14 @@ void launch_integrate32(const DevScene& d, hipStream_t s, int part = 0);
 // gr_adjoint.hip: one backward step (the forward step t must have just run)
 void launch_adjoint_step(const DevScene& d, const AdjBufs& a, uint32_t n_tables, hipStream_t s);
 // standalone GJK distance batches (GrainsTestDev workload)
+// shapes in host memory, at most kArgShapes and no polyhedra
+constexpr int kArgShapes = 8;
+void launch_gjk_batch_args64(const ShapeNP<double>* shapes, size_t count, const uint32_t* sa, const uint32_t* sb,
+                             const double* ta, const double* tb, uint64_t n, GjkArgs args, double* dist,
+                             int32_t* iters, hipStream_t s);
+void launch_gjk_batch_args32(const ShapeNP<float>* shapes, size_t count, const uint32_t* sa, const uint32_t* sb,
+                             const double* ta, const double* tb, uint64_t n, GjkArgs args, double* dist,
+                             int32_t* iters, hipStream_t s);
 void launch_gjk_batch64(const ShapeNP<double>* shapes, const double* verts, const uint32_t* sa,
                         const uint32_t* sb, const double* ta, const double* tb, uint64_t n,
                         GjkArgs args, double* dist, double* pa, double* pb, int32_t* iters,

@@ -555,9 +555,12 @@ __device__ __forceinline__ void obstacle_contact64(const DevScene& d, uint32_t s
 // force f and torque m, in FP64; returns whether they touch.  Walls whose plane is
 // farther from the centre than every point of the particle leave the support
 // point on its side: no contact, decided without it.
-__device__ __forceinline__ bool wall_contact64(const DevScene& d, const ShapeNP<double>& A, uint32_t o,
+template <bool BALLS = false>
+__device__ __forceinline__ bool wall_contact64(const DevScene& d, const ShapeNP<double>& A0, uint32_t o,
                                                uint32_t table, V3<double> xi, Qt<double> qi, V3<double> vel,
                                                V3<double> om, V3<double>& f, V3<double>& m) {
+  ShapeNP<double> A = A0;
+  if (BALLS) A.kind = GRAINS_SPHERE;
   const double* t = d.obs_tr + 12 * (size_t)o;
   const uint32_t os = d.obs_shape[o];
   Tr<double> a2w, b2w;
@@ -931,7 +934,7 @@ __global__ void __launch_bounds__(kBlock) k_integrate_obs(DevScene d, const uint
 // ALL: every particle instead of a queue -- a small bed's whole integration
 // in one launch, the step's last (1,000 spheres: 16 + 25 us in two launches -> 18 us;
 // 8,191 touching superquadrics: 22 + 90 us -> 27 us).
-template <class T, bool SO, bool ALL>
+template <class T, bool SO, bool ALL, bool BALLS = false>
 __global__ void __launch_bounds__(kBlock) k_integrate_walls(DevScene d, const uint32_t* __restrict__ list,
                                                            const uint32_t* __restrict__ count) {
   if (!d.nl[kNlRun]) return;
@@ -953,7 +956,7 @@ __global__ void __launch_bounds__(kBlock) k_integrate_walls(DevScene d, const ui
     for (uint32_t o0 = g.obs_begin; o0 < g.obs_end; o0 += G) {
       V3<double> f = {0.0, 0.0, 0.0}, m = f;
       const bool hit = o0 + sub < g.obs_end &&
-                       wall_contact64(d, d.np64[p.si], o0 + sub, g.table, p.xi, p.qi, p.vel, p.om, f, m);
+                       wall_contact64<BALLS>(d, d.np64[p.si], o0 + sub, g.table, p.xi, p.qi, p.vel, p.om, f, m);
       uint32_t hits = (uint32_t)(__ballot(hit) >> (lane - sub)) & ((1u << G) - 1u);
       for (; hits; hits &= hits - 1) {
         const int w = (int)(lane - sub) + __ffs(hits) - 1;
@@ -984,8 +987,11 @@ inline void launch_integrate_so(const DevScene& d, hipStream_t s, int part) {
   // queues are walked grid-stride over their device-held counts
   const dim3 og(std::min<unsigned>(grid.x, (unsigned)cu_count() * 8));
   if (part == 0 && d.nobs && !d.gen_obs && d.n <= kWideIntegrate) {
-    hipLaunchKernelGGL((k_integrate_walls<T, SO, true>), dim3((unsigned)((d.n * 8 + kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0, s, d, nullptr, nullptr);
+    const dim3 eight((unsigned)((d.n * 8 + kBlock - 1) / kBlock));
+    if (sizeof(T) == 8 && d.balls)
+      hipLaunchKernelGGL((k_integrate_walls<T, SO, true, sizeof(T) == 8>), eight, dim3(kBlock), 0, s, d, nullptr, nullptr);
+    else
+      hipLaunchKernelGGL((k_integrate_walls<T, SO, true>), eight, dim3(kBlock), 0, s, d, nullptr, nullptr);
     return;
   }
   if (part == 1)
@@ -1013,12 +1019,11 @@ inline void launch_integrate_t(const DevScene& d, hipStream_t s, int part) {
 
 // GrainsTestDev workload: GJK distance of independent pairs of full shapes.
 template <class T, bool SV>
-__global__ void __launch_bounds__(kBlock) k_gjk_batch(const ShapeNP<T>* __restrict__ shapes,
-                                                     const T* __restrict__ verts, const uint32_t* __restrict__ sa,
-                                                     const uint32_t* __restrict__ sb, const double* __restrict__ ta,
-                                                     const double* __restrict__ tb, uint64_t n, GjkArgs args,
-                                                     double* __restrict__ dist, double* __restrict__ pa,
-                                                     double* __restrict__ pb, int32_t* __restrict__ iters) {
+__device__ __forceinline__ void gjk_batch(const ShapeNP<T>* shapes, const T* verts, const uint32_t* __restrict__ sa,
+                                          const uint32_t* __restrict__ sb, const double* __restrict__ ta,
+                                          const double* __restrict__ tb, uint64_t n, const GjkArgs& args,
+                                          double* __restrict__ dist, double* __restrict__ pa,
+                                          double* __restrict__ pb, int32_t* __restrict__ iters) {
   const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const double* A12 = ta + 12 * k;
@@ -1060,6 +1065,44 @@ __global__ void __launch_bounds__(kBlock) k_gjk_batch(const ShapeNP<T>* __restri
     pb[3 * k + 1] = q.y;
     pb[3 * k + 2] = q.z;
   }
+}
+
+template <class T, bool SV>
+__global__ void __launch_bounds__(kBlock) k_gjk_batch(const ShapeNP<T>* __restrict__ shapes,
+                                                     const T* __restrict__ verts, const uint32_t* __restrict__ sa,
+                                                     const uint32_t* __restrict__ sb, const double* __restrict__ ta,
+                                                     const double* __restrict__ tb, uint64_t n, GjkArgs args,
+                                                     double* __restrict__ dist, double* __restrict__ pa,
+                                                     double* __restrict__ pb, int32_t* __restrict__ iters) {
+  gjk_batch<T, SV>(shapes, verts, sa, sb, ta, tb, n, args, dist, pa, pb, iters);
+}
+// A few shapes without vertices ride in the kernel's arguments instead of
+// memory allocated, filled and freed around the launch (614,400 pairs in FP32:
+// 215 -> 125 us; the witness points it does not return leave it 168
+// registers instead of 241, three waves per SIMD).
+template <class T>
+struct ArgShapes {
+  ShapeNP<T> s[kArgShapes];
+};
+template <class T, bool SV>
+__global__ void __launch_bounds__(kBlock, sizeof(T) == 4 && !SV ? 3 : 1) k_gjk_batch_args(ArgShapes<T> shapes, const uint32_t* __restrict__ sa,
+                                                          const uint32_t* __restrict__ sb,
+                                                          const double* __restrict__ ta,
+                                                          const double* __restrict__ tb, uint64_t n, GjkArgs args,
+                                                          double* __restrict__ dist, int32_t* __restrict__ iters) {
+  gjk_batch<T, SV>(shapes.s, nullptr, sa, sb, ta, tb, n, args, dist, nullptr, nullptr, iters);
+}
+template <class T>
+inline void launch_gjk_batch_args_t(const ShapeNP<T>* shapes, size_t count, const uint32_t* sa, const uint32_t* sb,
+                                    const double* ta, const double* tb, uint64_t n, GjkArgs args, double* dist,
+                                    int32_t* iters, hipStream_t s) {
+  ArgShapes<T> a{};
+  std::copy(shapes, shapes + count, a.s);
+  const dim3 grid((unsigned)((n + 63) / 64)), block(64);  // a wave's registers are free when it ends
+  if (args.flags & GRAINS_REF_QUIRKS)
+    hipLaunchKernelGGL((k_gjk_batch_args<T, false>), grid, block, 0, s, a, sa, sb, ta, tb, n, args, dist, iters);
+  else
+    hipLaunchKernelGGL((k_gjk_batch_args<T, true>), grid, block, 0, s, a, sa, sb, ta, tb, n, args, dist, iters);
 }
 
 }  // namespace gr

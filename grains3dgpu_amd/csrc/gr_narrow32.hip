@@ -30,6 +30,11 @@ void launch_narrow32(const DevScene& d, int pass, hipStream_t s) {
   }
 }
 void launch_integrate32(const DevScene& d, hipStream_t s, int part) { launch_integrate_t<float>(d, s, part); }
+void launch_gjk_batch_args32(const ShapeNP<float>* shapes, size_t count, const uint32_t* sa, const uint32_t* sb,
+                            const double* ta, const double* tb, uint64_t n, GjkArgs args, double* dist,
+                            int32_t* iters, hipStream_t s) {
+  launch_gjk_batch_args_t<float>(shapes, count, sa, sb, ta, tb, n, args, dist, iters, s);
+}
 void launch_gjk_batch32(const ShapeNP<float>* shapes, const float* verts, const uint32_t* sa,
                         const uint32_t* sb, const double* ta, const double* tb, uint64_t n, GjkArgs args,
                         double* dist, double* pa, double* pb, int32_t* iters, hipStream_t s) {

@@ -70,6 +70,11 @@ void launch_refine64(const DevScene& d, hipStream_t s) {
     launch_search64<1>(d, s);
 }
 void launch_integrate64(const DevScene& d, hipStream_t s, int part) { launch_integrate_t<double>(d, s, part); }
+void launch_gjk_batch_args64(const ShapeNP<double>* shapes, size_t count, const uint32_t* sa, const uint32_t* sb,
+                            const double* ta, const double* tb, uint64_t n, GjkArgs args, double* dist,
+                            int32_t* iters, hipStream_t s) {
+  launch_gjk_batch_args_t<double>(shapes, count, sa, sb, ta, tb, n, args, dist, iters, s);
+}
 void launch_gjk_batch64(const ShapeNP<double>* shapes, const double* verts, const uint32_t* sa,
                         const uint32_t* sb, const double* ta, const double* tb, uint64_t n, GjkArgs args,
                         double* dist, double* pa, double* pb, int32_t* iters, hipStream_t s) {
