@@ -53,7 +53,7 @@ OPS_PER_GJK_ITER = 222
 OPS_PER_GJK_PAIR = 390
 # per candidate entry: loads, periodic image, bounding-sphere test (20)
 OPS_PER_ENTRY = 20
-# Compulsory HBM bytes of one narrow-phase launch (k_narrow): each particle's
+# Compulsory HBM bytes of one narrow-phase launch (k_screen): each particle's
 # pose (pos 24 + quat 32, FP64) and shape and sim ids (8) once, each shape's
 # narrow-phase record (ShapeNP<float>, 96) once, each candidate entry's two
 # ids (8) and flag (4), each contact's force and torque (FP32, 24)
@@ -65,17 +65,15 @@ B_NP_CONTACT = 24
 # new one written, per candidate entry, plus each particle's record count
 B_NP_WARM_ENTRY = 32
 B_NP_WARM_PARTICLE = 8
-# Compulsory HBM bytes of one candidate-search launch: each particle's FP64
-# record (32) and FP32 record (16), key, sim and candidate count (12) once;
-# each candidate written (4)
-B_CAND_PARTICLE = 60
-B_CAND_ENTRY = 4
-# the half-shell search by cell (k_candidates_half): each particle's FP32
-# record (16) and FP64 record (32) once, its list count read and written
-# (8); each candidate written (4)
-B_HALF_PARTICLE = 56
-# Compulsory HBM bytes per particle-step of the FP32-mixed step at 3 radix
-# passes (state read 84 + write 80, key+index 8, sort 16 x 3, sorted key 4)
+# Compulsory HBM bytes of one step's integration: each particle's pose (64) and
+# velocity (48) records read and written, the position its lists were built
+# at (32), its shape's dynamics (64), its entries' offset and marks (12);
+# each candidate entry's flag (4); each contact's force and torque (24)
+B_INT_PARTICLE = 332
+B_INT_ENTRY = 4
+B_INT_CONTACT = 24
+# Compulsory HBM bytes per particle-step: the pose and velocity records read
+# and written (112 + 112); FP64 reads an FP64 shape record more of
 B_PS_FP32 = 224
 B_PS_FP64 = 272
 
@@ -225,7 +223,7 @@ def measured_traffic(traffic_file):
 
 
 def narrow_roofline(sc, r, K, traffic=None, warm=True):
-    """Roofline of the screening narrow pass (k_narrow<float,true,2,warm>,
+    """Roofline of the screening narrow pass (k_screen<float,warm>,
     one launch per step): compulsory bytes per launch over its HIP-event
     time."""
     st = r["stats"]
@@ -235,7 +233,7 @@ def narrow_roofline(sc, r, K, traffic=None, warm=True):
     if warm:
         nbytes += E * B_NP_WARM_ENTRY + sc.n * B_NP_WARM_PARTICLE
     achieved_gbs = nbytes / (nar_ms * 1e-3) / 1e9
-    kernel = "k_narrow<float,true,2,true>" if warm else "k_narrow<float,true,2,false>"
+    kernel = "k_screen<float,true>" if warm else "k_screen<float,false>"
     return dict(bound="hbm", kernel=kernel, achieved=achieved_gbs, peak=PEAK_HBM_GBS,
                 unit="GB/s", frac=achieved_gbs / PEAK_HBM_GBS, traffic=(traffic or {}).get(kernel),
                 bytes_per_launch=nbytes, avg_launch_ms=nar_ms,
@@ -245,37 +243,19 @@ def narrow_roofline(sc, r, K, traffic=None, warm=True):
                                                    "records" if warm else "") + "; the launch is gather-latency bound")
 
 
-def candidates_roofline(sc, r, K, kind, traffic=None):
-    """Roofline of the candidate search (one launch per step): compulsory
-    bytes per launch over its HIP-event time.  kind "staged"
-    (k_candidates_staged): each particle's FP64 and FP32 records (32 + 16 B),
-    its key, sim and count (12 B) once, each candidate written (4 B).  "half",
-    the half shell by cell (k_candidates_half, the default on beds of a few
-    particles per cell): each particle's FP32 and FP64 records (16 + 32 B)
-    and its list count read and written (8 B), each candidate written (4 B);
-    the cell offsets (4 B per cell, ~6 particles per cell on the beds) are
-    left out.  A cell's ~87 neighbourhood records are read by its group from
-    the caches; the tests are VALU work.  "half_wl", the same search with
-    several groups on a dense cell, taken from a work list (the library's
-    choice when particles outnumber cells 8 to 1): the same bytes; the
-    phase's time includes the work list's three small launches."""
+def integrate_roofline(sc, r, K, traffic=None):
+    """Roofline of the integration (k_integrate and the queues of particles
+    near obstacles): compulsory bytes per step over its HIP-event time."""
     st = r["stats"]
-    ms = r["phases"]["candidates"]
-    E = st["candidate_pairs"] / K
-    multi = "<true>" if len(sc.sims) > 1 else "<false>"
-    if kind == "staged":
-        nbytes = sc.n * B_CAND_PARTICLE + E * B_CAND_ENTRY
-        kernel = "k_candidates_staged"
-        what = "60 B per particle (FP64 + FP32 records, key, sim, count), 4 B per candidate"
-    else:
-        nbytes = sc.n * B_HALF_PARTICLE + E * B_CAND_ENTRY
-        kernel = ("k_candidates_half_wl" if kind == "half_wl" else "k_candidates_half") + multi
-        what = "56 B per particle (FP32 + FP64 records, list count read and written), 4 B per candidate"
+    ms = r["phases"]["integrate"]
+    nbytes = sc.n * B_INT_PARTICLE + st["candidate_pairs"] / K * B_INT_ENTRY + st["contacts"] / K * B_INT_CONTACT
     achieved_gbs = nbytes / (ms * 1e-3) / 1e9
+    kernel = "k_integrate<float,false>"
     return dict(bound="hbm", kernel=kernel, achieved=achieved_gbs, peak=PEAK_HBM_GBS, unit="GB/s",
                 frac=achieved_gbs / PEAK_HBM_GBS, traffic=(traffic or {}).get(kernel),
                 bytes_per_launch=nbytes, avg_launch_ms=ms,
-                note="candidate search; compulsory bytes: " + what)
+                note="integration; compulsory bytes: 332 B per particle (records read and written, dynamics, list "
+                     "position), 4 B per candidate entry, 24 B per contact")
 
 
 def valu_roofline(r, K):
@@ -284,7 +264,7 @@ def valu_roofline(r, K):
         OPS_PER_ENTRY * st["candidate_pairs"] / K
     nar_all_ms = r["phases"]["narrow"] + r["phases"]["narrow_deferred"]
     achieved = ops / (nar_all_ms * 1e-3) / 1e12
-    return dict(bound="valu", kernel="k_narrow<float,true,2|1>", achieved=achieved, peak=PEAK_FP32_TFLOPS,
+    return dict(bound="valu", kernel="k_screen<float>, k_complete<float>", achieved=achieved, peak=PEAK_FP32_TFLOPS,
                 unit="TFLOP/s", frac=achieved / PEAK_FP32_TFLOPS, ops_per_launch=ops,
                 note="no MFMA: no dense contraction on the path; peak = FP32 vector")
 
@@ -461,12 +441,13 @@ def bench_c1(args):
         agit = accuracy_1000(sa)
 
     # the dominant kernel's roofline: the screening narrow pass or the
-    # candidate search, whichever takes longer per step
+    # integration, whichever takes longer per step (the list builds, the
+    # candidate search among them, serve several steps each)
     traffic = measured_traffic("step_c1_1M_traffic.txt")
-    roof_cand = candidates_roofline(sc, r32, K, "half", traffic)
+    roof_int = integrate_roofline(sc, r32, K, traffic)
     roof_nar = narrow_roofline(sc, r32, K, traffic)
-    roofline, roof_other = ((roof_nar, roof_cand) if r32["phases"]["narrow"] >= r32["phases"]["candidates"]
-                            else (roof_cand, roof_nar))
+    roofline, roof_other = ((roof_nar, roof_int) if r32["phases"]["narrow"] >= r32["phases"]["integrate"]
+                            else (roof_int, roof_nar))
     step_ms = r32["wall_s"] * 1e3 / K
     roofline_step = dict(bound="hbm", bytes_per_particle_step=B_PS_FP32,
                          achieved=B_PS_FP32 * ps32 / 1e9, peak=PEAK_HBM_GBS, unit="GB/s",
@@ -593,7 +574,7 @@ def bench_c2(args):
         gjk_pair_tests_per_s=st["gjk_calls"] / 2 / r32["wall_s"],
         gjk_iterations_per_test=st["gjk_iterations"] / max(st["gjk_calls"], 1),
         step_stats=step_stats(st), phase_ms_per_step=r32["phases"],
-        roofline=candidates_roofline(sc, r32, K, "half_wl"), roofline_narrow=narrow_roofline(sc, r32, K),
+        roofline=integrate_roofline(sc, r32, K), roofline_narrow=narrow_roofline(sc, r32, K),
         roofline_valu=valu_roofline(r32, K), cpu_baseline=cpu,
         speedup_vs_cpu=None if cpu is None else ps32 / cpu["value"])
 
@@ -657,7 +638,7 @@ def bench_c3(args):
         fp32_mixed_error_vs_fp64=err,
         step_stats=step_stats(r32["stats"]), phase_ms_per_step=r32["phases"],
         gjk_pair_tests_per_s=r32["stats"]["gjk_calls"] / 2 / r32["wall_s"],
-        roofline=candidates_roofline(sc, r32, K, "staged" if tuned["candidate_staging"] == 2 else "half"),
+        roofline=integrate_roofline(sc, r32, K),
         roofline_narrow=narrow_roofline(sc, r32, K), roofline_valu=valu_roofline(r32, K), cpu_baseline=cpu,
         speedup_vs_cpu=None if cpu is None else ps32 / cpu["value"])
 

@@ -1,4 +1,5 @@
-// gr_broad.hip -- linked-cell broad phase on the device.
+// gr_broad.hip -- linked-cell broad phase on the device: the neighbour lists'
+// build (spheres grown by half the lists' skin), the state's planes and rows.
 //
 //   k_hash        cell key of every particle (LinkedCell::computeLinearCellHash,
 //                 LinkedCell.cpp:117-149), FP64 divide + floor as the reference
@@ -10,6 +11,8 @@
 //   k_cells       CSR cell offsets from the sorted keys (the cell start/end of
 //                 ComponentManagerGPU_Kernels.cpp:28-75), the inverse
 //                 permutation and the pose records in cell order
+//   k_candidates_half / _half_wl
+//                 per cell, each unordered pair tested once
 //   k_candidates_direct / _staged
 //                 per particle, the 27 cells in the reference order
 //                 (LinkedCell.cpp:41-70) and their residents ascending
@@ -1440,7 +1443,7 @@ __global__ void __launch_bounds__(kBlock) k_warm_carry(DevScene d) {
   }
 }
 
-void launch_expand(const DevScene& d, const uint32_t*, hipStream_t s) {
+void launch_expand(const DevScene& d, hipStream_t s) {
   const dim3 grid((unsigned)((d.n + d.block - 1) / d.block)), block(d.block);
   hipLaunchKernelGGL(k_expand, grid, block, 0, s, d);
   if (d.warm) hipLaunchKernelGGL(k_warm_carry, dim3((unsigned)cu_count() * 8), dim3(kBlock), 0, s, d);

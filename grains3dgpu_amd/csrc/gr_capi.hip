@@ -1114,7 +1114,6 @@ static int finalize(grains_ctx* ctx) {
   d.block = (uint32_t)ctx->cfg.block_size;
   d.narrow_blocks = (uint32_t)(cu_count() * ctx->cfg.narrow_blocks_per_cu);
   d.split = ctx->cfg.narrow_passes == 2 ? 1 : 0;
-  d.overlap = 1;
   d.cand_half = half_of(ctx->cfg.candidate_staging, ctx->sgrids);
   d.cand_staged = staging_of(ctx->cfg.candidate_staging, n, d.ncells, d.cand_half);
   // dense cells on average: the half-shell search takes its groups (several
@@ -1339,7 +1338,7 @@ static void enqueue_build(grains_ctx* ctx) {
   launch_candidates(d, ctx->keys_s, s);
   mark(ctx);
   launch_scan(d.cand_count, d.entry_off, d.n, d.scan_blocks, s, d.K);
-  launch_expand(d, ctx->keys_s, s);
+  launch_expand(d, s);
   mark(ctx);
 }
 
@@ -1357,7 +1356,7 @@ static void enqueue_step(grains_ctx* ctx, bool build) {
   // passes (physics semantics), the step not profiled phase by phase; a
   // small bed's integration is too short to be worth the second stream, and
   // spheres in FP64 have no second pass
-  const bool split = d.overlap && d.n > kWideIntegrate && !(d.balls && d.precision == GRAINS_FP64) && d.split > 0 && !(d.flags & GRAINS_REF_QUIRKS) && !ctx->adj_rec &&
+  const bool split = d.n > kWideIntegrate && !(d.balls && d.precision == GRAINS_FP64) && d.split > 0 && !(d.flags & GRAINS_REF_QUIRKS) && !ctx->adj_rec &&
                      !(ctx->profiling && !ctx->capturing);
   if (d.precision == GRAINS_FP64 && split) {
     launch_narrow64(d, 0, s);

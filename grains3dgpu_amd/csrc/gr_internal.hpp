@@ -255,7 +255,7 @@ struct DevScene {
   uint32_t* obs_count2;
   // Two narrow passes: pend[s] = 1 when the screen left an entry of sorted
   // position s undecided (both particles of the entry are marked; cleared by
-  // the integration).  With `overlap`, the integration of the other particles runs
+  // the integration).  On large beds the integration of the other particles runs
   // while the complete pass and the FP64 re-runs settle those entries, and
   // the marked particles (queued in pend_list, count pend_count, reset by
   // the screen) are integrated after both.
@@ -276,7 +276,6 @@ struct DevScene {
   uint32_t* pend;
   uint32_t* pend_list;
   uint32_t* pend_count;
-  int32_t overlap;
   // per particle outputs
   int32_t* contact_count;
   double *last_force, *last_torque;
@@ -332,7 +331,7 @@ void launch_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* block_
 // the start of a run of n steps: counters cleared, run words set; sort:
 // the sorted order no longer stands
 void launch_run_begin(const DevScene& d, uint32_t n, bool sort, hipStream_t s);
-void launch_expand(const DevScene& d, const uint32_t* keys_s, hipStream_t s);
+void launch_expand(const DevScene& d, hipStream_t s);
 int cu_count();
 // gr_narrow64.hip / gr_narrow32.hip
 // pass 0: every entry (complete, or screened with d.split);

@@ -170,11 +170,13 @@ typedef struct grains_config_t {
   int32_t narrow_blocks_per_cu; /* resident blocks per CU of the persistent
                                narrow-phase launch, in [1, 64] (0: 8;
                                above 64: GRAINS_EINVAL)                     */
-  int32_t narrow_passes;    /* physics semantics: 2 = a screening pass over
-                               every entry (bounding sphere, OBB, GJK's first
+  int32_t narrow_passes;    /* 2 = a screening pass over every entry (bounding
+                               sphere, OBB and, physics semantics, GJK's first
                                support pair) and a complete pass over the
                                undecided entries, compacted; 1 = one complete
-                               pass (0: 2).  Results do not depend on it.   */
+                               pass (0: 2; REF_QUIRKS in FP32 and FP64 beds of
+                               spheres take one).  Results do not depend on
+                               it.                                          */
   int32_t candidate_staging; /* broad phase: 1 = each unordered pair tested
                                once (the residents after it in its cell and
                                13 of the 26 neighbour cells), by cell, dense
@@ -212,7 +214,7 @@ typedef struct grains_stats_t {
   uint64_t fp64_refines;      /* FP32-mixed: GJK re-run in FP64               */
   uint64_t neighbor_overflow; /* candidates dropped: capacity exceeded         */
   uint32_t max_candidates;    /* largest per-particle candidate count seen    */
-  uint32_t sort_passes;       /* radix passes per step                         */
+  uint32_t sort_passes;       /* radix passes a sort of the reference's cells takes */
   double   elapsed_ms;        /* device time of the last grains_step call      */
   uint64_t narrow_deferred;   /* entries the screening pass queued for the
                                  complete narrow pass                          */
@@ -331,9 +333,11 @@ int grains_get_stats(grains_ctx_t* ctx, grains_stats_t* stats);
 /* Per-phase device time of the steps run while profiling is on: HIP events
  * on the context's stream around each kernel group, summed over the steps
  * of the last grains_step call.  Phases, in order: cell hash, radix sort,
- * cell ranges + sorted records, candidates, scan + expand, narrow phase +
- * force (first pass), narrow phase of the deferred entries (second pass),
- * FP64 re-run, reduction + walls + integration. */
+ * cell ranges + sorted records, candidates, scan + expand (these five: the
+ * neighbour lists' builds, each serving the steps until a particle has moved
+ * half the lists' skin), narrow phase + force (first pass), narrow phase of
+ * the deferred entries (second pass), FP64 re-run, reduction + walls +
+ * integration. */
 #define GRAINS_NUM_PHASES 9
 int grains_set_profiling(grains_ctx_t* ctx, int on);
 int grains_get_phase_times(grains_ctx_t* ctx, double* ms, int n_phases);
@@ -348,8 +352,10 @@ int grains_get_phase_times(grains_ctx_t* ctx, double* ms, int n_phases);
  * differentiation of the closest-point conditions).
  * grains_adjoint_record starts a trajectory at the current state and keeps a
  * checkpoint every `checkpoint_every` steps of the following grains_step /
- * grains_step_graph calls.  grains_adjoint then sweeps back over every
- * recorded step, re-running each block of steps from its checkpoint:
+ * grains_step_graph calls, and the states of the steps between while they
+ * take no more than 4 GiB (104 B per particle and step) and the device has
+ * them.  grains_adjoint then sweeps back over every recorded step, first
+ * re-running from its checkpoint a block whose states were not kept:
  * dL_dstate (13 n: pos n x 3, quat n x 4, vel n x 3, omega n x 3, the
  * gradient of the loss at the current state) -> dL_dparams (n_table_entries
  * x 4: kn, en, etat, muc, in the order of grains_set_contact_tables) and,
@@ -379,8 +385,9 @@ int grains_gjk_batch_device(grains_ctx_t* ctx, const uint32_t* shape_a_device,
                             float* elapsed_ms);
 /* grains_gjk_batch_device that allocates nothing: no counterpart in the
  * reference; for callers that cannot allocate device memory (code under HIP
- * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
- * context's shape tables are copied into a fixed 1 MiB device array that
+ * graph capture, tight serving loops, harnesses that forbid hipMalloc).  Up
+ * to eight shapes without polyhedra go as kernel arguments; larger sets' tables
+ * are copied into a fixed 1 MiB device array that
  * the library holds on each GPU until the process ends (at most ~6,500
  * shapes in FP64, ~10,900 in FP32, fewer with polyhedron vertices; larger
  * sets return GRAINS_EINVAL).  Results equal grains_gjk_batch_device's.
