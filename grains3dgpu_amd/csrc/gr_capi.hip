@@ -1379,10 +1379,10 @@ static void enqueue_step(grains_ctx* ctx, bool build) {
     // while the complete pass and the FP64 re-runs settle the others
     launch_narrow32(d, 0, s);
     (void)hipEventRecord(ctx->ev_fork, s);
+    launch_narrow32(d, 1, s);  // first: its few long searches must not wait for room beside the integration
     (void)hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0);
     launch_integrate32(d, ctx->side, 1);
     (void)hipEventRecord(ctx->ev_join, ctx->side);
-    launch_narrow32(d, 1, s);
     launch_refine64(d, s);
     (void)hipStreamWaitEvent(s, ctx->ev_join, 0);
     launch_integrate32(d, s, 2);

@@ -510,7 +510,7 @@ __global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 2) k_screen(DevSc
 // 149 -> 8 + 93 us.
 template <class T, bool WARM, bool SV = true>
 __global__ void __launch_bounds__(kBlock) k_complete(DevScene d) {
-  if ((uint64_t)defer_total(d) * 2 <= (uint64_t)gridDim.x * blockDim.x)
+  if ((uint64_t)defer_total(d) * 2 <= (uint64_t)d.narrow_blocks * blockDim.x)
     narrow<T, SV, 1, WARM, true>(d);
   else
     narrow<T, SV, 1, WARM, false>(d);

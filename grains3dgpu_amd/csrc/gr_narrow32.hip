@@ -23,10 +23,13 @@ void launch_narrow32(const DevScene& d, int pass, hipStream_t s) {
     else
       hipLaunchKernelGGL((k_narrow<float, false>), grid, block, 0, s, d);
   } else if (two) {
+    // as many blocks as are resident at once: eight per CU, most with nothing
+    // to do, queued behind the integration's (10^6 superquadrics: 100 -> 7 us)
+    const dim3 cg(std::min(grid.x, (unsigned)cu_count() * 2));
     if (warm)
-      hipLaunchKernelGGL((k_complete<float, true>), grid, block, 0, s, d);
+      hipLaunchKernelGGL((k_complete<float, true>), cg, block, 0, s, d);
     else
-      hipLaunchKernelGGL((k_complete<float, false>), grid, block, 0, s, d);
+      hipLaunchKernelGGL((k_complete<float, false>), cg, block, 0, s, d);
   }
 }
 void launch_integrate32(const DevScene& d, hipStream_t s, int part) { launch_integrate_t<float>(d, s, part); }
