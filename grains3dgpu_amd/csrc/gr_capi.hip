@@ -2085,15 +2085,17 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
       ctx->adj_save = ctx->adj_blk = nullptr;
       return rc;
     }
-    // the FP64 searches leave their results for the adjoint of their contacts
-    // (without the memory for them it searches again)
-    if (ctx->d.precision == GRAINS_FP64 && ctx->d.split > 0) (void)dalloc(ctx, &a.gjk, ecap * sizeof(GjkRec), L);
     a.max_obs = max_obs;
   }
   // blocks whose steps have to be run again from their checkpoint
   auto logged = [&](uint64_t bb) { return K == 1 || (ctx->adj_log_ok && ctx->adj_log[bb]); };
   for (uint64_t bb = 0; bb * K < T; ++bb)
     if (!logged(bb) && !ctx->adj_blk && (rc = dalloc(ctx, &ctx->adj_blk, K * 13 * n * 8, ctx->adj_allocs))) return rc;
+  // the FP64 searches of two passes leave their results for the adjoint of
+  // their contacts; in one pass, or without the memory for them, it searches
+  // again (the passes can change from one sweep to the next)
+  const bool rec = ctx->d.precision == GRAINS_FP64 && ctx->d.split > 0;
+  if (rec && !a.gjk) (void)dalloc(ctx, &a.gjk, ecap * sizeof(GjkRec), ctx->adj_allocs);
   // the state adjoint, rows -> planes
   {
     std::vector<double> planes(13 * n);
@@ -2120,7 +2122,7 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
   ctx->lists_ok = false;
   ctx->d.keep_torce = 1;
   launch_run_begin(ctx->d, 0u, true, s);
-  ctx->d.gjk_rec = a.gjk;
+  ctx->d.gjk_rec = rec ? a.gjk : nullptr;
   const uint64_t nblocks = (T + K - 1) / K;
   for (uint64_t bb = nblocks; bb-- > 0;) {
     const uint64_t t0 = bb * K, t1 = std::min(t0 + K, T);

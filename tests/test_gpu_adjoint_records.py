@@ -37,3 +37,24 @@ def test_recorded_searches_give_the_same_gradients(which):
     for a, b, c in zip(*out):
         np.testing.assert_array_equal(a, b)
         np.testing.assert_array_equal(a, c)
+
+
+def test_passes_changed_between_two_sweeps():
+    """The records are the step's own: a sweep in one pass, whose searches
+    leave none, does not take those of the sweep before it in two."""
+    from grains3dgpu_amd import engine
+    sc = lattice_superquadrics(n_side=5, n_rng=(2.0, 2.0))
+    rng = np.random.default_rng(6)
+    w = [rng.standard_normal((sc.n, k)) for k in (3, 4, 3, 3)]
+    e = S.load(engine.Engine(dt=sc.dt, precision=A.FP64, gjk_rel_tol=1e-12, narrow_passes=2), sc)
+    e.adjoint_record(5)
+    e.step(12)
+    out = []
+    for passes in (2, 1, 2, 1):
+        e.set_narrow_passes(passes)
+        g, g0 = e.adjoint(*w, want_state0=True)
+        out.append([g, *g0])
+    assert np.abs(out[0][0]).max() > 0
+    for o in out[1:]:
+        for a, b in zip(out[0], o):
+            np.testing.assert_array_equal(a, b)
