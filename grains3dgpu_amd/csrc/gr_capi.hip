@@ -806,6 +806,30 @@ static void adj_drop(grains_ctx* ctx) {
   ctx->adj_count = nullptr;
 }
 
+// The search's cells, and how it runs over them: with a skin those of
+// ctx->sgrids; without one the reference's (ctx->grids), every build for its
+// step alone and a list the step's own candidates, so that it needs no more
+// of max_neighbors than they do, whatever the cells' size.
+static const std::vector<SimGrid>& search_grids(const grains_ctx* ctx) { return ctx->d.skin ? ctx->sgrids : ctx->grids; }
+static void set_search(grains_ctx* ctx, bool skin) {
+  DevScene& d = ctx->d;
+  d.skin = skin ? 1 : 0;
+  const std::vector<SimGrid>& grids = search_grids(ctx);
+  const SimGrid& g = grids.back();
+  d.ncells = g.base + (uint32_t)((uint64_t)g.n3[0] * g.n3[1] * g.n3[2]);
+  int bits = 1;
+  while (bits < 32 && (1ull << bits) < d.ncells) ++bits;
+  // fewest LSD passes of digits up to kRadixMaxBits wide, digits at least 8
+  // bits: an 18-bit key sorts in 2 passes of 9 bits instead of 3 of 8
+  ctx->passes = (bits + kRadixMaxBits - 1) / kRadixMaxBits;
+  ctx->digit_bits = std::max(8, (bits + ctx->passes - 1) / ctx->passes);
+  d.cand_half = half_of(ctx->cfg.candidate_staging, grids);
+  d.cand_staged = staging_of(ctx->cfg.candidate_staging, ctx->n, d.ncells, d.cand_half);
+  // dense cells on average: the half-shell search takes its groups (several
+  // on a dense cell) from a work list built each step
+  d.half_wl = ctx->n > 8 * (uint64_t)d.ncells ? 1 : 0;
+}
+
 static int finalize(grains_ctx* ctx) {
   if (ctx->layout_ok) return GRAINS_OK;
   if (!ctx->n) return fail(ctx, GRAINS_ESTATE, "no particles");
@@ -894,9 +918,7 @@ static int finalize(grains_ctx* ctx) {
   // beds (369,564) 0.358 / 0.356 / 0.354 / 0.367; lists built every step:
   // 0.58, 0.52, 0.40, 0.58.
   // A periodic axis that would hold fewer than three such cells leaves the
-  // whole context without a skin: the lists are then built every step, in
-  // cells at least two radii wide, or where even those do not fit, in the
-  // reference's.
+  // whole context without a skin (set_search).
   std::vector<double> rmean(ns, 0.0);
   std::vector<uint64_t> rnum(ns, 0);
   for (uint64_t i = 0; i < ctx->n; ++i) {
@@ -904,45 +926,29 @@ static int finalize(grains_ctx* ctx) {
     rmean[ctx->psim[i]] += quirks ? h.rc : h.rc_exact;
     ++rnum[ctx->psim[i]];
   }
+  bool skin_fits = true;
   uint64_t sbase = 0;
-  for (int with = 1; with >= 0; --with) {
-    ctx->sgrids = ctx->grids;
-    d.skin = with;
-    sbase = 0;
-    for (uint32_t s = 0; s < ns; ++s) {
-      SimGrid& g = ctx->sgrids[s];
-      const double skin = with && rnum[s] ? 0.1 * rmean[s] / (double)rnum[s] : 0.0;
-      double h = std::max(g.h, (2.0 * lc[s] + skin) * (1.0 + 1e-9));
-      for (int k = 0; k < 3; ++k) {
-        if (!(skin > 1e-9 * g.L[k]) && rnum[s]) d.skin = 0;
-        if (((g.periodic >> k) & 1) && g.L[k] < 3.0 * h) {
-          d.skin = 0;
-          h = g.h;  // (without a skin: the reference's cells)
-        }
-      }
-      if (h != g.h)
-        for (int k = 0; k < 3; ++k) g.n3[k] = (uint32_t)std::max(1.0, g.L[k] / h);
-      g.h = h;
-      g.half_skin = 0.5 * skin;
-      g.move2 = 0.25 * skin * skin * (1.0 - 1e-6) * (1.0 - 1e-6);
-      g.base = (uint32_t)sbase;
-      sbase += (uint64_t)g.n3[0] * g.n3[1] * g.n3[2];
-      ctx->grids[s].move2 = g.move2;
-    }
-    if (d.skin == with) break;
+  ctx->sgrids = ctx->grids;
+  for (uint32_t s = 0; s < ns; ++s) {
+    SimGrid& g = ctx->sgrids[s];
+    const double skin = rnum[s] ? 0.1 * rmean[s] / (double)rnum[s] : 0.0;
+    const double h = std::max(g.h, (2.0 * lc[s] + skin) * (1.0 + 1e-9));
+    for (int k = 0; k < 3; ++k)
+      if ((rnum[s] && !(skin > 1e-9 * g.L[k])) || (((g.periodic >> k) & 1) && g.L[k] < 3.0 * h)) skin_fits = false;
+    if (h != g.h)
+      for (int k = 0; k < 3; ++k) g.n3[k] = (uint32_t)std::max(1.0, g.L[k] / h);
+    g.h = h;
+    g.half_skin = 0.5 * skin;
+    g.move2 = 0.25 * skin * skin * (1.0 - 1e-6) * (1.0 - 1e-6);
+    g.base = (uint32_t)sbase;
+    sbase += (uint64_t)g.n3[0] * g.n3[1] * g.n3[2];
+    ctx->grids[s].move2 = g.move2;
   }
-  d.ncells = (uint32_t)sbase;
-  int bits = 1;
-  while (bits < 32 && (1ull << bits) < sbase) ++bits;
-  // fewest LSD passes of digits up to kRadixMaxBits wide, digits at least 8
-  // bits: an 18-bit key sorts in 2 passes of 9 bits instead of 3 of 8
-  ctx->passes = (bits + kRadixMaxBits - 1) / kRadixMaxBits;
   {
     int ref = 1;
     while (ref < 32 && (1ull << ref) < base) ++ref;
     ctx->ref_passes = (ref + kRadixMaxBits - 1) / kRadixMaxBits;
   }
-  ctx->digit_bits = std::max(8, (bits + ctx->passes - 1) / ctx->passes);
   // shape tables
   const size_t S = ctx->shapes.size();
   std::vector<ShapeNP<double>> np64(S);
@@ -984,7 +990,7 @@ static int finalize(grains_ctx* ctx) {
     hk32[i] = {(float)t.kn, (float)t.en, (float)t.etat, (float)t.muc, (float)t.kr, (float)muen};
   }
   auto& L = ctx->allocs;
-  const uint64_t n = ctx->n;
+  const uint64_t n = ctx->n;  // (the arrays by cell hold the search's cells with and without a skin: never more than base)
   const uint32_t K = (uint32_t)ctx->cfg.max_neighbors;
   const uint64_t ecap = n * K;
   const uint64_t ntiles = (n + kTile - 1) / kTile;
@@ -993,7 +999,7 @@ static int finalize(grains_ctx* ctx) {
   const uint64_t max_nb = (uint64_t)cu_count() * kMaxNarrowPerCu;
   const uint64_t nhist = (uint64_t)kRadixMaxDigits * ntiles;  // histogram of the widest digit
   const uint64_t nblk = std::max(std::max((n + kTile - 1) / kTile, (nhist + kTile - 1) / kTile),
-                                 std::max((max_nb + kTile) / kTile, ((uint64_t)d.ncells + kTile) / kTile)) +
+                                 std::max((max_nb + kTile) / kTile, (base + kTile) / kTile)) +
                         2;
   // entry results in FP64 for the plain path and for FP32-mixed with FP64
   // contact geometry (whose contacts all come from FP64 re-runs)
@@ -1021,12 +1027,12 @@ static int finalize(grains_ctx* ctx) {
       (rc = dalloc(ctx, &potr, (otr.size() + 12) * sizeof(double), L)) ||
       (rc = dalloc(ctx, &d.key, n * 4, L)) || (rc = dalloc(ctx, &d.keyA, n * 4, L)) || (rc = dalloc(ctx, &d.idxA, n * 4, L)) ||
       (rc = dalloc(ctx, &d.keyB, n * 4, L)) || (rc = dalloc(ctx, &d.idxB, n * 4, L)) || (rc = dalloc(ctx, &d.rank, n * 4, L)) ||
-      (rc = dalloc(ctx, &d.cell_off, ((size_t)d.ncells + 1) * 4, L)) ||
+      (rc = dalloc(ctx, &d.cell_off, (base + 1) * 4, L)) ||
       (rc = dalloc(ctx, &d.bp, n * sizeof(double4), L)) || (rc = dalloc(ctx, &d.pk, n * sizeof(PoseRec), L)) ||
       (rc = dalloc(ctx, &d.vk, n * sizeof(VelRec), L)) || (rc = dalloc(ctx, &d.rws, n * 8, L)) ||
       (rc = dalloc(ctx, &d.bp32, n * sizeof(float4), L)) ||
-      (rc = dalloc(ctx, &d.cell_sph, ((size_t)d.ncells + 1) * sizeof(float4), L)) ||
-      (rc = dalloc(ctx, &d.half_goff, ((size_t)d.ncells + 1) * 4, L)) || (rc = dalloc(ctx, &d.half_glist, n * 4, L)) ||
+      (rc = dalloc(ctx, &d.cell_sph, (base + 1) * sizeof(float4), L)) ||
+      (rc = dalloc(ctx, &d.half_goff, (base + 1) * 4, L)) || (rc = dalloc(ctx, &d.half_glist, n * 4, L)) ||
       (rc = dalloc(ctx, &d.hist, (nhist + 1) * 4, L)) || (rc = dalloc(ctx, &d.scan_blocks, nblk * 4, L)) ||
       (rc = dalloc(ctx, &d.cand, ecap * 4, L)) || (rc = dalloc(ctx, &d.cand_count, n * 4, L)) ||
       (rc = dalloc(ctx, &d.entry_off, (n + 1) * 4, L)) || (rc = dalloc(ctx, &d.pair_i, ecap * 4, L)) ||
@@ -1078,7 +1084,8 @@ static int finalize(grains_ctx* ctx) {
   GR_HIP(hipMemcpy(ph64, hk64.data(), hk64.size() * sizeof(HookeP<double>), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(ph32, hk32.data(), hk32.size() * sizeof(HookeP<float>), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(pgr, ctx->grids.data(), ns * sizeof(SimGrid), hipMemcpyHostToDevice));
-  GR_HIP(hipMemcpy(psg, ctx->sgrids.data(), ns * sizeof(SimGrid), hipMemcpyHostToDevice));
+  set_search(ctx, skin_fits);
+  GR_HIP(hipMemcpy(psg, search_grids(ctx).data(), ns * sizeof(SimGrid), hipMemcpyHostToDevice));
   if (!osh.empty()) {
     GR_HIP(hipMemcpy(posh, osh.data(), osh.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     GR_HIP(hipMemcpy(potr, otr.data(), otr.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -1114,11 +1121,6 @@ static int finalize(grains_ctx* ctx) {
   d.block = (uint32_t)ctx->cfg.block_size;
   d.narrow_blocks = (uint32_t)(cu_count() * ctx->cfg.narrow_blocks_per_cu);
   d.split = ctx->cfg.narrow_passes == 2 ? 1 : 0;
-  d.cand_half = half_of(ctx->cfg.candidate_staging, ctx->sgrids);
-  d.cand_staged = staging_of(ctx->cfg.candidate_staging, n, d.ncells, d.cand_half);
-  // dense cells on average: the half-shell search takes its groups (several
-  // on a dense cell) from a work list built each step
-  d.half_wl = n > 8 * (uint64_t)d.ncells ? 1 : 0;
   // a small bed sorts in one block (measured: 1,000 particles 0.113 ->
   // 0.094 ms/step; 2,048, 4,096 and 8,192 slower than the radix passes and
   // the merge: 0.267, 0.352, 0.425 against 0.255, 0.320, 0.338 ms);
@@ -1438,15 +1440,13 @@ static void read_stats(grains_ctx* ctx, uint32_t steps) {
   st.sort_passes = (uint32_t)ctx->ref_passes;
 }
 
-// The lists with their skin (on) or without: every build then holds for its
-// step alone, and a list is the step's own candidates.
+// The lists with their skin (on) or without, from the next build on.
 static int use_skin(grains_ctx* ctx, bool on) {
-  std::vector<SimGrid> g = ctx->sgrids;
-  if (!on)
-    for (SimGrid& x : g) x.half_skin = 0.0;
   GR_HIP(hipStreamSynchronize(ctx->stream));
+  set_search(ctx, on);
+  const std::vector<SimGrid>& g = search_grids(ctx);
   GR_HIP(hipMemcpy((void*)ctx->d.sgrids, g.data(), g.size() * sizeof(SimGrid), hipMemcpyHostToDevice));
-  ctx->d.skin = on ? 1 : 0;
+  launch_fill_u32(ctx->d.sort_state, 3, 0u, ctx->stream);  // the standing order is that of other cells
   ctx->lists_ok = false;
   drop_graph(ctx);  // captured kernels hold the flag
   return GRAINS_OK;
@@ -1662,8 +1662,7 @@ extern "C" int grains_set_narrow_passes(grains_ctx_t* ctx, int passes) {
 extern "C" int grains_set_candidate_staging(grains_ctx_t* ctx, int mode) {
   if (!ctx || mode < 0 || mode > 3) return GRAINS_EINVAL;
   ctx->cfg.candidate_staging = mode;
-  ctx->d.cand_half = half_of(mode, ctx->sgrids);
-  ctx->d.cand_staged = staging_of(mode, ctx->d.n, ctx->d.ncells, ctx->d.cand_half);
+  if (ctx->layout_ok) set_search(ctx, ctx->d.skin != 0);
   drop_graph(ctx);  // a captured build holds the old kernel
   ctx->lists_ok = false;
   return GRAINS_OK;

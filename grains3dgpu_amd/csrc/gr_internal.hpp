@@ -183,7 +183,7 @@ struct DevScene {
   const HookeP<double>* hooke64;
   const HookeP<float>* hooke32;
   const SimGrid* grids;         // the reference's cells (keys, adjacency, visit order)
-  const SimGrid* sgrids;        // the search's cells (at least a list reach wide)
+  const SimGrid* sgrids;        // the search's cells (with a skin at least a list reach wide, else the reference's)
   const uint32_t* obs_shape;    // sorted by sim
   const double* obs_tr;         // 12 doubles each
   // broad phase

@@ -146,3 +146,20 @@ def test_state_between_the_steps_of_a_run(which, scheme):
     for a, b, c in zip(whole.get_torce(), cut.get_torce(), single.get_torce()):
         np.testing.assert_array_equal(a, b)
         np.testing.assert_array_equal(a, c)
+
+
+def test_lists_of_small_cells_hold_their_candidates_only():
+    """Cells smaller than the grains: pairs that overlap beyond neighbouring
+    cells are no candidates and take no room in max_neighbors (at most 8 of
+    the 13 overlapping neighbours of a sphere here)."""
+    from grains3dgpu_amd import engine
+    sc = dense_spheres(n=600, seed=5, vel=0.01)
+    sc.sims[0]["cell_size"] = 0.35e-3
+    full = S.load(engine.Engine(dt=sc.dt, max_neighbors=96), sc)
+    full.step(5)
+    most = full.get_stats()["max_candidates"]
+    assert most == 8
+    tight = S.load(engine.Engine(dt=sc.dt, max_neighbors=most), sc)
+    tight.step(5)
+    for a, b in zip(result(tight), result(full)):
+        np.testing.assert_array_equal(a, b)
