@@ -94,7 +94,7 @@ enum ListState {
   kNlLast,        // it is the run's last step
   kNlDone,        // steps of the run taken
   kNlTarget,      // steps of the run asked for
-  kNlOver,        // a list outgrew max_neighbors when the lists were built
+  kNlOver,        // a list outgrew max_neighbors when the lists were built (2: with its skin, and no step uses them)
   kNlOutside,     // a centre lay outside a periodic side when they were built
   kNlStale,       // the records by sorted position are ahead of the state's planes
   kNlWords = 8

@@ -163,3 +163,26 @@ def test_lists_of_small_cells_hold_their_candidates_only():
     tight.step(5)
     for a, b in zip(result(tight), result(full)):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("mode", [0, 3])
+def test_lists_that_outgrow_their_room_keep_the_warm_starts(mode):
+    """A bed drawn together until its lists with the skin outgrow
+    max_neighbors in the middle of a run: the directions its searches start
+    from outlast the build that did not fit."""
+    from grains3dgpu_amd import engine
+    sc = dense_superquadrics(n=400, seed=9, phi=0.12, vel=0.0, periodic=0, walls=False)
+    mid = 0.5 * np.asarray(sc.sims[0]["domain_max"])
+    sc.vel = -4000.0 * (sc.pos - mid)
+
+    def make(k):
+        return S.load(engine.Engine(dt=sc.dt, precision=A.FP32_MIXED, flags=A.WARM_START | A.FP64_CONTACTS,
+                                    max_neighbors=k, gjk_rel_tol=1e-6, candidate_staging=mode), sc)
+    roomy = make(128)
+    roomy.step(60)
+    most = roomy.get_stats()["max_candidates"]
+    tight = make(most)
+    tight.step(60)
+    assert tight.get_stats()["max_candidates"] == most
+    for a, b in zip(result(tight), result(roomy)):
+        np.testing.assert_array_equal(a, b)
