@@ -38,18 +38,20 @@ void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s) {
 }
 
 // ---- the start of a run -------------------------------------------------------------
-__global__ void k_run_begin(DevScene d, uint32_t n, int sort) {
+// fresh: the lists do not stand (nor the sorted order), and the planes hold
+// the state, whatever a run that stopped early left in the records.
+__global__ void k_run_begin(DevScene d, uint32_t n, int fresh) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < (uint32_t)kNumCounters * kCntSlots) d.counters[i] = 0ull;
   if (i == 0) {
     d.nl[kNlDone] = 0u;
     d.nl[kNlTarget] = n;
-    if (sort) d.sort_state[0] = d.sort_state[2] = 0u;
+    if (fresh) d.sort_state[0] = d.sort_state[2] = d.nl[kNlStale] = 0u;
   }
 }
-void launch_run_begin(const DevScene& d, uint32_t n, bool sort, hipStream_t s) {
+void launch_run_begin(const DevScene& d, uint32_t n, bool fresh, hipStream_t s) {
   constexpr unsigned words = kNumCounters * kCntSlots;
-  hipLaunchKernelGGL(k_run_begin, dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d, n, sort ? 1 : 0);
+  hipLaunchKernelGGL(k_run_begin, dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d, n, fresh ? 1 : 0);
 }
 
 // ---- cell hash --------------------------------------------------------------------
@@ -105,7 +107,7 @@ void launch_hash(const DevScene& d, const uint32_t* keys_prev, hipStream_t s) {
   hipLaunchKernelGGL(k_hash, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d, keys_prev);
 }
 
-// the planes of a run's state between two of its steps
+// the planes of the state a run has reached between two of its steps
 __global__ void k_store_state(DevScene d) {
   if (!d.nl[kNlStale]) return;
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -139,9 +141,12 @@ __global__ void k_log_state(DevScene d) {
 void launch_log_state(const DevScene& d, hipStream_t s) {
   hipLaunchKernelGGL(k_log_state, dim3((unsigned)((d.n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d);
 }
-__global__ void k_log_set(StateLog* log, StateLog v) { *log = v; }
-void launch_log_set(const DevScene& d, StateLog v, hipStream_t s) {
-  hipLaunchKernelGGL(k_log_set, dim3(1), dim3(1), 0, s, d.log, v);
+__global__ void k_log_set(DevScene d, StateLog v, uint32_t target) {
+  *d.log = v;
+  d.nl[kNlTarget] = target;
+}
+void launch_log_set(const DevScene& d, StateLog v, uint32_t target, hipStream_t s) {
+  hipLaunchKernelGGL(k_log_set, dim3(1), dim3(1), 0, s, d, v, target);
 }
 
 // Particles [i0, i0 + m) of the state's planes as rows, into the host's

@@ -406,6 +406,7 @@ struct grains_ctx {
   uint64_t adj_steps = 0;
   std::vector<void*> adj_cp;      // state every adj_every steps (13 planes)
   std::vector<void*> adj_allocs;  // sweep buffers
+  uint64_t adj_cap = 0;           // the most device bytes the recording and its sweeps hold (0: what the device has)
   std::vector<double*> adj_log;   // per block of adj_every steps, the states between (null: run again from its checkpoint)
   std::vector<void*> adj_log_allocs;
   bool adj_log_ok = false;        // the logged steps followed each other (no state set between)
@@ -558,6 +559,7 @@ extern "C" int grains_create(const grains_config_t* cfg, grains_ctx_t** out) {
     delete ctx;
     return GRAINS_EINVAL;
   }
+  if (const char* e = std::getenv("GRAINS_ADJOINT_BYTES")) ctx->adj_cap = std::strtoull(e, nullptr, 10);
   if (ctx->cfg.gjk_rel_tol_fp64 == 0) ctx->cfg.gjk_rel_tol_fp64 = 1e-10;
   if (ctx->cfg.narrow_blocks_per_cu <= 0) ctx->cfg.narrow_blocks_per_cu = 8;
   // the narrow phase's queue segments and their scan are sized for at most
@@ -791,6 +793,23 @@ static uint64_t defer_words(uint64_t ecap) {
   const uint64_t cus = (uint64_t)cu_count();
   return ecap + (kDeferQueues - 1) * (ecap / cus + 1) + (cus * kMaxNarrowPerCu + kDeferQueues) * 256 +
          64 * kXcds * kDeferQueues;
+}
+
+// Device memory of the recording and its sweeps, within adj_cap.
+template <class P>
+static int adj_dalloc(grains_ctx* ctx, P** p, size_t bytes, std::vector<void*>& list) {
+  if (ctx->adj_cap) {
+    uint64_t held = bytes;
+    for (const auto* l : {&ctx->adj_cp, &ctx->adj_allocs, &ctx->adj_log_allocs})
+      for (void* q : *l) {
+        size_t b = 0;
+        GR_HIP(hipMemPtrGetInfo(q, &b));
+        held += b;
+      }
+    if (held > ctx->adj_cap)
+      return fail(ctx, GRAINS_ENOMEM, std::to_string(bytes) + " bytes more for the adjoint pass GRAINS_ADJOINT_BYTES");
+  }
+  return dalloc(ctx, p, bytes, list);
 }
 
 static void adj_drop(grains_ctx* ctx) {
@@ -1463,32 +1482,34 @@ static int state_from(grains_ctx* ctx, const double* src) {
   return GRAINS_OK;
 }
 // after recorded steps (never past a checkpoint): a checkpoint every
-// adj_every steps
+// adj_every steps, of the planes that its step has written (log_chunk)
 static int adj_after_steps(grains_ctx* ctx, uint32_t steps) {
   ctx->adj_steps += steps;
   if (!steps || ctx->adj_steps % ctx->adj_every) return GRAINS_OK;
   double* cp;
-  int rc = dalloc(ctx, &cp, 13 * ctx->n * 8, ctx->adj_cp);
+  int rc = adj_dalloc(ctx, &cp, 13 * ctx->n * 8, ctx->adj_cp);
   if (rc) return rc;
-  launch_store_state(ctx->d, ctx->stream);
   return state_to(ctx, cp);
 }
 
 // The states of a recorded trajectory's steps are kept beside its checkpoints
 // while they fit kLogBytes (and the device), so that the sweep need not run
 // them again: its block's memory (null: no more), and the place of the steps
-// of a run of which `done` are taken.
+// of a run of which `done` are taken.  The step that reaches the next
+// checkpoint writes its results as a run's last does (target: the run's steps
+// up to there): a checkpoint copies them, and a run that stops there because
+// it finds no memory has them.
 constexpr uint64_t kLogBytes = 4ull << 30;
-static int log_chunk(grains_ctx* ctx, uint32_t done) {
+static int log_chunk(grains_ctx* ctx, uint32_t done, uint32_t target) {
   const uint64_t K = ctx->adj_every, blk = ctx->adj_steps / K, bytes = 13 * ctx->n * 8 * K;
   while (ctx->adj_log.size() <= blk) {
     double* p = nullptr;
     const uint64_t used = ctx->adj_log_allocs.size() * bytes;
     if (K > 1 && bytes / K / 13 / 8 == ctx->n && bytes <= kLogBytes && used <= kLogBytes - bytes)
-      (void)dalloc(ctx, &p, bytes, ctx->adj_log_allocs);
+      (void)adj_dalloc(ctx, &p, bytes, ctx->adj_log_allocs);
     ctx->adj_log.push_back(p);
   }
-  launch_log_set(ctx->d, {ctx->adj_log[blk], (int64_t)(ctx->adj_steps % K) - (int64_t)done, K}, ctx->stream);
+  launch_log_set(ctx->d, {ctx->adj_log[blk], (int64_t)(ctx->adj_steps % K) - (int64_t)done, K}, target, ctx->stream);
   GR_HIP(hipGetLastError());
   return GRAINS_OK;
 }
@@ -1497,9 +1518,8 @@ static int log_chunk(grains_ctx* ctx, uint32_t done) {
 // for; the kernels of a step whose lists no longer hold return at once, and
 // after each chunk the host reads how many were taken, builds new lists when
 // they ran out, and goes on.
-static int run_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
-  int rc = finalize(ctx);
-  if (rc) return rc;
+static int take_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
+  int rc;
   hipStream_t s = ctx->stream;
   launch_run_begin(ctx->d, n_steps, !ctx->lists_ok, s);
   // 0: the lists' build; otherwise that many steps
@@ -1545,8 +1565,10 @@ static int run_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
   uint32_t done = 0, nl[kNlWords] = {0};
   while (done < n_steps) {
     uint32_t m = n_steps - done;
-    if (ctx->adj_rec) m = std::min<uint32_t>(m, ctx->adj_every - (uint32_t)(ctx->adj_steps % ctx->adj_every));
-    if (ctx->adj_rec && (rc = log_chunk(ctx, done))) return rc;
+    if (ctx->adj_rec) {
+      m = std::min<uint32_t>(m, ctx->adj_every - (uint32_t)(ctx->adj_steps % ctx->adj_every));
+      if ((rc = log_chunk(ctx, done, done + m))) return rc;
+    }
     const bool each = !ctx->d.skin || ctx->interval <= 1;  // lists for one step at a time
     if (each) {
       m = std::min(m, 64u);
@@ -1615,6 +1637,20 @@ static int run_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
     return fail(ctx, GRAINS_EOVERFLOW, "candidate capacity max_neighbors exceeded (" +
                                            std::to_string(ctx->stats.max_candidates) + " needed)");
   return GRAINS_OK;
+}
+
+static int run_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
+  int rc = finalize(ctx);
+  if (rc) return rc;
+  rc = take_steps(ctx, n_steps, graph);
+  if (rc) {
+    // A run that stops early may have taken steps whose records are ahead of
+    // the planes: these take them, and the next run starts from the planes.
+    launch_store_state(ctx->d, ctx->stream);
+    (void)hipStreamSynchronize(ctx->stream);
+    ctx->lists_ok = false;
+  }
+  return rc;
 }
 
 extern "C" int grains_step(grains_ctx_t* ctx, uint32_t n_steps) {
@@ -2055,7 +2091,7 @@ extern "C" int grains_adjoint_record(grains_ctx_t* ctx, uint32_t checkpoint_ever
   ctx->adj_steps = 0;
   ctx->adj_rec = true;
   double* cp;
-  if ((rc = dalloc(ctx, &cp, 13 * ctx->n * 8, ctx->adj_cp)) || (rc = state_to(ctx, cp))) return rc;
+  if ((rc = adj_dalloc(ctx, &cp, 13 * ctx->n * 8, ctx->adj_cp)) || (rc = state_to(ctx, cp))) return rc;
   GR_HIP(hipStreamSynchronize(ctx->stream));
   return GRAINS_OK;
 }
@@ -2072,13 +2108,13 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
     uint32_t max_obs = 1;
     for (const SimGrid& g : ctx->grids) max_obs = std::max(max_obs, g.obs_end - g.obs_begin);
     auto& L = ctx->adj_allocs;
-    if ((rc = dalloc(ctx, &ctx->adj_save, 13 * n * 8, L)) ||
-        (rc = dalloc(ctx, &ctx->adj_count, n * 4, L)) || (rc = dalloc(ctx, &a.abar, 13 * n * 8, L)) ||
-        (rc = dalloc(ctx, &a.own, 13 * n * 8, L)) || (rc = dalloc(ctx, &a.Fb, 3 * n * 8, L)) ||
-        (rc = dalloc(ctx, &a.Mb, 3 * n * 8, L)) || (rc = dalloc(ctx, &a.part_i, ecap * 13 * 8, L)) ||
-        (rc = dalloc(ctx, &a.part_j, ecap * 13 * 8, L)) || (rc = dalloc(ctx, &a.entry_theta, ecap * 4 * 8, L)) ||
-        (rc = dalloc(ctx, &a.entry_tidx, ecap * 4, L)) || (rc = dalloc(ctx, &a.wall_theta, n * max_obs * 4 * 8, L)) ||
-        (rc = dalloc(ctx, &a.wall_tidx, n * max_obs * 4, L)) || (rc = dalloc(ctx, &a.dtheta, (size_t)ntab * 4 * 8, L))) {
+    if ((rc = adj_dalloc(ctx, &ctx->adj_save, 13 * n * 8, L)) ||
+        (rc = adj_dalloc(ctx, &ctx->adj_count, n * 4, L)) || (rc = adj_dalloc(ctx, &a.abar, 13 * n * 8, L)) ||
+        (rc = adj_dalloc(ctx, &a.own, 13 * n * 8, L)) || (rc = adj_dalloc(ctx, &a.Fb, 3 * n * 8, L)) ||
+        (rc = adj_dalloc(ctx, &a.Mb, 3 * n * 8, L)) || (rc = adj_dalloc(ctx, &a.part_i, ecap * 13 * 8, L)) ||
+        (rc = adj_dalloc(ctx, &a.part_j, ecap * 13 * 8, L)) || (rc = adj_dalloc(ctx, &a.entry_theta, ecap * 4 * 8, L)) ||
+        (rc = adj_dalloc(ctx, &a.entry_tidx, ecap * 4, L)) || (rc = adj_dalloc(ctx, &a.wall_theta, n * max_obs * 4 * 8, L)) ||
+        (rc = adj_dalloc(ctx, &a.wall_tidx, n * max_obs * 4, L)) || (rc = adj_dalloc(ctx, &a.dtheta, (size_t)ntab * 4 * 8, L))) {
       free_list(L);
       a = AdjBufs{};
       ctx->adj_save = ctx->adj_blk = nullptr;
@@ -2089,12 +2125,12 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
   // blocks whose steps have to be run again from their checkpoint
   auto logged = [&](uint64_t bb) { return K == 1 || (ctx->adj_log_ok && ctx->adj_log[bb]); };
   for (uint64_t bb = 0; bb * K < T; ++bb)
-    if (!logged(bb) && !ctx->adj_blk && (rc = dalloc(ctx, &ctx->adj_blk, K * 13 * n * 8, ctx->adj_allocs))) return rc;
+    if (!logged(bb) && !ctx->adj_blk && (rc = adj_dalloc(ctx, &ctx->adj_blk, K * 13 * n * 8, ctx->adj_allocs))) return rc;
   // the FP64 searches of two passes leave their results for the adjoint of
   // their contacts; in one pass, or without the memory for them, it searches
   // again (the passes can change from one sweep to the next)
   const bool rec = ctx->d.precision == GRAINS_FP64 && ctx->d.split > 0;
-  if (rec && !a.gjk) (void)dalloc(ctx, &a.gjk, ecap * sizeof(GjkRec), ctx->adj_allocs);
+  if (rec && !a.gjk) (void)adj_dalloc(ctx, &a.gjk, ecap * sizeof(GjkRec), ctx->adj_allocs);
   // the state adjoint, rows -> planes
   {
     std::vector<double> planes(13 * n);

@@ -91,9 +91,9 @@ enum Counter {
 enum ListState {
   kNlValid = 0,   // the lists cover the current positions (2: for one step only)
   kNlRun,         // this step runs (latched from kNlValid by its first kernel)
-  kNlLast,        // it is the run's last step
+  kNlLast,        // it is the run's last step, or a checkpoint's
   kNlDone,        // steps of the run taken
-  kNlTarget,      // steps of the run asked for
+  kNlTarget,      // steps of the run asked for (recorded: up to the next checkpoint)
   kNlOver,        // a list outgrew max_neighbors when the lists were built (2: with its skin, and no step uses them)
   kNlOutside,     // a centre lay outside a periodic side when they were built
   kNlStale,       // the records by sorted position are ahead of the state's planes
@@ -314,7 +314,7 @@ void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 // keys_prev: the sort's output buffer (the previous step's sorted keys)
 void launch_store_state(const DevScene& d, hipStream_t s);
 void launch_log_state(const DevScene& d, hipStream_t s);
-void launch_log_set(const DevScene& d, StateLog v, hipStream_t s);
+void launch_log_set(const DevScene& d, StateLog v, uint32_t target, hipStream_t s);
 void launch_state_rows(const DevScene& d, uint64_t i0, uint64_t m, double* out, hipStream_t s);
 void launch_hash(const DevScene& d, const uint32_t* keys_prev, hipStream_t s);
 // sorts (d.key, identity) into the returned buffers: `passes` LSD passes of
@@ -328,9 +328,9 @@ void launch_candidates(const DevScene& d, const uint32_t* keys_s, hipStream_t s)
 // the kernels return at once unless *gate == 0
 void launch_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* block_sums, hipStream_t s,
                  uint32_t clamp = 0xffffffffu, const uint32_t* gate = nullptr);
-// the start of a run of n steps: counters cleared, run words set; sort:
-// the sorted order no longer stands
-void launch_run_begin(const DevScene& d, uint32_t n, bool sort, hipStream_t s);
+// the start of a run of n steps: counters cleared, run words set; fresh: the
+// lists and the sorted order no longer stand, the planes hold the state
+void launch_run_begin(const DevScene& d, uint32_t n, bool fresh, hipStream_t s);
 void launch_expand(const DevScene& d, hipStream_t s);
 int cu_count();
 // gr_narrow64.hip / gr_narrow32.hip

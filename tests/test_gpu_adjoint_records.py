@@ -58,3 +58,57 @@ def test_passes_changed_between_two_sweeps():
     for o in out[1:]:
         for a, b in zip(out[0], o):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_checkpoint_that_finds_no_memory(graph, monkeypatch):
+    """A step call that stops because a checkpoint finds no memory leaves the
+    state of the steps it took, with their forces, counts and cell keys; a
+    state set afterwards is the one the next steps start from."""
+    from grains3dgpu_amd import engine
+    from grains3dgpu_amd.engine import GrainsError
+    sc = lattice_superquadrics(n_side=5, n_rng=(2.0, 2.0))
+
+    def make():
+        return S.load(engine.Engine(dt=sc.dt, precision=A.FP64, gjk_rel_tol=1e-12), sc)
+
+    def result(e):
+        return [*e.get_state(), *e.get_torce(), e.get_contact_count(), *e.get_cell_keys()]
+
+    want, want0 = make(), make()
+    want.step(10, graph=graph)
+    want0.step(4, graph=graph)
+    # room for the checkpoints of the start and of 5 steps, not of 10
+    monkeypatch.setenv("GRAINS_ADJOINT_BYTES", str(3 * 104 * sc.n - 1))
+    e = make()
+    e.adjoint_record(5)
+    with pytest.raises(GrainsError, match="GRAINS_ADJOINT_BYTES"):
+        e.step(13, graph=graph)
+    for a, b in zip(result(e), result(want)):
+        np.testing.assert_array_equal(a, b)
+    e.set_state(sc.pos, sc.quat, sc.vel, sc.omega)
+    e.reset_contact_count()
+    monkeypatch.delenv("GRAINS_ADJOINT_BYTES")
+    e.set_sims(sc)  # (a new layout ends the recording)
+    e.step(4, graph=graph)
+    for a, b in zip(result(e), result(want0)):
+        np.testing.assert_array_equal(a, b)
+
+
+def test_state_set_after_a_step_call_that_stopped(monkeypatch):
+    """As above, without a new layout between: the run that stopped left
+    records ahead of the state's planes."""
+    from grains3dgpu_amd import engine
+    from grains3dgpu_amd.engine import GrainsError
+    sc = lattice_superquadrics(n_side=5, n_rng=(2.0, 2.0))
+    monkeypatch.setenv("GRAINS_ADJOINT_BYTES", str(2 * 104 * sc.n - 1))
+    e = S.load(engine.Engine(dt=sc.dt, precision=A.FP64, gjk_rel_tol=1e-12), sc)
+    want = S.load(engine.Engine(dt=sc.dt, precision=A.FP64, gjk_rel_tol=1e-12), sc)
+    want.step(3)
+    e.adjoint_record(5)
+    with pytest.raises(GrainsError, match="GRAINS_ADJOINT_BYTES"):
+        e.step(8)
+    e.set_state(sc.pos, sc.quat, sc.vel, sc.omega)
+    e.step(3)
+    for a, b in zip(e.get_state(), want.get_state()):
+        np.testing.assert_array_equal(a, b)
