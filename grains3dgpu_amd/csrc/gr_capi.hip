@@ -1865,6 +1865,9 @@ extern "C" int grains_gjk_batch_device(grains_ctx_t* ctx, const uint32_t* sa, co
   float* pv32 = nullptr;
   hipStream_t s = ctx->stream;
   int rc;
+  // The call comes after what the caller has put on the default stream (the
+  // arrays may be its results), as the copies of the tables below do.
+  if (in_args) (void)hipStreamSynchronize(nullptr);
   if (!in_args) {
     if ((rc = dalloc(ctx, &p64, S * sizeof(ShapeNP<double>), tmp)) || (rc = dalloc(ctx, &p32, S * sizeof(ShapeNP<float>), tmp)) ||
         (rc = dalloc(ctx, &pv64, v64.size() * 8, tmp)) || (rc = dalloc(ctx, &pv32, v32.size() * 4, tmp))) {

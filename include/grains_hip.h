@@ -377,7 +377,8 @@ int grains_gjk_batch(grains_ctx_t* ctx, const uint32_t* shape_a,
                      const uint32_t* shape_b, const double* ta,
                      const double* tb, uint64_t n, double* dist, double* pa,
                      double* pb, int32_t* iters);
-/* Device-resident variant for timing: all pointers are device pointers. */
+/* Device-resident variant for timing: all pointers are device pointers; the
+ * call comes after what is on the device's default stream. */
 int grains_gjk_batch_device(grains_ctx_t* ctx, const uint32_t* shape_a_device,
                             const uint32_t* shape_b_device, const double* ta_device,
                             const double* tb_device, uint64_t n,

@@ -51,3 +51,33 @@ def test_shapes_in_arguments_equal_shapes_in_memory(n, precision, flags):
     else:
         # one arithmetic, contracted per kernel: the FP32 tolerance of the distances
         np.testing.assert_allclose(out[0][0], out[2][0], rtol=0, atol=1e-5 * 2e-3)
+
+
+@pytest.mark.parametrize("n_shapes", [8, 9])
+def test_batch_comes_after_the_default_stream(n_shapes):
+    """Poses that copies on the default stream are still to bring: the call
+    sees them, with the shapes in its arguments (8) as with them in memory (9)."""
+    import ctypes as C
+    from grains3dgpu_amd import engine
+    rng = np.random.default_rng(3)
+    e = engine.Engine(precision=A.FP64, gjk_rel_tol=1e-10)
+    e.set_shapes(_scene(rng, n_shapes))
+    n = 5000
+    sa, sb, ta, tb = _pairs(rng, n, 8)
+    dev = _Dev()
+    want = _run(e, dev, e.L.grains_gjk_batch_device, sa, sb, ta, tb)[0]
+    p = [dev.put(a) for a in (sa, sb, ta, ta, tb, np.zeros(n), np.zeros(n, np.int32))]
+    big = 1 << 30
+    work = [C.c_void_p(), C.c_void_p()]
+    for w in work:
+        assert dev.h.hipMalloc(C.byref(w), big) == 0
+        dev.bufs.append(w)
+    copy = dev.h.hipMemcpyAsync
+    copy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_void_p]
+    for _ in range(30):  # some 10 ms of work
+        assert copy(work[0], work[1], big, 3, None) == 0  # device to device
+    assert copy(p[3], p[4], tb.nbytes, 3, None) == 0      # b's poses, in the place of a's
+    assert e.L.grains_gjk_batch_device(e.h, p[0], p[1], p[2], p[3], n, p[5], p[6], None) == 0
+    got = dev.get(p[5], want)
+    dev.free()
+    np.testing.assert_array_equal(got, want)
