@@ -407,8 +407,10 @@ struct grains_ctx {
   std::vector<void*> adj_cp;      // state every adj_every steps (13 planes)
   std::vector<void*> adj_allocs;  // sweep buffers
   uint64_t adj_cap = 0;           // the most device bytes the recording and its sweeps hold (0: what the device has)
+  std::vector<void*> adj_gjk;     // the searches' records
   std::vector<double*> adj_log;   // per block of adj_every steps, the states between (null: run again from its checkpoint)
   std::vector<void*> adj_log_allocs;
+  bool adj_log_off = false;       // it gave way to what the recording and the sweep cannot do without
   bool adj_log_ok = false;        // the logged steps followed each other (no state set between)
   AdjBufs ab{};
   double *adj_blk = nullptr, *adj_save = nullptr;
@@ -797,10 +799,10 @@ static uint64_t defer_words(uint64_t ecap) {
 
 // Device memory of the recording and its sweeps, within adj_cap.
 template <class P>
-static int adj_dalloc(grains_ctx* ctx, P** p, size_t bytes, std::vector<void*>& list) {
+static int adj_spare(grains_ctx* ctx, P** p, size_t bytes, std::vector<void*>& list) {
   if (ctx->adj_cap) {
     uint64_t held = bytes;
-    for (const auto* l : {&ctx->adj_cp, &ctx->adj_allocs, &ctx->adj_log_allocs})
+    for (const auto* l : {&ctx->adj_cp, &ctx->adj_allocs, &ctx->adj_log_allocs, &ctx->adj_gjk})
       for (void* q : *l) {
         size_t b = 0;
         GR_HIP(hipMemPtrGetInfo(q, &b));
@@ -811,11 +813,27 @@ static int adj_dalloc(grains_ctx* ctx, P** p, size_t bytes, std::vector<void*>& 
   }
   return dalloc(ctx, p, bytes, list);
 }
+// The same for what cannot be done without: what is only kept to spare work,
+// the logged states and the searches' records, gives way to it.
+template <class P>
+static int adj_dalloc(grains_ctx* ctx, P** p, size_t bytes, std::vector<void*>& list) {
+  const int rc = adj_spare(ctx, p, bytes, list);
+  if (rc != GRAINS_ENOMEM || (ctx->adj_log_allocs.empty() && ctx->adj_gjk.empty())) return rc;
+  launch_log_set(ctx->d, StateLog{}, 0u, ctx->stream);  // (set again before the next steps)
+  GR_HIP(hipStreamSynchronize(ctx->stream));
+  ctx->adj_log_off = true;
+  ctx->adj_log.assign(ctx->adj_log.size(), nullptr);
+  ctx->ab.gjk = nullptr;
+  free_list(ctx->adj_log_allocs);
+  free_list(ctx->adj_gjk);
+  return adj_spare(ctx, p, bytes, list);
+}
 
 static void adj_drop(grains_ctx* ctx) {
   if (ctx->adj_rec) drop_graph(ctx);  // a recorded step logs its state
   free_list(ctx->adj_cp);
   free_list(ctx->adj_allocs);
+  free_list(ctx->adj_gjk);
   free_list(ctx->adj_log_allocs);
   ctx->adj_log.clear();
   ctx->adj_rec = false;
@@ -1505,8 +1523,8 @@ static int log_chunk(grains_ctx* ctx, uint32_t done, uint32_t target) {
   while (ctx->adj_log.size() <= blk) {
     double* p = nullptr;
     const uint64_t used = ctx->adj_log_allocs.size() * bytes;
-    if (K > 1 && bytes / K / 13 / 8 == ctx->n && bytes <= kLogBytes && used <= kLogBytes - bytes)
-      (void)adj_dalloc(ctx, &p, bytes, ctx->adj_log_allocs);
+    if (!ctx->adj_log_off && K > 1 && bytes / K / 13 / 8 == ctx->n && bytes <= kLogBytes && used <= kLogBytes - bytes)
+      (void)adj_spare(ctx, &p, bytes, ctx->adj_log_allocs);
     ctx->adj_log.push_back(p);
   }
   launch_log_set(ctx->d, {ctx->adj_log[blk], (int64_t)(ctx->adj_steps % K) - (int64_t)done, K}, target, ctx->stream);
@@ -2083,8 +2101,10 @@ extern "C" int grains_adjoint_record(grains_ctx_t* ctx, uint32_t checkpoint_ever
   // the sweep's buffers are sized by checkpoint_every: drop them
   free_list(ctx->adj_cp);
   free_list(ctx->adj_allocs);
+  free_list(ctx->adj_gjk);
   free_list(ctx->adj_log_allocs);
   ctx->adj_log.clear();
+  ctx->adj_log_off = false;
   ctx->adj_log_ok = true;
   ctx->ab = AdjBufs{};
   ctx->adj_blk = ctx->adj_save = nullptr;
@@ -2119,6 +2139,7 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
         (rc = adj_dalloc(ctx, &a.entry_tidx, ecap * 4, L)) || (rc = adj_dalloc(ctx, &a.wall_theta, n * max_obs * 4 * 8, L)) ||
         (rc = adj_dalloc(ctx, &a.wall_tidx, n * max_obs * 4, L)) || (rc = adj_dalloc(ctx, &a.dtheta, (size_t)ntab * 4 * 8, L))) {
       free_list(L);
+      free_list(ctx->adj_gjk);
       a = AdjBufs{};
       ctx->adj_save = ctx->adj_blk = nullptr;
       return rc;
@@ -2133,7 +2154,7 @@ extern "C" int grains_adjoint(grains_ctx_t* ctx, const double* dL_dstate, double
   // their contacts; in one pass, or without the memory for them, it searches
   // again (the passes can change from one sweep to the next)
   const bool rec = ctx->d.precision == GRAINS_FP64 && ctx->d.split > 0;
-  if (rec && !a.gjk) (void)adj_dalloc(ctx, &a.gjk, ecap * sizeof(GjkRec), ctx->adj_allocs);
+  if (rec && !a.gjk) (void)adj_spare(ctx, &a.gjk, ecap * sizeof(GjkRec), ctx->adj_gjk);
   // the state adjoint, rows -> planes
   {
     std::vector<double> planes(13 * n);

@@ -112,3 +112,37 @@ def test_state_set_after_a_step_call_that_stopped(monkeypatch):
     e.step(3)
     for a, b in zip(e.get_state(), want.get_state()):
         np.testing.assert_array_equal(a, b)
+
+
+def test_log_gives_way_to_checkpoints_and_sweep(monkeypatch):
+    """The logged states are kept where there is memory to spare: with room for
+    the checkpoints, or for them, the sweep's buffers and a block run again,
+    but not for the log as well, recording and sweep go on without it.  Bytes a
+    particle: a state 104, ten steps to a block, five checkpoints; the sweep
+    364, 244 for each of max_neighbors, 36 for each of six walls."""
+    from grains3dgpu_amd import engine
+    sc = lattice_superquadrics(n_side=5, n_rng=(2.0, 2.0))
+    rng = np.random.default_rng(7)
+    w = [rng.standard_normal((sc.n, k)) for k in (3, 4, 3, 3)]
+    K = 16
+    sweep = 364 + 244 * K + 36 * 6
+
+    def run(per_particle):
+        monkeypatch.setenv("GRAINS_ADJOINT_BYTES", str(per_particle * sc.n))
+        e = S.load(engine.Engine(dt=sc.dt, precision=A.FP64, gjk_rel_tol=1e-12, max_neighbors=K), sc)
+        e.adjoint_record(10)
+        e.step(42)
+        return e
+
+    want = run(0)
+    # two blocks logged and two checkpoints, but not the third checkpoint
+    short = run(2 * 11 * 104 + 52)
+    for a, b in zip(short.get_state(), want.get_state()):
+        np.testing.assert_array_equal(a, b)
+    # all of the recording, but not the sweep beside it (1 %: allocations rounded up)
+    tight = run(int(1.01 * (15 * 104 + sweep)) + 100)
+    g, g0 = want.adjoint(*w, want_state0=True)
+    h, h0 = tight.adjoint(*w, want_state0=True)
+    assert np.abs(g).max() > 0
+    for a, b in zip([g, *g0], [h, *h0]):
+        np.testing.assert_array_equal(a, b)
