@@ -389,7 +389,8 @@ struct grains_ctx {
   bool interval_known = false;
   unsigned char* host_words = nullptr;  // pinned: the counters and the list words, read back together
   // grains_get_state: rows of up to rows_cap particles in pinned memory, two
-  // of them when the state takes several
+  // of them when the state takes several (the events are the context's GPU's,
+  // whichever is current when the state is read)
   std::mutex rows_mu;
   double* rows[2] = {nullptr, nullptr};
   hipEvent_t rows_ev[2] = {nullptr, nullptr};
@@ -596,6 +597,8 @@ extern "C" int grains_create(const grains_config_t* cfg, grains_ctx_t** out) {
       hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&ctx->ev_fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&ctx->ev_join, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&ctx->rows_ev[0], hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&ctx->rows_ev[1], hipEventDisableTiming) != hipSuccess ||
       hipHostMalloc((void**)&ctx->host_words, kWordBytes, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     grains_destroy(ctx);
@@ -623,6 +626,8 @@ extern "C" void grains_destroy(grains_ctx_t* ctx) {
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
   if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
+  for (hipEvent_t e : ctx->rows_ev)
+    if (e) (void)hipEventDestroy(e);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
@@ -1238,16 +1243,13 @@ static void copy_rows_threads(const StateDst& o, const double* rows, uint64_t i0
 static void free_rows(grains_ctx* ctx) {
   for (int k = 0; k < 2; ++k) {
     if (ctx->rows[k]) (void)hipHostFree(ctx->rows[k]);
-    if (ctx->rows_ev[k]) (void)hipEventDestroy(ctx->rows_ev[k]);
     ctx->rows[k] = nullptr;
-    ctx->rows_ev[k] = nullptr;
   }
   ctx->rows_cap = 0;
 }
 static bool alloc_rows(grains_ctx* ctx, uint64_t cap, int count) {
   for (int k = 0; k < count; ++k)
-    if (hipHostMalloc((void**)&ctx->rows[k], 13 * cap * sizeof(double), hipHostMallocDefault) != hipSuccess ||
-        hipEventCreateWithFlags(&ctx->rows_ev[k], hipEventDisableTiming) != hipSuccess) {
+    if (hipHostMalloc((void**)&ctx->rows[k], 13 * cap * sizeof(double), hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
       free_rows(ctx);
       return false;

@@ -7,6 +7,7 @@ import pytest
 
 from grains3dgpu_amd import _abi as A
 from grains3dgpu_amd import scene as S
+from tests.scenes import dense_spheres
 
 pytestmark = pytest.mark.gpu
 
@@ -29,3 +30,21 @@ def test_state_round_trip(n):
     v = np.zeros((n, 3))
     assert e.L.grains_get_state(e.h, None, None, A.dptr(v), None, C.c_uint64(n)) == 0
     np.testing.assert_array_equal(v, want[2])
+
+
+def test_state_read_while_another_gpu_is_current():
+    """A context's state is read whichever GPU the thread has set."""
+    from grains3dgpu_amd import engine
+    engine.lib()
+    h = C.CDLL("libamdhip64.so.7")
+    count = C.c_int()
+    if h.hipGetDeviceCount(C.byref(count)) or count.value < 2:
+        pytest.skip("needs two GPUs")
+    sc = dense_spheres(n=500, seed=1)
+    e = S.load(engine.Engine(dt=sc.dt), sc)
+    assert h.hipSetDevice(1) == 0
+    try:
+        for a, b in zip(e.get_state(), (sc.pos, sc.quat, sc.vel, sc.omega)):
+            np.testing.assert_array_equal(a, b)
+    finally:
+        h.hipSetDevice(0)
