@@ -43,7 +43,12 @@ constexpr double kPrefilterSlack = 1.e-10;
 constexpr int kMaxMovers = 4096;     // particles that change cell in a step, merged into the previous order
 constexpr uint32_t kSmallSort = 8192; // the most particles k_sort_small can hold (64 KB of LDS)
 constexpr uint32_t kSmallSortDefault = 1024;  // beds up to this size sort in one block by default
-constexpr uint64_t kWideIntegrate = 16384;  // beds up to this size integrate every particle with its walls in one launch
+// beds up to this size integrate every particle with its walls in one launch:
+// touching superquadrics, one launch and two, us: 2,000 30 and 49, 8,000 27 and
+// 51, 16,000 31 and 51, 20,000 36 and 51, 30,000 51 and 52, 45,000 58 and 54
+// (larger beds also integrate beside the searches; spheres by 32,000: 52 and
+// 60 us a step)
+constexpr uint64_t kWideIntegrate = 16384;
 constexpr uint32_t kXcds = 8;          // dies of the card, each with its own L2; blocks go to them in turn
 constexpr int kMaxNarrowPerCu = 64;  // resident narrow-phase blocks per CU the queue buffers are sized for
 

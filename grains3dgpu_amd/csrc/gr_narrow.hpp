@@ -500,17 +500,20 @@ __global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 2) k_screen(DevSc
   count_add(d.counters, kCntGjk, c_gjk);
 }
 
-// The complete pass over the screen's queue: two lanes per entry when the
-// grid holds the queue twice over, else one.  (One launch: the two forms as
-// launches of their own cost a graph node of ~5 us each, and the one with
-// nothing to do had to wait for room beside the integration: 0.13 ms on the
-// bed of 10^6.)
+// The complete pass over the screen's queue: two lanes per entry where the
+// launched lanes hold the queue twice over, else one.  (One launch: the two
+// forms as launches of their own cost a graph node of ~5 us each, and the one
+// with nothing to do had to wait for room beside the integration: 0.13 ms on
+// the bed of 10^6.)  FP32 in 256 threads, 131,072 lanes, ms by two lanes and
+// by one: 11,000 entries 0.109 and 0.123, 28,000 0.111 and 0.118, 63,000 0.124
+// and 0.119; past the lanes two take another turn: 80,000 0.199 and 0.129,
+// 173,000 0.318 and 0.212, 262,000 0.425 and 0.289.
 // REF_QUIRKS in FP64 takes the two passes too: in one pass a wave searched
 // with the fifth of its lanes that reach GJK.  4,001 boxes and superquadrics
 // 149 -> 8 + 93 us.
 template <class T, bool WARM, bool SV = true>
 __global__ void __launch_bounds__(kBlock) k_complete(DevScene d) {
-  if ((uint64_t)defer_total(d) * 2 <= (uint64_t)d.narrow_blocks * blockDim.x)
+  if ((uint64_t)defer_total(d) * 2 <= (uint64_t)gridDim.x * blockDim.x)
     narrow<T, SV, 1, WARM, true>(d);
   else
     narrow<T, SV, 1, WARM, false>(d);

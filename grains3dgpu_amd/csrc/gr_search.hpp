@@ -329,8 +329,11 @@ __device__ __forceinline__ SvBest sv_closest_quad(V3<double> a, V3<double> b, V3
 // queue therefore takes one lane per entry (L = 1); a short one four: two per
 // body, which take the independent pow calls of a support side by side, one
 // per face of the simplex (L = 4).  Four lanes issue about twice the
-// instructions per entry: the line lies where one lane per entry fills the
-// waves (46,700 entries: 0.56 ms by four; 173,000: 1.10 ms by one).
+// instructions per entry: the line lies where one lane per entry begins to fill
+// the waves.  Touching superquadrics, ms by four and by one: 28,000 entries
+// 0.364 and 0.805, 46,000 0.46 and 0.80, 69,000 0.80 and 0.88, 80,000 0.82 and
+// 0.81, 98,000 0.99 and 0.82, 127,000 1.23 and 0.85, 173,000 1.60 and 1.08 (the
+// two meet at 80,000, below the line).
 //
 // A lane whose search has ended waits until a quarter of the wave's entries
 // have, then those store their results and take the next entries together

@@ -7,7 +7,7 @@ import pytest
 
 from grains3dgpu_amd import _abi as A
 from grains3dgpu_amd import scene as S
-from tests.scenes import dense_cylinders_cones, dense_spheres, dense_superquadrics
+from tests.scenes import dense_cylinders_cones, dense_spheres, dense_superquadrics, lattice_superquadrics
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +88,22 @@ def test_spheres_alone_equal_spheres_beside_a_box(n, flags):
     assert out[0][2] == out[1][2] and (n < 300 or out[0][2] > 0)
     for a, b in zip(out[0][0] + out[0][1], out[1][0] + out[1][1]):
         np.testing.assert_array_equal(a, b[:m])
+
+
+@pytest.mark.parametrize("flags", [0, A.WARM_START | A.FP64_CONTACTS])
+def test_complete_pass_by_one_lane_and_by_two(flags):
+    """Launches whose lanes hold the queue (9,000 entries) twice over search
+    each entry by two lanes, narrower ones by one: the same results."""
+    from grains3dgpu_amd import engine
+    sc = lattice_superquadrics(n_side=12, seed=36)
+    out = []
+    for block, per_cu in ((64, 1), (64, 8), (128, 2), (256, 8)):
+        e = S.load(engine.Engine(dt=sc.dt, precision=A.FP32_MIXED, flags=flags, gjk_rel_tol=1e-6, block_size=block,
+                                 narrow_blocks_per_cu=per_cu), sc)
+        e.step(3)
+        st = e.get_stats()
+        assert 3 * 8192 < st["narrow_deferred"] < 3 * 16384
+        out.append([*e.get_state(), e.get_pairs(A.PAIRS_CONTACT), np.array(st["contacts"])])
+    for o in out[1:]:
+        for a, b in zip(o, out[0]):
+            np.testing.assert_array_equal(a, b)
