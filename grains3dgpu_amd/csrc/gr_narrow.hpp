@@ -290,18 +290,21 @@ __device__ __forceinline__ void defer_flush(const DevScene& d, DeferLds& L, uint
 
 // One lane per list entry, grid-stride.  SV: physics semantics (signed-volume
 // GJK); !SV: REF_QUIRKS.
-// PASS 0: every entry, complete.  With two passes (physics semantics) the
-// screen settles most entries and queues the rest; PASS 1 runs the queued
-// entries, packed lane-dense, complete.  A wave costs as much as its slowest
-// lane, so the long searches are kept together and the screen's waves stay
-// short.  The queued searches start from scratch with the same arithmetic:
-// results equal those of PASS 0 bit for bit.
+// PASS 0 (the step's only pass): every list entry, complete.  PASS 1: the
+// entries that a pass before it queued -- the screen, which settles most, or
+// the filter, which leaves out those beyond the prefilter -- packed
+// lane-dense, complete.  A wave costs as much as its slowest lane, so the long
+// searches are kept together and the first pass's waves stay short.  The
+// queued searches start from scratch with the same arithmetic: results equal
+// those of a single pass bit for bit.
 // WARM: FP32 searches start from the pair's previous direction (d.warm).
-// PAIR (PASS 1, physics semantics): two lanes per queued entry, sharing its
+// PAIR (PASS 1): two lanes per queued entry, sharing its
 // support evaluations (pair_force<PAIR>): the queue is short on beds, and
 // the pass lasts as long as its longest search (k_complete chooses).
 // BALLS (PASS 0, FP64): every particle is a sphere -- no search, no second pass.
-template <class T, bool SV, int PASS, bool WARM = false, bool PAIR = false, bool BALLS = false>
+// PACK (PASS 0): a wave takes 64 entries at a time that pass the prefilter
+// from the list, which holds the skin's too, half as many again (kPackNarrow).
+template <class T, bool SV, int PASS, bool WARM = false, bool PAIR = false, bool BALLS = false, bool PACK = false>
 __device__ __forceinline__ void narrow(const DevScene& d) {
   constexpr bool first = PASS != 1;  // the step's first kernel
   if constexpr (first) {
@@ -315,28 +318,16 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x / L2;
   const bool lead = gid % L2 == 0;  // the lane that stores the entry's results
   const uint32_t lane = __lane_id();
-  // whole waves take turns (the queue appends are wave-wide)
-  for (uint64_t kw = (gid - lane) / L2; kw < E; kw += stride) {
-    const uint64_t k = kw + lane / L2;
-    const bool in = k < E;
-    uint32_t e = 0, flag = 0;
+  auto turn = [&](uint32_t e, bool in) {  // an entry per lane (or pair of lanes), whole waves
+    uint32_t flag = 0;
     NpStats st = {0u, 0};
     bool refine = false;
     if (in) {
-      e = PASS == 1 ? defer_entry(d, (uint32_t)k) : (uint32_t)k;
       PairRes<T> r;
       V3<T> dir = {T(0), T(0), T(0)};
-      flag = pair_force<T, T, SV, WARM, PAIR, first, BALLS>(d, d.pair_i[e], d.pair_j[e], r, st, e,
+      flag = pair_force<T, T, SV, WARM, PAIR, first && !PACK, BALLS>(d, d.pair_i[e], d.pair_j[e], r, st, e,
                                                             sizeof(T) == 4 && SV ? &dir : nullptr);
-      if constexpr (first) {
-        c_cand += (flag & kFlagCand) != 0;
-        if constexpr (WARM) {
-          // a pair that left the prefilter's reach forgets its direction
-          if (!flag && (d.pair_flag[e] & kFlagCand))
-            d.ws[(uint64_t)(*d.ws_par) * ((uint64_t)d.K * d.n) + e] =
-                make_float4(0.f, 0.f, 0.f, __uint_as_float(d.sidx[d.pair_j[e]]));
-        }
-      }
+      if constexpr (first) c_cand += (flag & kFlagCand) != 0;
       // FP32-mixed: re-run in FP64 when the search ended on rounding instead
       // of the gap test, the cores overlap (the contact normal switches to the
       // centre line there), the contact decision lay within FP32's rounding
@@ -374,6 +365,59 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
       }
     }
     if constexpr (sizeof(T) == 4) wave_append(d.refine_list, d.refine_count, refine && lead, e);
+  };
+  // whole waves take turns (the queue appends are wave-wide)
+  if constexpr (PACK) {
+    __shared__ uint32_t packed[kBlock / 64][128];
+    uint32_t* mine = packed[threadIdx.x / 64];
+    uint32_t have = 0;  // the wave's entries in it
+    const bool outside = d.nl[kNlOutside] != 0;
+    // a share of the list dealt to each wave, the rest handed out through a
+    // counter (the first queue's: no pass queues entries here)
+    const uint64_t dealt = stride / 64;
+    const uint32_t share = 64u * (uint32_t)min((uint64_t)8, max((uint64_t)1, (uint64_t)E / (dealt * 64 * 8)));
+    uint64_t kw = (gid / 64) * share, end = min((uint64_t)E, kw + share);
+    bool more = dealt * share < E;
+    for (;;) {
+      while (have < 64) {
+        if (kw >= end) {
+          if (!more) break;
+          uint32_t next = 0;
+          if (lane == 0) next = atomicAdd(d.defer_count, share);
+          kw = dealt * share + __shfl(next, 0);
+          end = min((uint64_t)E, kw + share);
+          more = end < E;
+          if (kw >= end) break;
+        }
+        const uint32_t e = (uint32_t)kw + lane;
+        bool cand = false;
+        if (kw + lane < end) {
+          const uint32_t si = d.pair_i[e], sj = d.pair_j[e];
+          const PoseRec pi = d.pk[si], pj = d.pk[sj];
+          cand = is_candidate(d.grids[pi.sim], V3<double>{pi.x, pi.y, pi.z}, V3<double>{pj.x, pj.y, pj.z}, d.rcs[si],
+                              d.rcs[sj], outside);
+          if (!cand) d.pair_flag[e] = 0u;
+        }
+        const uint64_t m = __ballot(cand);
+        if (cand) mine[have + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = e;
+        have += (uint32_t)__popcll(m);
+        kw += 64;
+      }
+      if (!have) break;
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the wave's LDS writes are done
+      const bool in = lane < have;
+      turn(in ? mine[lane] : 0u, in);
+      have -= min(have, 64u);
+      const uint32_t rest = lane < have ? mine[64 + lane] : 0u;
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // read before the list is refilled
+      if (lane < have) mine[lane] = rest;
+    }
+  } else {
+    for (uint64_t kw = (gid - lane) / L2; kw < E; kw += stride) {
+      const uint64_t k = kw + lane / L2;
+      const bool in = k < E;
+      turn(!in ? 0u : (PASS == 1 ? defer_entry(d, (uint32_t)k) : (uint32_t)k), in);
+    }
   }
   if constexpr (first) count_add(d.counters, kCntCandidates, c_cand);
   count_add(d.counters, kCntGjk, c_gjk);
@@ -385,9 +429,26 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
   count_max(d.counters, kCntMaxIters, c_maxit);
 }
 
-template <class T, bool SV, bool WARM = false>
+// The reference semantics in one pass.  A list taken as it stands costs as
+// many waves as it is long, the skin's entries among them: on large beds more
+// than the lists' builds it saves, so those pack it, with as many waves as are
+// resident at once; small beds have lanes to spare, and spheres no search.
+// Boxes and superquadrics, ms a step with lists built for every step, kept and
+// unpacked, packed: FP32 5,000 grains 0.363, 0.238, 0.244, 20,000 0.463, 0.390,
+// 0.377, 150,000 1.055, 1.065, 0.927, 500,000 2.77, 2.94, 2.68; FP64 5,000
+// 0.348, 0.265, 0.282, 20,000 0.578, 0.596, 0.480, 150,000 2.44, 2.87, 2.12.
+constexpr uint64_t kPackNarrow = 10000;  // the largest bed whose list is taken as it stands
+template <class T, bool PACK>
 __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
-  narrow<T, SV, 0, WARM>(d);
+  narrow<T, false, 0, false, false, false, PACK>(d);
+}
+template <class T>
+inline void launch_narrow_ref(const DevScene& d, hipStream_t s) {
+  if (d.balls || d.n <= kPackNarrow)
+    hipLaunchKernelGGL((k_narrow<T, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
+  else
+    hipLaunchKernelGGL((k_narrow<T, true>), dim3(std::min(d.narrow_blocks, (unsigned)(cu_count() * kBlock) / d.block)),
+                       dim3(d.block), 0, s, d);
 }
 
 // Beds of spheres in FP64 (either semantics) take one small pass: screen and
@@ -513,7 +574,11 @@ __global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 2) k_screen(DevSc
 // 149 -> 8 + 93 us.
 template <class T, bool WARM, bool SV = true>
 __global__ void __launch_bounds__(kBlock) k_complete(DevScene d) {
-  if ((uint64_t)defer_total(d) * 2 <= (uint64_t)gridDim.x * blockDim.x)
+  // (the FP64 filter's queue: by one lane, in pairs a wave's registers are two
+  // waves' work and most entries end at once: 3,001 cylinders and cones 0.307
+  // and 0.419 ms a step)
+  constexpr bool filtered = sizeof(T) == 8 && SV;
+  if (!filtered && (uint64_t)defer_total(d) * 2 <= (uint64_t)gridDim.x * blockDim.x)
     narrow<T, SV, 1, WARM, true>(d);
   else
     narrow<T, SV, 1, WARM, false>(d);

@@ -107,3 +107,27 @@ def test_complete_pass_by_one_lane_and_by_two(flags):
     for o in out[1:]:
         for a, b in zip(o, out[0]):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("block,per_cu", [(64, 1), (128, 2), (256, 8)])
+def test_reference_semantics_in_one_packed_pass(block, per_cu):
+    """REF_QUIRKS on a bed whose one pass packs its candidates from the lists
+    (more than 10,000 grains), its waves taking shares of one to eight turns:
+    FP64 equals two passes, FP32 itself in another launch and FP64's contacts."""
+    from grains3dgpu_amd import engine
+    sc = dense_superquadrics(n=11000, seed=37, phi=0.2, vel=0.5, box_frac=0.3)
+
+    def run(precision, passes, **launch):
+        e = S.load(engine.Engine(dt=sc.dt, precision=precision, flags=A.REF_QUIRKS, narrow_passes=passes, **launch), sc)
+        e.step(3)
+        st = e.get_stats()
+        assert st["contacts"] > 0
+        return [*e.get_state(), e.get_pairs(A.PAIRS_CONTACT),
+                np.array([st[k] for k in ("candidate_pairs", "gjk_calls", "gjk_iterations", "contacts")])]
+
+    launch = dict(block_size=block, narrow_blocks_per_cu=per_cu)
+    for a, b in zip(run(A.FP64, 1, **launch), run(A.FP64, 2)):
+        np.testing.assert_array_equal(a, b)
+    one = run(A.FP32_MIXED, 1, **launch)
+    for a, b in zip(one, run(A.FP32_MIXED, 1, block_size=64, narrow_blocks_per_cu=16)):
+        np.testing.assert_array_equal(a, b)
