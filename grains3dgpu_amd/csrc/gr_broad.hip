@@ -537,6 +537,16 @@ __global__ void __launch_bounds__(1024) k_sort_small(DevScene d, uint32_t* __res
   }
 }
 
+static void radix_passes(DevScene& d, int passes, int digit_bits, const uint32_t*& kin, const uint32_t*& iin,
+                         hipStream_t s) {
+  switch (digit_bits) {
+    case 8: run_sort_passes<8>(d, passes, kin, iin, s); break;
+    case 9: run_sort_passes<9>(d, passes, kin, iin, s); break;
+    case 10: run_sort_passes<10>(d, passes, kin, iin, s); break;
+    default: run_sort_passes<11>(d, passes, kin, iin, s); break;
+  }
+}
+
 void launch_sort(DevScene& d, int passes, int digit_bits, uint32_t** keys_sorted, uint32_t** idx_sorted,
                  hipStream_t s) {
   if (d.small_sort) {
@@ -547,12 +557,7 @@ void launch_sort(DevScene& d, int passes, int digit_bits, uint32_t** keys_sorted
   }
   const uint32_t* kin = d.skey;
   const uint32_t* iin = nullptr;
-  switch (digit_bits) {
-    case 8: run_sort_passes<8>(d, passes, kin, iin, s); break;
-    case 9: run_sort_passes<9>(d, passes, kin, iin, s); break;
-    case 10: run_sort_passes<10>(d, passes, kin, iin, s); break;
-    default: run_sort_passes<11>(d, passes, kin, iin, s); break;
-  }
+  radix_passes(d, passes, digit_bits, kin, iin, s);
   uint32_t* ks = const_cast<uint32_t*>(kin);
   uint32_t* is = const_cast<uint32_t*>(iin);
   // the merge (mode 1) works in the other buffer pair
@@ -565,6 +570,27 @@ void launch_sort(DevScene& d, int passes, int digit_bits, uint32_t** keys_sorted
   hipLaunchKernelGGL(k_merge_copy, grid, dim3(kBlock), 0, s, d, ko, io, ks, is);
   *keys_sorted = ks;
   *idx_sorted = is;
+}
+
+// The particles by (key, id) of the reference's cells (d.key), between two
+// steps: through the radix passes (or the one block) in arrays that only a step
+// or a build fills -- the obstacles', the marked particles' and the candidates'
+// -- with a count that is zero then as the sort's state (mode 0).
+const uint32_t* launch_key_order(const DevScene& d, int passes, int digit_bits, hipStream_t s) {
+  DevScene t = d;
+  t.skey = d.key;
+  t.keyA = d.obs_list;
+  t.idxA = d.obs_list2;
+  t.keyB = d.pend_list;
+  t.idxB = d.cand;
+  t.sort_state = d.refine_count;
+  const uint32_t *kin = t.skey, *iin = nullptr;
+  if (d.small_sort) {
+    hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(1024), 0, s, t, t.keyA, t.idxA);
+    return t.idxA;
+  }
+  radix_passes(t, passes, digit_bits, kin, iin, s);
+  return iin;
 }
 
 // ---- cell ranges and sorted records -----------------------------------------------
@@ -1458,6 +1484,64 @@ void launch_expand(const DevScene& d, hipStream_t s) {
   const dim3 grid((unsigned)((d.n + d.block - 1) / d.block)), block(d.block);
   hipLaunchKernelGGL(k_expand, grid, block, 0, s, d);
   if (d.warm) hipLaunchKernelGGL(k_warm_carry, dim3((unsigned)cu_count() * 8), dim3(kBlock), 0, s, d);
+}
+
+// ---- the step's pairs, read out -----------------------------------------------------
+// The entries flagged `want`, particle by particle (by id), each one's by
+// (neighbour cell in the visit order, id) at the positions of the step: the
+// lists' own order, unless one of them is in another cell than when the lists
+// were built.  Between two steps, in arrays that only a step or a build fills.
+__global__ void __launch_bounds__(kBlock) k_pair_count(DevScene d, uint32_t want, uint32_t* __restrict__ count) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= d.n) return;
+  const uint32_t s = d.rank[i];
+  uint32_t c = 0;
+  for (uint32_t e = d.entry_off[s]; e < d.entry_off[s + 1]; ++e) c += (d.pair_flag[e] & want) != 0;
+  count[i] = c;
+}
+__global__ void __launch_bounds__(kBlock) k_pair_list(DevScene d, uint32_t want, const uint32_t* __restrict__ off,
+                                                      uint32_t* __restrict__ nb) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= d.n) return;
+  const uint32_t s = d.rank[i], e0 = d.entry_off[s], e1 = d.entry_off[s + 1];
+  const SimGrid& g = d.grids[d.sim[i]];
+  uint32_t k = off[i];
+  bool again = d.rkey[s] != d.key[i];
+  for (uint32_t e = e0; e < e1; ++e) {
+    if (!(d.pair_flag[e] & want)) continue;
+    const uint32_t t = d.pair_j[e], j = d.sidx[t];
+    again |= d.rkey[t] != d.key[j];
+    nb[k++] = j;
+  }
+  if (!again) return;
+  auto cell = [&](uint32_t key, uint32_t* c) {
+    const uint32_t l = key - g.base;
+    c[0] = l % g.n3[0];
+    c[1] = (l / g.n3[0]) % g.n3[1];
+    c[2] = l / (g.n3[0] * g.n3[1]);
+  };
+  uint32_t ci[3];
+  cell(d.key[i], ci);
+  auto order = [&](uint32_t e) -> uint64_t {
+    const uint32_t j = d.sidx[d.pair_j[e]];
+    uint32_t cj[3];
+    cell(d.key[j], cj);
+    return ((uint64_t)(uint32_t)cell_slot(g, ci, cj) << 32) | j;
+  };
+  for (uint32_t e = e0; e < e1; ++e) {
+    if (!(d.pair_flag[e] & want)) continue;
+    const uint64_t me = order(e);
+    uint32_t place = off[i];
+    for (uint32_t f = e0; f < e1; ++f) place += (d.pair_flag[f] & want) && order(f) < me;
+    nb[place] = (uint32_t)me;
+  }
+}
+PairLists launch_pair_lists(const DevScene& d, uint32_t want, bool list, hipStream_t s) {
+  const dim3 grid((unsigned)((d.n + kBlock - 1) / kBlock));
+  hipLaunchKernelGGL(k_pair_count, grid, dim3(kBlock), 0, s, d, want, d.obs_list2);
+  launch_scan(d.obs_list2, d.obs_list, d.n, d.scan_blocks, s);
+  if (list) hipLaunchKernelGGL(k_pair_list, grid, dim3(kBlock), 0, s, d, want, d.obs_list, d.cand);
+  return {d.obs_list, d.cand};
 }
 
 int cu_count() {

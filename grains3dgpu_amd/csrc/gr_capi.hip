@@ -10,6 +10,7 @@
 #include <cstring>
 #include <string>
 #include <limits>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -368,7 +369,8 @@ struct grains_ctx {
   std::vector<void*> state_allocs; // particle state
   int passes = 1;      // LSD radix passes of the cell keys
   int digit_bits = 8;  // bits per pass
-  int ref_passes = 1;  // passes the reference's cell keys take (grains_stats_t.sort_passes)
+  int ref_passes = 1;  // passes the reference's cell keys take (grains_stats_t.sort_passes), and their digits
+  int ref_digit_bits = 8;
   uint32_t *keys_s = nullptr, *idx_s = nullptr;
   hipGraph_t graph = nullptr;            // one step
   hipGraphExec_t graph_exec = nullptr;
@@ -990,6 +992,7 @@ static int finalize(grains_ctx* ctx) {
     int ref = 1;
     while (ref < 32 && (1ull << ref) < base) ++ref;
     ctx->ref_passes = (ref + kRadixMaxBits - 1) / kRadixMaxBits;
+    ctx->ref_digit_bits = std::max(8, (ref + ctx->ref_passes - 1) / ctx->ref_passes);
   }
   // shape tables
   const size_t S = ctx->shapes.size();
@@ -1080,7 +1083,7 @@ static int finalize(grains_ctx* ctx) {
       (rc = dalloc(ctx, &d.entry_off, (n + 1) * 4, L)) || (rc = dalloc(ctx, &d.pair_i, ecap * 4, L)) ||
       (rc = dalloc(ctx, &d.pair_j, ecap * 4, L)) || (rc = dalloc(ctx, &d.pair_flag, ecap * 4, L)) ||
       (rc = dalloc(ctx, &d.pair_res, ecap * res_sz, L)) || (rc = dalloc(ctx, &d.refine_list, ecap * 4, L)) ||
-      (rc = dalloc(ctx, &d.refine_count, 16, L)) || (rc = dalloc(ctx, &d.obs_list, n * 4, L)) ||
+      (rc = dalloc(ctx, &d.refine_count, 16, L)) || (rc = dalloc(ctx, &d.obs_list, (n + 1) * 4, L)) ||
       (rc = dalloc(ctx, &d.obs_list2, n * 4, L)) ||
       (rc = dalloc(ctx, &d.obs_count, 16, L)) || (rc = dalloc(ctx, &d.pend, n * 4, L)) ||
       (rc = dalloc(ctx, &d.pend_list, n * 4, L)) || (rc = dalloc(ctx, &d.sort_state, 16, L)) ||
@@ -1182,6 +1185,7 @@ static int finalize(grains_ctx* ctx) {
   GR_HIP(hipGetLastError());
   GR_HIP(hipStreamSynchronize(ctx->stream));
   ctx->layout_ok = true;
+  ctx->keys_s = ctx->idx_s = nullptr;  // no lists yet
   ctx->lists_ok = false;
   ctx->interval = 8;
   ctx->interval_known = false;
@@ -1220,24 +1224,30 @@ static void copy_rows(const StateDst& o, const double* rows, uint64_t i0, uint64
   };
   put(o.pos, 0, 3), put(o.quat, 3, 4), put(o.vel, 7, 3), put(o.omega, 10, 3);
 }
-// The same by several threads: a caller's array that has not been written
-// before costs a page fault per 4 KB, 104 MB of them 20 ms on one thread.
-static void copy_rows_threads(const StateDst& o, const double* rows, uint64_t i0, uint64_t m) {
-  const uint64_t parts = std::min<uint64_t>(std::max(1u, std::min(8u, std::thread::hardware_concurrency())),
-                                            m / kRowsPerThread + 1);
+// f(a, b) for the parts [a, b) of [0, n), at least `per` long, by up to
+// eight threads.
+template <class F>
+static void in_parts(uint64_t n, uint64_t per, const F& f) {
+  const uint64_t parts =
+      std::min<uint64_t>(std::max(1u, std::min(8u, std::thread::hardware_concurrency())), n / per + 1);
   uint64_t left = parts;  // parts [0, left) are this thread's
   std::vector<std::thread> th;
   try {
     th.reserve(parts);
     while (left > 1) {
-      const uint64_t a = m * (left - 1) / parts, b = m * left / parts;
-      th.emplace_back([=] { copy_rows(o, rows, i0, m, a, b); });
+      const uint64_t a = n * (left - 1) / parts, b = n * left / parts;
+      th.emplace_back([=, &f] { f(a, b); });
       --left;
     }
-  } catch (const std::exception&) {  // no more threads: the rest is copied here
+  } catch (const std::exception&) {  // no more threads: the rest is done here
   }
-  copy_rows(o, rows, i0, m, 0, m * left / parts);
+  f(0, n * left / parts);
   for (std::thread& t : th) t.join();
+}
+// The same by several threads: a caller's array that has not been written
+// before costs a page fault per 4 KB, 104 MB of them 20 ms on one thread.
+static void copy_rows_threads(const StateDst& o, const double* rows, uint64_t i0, uint64_t m) {
+  in_parts(m, kRowsPerThread, [&](uint64_t a, uint64_t b) { copy_rows(o, rows, i0, m, a, b); });
 }
 
 static void free_rows(grains_ctx* ctx) {
@@ -1740,26 +1750,12 @@ extern "C" int grains_get_cell_keys(grains_ctx_t* ctx, uint32_t* keys, uint32_t*
   if (!ctx) return GRAINS_EINVAL;
   if (n != ctx->n || !ctx->layout_ok || !ctx->idx_s) return fail(ctx, GRAINS_ESTATE, "no step run yet");
   GR_HIP(hipStreamSynchronize(ctx->stream));
-  std::vector<uint32_t> own;
-  uint32_t* k = keys;
-  if (!k) {
-    own.resize(n);
-    k = own.data();
-  }
-  GR_HIP(hipMemcpy(k, ctx->d.key, n * 4, hipMemcpyDeviceToHost));
-  if (sorted) {  // stable, two counting passes of 16 bits
-    std::vector<uint32_t> tmp(n);
-    for (int p = 0; p < 2; ++p) {
-      std::vector<uint32_t> off(65537, 0u);
-      const uint32_t* in = p ? tmp.data() : nullptr;
-      uint32_t* out = p ? sorted : tmp.data();
-      for (uint64_t i = 0; i < n; ++i) ++off[((k[i] >> (16 * p)) & 0xffffu) + 1];
-      for (int v = 0; v < 65536; ++v) off[v + 1] += off[v];
-      for (uint64_t i = 0; i < n; ++i) {
-        const uint32_t id = in ? in[i] : (uint32_t)i;
-        out[off[(k[id] >> (16 * p)) & 0xffffu]++] = id;
-      }
-    }
+  if (keys) GR_HIP(hipMemcpy(keys, ctx->d.key, n * 4, hipMemcpyDeviceToHost));
+  if (sorted) {
+    const uint32_t* order = launch_key_order(ctx->d, ctx->ref_passes, ctx->ref_digit_bits, ctx->stream);
+    GR_HIP(hipGetLastError());
+    GR_HIP(hipStreamSynchronize(ctx->stream));
+    GR_HIP(hipMemcpy(sorted, order, n * 4, hipMemcpyDeviceToHost));
   }
   return GRAINS_OK;
 }
@@ -1769,58 +1765,23 @@ extern "C" int grains_get_pairs(grains_ctx_t* ctx, int which, uint32_t* ij, uint
   if (!ctx->layout_ok || !ctx->idx_s) return fail(ctx, GRAINS_ESTATE, "no step run yet");
   GR_HIP(hipStreamSynchronize(ctx->stream));
   const uint64_t n = ctx->n;
-  std::vector<uint32_t> off(n + 1), rank(n), sidx(n);
-  GR_HIP(hipMemcpy(off.data(), ctx->d.entry_off, (n + 1) * 4, hipMemcpyDeviceToHost));
-  GR_HIP(hipMemcpy(rank.data(), ctx->d.rank, n * 4, hipMemcpyDeviceToHost));
-  GR_HIP(hipMemcpy(sidx.data(), ctx->idx_s, n * 4, hipMemcpyDeviceToHost));
-  const uint64_t E = off[n];
-  std::vector<uint32_t> pj(E), fl(E), key(n);
-  GR_HIP(hipMemcpy(key.data(), ctx->d.key, n * 4, hipMemcpyDeviceToHost));
-  if (E) {
-    GR_HIP(hipMemcpy(pj.data(), ctx->d.pair_j, E * 4, hipMemcpyDeviceToHost));
-    GR_HIP(hipMemcpy(fl.data(), ctx->d.pair_flag, E * 4, hipMemcpyDeviceToHost));
-  }
   const uint32_t want = which == GRAINS_PAIRS_CONTACT ? kFlagContact : kFlagCand;
-  uint64_t k = 0;
-  std::vector<uint64_t> row;
-  for (uint64_t i = 0; i < n; ++i) {
-    // the particle's pairs by (neighbour cell in the visit order, id), at the
-    // positions of the step
-    const uint32_t s = rank[i];
-    const SimGrid& g = ctx->grids[ctx->psim[i]];
-    auto cell = [&](uint32_t id, uint32_t* c) {
-      const uint32_t l = key[id] - g.base;
-      c[0] = l % g.n3[0];
-      c[1] = (l / g.n3[0]) % g.n3[1];
-      c[2] = l / (g.n3[0] * g.n3[1]);
-    };
-    uint32_t ci[3];
-    cell((uint32_t)i, ci);
-    row.clear();
-    for (uint32_t e = off[s]; e < off[s + 1]; ++e) {
-      if (!(fl[e] & want)) continue;
-      const uint32_t j = sidx[pj[e]];  // entries hold sorted positions
-      uint32_t cj[3];
-      cell(j, cj);
-      uint64_t slot = 0;
-      for (int a = 2; a >= 0; --a) {
-        const int m = (int)g.n3[a];
-        int v = (int)cj[a] - (int)ci[a];
-        if ((g.periodic >> a) & 1) v = v == m - 1 ? -1 : (v == 1 - m ? 1 : v);
-        slot = slot * 3 + (uint64_t)(v + 1);
-      }
-      row.push_back((slot << 32) | j);
-    }
-    std::sort(row.begin(), row.end());
-    for (uint64_t r : row) {
-      if (ij && k < cap) {
-        ij[2 * k] = (uint32_t)i;
-        ij[2 * k + 1] = (uint32_t)r;
-      }
-      ++k;
-    }
+  const PairLists dev = launch_pair_lists(ctx->d, want, ij != nullptr, ctx->stream);
+  GR_HIP(hipGetLastError());
+  GR_HIP(hipStreamSynchronize(ctx->stream));
+  uint32_t total = 0;
+  GR_HIP(hipMemcpy(&total, dev.off + n, 4, hipMemcpyDeviceToHost));
+  if (ij && total) {
+    // (not vectors: their zeros cost as much as the copies into them)
+    std::unique_ptr<uint32_t[]> off(new uint32_t[n + 1]), nb(new uint32_t[total]);
+    GR_HIP(hipMemcpy(off.get(), dev.off, (n + 1) * 4, hipMemcpyDeviceToHost));
+    GR_HIP(hipMemcpy(nb.get(), dev.nb, (uint64_t)total * 4, hipMemcpyDeviceToHost));
+    in_parts(n, kRowsPerThread, [&](uint64_t a, uint64_t b) {
+      for (uint64_t i = a; i < b; ++i)
+        for (uint64_t k = off[i]; k < off[i + 1] && k < cap; ++k) ij[2 * k] = (uint32_t)i, ij[2 * k + 1] = nb[k];
+    });
   }
-  *m = k;
+  *m = total;
   return GRAINS_OK;
 }
 

@@ -327,6 +327,12 @@ void launch_hash(const DevScene& d, const uint32_t* keys_prev, hipStream_t s);
 void launch_sort(DevScene& d, int passes, int digit_bits, uint32_t** keys_sorted, uint32_t** idx_sorted,
                  hipStream_t s);
 // cell ranges, inverse permutation and the sorted pose records
+// the step's pairs by particle: off[n + 1] (off[n] their number), nb their neighbours
+struct PairLists {
+  const uint32_t *off, *nb;
+};
+PairLists launch_pair_lists(const DevScene& d, uint32_t want, bool list, hipStream_t s);
+const uint32_t* launch_key_order(const DevScene& d, int passes, int digit_bits, hipStream_t s);
 void launch_cells(const DevScene& d, const uint32_t* keys_s, const uint32_t* idx_s, hipStream_t s);
 void launch_candidates(const DevScene& d, const uint32_t* keys_s, hipStream_t s);
 // exclusive scan of min(in[i], clamp) into out[0 .. n]; gate (optional):

@@ -186,3 +186,34 @@ def test_lists_that_outgrow_their_room_keep_the_warm_starts(mode):
     assert tight.get_stats()["max_candidates"] == most
     for a, b in zip(result(tight), result(roomy)):
         np.testing.assert_array_equal(a, b)
+
+
+def test_pairs_and_keys_of_a_new_layout_are_refused():
+    """Pairs and cell keys are those of a step: none before a layout's first."""
+    from grains3dgpu_amd import engine
+    from grains3dgpu_amd.engine import GrainsError
+    sc = dense_spheres(n=300, seed=14)
+    e = S.load(engine.Engine(dt=sc.dt), sc)
+    e.step(2)
+    assert len(e.get_pairs(A.PAIRS_CANDIDATE))
+    e.set_sims(sc)
+    e.step(0)
+    for read in (e.get_pairs, e.get_cell_keys):
+        with pytest.raises(GrainsError, match="no step"):
+            read()
+    e.step(1)
+    assert len(e.get_pairs(A.PAIRS_CANDIDATE))
+
+
+@pytest.mark.parametrize("n", [1, 3, 300, 1025, 20000])
+def test_key_order_is_stable(n):
+    """The particles by (cell key, id), through one block or the radix passes,
+    after a step that has changed cells."""
+    import dataclasses
+    from grains3dgpu_amd import engine
+    sc = dense_spheres(n=max(n, 300), seed=15, vel=20.0, periodic=0b011)
+    sc = dataclasses.replace(sc, **{k: getattr(sc, k)[:n] for k in ("pos", "quat", "vel", "omega", "particle_shape")})
+    e = S.load(engine.Engine(dt=sc.dt, max_neighbors=64), sc)
+    e.step(20)
+    key, order = e.get_cell_keys()
+    np.testing.assert_array_equal(order, np.argsort(key, kind="stable"))
