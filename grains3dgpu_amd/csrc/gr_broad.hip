@@ -37,6 +37,25 @@ void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s) {
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, p, n, v);
 }
 
+// ---- shapes -----------------------------------------------------------------------
+// (FP64 division rounds here as on the host; 10^6 shapes' records were 64 MB
+// of divisions and a copy of a new layout)
+__global__ void __launch_bounds__(kBlock) k_sq_pow(const ShapeNP<double>* __restrict__ np, SqPow* __restrict__ out,
+                                                   uint64_t n) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  SqPow r = {};
+  if (np[i].kind == GRAINS_SUPERQUADRIC) {
+    const double a = np[i].core[0], b = np[i].core[1], c = np[i].core[2], n1 = np[i].core[3], n2 = np[i].core[4];
+    r = {1.0 / (n2 - 1.0), 1.0 / (n1 - 1.0), (n1 - n2) / (n2 * (n1 - 1.0)), n1 / n2, 1.0 / n1,
+         b / a,            c / a,            c / b};
+  }
+  out[i] = r;
+}
+void launch_sq_pow(const ShapeNP<double>* np, SqPow* out, uint64_t n, hipStream_t s) {
+  hipLaunchKernelGGL(k_sq_pow, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, np, out, n);
+}
+
 // ---- the start of a run -------------------------------------------------------------
 // fresh: the lists do not stand (nor the sorted order), and the planes hold
 // the state, whatever a run that stopped early left in the records.

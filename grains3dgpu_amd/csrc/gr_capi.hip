@@ -911,10 +911,15 @@ static int finalize(grains_ctx* ctx) {
   }
   // linked cells per sim (Grains.cpp:226-247, LinkedCell.cpp:16-29)
   ctx->grids.assign(ns, SimGrid());
-  std::vector<double> lc(ns, 0.0);
+  std::vector<double> lc(ns, 0.0), rmean(ns, 0.0);  // largest radius, sum of the radii
+  std::vector<uint64_t> rnum(ns, 0);
   for (uint64_t i = 0; i < ctx->n; ++i) {
     const HostShape& h = ctx->shapes[ctx->pshape[i]];
-    lc[ctx->psim[i]] = std::max(lc[ctx->psim[i]], quirks ? h.rc : h.rc_exact);
+    const uint32_t s = ctx->psim[i];
+    const double rc = quirks ? h.rc : h.rc_exact;
+    lc[s] = std::max(lc[s], rc);
+    rmean[s] += rc;
+    ++rnum[s];
   }
   uint64_t base = 0;
   const uint32_t per = ctx->nmat * (ctx->nmat + 1) / 2;
@@ -963,13 +968,6 @@ static int finalize(grains_ctx* ctx) {
   // 0.58, 0.52, 0.40, 0.58.
   // A periodic axis that would hold fewer than three such cells leaves the
   // whole context without a skin (set_search).
-  std::vector<double> rmean(ns, 0.0);
-  std::vector<uint64_t> rnum(ns, 0);
-  for (uint64_t i = 0; i < ctx->n; ++i) {
-    const HostShape& h = ctx->shapes[ctx->pshape[i]];
-    rmean[ctx->psim[i]] += quirks ? h.rc : h.rc_exact;
-    ++rnum[ctx->psim[i]];
-  }
   bool skin_fits = true;
   uint64_t sbase = 0;
   ctx->sgrids = ctx->grids;
@@ -998,7 +996,6 @@ static int finalize(grains_ctx* ctx) {
   const size_t S = ctx->shapes.size();
   std::vector<ShapeNP<double>> np64(S);
   std::vector<ShapeNP<float>> np32(S);
-  std::vector<SqPow> sq64(S, SqPow{});
   std::vector<ShapeDyn> dyn(S);
   std::vector<double> rcpf(S), v64, cv64;
   for (size_t i = 0; i < S; ++i) {
@@ -1006,11 +1003,6 @@ static int finalize(grains_ctx* ctx) {
     int32_t voff = (int32_t)(v64.size() / 3);
     np64[i] = to_np<double>(h, quirks, voff);
     np32[i] = to_np<float>(h, quirks, voff);
-    if (h.s.kind == GRAINS_SUPERQUADRIC) {
-      const double a = h.core[0], b = h.core[1], c = h.core[2], n1 = h.core[3], n2 = h.core[4];
-      sq64[i] = {1.0 / (n2 - 1.0), 1.0 / (n1 - 1.0), (n1 - n2) / (n2 * (n1 - 1.0)), n1 / n2, 1.0 / n1,
-                 b / a,            c / a,            c / b};
-    }
     ShapeDyn& y = dyn[i];
     y = ShapeDyn{};
     y.mass = h.mass;
@@ -1119,7 +1111,7 @@ static int finalize(grains_ctx* ctx) {
   }
   GR_HIP(hipMemcpy(p64, np64.data(), S * sizeof(ShapeNP<double>), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(p32, np32.data(), S * sizeof(ShapeNP<float>), hipMemcpyHostToDevice));
-  GR_HIP(hipMemcpy(psq, sq64.data(), S * sizeof(SqPow), hipMemcpyHostToDevice));
+  launch_sq_pow(p64, psq, S, ctx->stream);
   GR_HIP(hipMemcpy(pdyn, dyn.data(), S * sizeof(ShapeDyn), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(prc, rcpf.data(), S * sizeof(double), hipMemcpyHostToDevice));
   GR_HIP(hipMemcpy(pv64, v64.data(), v64.size() * sizeof(double), hipMemcpyHostToDevice));

@@ -317,6 +317,7 @@ struct AdjBufs {
 // gr_broad.hip
 void launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 // keys_prev: the sort's output buffer (the previous step's sorted keys)
+void launch_sq_pow(const ShapeNP<double>* np, SqPow* out, uint64_t n, hipStream_t s);
 void launch_store_state(const DevScene& d, hipStream_t s);
 void launch_log_state(const DevScene& d, hipStream_t s);
 void launch_log_set(const DevScene& d, StateLog v, uint32_t target, hipStream_t s);
