@@ -4,17 +4,22 @@ Times short windows of real steps on the scene itself and keeps the fastest
 setting, by coordinate descent: first the cell-size factor
 (CellSizeFactor >= 1 scales the cell edge 2 max R_c, Grains.cpp:232-242),
 then the block size of the per-particle / per-entry kernels, then the number
-of resident blocks per CU of the persistent narrow-phase launch, then one
+of blocks per CU of the persistent narrow-phase launches, then one
 narrow pass or a screening pass plus a pass over the queued entries, then
 the candidate search with or without LDS staging.  Every
 window replays a captured graph, the production mode.  The state
 is restored from a snapshot before every window, so all candidates run the
-same steps.
+same steps.  A restored state has its neighbour lists built by the first
+step, and a run keeps them for many: a window times the first step apart and
+charges what it took beyond the others to HELD steps.
 """
 import time
 
 from . import _abi as A
 from .scene import load
+
+
+HELD = 64  # steps a list build serves (30 to 200 on beds; one without a skin, where every step is timed with its build)
 
 
 def _window(eng, blob, steps):
@@ -24,8 +29,11 @@ def _window(eng, blob, steps):
     eng.step(1, graph=True)
     eng.restore(blob)
     t0 = time.perf_counter()
+    eng.step(1, graph=True)
+    t1 = time.perf_counter()
     eng.step(steps, graph=True)
-    return (time.perf_counter() - t0) / steps
+    per_step = (time.perf_counter() - t1) / steps
+    return per_step + max(0.0, t1 - t0 - per_step) / HELD
 
 
 def autotune(scene, precision=A.FP32_MIXED, flags=0, gjk_rel_tol=0.0, steps=10,
