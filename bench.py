@@ -102,7 +102,8 @@ EAGER = False
 
 def run_engine(sc, precision, warmup, steps, profile=True, flags=0, gjk_tol=None, graph=True, profile_steps=100,
                max_neighbors=64, graph_steps=1, **launch):
-    """W warm-up steps, then (profile) min(profile_steps, steps) eagerly
+    """W warm-up steps as the timed ones are launched (their graphs are captured
+    here), then (profile) min(profile_steps, steps) eagerly
     launched steps with HIP events around every phase, then `steps` timed
     steps replayed from a captured graph (the production mode).  Returns the
     timed wall time, the counters of the timed steps and per-step phase
@@ -113,8 +114,9 @@ def run_engine(sc, precision, warmup, steps, profile=True, flags=0, gjk_tol=None
     e = S.load(Engine(dt=sc.dt, precision=precision, max_neighbors=max_neighbors, gjk_rel_tol=tol, flags=flags,
                       **launch), sc)
     e.set_graph_steps(graph_steps)
+    graph = graph and not EAGER
     if warmup:
-        e.step(warmup)
+        e.step(warmup, graph=graph)
     phases = None
     if profile:
         kp = min(profile_steps, steps)
@@ -124,8 +126,7 @@ def run_engine(sc, precision, warmup, steps, profile=True, flags=0, gjk_tol=None
         e.set_profiling(False)
         log(f"    {kp} profiled steps: {', '.join(f'{p} {v:.3f}' for p, v in phases.items())} ms")
     # timed in at most 10 chunks so a long run keeps reporting progress
-    graph = graph and not EAGER
-    chunk = max(1, -(-steps // 10))
+    chunk = max(100, -(-steps // 10))
     done, wall, stats = 0, 0.0, None
     while done < steps:
         k = min(chunk, steps - done)
