@@ -574,11 +574,12 @@ __global__ void __launch_bounds__(kBlock, sizeof(T) == 4 ? 4 : 2) k_screen(DevSc
 // 149 -> 8 + 93 us.
 template <class T, bool WARM, bool SV = true>
 __global__ void __launch_bounds__(kBlock) k_complete(DevScene d) {
-  // (the FP64 filter's queue: by one lane, in pairs a wave's registers are two
-  // waves' work and most entries end at once: 3,001 cylinders and cones 0.307
-  // and 0.419 ms a step)
-  constexpr bool filtered = sizeof(T) == 8 && SV;
-  if (!filtered && (uint64_t)defer_total(d) * 2 <= (uint64_t)gridDim.x * blockDim.x)
+  // (the FP64 filter's queue may be long: two lanes while they are resident at
+  // once, a wave per SIMD.  ms a step by one and by two: 1,000 touching
+  // superquadrics, 7,900 entries, 0.71 and 0.48; 3,001 cylinders and cones,
+  // 41,000, 0.31 and 0.42)
+  constexpr uint64_t resident = sizeof(T) == 8 && SV ? 65536 : ~0ull;
+  if ((uint64_t)defer_total(d) * 2 <= min((uint64_t)gridDim.x * blockDim.x, resident))
     narrow<T, SV, 1, WARM, true>(d);
   else
     narrow<T, SV, 1, WARM, false>(d);
