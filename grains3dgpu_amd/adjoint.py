@@ -9,8 +9,9 @@ stiffness, restitution (which sets the normal damping) and friction -- in
 the row order of the scene's contact tables; the tangential damping and
 kr stay as the scene holds them.  `final` is (pos, quat, vel, omega) after
 n_steps from the scene's state, as float64 tensors; any loss of them
-backpropagates to `params` through one reverse sweep on the device, which
-re-runs every block of `checkpoint_every` steps from its checkpoint.
+backpropagates to `params` through one reverse sweep on the device, over the
+recorded steps' states where they were kept (at most 4 GiB), else over those
+of a block of `checkpoint_every` steps run again from its checkpoint.
 
 Tensors are host memory (the engine's boundary takes host buffers); torch is
 only the autograd plumbing here.

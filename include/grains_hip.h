@@ -174,7 +174,8 @@ typedef struct grains_config_t {
                                sphere, OBB and, physics semantics, GJK's first
                                support pair) and a complete pass over the
                                undecided entries, compacted; 1 = one complete
-                               pass (0: 2; REF_QUIRKS in FP32 and FP64 beds of
+                               pass over the entries that pass the prefilter
+                               (0: 2; REF_QUIRKS in FP32 and FP64 beds of
                                spheres take one).  Results do not depend on
                                it.                                          */
   int32_t candidate_staging; /* broad phase: 1 = each unordered pair tested
@@ -354,7 +355,8 @@ int grains_get_phase_times(grains_ctx_t* ctx, double* ms, int n_phases);
  * checkpoint every `checkpoint_every` steps of the following grains_step /
  * grains_step_graph calls, and the states of the steps between while they
  * take no more than 4 GiB (104 B per particle and step) and the device has
- * them.  grains_adjoint then sweeps back over every recorded step, first
+ * them (they are freed when a checkpoint or the sweep finds no memory).
+ * grains_adjoint then sweeps back over every recorded step, first
  * re-running from its checkpoint a block whose states were not kept:
  * dL_dstate (13 n: pos n x 3, quat n x 4, vel n x 3, omega n x 3, the
  * gradient of the loss at the current state) -> dL_dparams (n_table_entries
