@@ -350,7 +350,6 @@ int cu_count();
 // pass 1: the entries the screen queued (no launch unless d.split)
 void launch_narrow64(const DevScene& d, int pass, hipStream_t s);
 void launch_narrow32(const DevScene& d, int pass, hipStream_t s);
-void launch_filter(const DevScene& d, hipStream_t s);
 void launch_refine64(const DevScene& d, hipStream_t s);
 // part 0: every particle; 1: the particles the screen did not mark (the
 // marked ones queued); 2: the queued ones.  Each part then integrates the

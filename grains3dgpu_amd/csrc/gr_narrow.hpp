@@ -291,8 +291,8 @@ __device__ __forceinline__ void defer_flush(const DevScene& d, DeferLds& L, uint
 // One lane per list entry, grid-stride.  SV: physics semantics (signed-volume
 // GJK); !SV: REF_QUIRKS.
 // PASS 0 (the step's only pass): every list entry, complete.  PASS 1: the
-// entries that a pass before it queued -- the screen, which settles most, or
-// the filter, which leaves out those beyond the prefilter -- packed
+// entries that a pass before it queued -- the screen, which settles most, or in
+// FP64 the filter, which leaves out those beyond the prefilter -- packed
 // lane-dense, complete.  A wave costs as much as its slowest lane, so the long
 // searches are kept together and the first pass's waves stay short.  The
 // queued searches start from scratch with the same arithmetic: results equal
@@ -303,7 +303,10 @@ __device__ __forceinline__ void defer_flush(const DevScene& d, DeferLds& L, uint
 // the pass lasts as long as its longest search (k_complete chooses).
 // BALLS (PASS 0, FP64): every particle is a sphere -- no search, no second pass.
 // PACK (PASS 0): a wave takes 64 entries at a time that pass the prefilter
-// from the list, which holds the skin's too, half as many again (kPackNarrow).
+// from the list, which holds the skin's too, a quarter to a half as many again
+// (FP32 from cold, 40,000 touching superquadrics, ms a step with lists built
+// for every step, entries where they stand, packed: 0.986, 1.055, 0.913;
+// the reference semantics: kPackNarrow).
 template <class T, bool SV, int PASS, bool WARM = false, bool PAIR = false, bool BALLS = false, bool PACK = false>
 __device__ __forceinline__ void narrow(const DevScene& d) {
   constexpr bool first = PASS != 1;  // the step's first kernel
@@ -372,19 +375,26 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
     uint32_t* mine = packed[threadIdx.x / 64];
     uint32_t have = 0;  // the wave's entries in it
     const bool outside = d.nl[kNlOutside] != 0;
-    // a share of the list dealt to each wave, the rest handed out through a
-    // counter (the first queue's: no pass queues entries here)
+    // a share of the list dealt to each wave, the rest in turn (FP32, physics
+    // semantics: most entries end at once) or handed out through a counter (the
+    // first queue's: no pass queues entries here)
+    constexpr bool turns = sizeof(T) == 4 && SV;
     const uint64_t dealt = stride / 64;
-    const uint32_t share = 64u * (uint32_t)min((uint64_t)8, max((uint64_t)1, (uint64_t)E / (dealt * 64 * 8)));
+    const uint32_t share =
+        64u * (turns ? 1u : (uint32_t)min((uint64_t)8, max((uint64_t)1, (uint64_t)E / (dealt * 64 * 8))));
     uint64_t kw = (gid / 64) * share, end = min((uint64_t)E, kw + share);
     bool more = dealt * share < E;
     for (;;) {
       while (have < 64) {
         if (kw >= end) {
           if (!more) break;
-          uint32_t next = 0;
-          if (lane == 0) next = atomicAdd(d.defer_count, share);
-          kw = dealt * share + __shfl(next, 0);
+          if constexpr (turns) {
+            kw += stride - 64;
+          } else {
+            uint32_t next = 0;
+            if (lane == 0) next = atomicAdd(d.defer_count, share);
+            kw = dealt * share + __shfl(next, 0);
+          }
           end = min((uint64_t)E, kw + share);
           more = end < E;
           if (kw >= end) break;
@@ -396,7 +406,15 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
           const PoseRec pi = d.pk[si], pj = d.pk[sj];
           cand = is_candidate(d.grids[pi.sim], V3<double>{pi.x, pi.y, pi.z}, V3<double>{pj.x, pj.y, pj.z}, d.rcs[si],
                               d.rcs[sj], outside);
-          if (!cand) d.pair_flag[e] = 0u;
+          if (!cand) {
+            if constexpr (WARM) {
+              // a pair that left the prefilter's reach forgets its direction
+              if (d.pair_flag[e] & kFlagCand)
+                d.ws[(uint64_t)(*d.ws_par) * ((uint64_t)d.K * d.n) + e] =
+                    make_float4(0.f, 0.f, 0.f, __uint_as_float(d.sidx[sj]));
+            }
+            d.pair_flag[e] = 0u;
+          }
         }
         const uint64_t m = __ballot(cand);
         if (cand) mine[have + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = e;
@@ -429,7 +447,7 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
   count_max(d.counters, kCntMaxIters, c_maxit);
 }
 
-// The reference semantics in one pass.  A list taken as it stands costs as
+// One pass, but FP64 under the physics semantics.  The reference's: a list taken as it stands costs as
 // many waves as it is long, the skin's entries among them: on large beds more
 // than the lists' builds it saves, so those pack it, with as many waves as are
 // resident at once; small beds have lanes to spare, and spheres no search.
@@ -438,9 +456,9 @@ __device__ __forceinline__ void narrow(const DevScene& d) {
 // 0.377, 150,000 1.055, 1.065, 0.927, 500,000 2.77, 2.94, 2.68; FP64 5,000
 // 0.348, 0.265, 0.282, 20,000 0.578, 0.596, 0.480, 150,000 2.44, 2.87, 2.12.
 constexpr uint64_t kPackNarrow = 10000;  // the largest bed whose list is taken as it stands
-template <class T, bool PACK>
+template <class T, bool PACK, bool SV = false, bool WARM = false>
 __global__ void __launch_bounds__(kBlock) k_narrow(DevScene d) {
-  narrow<T, false, 0, false, false, false, PACK>(d);
+  narrow<T, SV, 0, WARM, false, false, PACK>(d);
 }
 template <class T>
 inline void launch_narrow_ref(const DevScene& d, hipStream_t s) {

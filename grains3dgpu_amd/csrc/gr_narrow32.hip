@@ -14,27 +14,25 @@ void launch_narrow32(const DevScene& d, int pass, hipStream_t s) {
   // The complete pass: no more threads than are resident at once, 512 a CU
   // whatever the block's size: more blocks, most with nothing to do, queue
   // behind the integration's (10^6 superquadrics at rest, 8 blocks per CU and 2:
-  // 0.360 and 0.352 ms a step; agitated beds and 64 ensembles within 1 %).
-  auto complete = [&] {
-    const dim3 cg(std::min(grid.x, (unsigned)cu_count() * 2 * (unsigned)(kBlock / d.block)));
-    if (warm)
-      hipLaunchKernelGGL((k_complete<float, true>), cg, block, 0, s, d);
-    else
-      hipLaunchKernelGGL((k_complete<float, false>), cg, block, 0, s, d);
-  };
+  // 0.360 and 0.352 ms a step; agitated beds and 64 ensembles within 1 %).  The
+  // single pass likewise, its waves packing the list.
+  const dim3 cg(std::min(grid.x, (unsigned)cu_count() * 2 * (unsigned)(kBlock / d.block)));
   if (pass == 0) {
     if (two && warm) {
       hipLaunchKernelGGL((k_screen<float, true>), grid, block, 0, s, d);
     } else if (two) {
       hipLaunchKernelGGL((k_screen<float, false>), grid, block, 0, s, d);
+    } else if (warm) {
+      hipLaunchKernelGGL((k_narrow<float, true, true, true>), cg, block, 0, s, d);
     } else if (sv) {
-      launch_filter(d, s);
-      complete();
+      hipLaunchKernelGGL((k_narrow<float, true, true>), cg, block, 0, s, d);
     } else {
       launch_narrow_ref<float>(d, s);
     }
+  } else if (two && warm) {
+    hipLaunchKernelGGL((k_complete<float, true>), cg, block, 0, s, d);
   } else if (two) {
-    complete();
+    hipLaunchKernelGGL((k_complete<float, false>), cg, block, 0, s, d);
   }
 }
 void launch_integrate32(const DevScene& d, hipStream_t s, int part) { launch_integrate_t<float>(d, s, part); }

@@ -37,14 +37,13 @@ __global__ void __launch_bounds__(kBlock) k_refine64_ref(DevScene d) {
   count_max(d.counters, kCntRefMaxIters, c_maxit);
 }
 
-// One narrow pass under the physics semantics: the entries that pass the
-// prefilter, queued for the complete pass (both precisions).  The lists hold
+// One narrow pass in FP64 under the physics semantics: the entries that pass the
+// prefilter, queued for the complete pass.  The lists hold
 // their skin's pairs too, a quarter to a third of the entries; the others,
 // searched in the lanes they stand in, take as many waves as the list has, not
 // as the step has candidates.  ms a step with lists built for every step,
-// entries where they stand, queued: FP64, 40,000 touching superquadrics 3.67,
-// 5.25, 3.54, 8,191 1.36, 1.28, 1.24, 300,000 loose ones 1.00, 1.07, 0.90;
-// FP32 from cold, 40,000 touching 0.986, 1.053, 0.861.
+// entries where they stand, queued: 40,000 touching superquadrics 3.67,
+// 5.25, 3.52, 8,191 1.36, 1.28, 1.23, 300,000 loose ones 1.00, 1.07, 0.91.
 __global__ void __launch_bounds__(kBlock) k_filter(DevScene d) {
   if (!step_begin(d)) return;
   __shared__ DeferLds L;
@@ -60,13 +59,7 @@ __global__ void __launch_bounds__(kBlock) k_filter(DevScene d) {
       const PoseRec pi = d.pk[si], pj = d.pk[sj];
       cand = is_candidate(d.grids[pi.sim], V3<double>{pi.x, pi.y, pi.z}, V3<double>{pj.x, pj.y, pj.z}, d.rcs[si],
                           d.rcs[sj], outside);
-      if (!cand) {
-        // a pair that left the prefilter's reach forgets its direction
-        if (d.warm && (d.pair_flag[e] & kFlagCand))
-          d.ws[(uint64_t)(*d.ws_par) * ((uint64_t)d.K * d.n) + e] =
-              make_float4(0.f, 0.f, 0.f, __uint_as_float(d.sidx[sj]));
-        d.pair_flag[e] = 0u;
-      }
+      if (!cand) d.pair_flag[e] = 0u;
       c_cand += cand;
     }
     defer_push(d, L, nq, cand, (uint32_t)e);
@@ -74,10 +67,6 @@ __global__ void __launch_bounds__(kBlock) k_filter(DevScene d) {
   defer_flush(d, L, nq);
   count_add(d.counters, kCntCandidates, c_cand);
 }
-void launch_filter(const DevScene& d, hipStream_t s) {
-  hipLaunchKernelGGL(k_filter, dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
-}
-
 // One wave per block, two per SIMD (the registers' limit).
 template <int MODE>
 static void launch_search64(const DevScene& d, hipStream_t s) {
@@ -95,7 +84,7 @@ void launch_narrow64(const DevScene& d, int pass, hipStream_t s) {
     else if (two)
       hipLaunchKernelGGL((k_screen<double, false, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
     else if (sv) {
-      launch_filter(d, s);
+      hipLaunchKernelGGL(k_filter, dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
       hipLaunchKernelGGL((k_complete<double, false>), dim3(d.narrow_blocks), dim3(d.block), 0, s, d);
     } else {
       launch_narrow_ref<double>(d, s);
