@@ -76,9 +76,9 @@ void launch_run_begin(const DevScene& d, uint32_t n, bool fresh, hipStream_t s) 
 // ---- cell hash --------------------------------------------------------------------
 // The first kernel of a list build (no other kernel runs beside it on the
 // stream): ws_par (warm starts on), the warm-start buffer of the lists, is
-// flipped here, unless the build before was of no use (kNlOver = 2): its
-// lists were cut, and with them the records carried over to them, so the ones
-// before it are carried over again.  Keys are those of the search's cells (d.sgrids).
+// flipped here, unless the build before was of no use (kNlOver >= 2): the
+// records carried over to its lists are left, and the ones before it carried
+// over again.  Keys are those of the search's cells (d.sgrids).
 // With a sorted order of the previous build in place (sort_state[0]), a
 // particle whose key differs from its key there (ks_prev at its previous
 // position rank[i]) has changed cell: it is counted in sort_state[2] and the
@@ -90,7 +90,7 @@ __global__ void k_hash(DevScene d, const uint32_t* __restrict__ ks_prev) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool mover = false;
   if (i == 0) {
-    if (d.warm && d.nl[kNlOver] != 2u) d.ws_par[0] = 1u - d.ws_par[0];
+    if (d.warm && d.nl[kNlOver] < 2u) d.ws_par[0] = 1u - d.ws_par[0];
     d.nl[kNlValid] = 0u;
     d.nl[kNlOver] = 0u;
     d.nl[kNlOutside] = 0u;
@@ -741,7 +741,7 @@ __global__ void k_cells(DevScene d, const uint32_t* __restrict__ ks, const uint3
   cell_of(gr, p, c);
   d.rkey[s] = cell_key(gr, c);
   // a centre outside a periodic side is folded into a border cell now and
-  // wrapped by the step: these lists hold for that step only
+  // wrapped by the step
   bool out = false;
 #pragma unroll
   for (int k = 0; k < 3; ++k) out |= ((g.periodic >> k) & 1) && (p[k] < g.lo[k] || p[k] >= g.hi[k]);
@@ -1384,9 +1384,11 @@ __global__ void k_expand(DevScene d) {
   const uint32_t* cand = d.cand;
   const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s == 0) {
-    const bool cut = d.nl[kNlOver] && d.skin;
-    d.nl[kNlValid] = cut ? 0u : (d.nl[kNlOutside] || !d.skin ? 2u : 1u);
-    if (cut) d.nl[kNlOver] = 2u;
+    // with a skin: no use when a list is cut, or when a centre lies outside a
+    // periodic side, whose neighbours are those of the reference's border cell
+    const uint32_t no_use = !d.skin ? 0u : (d.nl[kNlOver] ? 2u : (d.nl[kNlOutside] ? 3u : 0u));
+    d.nl[kNlValid] = no_use ? 0u : (d.skin ? 1u : 2u);
+    if (no_use) d.nl[kNlOver] = no_use;
   }
   uint32_t raw = 0;
   if (s < n) {

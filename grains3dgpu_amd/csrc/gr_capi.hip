@@ -386,6 +386,7 @@ struct grains_ctx {
   // the steps themselves moves the particles; lists_ok is cleared wherever
   // the state or the layout is set.
   bool lists_ok = false;
+  bool skin_back = false;       // without a skin for one step: its centres lie outside a periodic side
   uint32_t since_build = 0;     // steps taken since they were built
   uint32_t interval = 8;        // steps they are expected to hold, and whether a build has shown it
   bool interval_known = false;
@@ -1179,6 +1180,7 @@ static int finalize(grains_ctx* ctx) {
   ctx->layout_ok = true;
   ctx->keys_s = ctx->idx_s = nullptr;  // no lists yet
   ctx->lists_ok = false;
+  ctx->skin_back = false;
   ctx->interval = 8;
   ctx->interval_known = false;
   return GRAINS_OK;
@@ -1593,7 +1595,7 @@ static int take_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
     }
     const bool each = !ctx->d.skin || ctx->interval <= 1;  // lists for one step at a time
     if (each) {
-      m = std::min(m, 64u);
+      m = std::min(m, ctx->skin_back ? 1u : 64u);
       for (uint32_t k = 0; k < m; ++k) {
         if (ctx->profiling && !graph) {
           enqueue_step(ctx, true);
@@ -1601,7 +1603,7 @@ static int take_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
           if ((rc = build()) || (rc = steps(1))) return rc;
         }
       }
-      ctx->interval = 4;
+      if (!ctx->skin_back) ctx->interval = 4;
     } else {
       bool fresh = !ctx->lists_ok;
       if (fresh) ctx->since_build = 0;
@@ -1618,11 +1620,17 @@ static int take_steps(grains_ctx* ctx, uint32_t n_steps, bool graph) {
     if ((rc = read_words(ctx, nl))) return rc;
     const uint32_t took = nl[kNlDone] - done;
     if (ctx->d.skin && nl[kNlOver]) {
-      // a list outgrew max_neighbors with the skin; the step's own
-      // candidates may still fit
+      // a list outgrew max_neighbors with the skin, and the step's own
+      // candidates may still fit; or centres lie outside a periodic side, and
+      // the next step, which wraps them, takes the reference's cells
       if ((rc = use_skin(ctx, false))) return rc;
+      ctx->skin_back = nl[kNlOver] == 3u;
+    } else if (!took) {
+      return fail(ctx, GRAINS_EDEVICE, "a step did not run");
+    } else if (ctx->skin_back) {
+      ctx->skin_back = false;
+      if ((rc = use_skin(ctx, true))) return rc;
     } else {
-      if (!took) return fail(ctx, GRAINS_EDEVICE, "a step did not run");
       ctx->lists_ok = nl[kNlValid] != 0;
       ctx->since_build = each ? 1u : ctx->since_build + took;
       if (!each && !ctx->lists_ok) {

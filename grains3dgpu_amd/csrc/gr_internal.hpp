@@ -99,7 +99,8 @@ enum ListState {
   kNlLast,        // it is the run's last step, or a checkpoint's
   kNlDone,        // steps of the run taken
   kNlTarget,      // steps of the run asked for (recorded: up to the next checkpoint)
-  kNlOver,        // a list outgrew max_neighbors when the lists were built (2: with its skin, and no step uses them)
+  kNlOver,        // a list outgrew max_neighbors when the lists were built; 2: with its skin, 3: kNlOutside with
+                  // a skin -- no step uses such lists
   kNlOutside,     // a centre lay outside a periodic side when they were built
   kNlStale,       // the records by sorted position are ahead of the state's planes
   kNlWords = 8

@@ -217,3 +217,28 @@ def test_key_order_is_stable(n):
     e.step(20)
     key, order = e.get_cell_keys()
     np.testing.assert_array_equal(order, np.argsort(key, kind="stable"))
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_centres_outside_periodic_sides_as_the_oracle(warm, oracle_lib):
+    """A run that starts with centres outside periodic sides: they take the
+    neighbours of the border cell they are folded into, as in the reference's
+    cells, until the step wraps them; then the run goes on as from there."""
+    from grains3dgpu_amd import engine
+    sc = dense_spheres(n=1500, seed=16, vel=0.5, periodic=0b011)
+    sc.pos[::5, :2] -= 0.12 * np.asarray(sc.sims[0]["domain_max"])[:2]
+    kw = dict(precision=A.FP32_MIXED, flags=A.WARM_START | A.FP64_CONTACTS, gjk_rel_tol=1e-6) if warm else {}
+    e = S.load(engine.Engine(dt=sc.dt, max_neighbors=96, **kw), sc)
+    o = S.load(oracle_lib.Oracle(dt=sc.dt), sc)
+    o.step(1)
+    e.step(1)
+    assert e.get_stats()["out_of_domain"] > 0
+    for which in (A.PAIRS_CANDIDATE, A.PAIRS_CONTACT):
+        np.testing.assert_array_equal(e.get_pairs(which), o.get_pairs(which))
+    # in one run, by graph, and cut after the first step by a state put back
+    whole, cut = [S.load(engine.Engine(dt=sc.dt, max_neighbors=96, **kw), sc) for _ in range(2)]
+    whole.step(12, graph=True)
+    cut.step(1)
+    cut.step(11)
+    for a, b in zip(result(whole), result(cut)):
+        np.testing.assert_array_equal(a, b)
